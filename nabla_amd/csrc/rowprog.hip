@@ -1,335 +1,23 @@
-// Row-program interpreter: fused elementwise chains and last-axis reductions.
+// Row programs: fused elementwise chains and last-axis reductions.
 //
-// Two launch shapes share one instruction interpreter:
-//   * flat  (has_reduce = 0): one lane per 4-column chunk of the rows x C
-//     domain, no cross-lane traffic;
-//   * block (has_reduce = 1): one workgroup per row.  Lanes sweep the row in
-//     4-column chunks (coalesced 16-byte accesses), partial results are
-//     combined with 64-wide wavefront shuffles and an LDS tree across the
-//     waves of the group.  Rows that are read in more than one phase can be
-//     pre-loaded into LDS so HBM sees them once.
-//
-// Registers live in VGPRs: the 16 vector registers are four 16-wide vectors
-// (one per chunk component) indexed with a wave-uniform index, which the
-// compiler turns into VGPR-relative moves instead of scratch memory.
+// Checks a program, finds the compiled kernel the library carries for it (generated ahead of time
+// or written by hand) and launches that, or hands the program to the interpreter (rowprog_vm.hip).
 #include "nbk_common.h"
-#include "rowprog_device.h"
 #include "rowprog_spec.h"
+#include "rowprog_vm.h"
 #include <stddef.h>
 #include <mutex>
 #include <unordered_map>
 
-typedef float vf16 __attribute__((ext_vector_type(16)));
-typedef float vf4 __attribute__((ext_vector_type(4)));
-
-struct RpRegs {
-  vf16 x, y, z, w;  // vector registers 0..15, by chunk component
-  vf16 s;           // per-row scalar registers 16..31
-  vf4 acc;          // reduction accumulators
-};
-
-__device__ __forceinline__ float4 rp_read(const RpRegs& R, int i) {
-  if (i < NBK_RP_NVEC) {
-    return make_float4(R.x[i], R.y[i], R.z[i], R.w[i]);
-  }
-  float s = R.s[i - NBK_RP_NVEC];
-  return make_float4(s, s, s, s);
-}
-__device__ __forceinline__ void rp_write(RpRegs& R, int i, float4 v) {
-  R.x[i] = v.x; R.y[i] = v.y; R.z[i] = v.z; R.w[i] = v.w;
-}
-
-// readfirstlane returns a SIGNED int: widening it directly to 64 bits would
-// sign-extend and corrupt the high half of a pointer, so go through uint32_t.
-__device__ __forceinline__ uint32_t rp_sgpr(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_readfirstlane(v);
-}
-__device__ __forceinline__ uint64_t rp_sgpr64(uint2 v) {
-  return (uint64_t)rp_sgpr(v.x) | ((uint64_t)rp_sgpr(v.y) << 32);
-}
-
-__device__ __forceinline__ nbk_operand rp_operand(const nbk_rowprog& S, int i, int n_lead);
-
-__host__ __device__ __forceinline__ bool rp_is_unary(int op) {
+static bool rp_is_unary(int op) {
   return (op >= NBK_OP_MOV && op < NBK_OP_ADD) || op == NBK_OP_DGELU || op == NBK_OP_SIN ||
          op == NBK_OP_COS || (op >= NBK_OP_INEG && op <= NBK_OP_INEZ);
 }
-__host__ __device__ __forceinline__ bool rp_is_binary(int op) {
+static bool rp_is_binary(int op) {
   return (op >= NBK_OP_ADD && op < NBK_OP_WHERE) || (op >= NBK_OP_IADD && op <= NBK_OP_ILE);
 }
-__host__ __device__ __forceinline__ bool rp_is_ew(int op) {
+static bool rp_is_ew(int op) {
   return rp_is_unary(op) || rp_is_binary(op) || op == NBK_OP_WHERE || op == NBK_OP_FMA;
-}
-
-// One body instruction on one chunk.
-template <typename IDX>
-__device__ __forceinline__ void rp_exec_body(const nbk_rowprog& P, const nbk_ins in, RpRegs& R,
-                                             const IDX* lead_idx, int64_t col, int valid,
-                                             const float* stage, int64_t c_pad, int n_lead) {
-  const int op = in.op;
-  if (rp_is_binary(op)) {
-    float4 a = rp_read(R, in.a), b = rp_read(R, in.b), r;
-    switch (op) {  // the hot ones without a per-component switch
-      case NBK_OP_ADD: r = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); break;
-      case NBK_OP_SUB: r = make_float4(a.x - b.x, a.y - b.y, a.z - b.z, a.w - b.w); break;
-      case NBK_OP_MUL: r = make_float4(a.x * b.x, a.y * b.y, a.z * b.z, a.w * b.w); break;
-      default:
-        r = make_float4(rp_binary(op, a.x, b.x), rp_binary(op, a.y, b.y),
-                        rp_binary(op, a.z, b.z), rp_binary(op, a.w, b.w));
-    }
-    rp_write(R, in.dst, r);
-  } else if (rp_is_unary(op)) {
-    float4 a = rp_read(R, in.a);
-    float4 r = make_float4(rp_unary(op, a.x), rp_unary(op, a.y), rp_unary(op, a.z),
-                           rp_unary(op, a.w));
-    rp_write(R, in.dst, r);
-  } else if (op == NBK_OP_LDG) {
-    const nbk_operand o = rp_operand(P, in.a, n_lead);
-    float4 r;
-    if (o.stage_slot >= 0 && stage != nullptr) {
-      r = *(const float4*)(stage + o.stage_slot * c_pad + col);
-    } else {
-      r = rp_load4(o, rp_row_offset(o, lead_idx, n_lead), col, valid);
-    }
-    rp_write(R, in.dst, r);
-  } else if (op == NBK_OP_STG) {
-    const nbk_operand o = rp_operand(P, in.dst, n_lead);
-    rp_store4(o, rp_row_offset(o, lead_idx, n_lead), col, valid, rp_read(R, in.a));
-  } else if (op == NBK_OP_ACC) {
-    float4 a = rp_read(R, in.a);
-    const int kind = in.b;
-    float v = R.acc[in.dst];
-    if (valid > 0) v = rp_combine(v, a.x, kind);
-    if (valid > 1) v = rp_combine(v, a.y, kind);
-    if (valid > 2) v = rp_combine(v, a.z, kind);
-    if (valid > 3) v = rp_combine(v, a.w, kind);
-    R.acc[in.dst] = v;
-  } else if (op == NBK_OP_WHERE) {
-    float4 c = rp_read(R, in.a), a = rp_read(R, in.b), b = rp_read(R, in.c);
-    rp_write(R, in.dst, rp_where4(c, a, b));
-  } else if (op == NBK_OP_FMA) {
-    float4 a = rp_read(R, in.a), b = rp_read(R, in.b), c = rp_read(R, in.c);
-    rp_write(R, in.dst, make_float4(fmaf(a.x, b.x, c.x), fmaf(a.y, b.y, c.y),
-                                    fmaf(a.z, b.z, c.z), fmaf(a.w, b.w, c.w)));
-  } else if (op == NBK_OP_COLIDX) {
-    rp_write(R, in.dst, rp_colidx4(col, in.a != 0));
-  }
-}
-
-// Prologue (per-row, scalar-register) instruction.  Returns through R.
-template <typename IDX>
-__device__ __forceinline__ void rp_exec_scalar(const nbk_rowprog& P, const nbk_ins in, RpRegs& R,
-                                               const IDX* lead_idx, bool writer, float* red_buf,
-                                               int n_lead) {
-  const int op = in.op;
-  const int d = in.dst - NBK_RP_NVEC;
-  if (op == NBK_OP_IMM) {
-    R.s[d] = __uint_as_float(rp_sgpr(__float_as_uint(P.imm[in.a])));
-  } else if (op == NBK_OP_LDR) {
-    const nbk_operand o = rp_operand(P, in.a, n_lead);
-    R.s[d] = rp_load1(o.ptr, rp_row_offset(o, lead_idx, n_lead), o.dtype);
-  } else if (op == NBK_OP_STR) {
-    const nbk_operand o = rp_operand(P, in.dst, n_lead);
-    if (writer) {
-      rp_store1(o.ptr, rp_row_offset(o, lead_idx, n_lead), o.dtype, R.s[in.a - NBK_RP_NVEC]);
-    }
-  } else if (op == NBK_OP_LEADIDX) {
-    const int k = in.a;
-    const int li = (int)(k == 0 ? lead_idx[0] : k == 1 ? lead_idx[1] : k == 2 ? lead_idx[2] : lead_idx[3]);
-    R.s[d] = in.b != 0 ? rp_ibits(li) : (float)li;
-  } else if (op == NBK_OP_ACCINIT) {
-    R.acc[in.dst] = rp_identity(in.a);
-  } else if (op == NBK_OP_RED) {
-    R.s[d] = rp_block_reduce(R.acc[in.a], in.b, red_buf);
-  } else if (rp_is_binary(op)) {
-    R.s[d] = rp_binary(op, R.s[in.a - NBK_RP_NVEC], R.s[in.b - NBK_RP_NVEC]);
-  } else if (rp_is_unary(op)) {
-    R.s[d] = rp_unary(op, R.s[in.a - NBK_RP_NVEC]);
-  } else if (op == NBK_OP_WHERE) {
-    R.s[d] = rp_where(R.s[in.a - NBK_RP_NVEC], R.s[in.b - NBK_RP_NVEC], R.s[in.c - NBK_RP_NVEC]);
-  } else if (op == NBK_OP_FMA) {
-    R.s[d] = fmaf(R.s[in.a - NBK_RP_NVEC], R.s[in.b - NBK_RP_NVEC], R.s[in.c - NBK_RP_NVEC]);
-  }
-}
-
-// ---------------------------------------------------------------- program staging
-// Kernel arguments live in uncached memory: a scalar load from them costs a full
-// memory round trip, far too slow for an instruction stream that is re-read for
-// every chunk.  Each workgroup therefore copies the program into LDS once and
-// then walks rows persistently; the interpreter fetches instructions and operand
-// descriptors from LDS and turns them into scalars with readfirstlane.
-#define RP_WORDS ((int)(sizeof(nbk_rowprog) / 4))
-static_assert(sizeof(nbk_rowprog) % 4 == 0, "program is copied word by word");
-static_assert(sizeof(nbk_operand) % 8 == 0 && offsetof(nbk_rowprog, operand) % 8 == 0 &&
-                  offsetof(nbk_operand, col_stride) % 8 == 0 && offsetof(nbk_operand, vec_ok) % 8 == 0,
-              "operand descriptors are read from LDS with 8-byte accesses");
-static_assert(sizeof(nbk_ins) == 8 && offsetof(nbk_rowprog, ins) % 8 == 0,
-              "instructions are read from LDS with 8-byte accesses");
-
-__device__ __forceinline__ void rp_copy_program(const nbk_rowprog& P, uint32_t* dst) {
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(&P);
-  for (int i = threadIdx.x; i < RP_WORDS; i += blockDim.x) dst[i] = src[i];
-  __syncthreads();
-}
-
-__device__ __forceinline__ nbk_ins rp_fetch(const nbk_rowprog& S, int q) {
-  const uint2 u = *reinterpret_cast<const uint2*>(&S.ins[q]);
-  const uint32_t lo = rp_sgpr(u.x);
-  const uint32_t hi = rp_sgpr(u.y);
-  nbk_ins in;
-  in.op = lo & 0xff; in.dst = (lo >> 8) & 0xff; in.a = (lo >> 16) & 0xff; in.b = lo >> 24;
-  in.c = hi & 0xff; in.pad = 0; in.aux = (uint16_t)(hi >> 16);
-  return in;
-}
-
-// Scalar copy of one operand descriptor out of LDS.
-__device__ __forceinline__ nbk_operand rp_operand(const nbk_rowprog& S, int i, int n_lead) {
-  const nbk_operand& o = S.operand[i];
-  nbk_operand r;
-  r.ptr = reinterpret_cast<void*>(rp_sgpr64(*reinterpret_cast<const uint2*>(&o.ptr)));
-  // descriptors are 56 bytes apart, so only 8-byte alignment is guaranteed here
-  const uint2 t0 = *reinterpret_cast<const uint2*>(&o.col_stride);
-  const uint2 t1 = *reinterpret_cast<const uint2*>(&o.vec_ok);
-  r.col_stride = (int32_t)rp_sgpr(t0.x);
-  r.dtype = (int32_t)rp_sgpr(t0.y);
-  r.vec_ok = (int32_t)rp_sgpr(t1.x);
-  r.stage_slot = (int32_t)rp_sgpr(t1.y);
-  // the host zero-fills strides beyond n_lead
-  (void)n_lead;
-#pragma unroll
-  for (int k = 0; k < NBK_RP_MAX_LEAD; ++k) {
-    r.lead_stride[k] = (int64_t)rp_sgpr64(*reinterpret_cast<const uint2*>(&o.lead_stride[k]));
-  }
-  return r;
-}
-
-// ---------------------------------------------------------------- block mode
-extern __shared__ __align__(16) float rp_stage_lds[];
-
-__global__ __launch_bounds__(512) void rp_block_kernel(const nbk_rowprog P, int64_t rows) {
-  __shared__ float red_buf[16];
-  __shared__ __align__(16) uint32_t prog_lds[RP_WORDS];
-  rp_copy_program(P, prog_lds);
-  const nbk_rowprog& S = *reinterpret_cast<const nbk_rowprog*>(prog_lds);
-  RpRegs R;
-  R.acc = (vf4)(0.f);
-  const int64_t C = P.C;
-  const int64_t c_pad = (C + 3) & ~(int64_t)3;
-  const int64_t n_chunks = c_pad >> 2;
-  const int n_lead = P.n_lead;
-  const int n_ins = P.n_ins;
-  const int n_operands = P.n_operands;
-  const int n_stage = P.n_stage;
-  int64_t lead_dim[NBK_RP_MAX_LEAD];
-#pragma unroll
-  for (int k = 0; k < NBK_RP_MAX_LEAD; ++k) lead_dim[k] = P.lead_dim[k];
-  const float* stage = n_stage > 0 ? rp_stage_lds : nullptr;
-  const bool writer = threadIdx.x == 0;
-
-  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
-    // decompose the row index over the leading dims (wave-uniform)
-    // unused leading dims have extent 1, so the same three divisions serve every n_lead
-    int64_t lead_idx[NBK_RP_MAX_LEAD];
-    {
-      int64_t rem = row, q;
-      q = rem / lead_dim[3]; lead_idx[3] = rem - q * lead_dim[3]; rem = q;
-      q = rem / lead_dim[2]; lead_idx[2] = rem - q * lead_dim[2]; rem = q;
-      q = rem / lead_dim[1]; lead_idx[1] = rem - q * lead_dim[1]; rem = q;
-      lead_idx[0] = rem;
-    }
-
-    // pre-load staged operands: every lane stages exactly the chunks it will
-    // later read back, so no barrier is needed between the two.
-    if (n_stage > 0) {
-      for (int oi = 0; oi < n_operands; ++oi) {
-        const nbk_operand o = rp_operand(S, oi, n_lead);
-        if (o.stage_slot < 0) continue;
-        rp_stage_row(o, rp_row_offset(o, lead_idx, n_lead), rp_stage_lds + o.stage_slot * c_pad, C,
-                     n_chunks);
-      }
-    }
-
-    int pc = 0;
-    while (pc < n_ins) {
-      const nbk_ins in = rp_fetch(S, pc);
-      if (in.op == NBK_OP_HALT) break;
-      if (in.op == NBK_OP_BODY) {
-        const int b0 = pc + 1, b1 = pc + 1 + in.aux;
-        for (int64_t ch = threadIdx.x; ch < n_chunks; ch += blockDim.x) {
-          const int64_t col = ch << 2;
-          const int64_t left = C - col;
-          const int valid = left >= 4 ? 4 : (int)left;
-          nbk_ins nxt = rp_fetch(S, b0);
-#pragma unroll 1
-          for (int q = b0; q < b1; ++q) {
-            const nbk_ins cur = nxt;
-            if (q + 1 < b1) nxt = rp_fetch(S, q + 1);  // fetch ahead of the decode
-            rp_exec_body(S, cur, R, lead_idx, col, valid, stage, c_pad, n_lead);
-          }
-        }
-        pc = b1;
-      } else {
-        rp_exec_scalar(S, in, R, lead_idx, writer, red_buf, n_lead);
-        ++pc;
-      }
-    }
-    // rows reuse the staging buffer and red_buf; RED already ends with a barrier,
-    // the staging area is private per lane, so no extra barrier is needed here
-  }
-}
-
-// ----------------------------------------------------------------- flat mode
-__global__ __launch_bounds__(256) void rp_flat_kernel(const nbk_rowprog P, uint32_t cpr,
-                                                      uint64_t total_chunks) {
-  __shared__ __align__(16) uint32_t prog_lds[RP_WORDS];
-  rp_copy_program(P, prog_lds);
-  const nbk_rowprog& S = *reinterpret_cast<const nbk_rowprog*>(prog_lds);
-  RpRegs R;
-  R.acc = (vf4)(0.f);
-  const int n_lead = P.n_lead;
-  const int n_ins = P.n_ins;
-  const int64_t C = P.C;
-  uint32_t lead_dim[NBK_RP_MAX_LEAD];
-#pragma unroll
-  for (int k = 0; k < NBK_RP_MAX_LEAD; ++k) lead_dim[k] = (uint32_t)P.lead_dim[k];
-  const uint64_t stride = (uint64_t)gridDim.x * 256u;
-  for (uint64_t g = (uint64_t)blockIdx.x * 256u + threadIdx.x; g < total_chunks; g += stride) {
-    uint32_t row, cc;
-    if (cpr == 1) { row = (uint32_t)g; cc = 0; }
-    else if (total_chunks <= cpr) { row = 0; cc = (uint32_t)g; }
-    else { row = (uint32_t)(g / cpr); cc = (uint32_t)(g - (uint64_t)row * cpr); }
-    uint32_t lead_idx[NBK_RP_MAX_LEAD] = {0, 0, 0, 0};
-    if (n_lead > 0) {
-      uint32_t rem = row, q;
-      q = rem / lead_dim[3]; lead_idx[3] = rem - q * lead_dim[3]; rem = q;
-      q = rem / lead_dim[2]; lead_idx[2] = rem - q * lead_dim[2]; rem = q;
-      q = rem / lead_dim[1]; lead_idx[1] = rem - q * lead_dim[1]; rem = q;
-      lead_idx[0] = rem;
-    }
-    const int64_t col = (int64_t)cc << 2;
-    const int64_t left = C - col;
-    const int valid = left >= 4 ? 4 : (int)left;
-    int pc = 0;
-    while (pc < n_ins) {
-      const nbk_ins in = rp_fetch(S, pc);
-      if (in.op == NBK_OP_HALT) break;
-      if (in.op == NBK_OP_BODY) {
-        const int b1 = pc + 1 + in.aux;
-        nbk_ins nxt = rp_fetch(S, pc + 1);
-#pragma unroll 1
-        for (int q = pc + 1; q < b1; ++q) {
-          const nbk_ins cur = nxt;
-          if (q + 1 < b1) nxt = rp_fetch(S, q + 1);
-          rp_exec_body(S, cur, R, lead_idx, col, valid, nullptr, 0, n_lead);
-        }
-        pc = b1;
-      } else {
-        // one lane per row writes row scalars: the lane that owns chunk 0
-        rp_exec_scalar(S, in, R, lead_idx, cc == 0, nullptr, n_lead);
-        ++pc;
-      }
-    }
-  }
 }
 
 // ------------------------------------------------------------------ host side
@@ -583,15 +271,6 @@ extern "C" int nbk_rowprog_launch(const nbk_rowprog* prog, void* stream) {
     NBK_REQUIRE(p->n_stage >= 0 && p->n_stage <= NBK_RP_MAX_STAGE, "rowprog: n_stage %d",
                 p->n_stage);
     NBK_REQUIRE(lds <= 64 * 1024, "rowprog: staging %zu bytes of LDS exceeds 64 KiB", lds);
-    if (lds > 32 * 1024) {
-      // static (program copy) + dynamic (staging) LDS exceeds the 64 KiB default cap
-      static bool attr_set = false;  // idempotent, a race only repeats the call
-      if (!attr_set) {
-        NBK_HIP(hipFuncSetAttribute((const void*)rp_block_kernel,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
-        attr_set = true;
-      }
-    }
     // persistent workgroups: enough to fill every CU at this block size / LDS use
     const int per_cu = lds > 48 * 1024 ? 2 : (block >= 512 ? 2 : (block >= 256 ? 4 : 8));
     int64_t grid = (int64_t)nbk_num_cus() * per_cu;
@@ -662,8 +341,7 @@ extern "C" int nbk_rowprog_launch(const nbk_rowprog* prog, void* stream) {
       NBK_HIP(hipLaunchKernel(spec->kernel[0], dim3((unsigned)grid), dim3(block), args, lds, st));
       return NBK_OK;
     }
-    hipLaunchKernelGGL(rp_block_kernel, dim3((unsigned)grid), dim3(block), lds, st, *p, rows);
-    return nbk_check_launch("rp_block_kernel");
+    return rp_vm_launch(p, rows, st);
   }
   NBK_REQUIRE(rows <= 0xffffffffLL, "rowprog: %lld rows exceed 2^32", (long long)rows);
   for (int k = 0; k < p->n_lead; ++k)
@@ -682,7 +360,5 @@ extern "C" int nbk_rowprog_launch(const nbk_rowprog* prog, void* stream) {
     NBK_HIP(hipLaunchKernel(fn, dim3((unsigned)blocks), dim3(256), args, 0, st));
     return NBK_OK;
   }
-  hipLaunchKernelGGL(rp_flat_kernel, dim3((unsigned)blocks), dim3(256), 0, st, *p, (uint32_t)cpr,
-                     total);
-  return nbk_check_launch("rp_flat_kernel");
+  return rp_vm_launch(p, rows, st);
 }

@@ -53,90 +53,94 @@ __device__ __forceinline__ void rp_store1(void* p, int64_t i, int dt, float v) {
   else nbk_store_from_f32(p, i, dt, v);
 }
 
-__device__ __forceinline__ float4 rp_load4(const nbk_operand& o, int64_t off, int64_t col,
-                                           int valid) {
-  const int dt = o.dtype;
-  const int64_t cs = o.col_stride;
+// Vector accesses of 16, 8 and 4 bytes at element alignment: the memory unit takes them at any
+// address, so a row that starts at an odd element still moves in whole chunks (four narrow
+// accesses per chunk before: rows of 1003 floats read at a quarter of the rate).
+typedef uint32_t rp_u4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t rp_u2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t rp_u1 __attribute__((aligned(1)));
+typedef long long rp_ll2 __attribute__((ext_vector_type(2), aligned(8)));
+
+// Four columns at element `e` with column stride `cs`, `valid` of them inside the row.
+__device__ __forceinline__ float4 rp_load4_any(const void* ptr, int dt, int64_t e, int64_t cs, int valid) {
   float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (o.vec_ok && valid == 4) {
-    const int64_t e = off + col;
-    if (dt == NBK_F32) {
-      r = *(const float4*)((const float*)o.ptr + e);
+  if (valid == 4 && cs == 1) {
+    if (dt == NBK_F32 || dt == NBK_I32) {  // (an int32's bits as they are)
+      const rp_u4 u = *(const rp_u4*)((const float*)ptr + e);
+      r = make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
     } else if (dt == NBK_BF16) {
-      uint2 u = *(const uint2*)((const uint16_t*)o.ptr + e);
+      const rp_u2 u = *(const rp_u2*)((const uint16_t*)ptr + e);
       r.x = __uint_as_float(u.x << 16);
       r.y = __uint_as_float(u.x & 0xffff0000u);
       r.z = __uint_as_float(u.y << 16);
       r.w = __uint_as_float(u.y & 0xffff0000u);
     } else if (dt == NBK_F16) {
-      const __half* h = (const __half*)o.ptr + e;
-      uint2 u = *(const uint2*)h;
-      __half2 a = *(__half2*)&u.x, b = *(__half2*)&u.y;
-      float2 fa = __half22float2(a), fb = __half22float2(b);
+      const rp_u2 u = *(const rp_u2*)((const uint16_t*)ptr + e);
+      const uint32_t ux = u.x, uy = u.y;
+      const float2 fa = __half22float2(__builtin_bit_cast(__half2, ux)),
+                   fb = __half22float2(__builtin_bit_cast(__half2, uy));
       r = make_float4(fa.x, fa.y, fb.x, fb.y);
-    } else if (dt == NBK_I32) {
-      r = *(const float4*)((const int32_t*)o.ptr + e);  // the bits as they are
     } else if (dt == NBK_I64) {
-      const int64_t* p = (const int64_t*)o.ptr + e;
-      longlong2 u0 = *(const longlong2*)p, u1 = *(const longlong2*)(p + 2);
+      const int64_t* p = (const int64_t*)ptr + e;
+      const rp_ll2 u0 = *(const rp_ll2*)p, u1 = *(const rp_ll2*)(p + 2);
       r = make_float4(rp_ibits(rp_sat32(u0.x)), rp_ibits(rp_sat32(u0.y)), rp_ibits(rp_sat32(u1.x)),
                       rp_ibits(rp_sat32(u1.y)));
     } else {
-      uint32_t u = *(const uint32_t*)((const uint8_t*)o.ptr + e);
+      const uint32_t u = *(const rp_u1*)((const uint8_t*)ptr + e);
       r = make_float4((float)(u & 0xff), (float)((u >> 8) & 0xff), (float)((u >> 16) & 0xff),
                       (float)(u >> 24));
     }
     return r;
   }
-  const int64_t e0 = off + col * cs;
-  if (valid > 0) r.x = rp_load1(o.ptr, e0, dt);
+  if (valid > 0) r.x = rp_load1(ptr, e, dt);
   if (cs == 0) {
     r.y = r.z = r.w = r.x;
     return r;
   }
-  if (valid > 1) r.y = rp_load1(o.ptr, e0 + cs, dt);
-  if (valid > 2) r.z = rp_load1(o.ptr, e0 + 2 * cs, dt);
-  if (valid > 3) r.w = rp_load1(o.ptr, e0 + 3 * cs, dt);
+  if (valid > 1) r.y = rp_load1(ptr, e + cs, dt);
+  if (valid > 2) r.z = rp_load1(ptr, e + 2 * cs, dt);
+  if (valid > 3) r.w = rp_load1(ptr, e + 3 * cs, dt);
   return r;
 }
 
-__device__ __forceinline__ void rp_store4(const nbk_operand& o, int64_t off, int64_t col,
-                                          int valid, float4 v) {
-  const int dt = o.dtype;
-  const int64_t cs = o.col_stride;
-  if (o.vec_ok && valid == 4) {
-    const int64_t e = off + col;
-    if (dt == NBK_F32) {
-      *(float4*)((float*)o.ptr + e) = v;
+__device__ __forceinline__ void rp_store4_any(void* ptr, int dt, int64_t e, int64_t cs, int valid, float4 v) {
+  if (valid == 4 && cs == 1) {
+    if (dt == NBK_F32 || dt == NBK_I32) {
+      const rp_u4 u = {__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)};
+      *(rp_u4*)((float*)ptr + e) = u;
     } else if (dt == NBK_BF16) {
-      uint2 u;
+      rp_u2 u;
       u.x = (uint32_t)nbk_f32_to_bf16(v.x) | ((uint32_t)nbk_f32_to_bf16(v.y) << 16);
       u.y = (uint32_t)nbk_f32_to_bf16(v.z) | ((uint32_t)nbk_f32_to_bf16(v.w) << 16);
-      *(uint2*)((uint16_t*)o.ptr + e) = u;
+      *(rp_u2*)((uint16_t*)ptr + e) = u;
     } else if (dt == NBK_F16) {
-      __half2 a = __floats2half2_rn(v.x, v.y), b = __floats2half2_rn(v.z, v.w);
-      uint2 u;
-      u.x = *(uint32_t*)&a;
-      u.y = *(uint32_t*)&b;
-      *(uint2*)((__half*)o.ptr + e) = u;
-    } else if (dt == NBK_I32) {
-      *(float4*)((int32_t*)o.ptr + e) = v;
+      rp_u2 u;
+      u.x = __builtin_bit_cast(uint32_t, __floats2half2_rn(v.x, v.y));
+      u.y = __builtin_bit_cast(uint32_t, __floats2half2_rn(v.z, v.w));
+      *(rp_u2*)((uint16_t*)ptr + e) = u;
     } else if (dt == NBK_I64) {
-      longlong2* p = (longlong2*)((int64_t*)o.ptr + e);
-      p[0] = make_longlong2((int64_t)rp_int(v.x), (int64_t)rp_int(v.y));
-      p[1] = make_longlong2((int64_t)rp_int(v.z), (int64_t)rp_int(v.w));
+      rp_ll2* p = (rp_ll2*)((int64_t*)ptr + e);
+      const rp_ll2 u0 = {(long long)rp_int(v.x), (long long)rp_int(v.y)};
+      const rp_ll2 u1 = {(long long)rp_int(v.z), (long long)rp_int(v.w)};
+      p[0] = u0;
+      p[1] = u1;
     } else {
-      uint32_t u = (uint32_t)(v.x != 0.f) | ((uint32_t)(v.y != 0.f) << 8) |
-                   ((uint32_t)(v.z != 0.f) << 16) | ((uint32_t)(v.w != 0.f) << 24);
-      *(uint32_t*)((uint8_t*)o.ptr + e) = u;
+      *(rp_u1*)((uint8_t*)ptr + e) = (uint32_t)(v.x != 0.f) | ((uint32_t)(v.y != 0.f) << 8) |
+                                     ((uint32_t)(v.z != 0.f) << 16) | ((uint32_t)(v.w != 0.f) << 24);
     }
     return;
   }
-  const int64_t e0 = off + col * cs;
-  if (valid > 0) rp_store1(o.ptr, e0, dt, v.x);
-  if (valid > 1) rp_store1(o.ptr, e0 + cs, dt, v.y);
-  if (valid > 2) rp_store1(o.ptr, e0 + 2 * cs, dt, v.z);
-  if (valid > 3) rp_store1(o.ptr, e0 + 3 * cs, dt, v.w);
+  if (valid > 0) rp_store1(ptr, e, dt, v.x);
+  if (valid > 1) rp_store1(ptr, e + cs, dt, v.y);
+  if (valid > 2) rp_store1(ptr, e + 2 * cs, dt, v.z);
+  if (valid > 3) rp_store1(ptr, e + 3 * cs, dt, v.w);
+}
+
+__device__ __forceinline__ float4 rp_load4(const nbk_operand& o, int64_t off, int64_t col, int valid) {
+  return rp_load4_any(o.ptr, o.dtype, off + col * o.col_stride, o.col_stride, valid);
+}
+__device__ __forceinline__ void rp_store4(const nbk_operand& o, int64_t off, int64_t col, int valid, float4 v) {
+  rp_store4_any(o.ptr, o.dtype, off + col * o.col_stride, o.col_stride, valid, v);
 }
 
 // ---- elementwise functions --------------------------------------------------

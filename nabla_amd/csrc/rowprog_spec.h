@@ -9,8 +9,8 @@ struct rp_spec_entry {
   uint64_t hash;
   // [0]: generic form (any row length).  [1..4]: register-resident forms for
   // reduction programs whose lanes own exactly 1 / 2 / 4 / 8 chunks of a row;
-  // nullptr where that form was not generated.  All have the signature of
-  // rp_block_kernel / rp_flat_kernel.
+  // nullptr where that form was not generated.  Reduction programs take (nbk_rowprog,
+  // int64_t rows), the others (nbk_rowprog, uint32_t chunks per row, uint64_t chunks).
   const void* kernel[5];
   // [1..4]: the same register-resident forms compiled for rows of exactly
   // 1 / 2 / 4 / 8 chunks per lane (no masked lanes or elements); [0] unused.
@@ -30,7 +30,7 @@ struct rp_spec_entry {
 };
 
 // A hand-scheduled kernel for one program (rowprog_hand.hip), attached by hash to that program's
-// entry above.  Signature of rp_block_kernel; launched with `block` lanes per row when
+// entry above.  Signature of a generated reduction kernel; launched with `block` lanes per row when
 // `fits(program)` holds, `kernel_stream` (non-temporal loads and stores) for launches that move
 // more than the last-level cache holds.
 struct rp_hand_entry {
