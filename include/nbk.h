@@ -388,14 +388,15 @@ int nbk_avgpool2d_bwd(const nbk_pool_desc* d, const void* dy, void* dx, void* st
  * log-sum-exp per score row (lse, fp32 [B, H, S]) and the backward recomputes.
  * Tensors are [B, S, H, hd] addressed through element strides (sb, ss, sh) with
  * hd contiguous, so heads are read and written in place of a transpose.
- * dtype NBK_BF16, hd 64 or 128, S a multiple of 128; pointers 16-byte aligned,
- * strides multiples of 8.  causal != 0 masks key > query. */
+ * dtype NBK_BF16, hd 64 or 128; S a multiple of 128 unless any_length is set (then any S, each
+ * tensor S rows long); pointers 16-byte aligned, strides multiples of 8.  causal != 0 masks
+ * key > query. */
 typedef struct nbk_attn_desc {
   int64_t B, H, S, hd;
   float scale;
   int32_t causal;
   int32_t dtype;
-  int32_t reserved;
+  int32_t any_length;
 } nbk_attn_desc;
 typedef struct nbk_attn_tensor {
   void* ptr;

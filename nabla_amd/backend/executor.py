@@ -272,6 +272,7 @@ class BoundPlan:
                 d.B, d.H, d.S, d.hd = a["B"], a["H"], a["S"], a["hd"]
                 d.scale = a["scale"]
                 d.causal = 1 if a["causal"] else 0
+                d.any_length = 1
                 d.dtype = a["q"].dtype.abi
                 keep_alive = [d]
 
@@ -279,7 +280,9 @@ class BoundPlan:
                     """[B, H, S, hd] view -> (batch, sequence, head) strides."""
                     t = lib.AttnTensor()
                     sb, sh, ss, _ = ref.strides
-                    t.sb, t.ss, t.sh = sb, ss, (sh if ref.shape[1] > 1 else a["hd"])
+                    t.sb = sb
+                    t.ss = ss if ref.shape[2] > 1 else a["hd"]
+                    t.sh = sh if ref.shape[1] > 1 else a["hd"]
                     if ref.shape[0] == 1:
                         t.sb = 0
                     ptr_field(t, "ptr", ref.buf, ref.offset * ref.dtype.size_in_bytes)

@@ -114,7 +114,7 @@ class PoolDesc(C.Structure):
 class AttnDesc(C.Structure):
     _fields_ = [
         ("B", C.c_int64), ("H", C.c_int64), ("S", C.c_int64), ("hd", C.c_int64),
-        ("scale", C.c_float), ("causal", C.c_int32), ("dtype", C.c_int32), ("reserved", C.c_int32),
+        ("scale", C.c_float), ("causal", C.c_int32), ("dtype", C.c_int32), ("any_length", C.c_int32),
     ]
 
 

@@ -4,8 +4,15 @@
 //   backward: dQ, dK, dV from (Q, K, V, O, LSE, dO) with the probabilities recomputed
 //
 // The S x S score matrix never reaches memory.  Tensors are [B, S, H, hd] in any
-// strides with a unit stride along hd (heads are read in place), hd = 64 or 128,
-// S a multiple of 128.
+// strides with a unit stride along hd (heads are read in place), hd = 64 or 128.
+//
+// Every kernel works on whole tiles of 128 owned rows and 64 walked rows.  Where S is a multiple
+// of 128 nothing else exists (RAG = false).  For any other S (RAG = true) the rows past the end
+// are read from row S - 1 (an address inside the tensor, finite values), walked rows past the end
+// get probability zero in the tile that holds them, owned ones are not stored, and a wave
+// without an owned row inside skips the arithmetic.  B1 H8 S1800 hd128, causal: 44 us; as batched
+// products around a softmax program (which wrote the scores three times) it took 260 us, and a
+// training step of a B6 S333 H8 hd64 block 756 us where it takes 566 with these kernels.
 //
 // Register layouts of v_mfma_f32_32x32x16_bf16 (lane l, li = l % 32, h = l / 32):
 //   A: lane holds A[row li][k = 8h .. 8h+7]      B: lane holds B[k = 8h .. 8h+7][col li]
@@ -89,12 +96,13 @@ struct AtRowTile {
     if constexpr (NCH == 8) return (row & 7) ^ ((row >> 3) & 1);  // 128-byte rows: two per window
     else return row & 15;
   }
-  __device__ __forceinline__ void load(const uint16_t* base, int64_t row_stride, int row0) {
+  // (rows past `last` repeat it)
+  __device__ __forceinline__ void load(const uint16_t* base, int64_t row_stride, int row0, int last) {
 #pragma unroll
     for (int s = 0; s < NREG; ++s) {
       const int t = threadIdx.x + s * 256;
       const int row = t / NCH, c = t % NCH;
-      reg[s] = *(const at_u32x4*)(base + (int64_t)(row0 + row) * row_stride + c * 8);
+      reg[s] = *(const at_u32x4*)(base + (int64_t)min(row0 + row, last) * row_stride + c * 8);
     }
   }
   __device__ __forceinline__ void store(at_u32x4* lds) const {
@@ -126,12 +134,12 @@ struct AtTransTile {
     kb = (t >> 2) % NKB;
     db = (t & 3) + 4 * (t / (4 * NKB));
   }
-  __device__ __forceinline__ void load(const uint16_t* base, int64_t row_stride, int row0) {
+  __device__ __forceinline__ void load(const uint16_t* base, int64_t row_stride, int row0, int last) {
     int kb, db;
     block_of(kb, db);
 #pragma unroll
     for (int r = 0; r < KPB; ++r)
-      reg[r] = *(const at_u32x4*)(base + (int64_t)(row0 + kb * KPB + r) * row_stride + db * 8);
+      reg[r] = *(const at_u32x4*)(base + (int64_t)min(row0 + kb * KPB + r, last) * row_stride + db * 8);
   }
   __device__ __forceinline__ void store(uint16_t* lds) const {
     int kb, db;
@@ -224,8 +232,8 @@ constexpr float AT_SLACK = 8.0f;
 constexpr float AT_LOG2E = 1.4426950408889634f;
 constexpr float AT_LN2 = 0.6931471805599453f;
 
-template <int HD>
-__global__ __launch_bounds__(256, HD == 64 ? 4 : 2) void attn_fwd_kernel(const AttnArgs g) {
+template <int HD, bool RAG>
+__global__ __launch_bounds__(256, HD == 64 ? (RAG ? 3 : 4) : 2) void attn_fwd_kernel(const AttnArgs g) {
   constexpr int KSTEPS = HD / 16, DT = HD / 32, NCH = HD / 8;
   constexpr int TILE = 64 * HD * 2, STAGE = 2 * TILE;
   extern __shared__ __align__(16) unsigned char at_lds[];
@@ -244,13 +252,15 @@ __global__ __launch_bounds__(256, HD == 64 ? 4 : 2) void attn_fwd_kernel(const A
   const uint16_t* V = g.v.p + (int64_t)b * g.v.sb + (int64_t)hh * g.v.sh;
   const int wq0 = q0 + wave * 32;  // first query of the wave
   const int my_q = wq0 + li;
+  const int last = g.S - 1;
+  const int row_q = RAG ? min(my_q, last) : my_q;  // the row this lane reads for its query
   const float c = g.scale * AT_LOG2E;
 
   // the wave's queries as B fragments of the score MFMA
   at_bf16x8 qf[KSTEPS];
 #pragma unroll
   for (int s = 0; s < KSTEPS; ++s) {
-    const at_u32x4 u = *(const at_u32x4*)(Q + (int64_t)my_q * g.q.ss + s * 16 + h * 8);
+    const at_u32x4 u = *(const at_u32x4*)(Q + (int64_t)row_q * g.q.ss + s * 16 + h * 8);
     qf[s] = __builtin_bit_cast(at_bf16x8, u);
   }
 
@@ -266,7 +276,8 @@ __global__ __launch_bounds__(256, HD == 64 ? 4 : 2) void attn_fwd_kernel(const A
   // log-sum-exp, with which the probabilities that the backward pass recomputes sum to one too.
   float l_r = 0.f;
 
-  const int n_tiles = g.causal ? (q0 + 128) / 64 : g.S / 64;
+  const int all_tiles = RAG ? (g.S + 63) / 64 : g.S / 64;
+  const int n_tiles = !g.causal ? all_tiles : RAG ? min((q0 + 128) / 64, all_tiles) : (q0 + 128) / 64;
   // K and V tiles go from memory into LDS without passing through registers: a wave instruction
   // deposits 64 x 16 bytes in a row (four rows of a 128-wide tile, eight of a 64-wide one), so
   // the swizzle is applied to the address each lane fetches from.
@@ -281,6 +292,18 @@ __global__ __launch_bounds__(256, HD == 64 ? 4 : 2) void attn_fwd_kernel(const A
   auto request = [&](int kt, int buf) {
     const uint16_t* ks = K + (int64_t)kt * 64 * g.k.ss;
     const uint16_t* vs = V + (int64_t)kt * 64 * g.v.ss;
+    if (RAG && kt * 64 + 63 > last) {  // (the last tile: rows past the end repeat the last one)
+#pragma unroll
+      for (int j = 0; j < PER_WAVE; ++j) {
+        const int slot = (wave * PER_WAVE + j) * 64 + lane, row = slot / NCH;
+        const int back = max(kt * 64 + row - last, 0);
+        __builtin_amdgcn_global_load_lds((at_glb_void*)(ks + src_off_k[j] - back * (int)g.k.ss),
+                                         (at_lds_void*)(k_tile(buf) + (wave * PER_WAVE + j) * 64), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((at_glb_void*)(vs + src_off_v[j] - back * (int)g.v.ss),
+                                         (at_lds_void*)(v_tile(buf) + (wave * PER_WAVE + j) * 64), 16, 0, 0);
+      }
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < PER_WAVE; ++j) {
       __builtin_amdgcn_global_load_lds((at_glb_void*)(ks + src_off_k[j]),
@@ -313,6 +336,7 @@ __global__ __launch_bounds__(256, HD == 64 ? 4 : 2) void attn_fwd_kernel(const A
     const unsigned char* base = (const unsigned char*)tile + k16 * 16 * (HD * 2);
     return at_tr_pair(base + tr_lo + ((tr_x_lo ^ (dd << 2)) << 4), base + tr_hi + ((tr_x_hi ^ (dd << 2)) << 4));
   };
+  const int seen = g.causal ? (RAG ? min(my_q, last) : my_q) : last;  // the last key this lane's query sees
   request(0, 0);
   tile_barrier();
   for (int kt = 0; kt < n_tiles; ++kt) {
@@ -346,7 +370,7 @@ __global__ __launch_bounds__(256, HD == 64 ? 4 : 2) void attn_fwd_kernel(const A
         for (int r = 0; r < 16; ++r) {
           if (MASK) {
             const int key = k0 + kt2 * 32 + (r >> 2) * 8 + 4 * h + (r & 3);
-            if (key > my_q) st[kt2][r] = at_neg_big();
+            if (key > seen) st[kt2][r] = at_neg_big();
           }
           mx = fmaxf(mx, st[kt2][r]);
         }
@@ -383,13 +407,16 @@ __global__ __launch_bounds__(256, HD == 64 ? 4 : 2) void attn_fwd_kernel(const A
         }
     };
     // keys of this tile against the wave's queries: all visible, some, or none
-    if (!g.causal || k0 + 63 <= wq0) tile(std::false_type{});
-    else if (k0 <= wq0 + 31) tile(std::true_type{});
+    const bool whole = !RAG || k0 + 63 <= last;
+    if (RAG && wq0 > last) {}
+    else if (whole && (!g.causal || k0 + 63 <= wq0)) tile(std::false_type{});
+    else if (!g.causal || k0 <= wq0 + 31) tile(std::true_type{});
     tile_barrier();
   }
-  // normalise and write: register r of tile d is O[my_q][32 d + (r/4)*8 + 4h + r%4]
   l_i += at_xhalf(l_i);
   l_r += at_xhalf(l_r);
+  if (RAG && my_q > last) return;
+  // normalise and write: register r of tile d is O[my_q][32 d + (r/4)*8 + 4h + r%4]
   const float inv = 1.0f / l_r;
   uint16_t* O = (uint16_t*)g.o.p + (int64_t)b * g.o.sb + (int64_t)hh * g.o.sh + (int64_t)my_q * g.o.ss;
 #pragma unroll
@@ -430,7 +457,7 @@ __global__ __launch_bounds__(256, HD == 64 ? 4 : 2) void attn_fwd_kernel(const A
 //   dP[q, key] = dO V^T         (A: dO tile rows, B: the wave's V fragments)
 //   dS         = P * (dP - delta[q])
 //   dK^T[d,key] += Q^T[d, q] dS[q, key]         (A: transposed Q tile, B: dS registers; * scale at the end)
-template <int HD>
+template <int HD, bool RAG>
 __global__ __launch_bounds__(256) void attn_bwd_kv_kernel(const AttnArgs g) {
   using RowT = AtRowTile<HD>;
   using TrT = AtTransTile<HD>;
@@ -454,12 +481,14 @@ __global__ __launch_bounds__(256) void attn_bwd_kv_kernel(const AttnArgs g) {
   const float* LSE = g.lse + ((int64_t)b * g.H + hh) * g.S;
   const float* DEL = g.delta + ((int64_t)b * g.H + hh) * g.S;
   const int my_k = k0 + wave * 32 + li;
+  const int last = RAG ? g.S - 1 : 0x7fffffff;  // (no row is past the end of whole tiles)
+  const int row_k = min(my_k, last);
 
   at_bf16x8 kf[KSTEPS], vf[KSTEPS];
 #pragma unroll
   for (int s = 0; s < KSTEPS; ++s) {
-    const at_u32x4 uk = *(const at_u32x4*)(K + (int64_t)my_k * g.k.ss + s * 16 + h * 8);
-    const at_u32x4 uv = *(const at_u32x4*)(V + (int64_t)my_k * g.v.ss + s * 16 + h * 8);
+    const at_u32x4 uk = *(const at_u32x4*)(K + (int64_t)row_k * g.k.ss + s * 16 + h * 8);
+    const at_u32x4 uv = *(const at_u32x4*)(V + (int64_t)row_k * g.v.ss + s * 16 + h * 8);
     kf[s] = __builtin_bit_cast(at_bf16x8, uk);
     vf[s] = __builtin_bit_cast(at_bf16x8, uv);
   }
@@ -471,17 +500,17 @@ __global__ __launch_bounds__(256) void attn_bwd_kv_kernel(const AttnArgs g) {
   }
 
   const int first = g.causal ? k0 / 64 : 0;  // first query tile that sees key k0
-  const int n_tiles = g.S / 64;
+  const int n_tiles = RAG ? (g.S + 63) / 64 : g.S / 64;
   RowT ql, dol;
   TrT qtl, dotl;
   float lreg = 0.f;  // lanes 0..63: LSE, 64..127: delta of the tile's queries
   auto load_all = [&](int qt) {
-    ql.load(Q, g.q.ss, qt * 64);
-    dol.load(DO, g.dout.ss, qt * 64);
-    qtl.load(Q, g.q.ss, qt * 64);
-    dotl.load(DO, g.dout.ss, qt * 64);
-    if (threadIdx.x < 64) lreg = LSE[qt * 64 + threadIdx.x] * AT_LOG2E;
-    else if (threadIdx.x < 128) lreg = DEL[qt * 64 + threadIdx.x - 64];
+    ql.load(Q, g.q.ss, qt * 64, last);
+    dol.load(DO, g.dout.ss, qt * 64, last);
+    qtl.load(Q, g.q.ss, qt * 64, last);
+    dotl.load(DO, g.dout.ss, qt * 64, last);
+    if (threadIdx.x < 64) lreg = LSE[min(qt * 64 + (int)threadIdx.x, last)] * AT_LOG2E;
+    else if (threadIdx.x < 128) lreg = DEL[min(qt * 64 + (int)threadIdx.x - 64, last)];
   };
   auto store_all = [&](int buf) {
     ql.store(q_tile(buf));
@@ -492,6 +521,7 @@ __global__ __launch_bounds__(256) void attn_bwd_kv_kernel(const AttnArgs g) {
   };
   const int wk0 = k0 + wave * 32;  // first key of the wave
   const float c = g.scale * AT_LOG2E;
+  const int see = g.causal ? 0 : 0x3fffffff;  // how far past itself a query sees
   load_all(first);
   store_all(0);
   __syncthreads();
@@ -536,7 +566,7 @@ __global__ __launch_bounds__(256) void attn_bwd_kv_kernel(const AttnArgs g) {
         for (int e = 0; e < 4; ++e) {
           const int r = gq * 4 + e;
           float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[r], c, -lv[e]));
-          if (MASK && my_k > q0 + qb + e) pv = 0.f;
+          if (MASK && (my_k > q0 + qb + e + (RAG ? see : 0) || (RAG && q0 + qb + e > last))) pv = 0.f;
           p[r] = pv;
           ds[r] = pv * (dp_acc[r] - dv[e]);
         }
@@ -556,12 +586,15 @@ __global__ __launch_bounds__(256) void attn_bwd_kv_kernel(const AttnArgs g) {
 #pragma unroll
     for (int qt2 = 0; qt2 < 2; ++qt2) {
       const int sq0 = q0 + qt2 * 32;  // queries sq0 .. sq0 + 31 against keys wk0 .. wk0 + 31
-      if (!g.causal || wk0 + 31 <= sq0) subtile(std::false_type{}, qt2);
-      else if (wk0 <= sq0 + 31) subtile(std::true_type{}, qt2);
+      const bool whole = !RAG || sq0 + 31 <= last;
+      if (RAG && (sq0 > last || wk0 > last)) {}
+      else if (whole && (!g.causal || wk0 + 31 <= sq0)) subtile(std::false_type{}, qt2);
+      else if (!g.causal || wk0 <= sq0 + 31) subtile(std::true_type{}, qt2);
     }
     if (more) store_all(cur ^ 1);
     __syncthreads();
   }
+  if (RAG && my_k > last) return;
   uint16_t* DK = (uint16_t*)g.dk.p + (int64_t)b * g.dk.sb + (int64_t)hh * g.dk.sh + (int64_t)my_k * g.dk.ss;
   uint16_t* DV = (uint16_t*)g.dv.p + (int64_t)b * g.dv.sb + (int64_t)hh * g.dv.sh + (int64_t)my_k * g.dv.ss;
 #pragma unroll
@@ -593,7 +626,7 @@ __global__ __launch_bounds__(256) void attn_bwd_kv_kernel(const AttnArgs g) {
 // sw(r) = 4 (r % 4) + (r / 4) % 4.  Sixteen consecutive rows send one chunk to sixteen different
 // 16-byte slots (the fragment reads of 16 lanes), and four consecutive rows send a 64-byte piece
 // to four different 64-byte windows (the transposing read of half a wave).
-template <int HD>
+template <int HD, bool RAG>
 __global__ __launch_bounds__(512) void attn_bwd_kv8_kernel(const AttnArgs g) {
   constexpr int KSTEPS = HD / 16, DT = HD / 32, NCH = HD / 8;
   constexpr int TILE = 64 * HD * 2;    // a 64-row tile
@@ -617,13 +650,14 @@ __global__ __launch_bounds__(512) void attn_bwd_kv8_kernel(const AttnArgs g) {
   const float* LSE = g.lse + ((int64_t)b * g.H + hh) * g.S;
   const float* DEL = g.delta + ((int64_t)b * g.H + hh) * g.S;
   const int my_k = k0 + kw * 32 + li;
+  const int last = RAG ? g.S - 1 : 0x7fffffff;  // (no row is past the end of whole tiles)
 
   // K and V rows of the workgroup -> LDS (512 lanes, 16 bytes each)
 #pragma unroll
   for (int s = 0; s < 128 * NCH / 512; ++s) {
     const int t = tid + s * 512, row = t / NCH, c = t % NCH;
-    Ks[row * NCH + (c ^ at_sw<NCH>(row))] = *(const at_u32x4*)(K + (int64_t)(k0 + row) * g.k.ss + c * 8);
-    Vs[row * NCH + (c ^ at_sw<NCH>(row))] = *(const at_u32x4*)(V + (int64_t)(k0 + row) * g.v.ss + c * 8);
+    Ks[row * NCH + (c ^ at_sw<NCH>(row))] = *(const at_u32x4*)(K + (int64_t)min(k0 + row, last) * g.k.ss + c * 8);
+    Vs[row * NCH + (c ^ at_sw<NCH>(row))] = *(const at_u32x4*)(V + (int64_t)min(k0 + row, last) * g.v.ss + c * 8);
   }
 
   at_f32x16 dk_acc[DT], dv_acc[DT];
@@ -634,7 +668,7 @@ __global__ __launch_bounds__(512) void attn_bwd_kv8_kernel(const AttnArgs g) {
   }
 
   const int first = g.causal ? k0 / 64 : 0;  // first query tile that sees key k0
-  const int n_tiles = g.S / 64;
+  const int n_tiles = RAG ? (g.S + 63) / 64 : g.S / 64;
   constexpr int TP = 64 * NCH / 512;  // passes over a 64-row tile
   at_u32x4 qreg[TP], doreg[TP];
   float lreg = 0.f;  // lanes 0..63: LSE, 64..127: delta of the tile's queries
@@ -642,11 +676,11 @@ __global__ __launch_bounds__(512) void attn_bwd_kv8_kernel(const AttnArgs g) {
 #pragma unroll
     for (int s = 0; s < TP; ++s) {
       const int t = tid + s * 512, row = t / NCH, c = t % NCH;
-      qreg[s] = *(const at_u32x4*)(Q + (int64_t)(qt * 64 + row) * g.q.ss + c * 8);
-      doreg[s] = *(const at_u32x4*)(DO + (int64_t)(qt * 64 + row) * g.dout.ss + c * 8);
+      qreg[s] = *(const at_u32x4*)(Q + (int64_t)min(qt * 64 + row, last) * g.q.ss + c * 8);
+      doreg[s] = *(const at_u32x4*)(DO + (int64_t)min(qt * 64 + row, last) * g.dout.ss + c * 8);
     }
-    if (tid < 64) lreg = LSE[qt * 64 + tid] * AT_LOG2E;
-    else if (tid < 128) lreg = DEL[qt * 64 + tid - 64];
+    if (tid < 64) lreg = LSE[min(qt * 64 + tid, last)] * AT_LOG2E;
+    else if (tid < 128) lreg = DEL[min(qt * 64 + tid - 64, last)];
   };
   auto store_all = [&](int buf) {
     at_u32x4* qd = q_tile(buf);
@@ -684,6 +718,7 @@ __global__ __launch_bounds__(512) void attn_bwd_kv8_kernel(const AttnArgs g) {
 
   const int wk0 = k0 + kw * 32;  // first key of the wave
   const float c = g.scale * AT_LOG2E;
+  const int see = g.causal ? 0 : 0x3fffffff;  // how far past itself a query sees
   load_all(first);
   store_all(0);
   __syncthreads();
@@ -725,7 +760,7 @@ __global__ __launch_bounds__(512) void attn_bwd_kv8_kernel(const AttnArgs g) {
         for (int e = 0; e < 4; ++e) {
           const int r = gq * 4 + e;
           float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[r], c, -lv[e]));
-          if (MASK && my_k > qt * 64 + qb + e) pv = 0.f;
+          if (MASK && (my_k > qt * 64 + qb + e + (RAG ? see : 0) || (RAG && qt * 64 + qb + e > last))) pv = 0.f;
           s_acc[r] = pv;                          // P in place of S
           dp_acc[r] = pv * (dp_acc[r] - dv[e]);   // dS in place of dP
         }
@@ -740,8 +775,10 @@ __global__ __launch_bounds__(512) void attn_bwd_kv8_kernel(const AttnArgs g) {
         }
       }
     };
-    if (!g.causal || wk0 + 31 <= sq0) subtile(std::false_type{});
-    else if (wk0 <= sq0 + 31) subtile(std::true_type{});
+    const bool whole = !RAG || sq0 + 31 <= last;
+    if (RAG && (sq0 > last || wk0 > last)) {}
+    else if (whole && (!g.causal || wk0 + 31 <= sq0)) subtile(std::false_type{});
+    else if (!g.causal || wk0 <= sq0 + 31) subtile(std::true_type{});
     if (more) store_all(cur ^ 1);
     __syncthreads();
   }
@@ -758,7 +795,7 @@ __global__ __launch_bounds__(512) void attn_bwd_kv8_kernel(const AttnArgs g) {
       }
   }
   __syncthreads();
-  if (qh == 1) return;
+  if (qh == 1 || (RAG && my_k > last)) return;
   uint16_t* DK = (uint16_t*)g.dk.p + (int64_t)b * g.dk.sb + (int64_t)hh * g.dk.sh + (int64_t)my_k * g.dk.ss;
   uint16_t* DV = (uint16_t*)g.dv.p + (int64_t)b * g.dv.sb + (int64_t)hh * g.dv.sh + (int64_t)my_k * g.dv.ss;
 #pragma unroll
@@ -785,7 +822,7 @@ __global__ __launch_bounds__(512) void attn_bwd_kv8_kernel(const AttnArgs g) {
 // There is no transposed copy of K: the A operand of the last product comes out of the row-major
 // K tile through the transposing LDS read, in the layout of the eight-wave dK / dV kernel above.
 // Two stages of K and V (32 KB each with 128-wide heads) fit twice on a CU.
-template <int HD>
+template <int HD, bool RAG>
 __global__ __launch_bounds__(256, 2) void attn_bwd_q_tr_kernel(const AttnArgs g) {
   constexpr int KSTEPS = HD / 16, DT = HD / 32, NCH = HD / 8;
   constexpr int TILE = 64 * HD * 2, STAGE = 2 * TILE;
@@ -802,7 +839,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_tr_kernel(const AttnArgs g)
   const uint16_t* V = g.v.p + (int64_t)b * g.v.sb + (int64_t)hh * g.v.sh;
   const uint16_t* DO = g.dout.p + (int64_t)b * g.dout.sb + (int64_t)hh * g.dout.sh;
   const int my_q = q0 + wave * 32 + li;
-  const float my_lse = g.lse[((int64_t)b * g.H + hh) * g.S + my_q] * AT_LOG2E;
+  const int last = RAG ? g.S - 1 : 0x7fffffff;  // (no row is past the end of whole tiles)
+  const int row_q = min(my_q, last);
+  const float my_lse = g.lse[((int64_t)b * g.H + hh) * g.S + row_q] * AT_LOG2E;
   const int wq0 = q0 + wave * 32;  // first query of the wave
   const float c = g.scale * AT_LOG2E;
 
@@ -810,15 +849,16 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_tr_kernel(const AttnArgs g)
 #pragma unroll
   for (int d = 0; d < DT; ++d) dq_acc[d] = (at_f32x16)(0.f);
 
-  const int n_tiles = g.causal ? (q0 + 128) / 64 : g.S / 64;
+  const int all_tiles = RAG ? (g.S + 63) / 64 : g.S / 64;
+  const int n_tiles = !g.causal ? all_tiles : RAG ? min((q0 + 128) / 64, all_tiles) : (q0 + 128) / 64;
   constexpr int TP = 64 * NCH / 256;  // passes over a 64-row tile
   at_u32x4 kreg[TP], vreg[TP];
   auto load_all = [&](int kt) {
 #pragma unroll
     for (int s = 0; s < TP; ++s) {
       const int t = tid + s * 256, row = t / NCH, ch = t % NCH;
-      kreg[s] = *(const at_u32x4*)(K + (int64_t)(kt * 64 + row) * g.k.ss + ch * 8);
-      vreg[s] = *(const at_u32x4*)(V + (int64_t)(kt * 64 + row) * g.v.ss + ch * 8);
+      kreg[s] = *(const at_u32x4*)(K + (int64_t)min(kt * 64 + row, last) * g.k.ss + ch * 8);
+      vreg[s] = *(const at_u32x4*)(V + (int64_t)min(kt * 64 + row, last) * g.v.ss + ch * 8);
     }
   };
   auto store_all = [&](int buf) {
@@ -866,19 +906,20 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_tr_kernel(const AttnArgs g)
   load_all(0);
 #pragma unroll
   for (int s = 0; s < KSTEPS; ++s) {
-    const at_u32x4 uq = *(const at_u32x4*)(Q + (int64_t)my_q * g.q.ss + s * 16 + h * 8);
-    const at_u32x4 ud = *(const at_u32x4*)(DO + (int64_t)my_q * g.dout.ss + s * 16 + h * 8);
+    const at_u32x4 uq = *(const at_u32x4*)(Q + (int64_t)row_q * g.q.ss + s * 16 + h * 8);
+    const at_u32x4 ud = *(const at_u32x4*)(DO + (int64_t)row_q * g.dout.ss + s * 16 + h * 8);
     qf[s] = __builtin_bit_cast(at_bf16x8, uq);
     dof[s] = __builtin_bit_cast(at_bf16x8, ud);
   }
 #pragma unroll
   for (int s = 0; s < KSTEPS; ++s) {
-    uo[s] = *(const at_u32x4*)(O + (int64_t)my_q * g.o.ss + s * 16 + h * 8);
+    uo[s] = *(const at_u32x4*)(O + (int64_t)row_q * g.o.ss + s * 16 + h * 8);
     ul[s] = (at_u32x4){0u, 0u, 0u, 0u};
-    if (OL != nullptr) ul[s] = *(const at_u32x4*)(OL + (int64_t)my_q * g.o_lo.ss + s * 16 + h * 8);
+    if (OL != nullptr) ul[s] = *(const at_u32x4*)(OL + (int64_t)row_q * g.o_lo.ss + s * 16 + h * 8);
   }
   store_all(0);
   __syncthreads();
+  const int seen = g.causal ? row_q : last;  // the last key this lane's query sees
   float my_delta = 0.f;
 #pragma unroll
   for (int s = 0; s < KSTEPS; ++s) {
@@ -891,7 +932,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_tr_kernel(const AttnArgs g)
     }
   }
   my_delta += at_xhalf(my_delta);
-  if (h == 0) g.delta[((int64_t)b * g.H + hh) * g.S + my_q] = my_delta;
+  if (h == 0 && my_q <= last) g.delta[((int64_t)b * g.H + hh) * g.S + my_q] = my_delta;
   for (int kt = 0; kt < n_tiles; ++kt) {
     const int cur = kt & 1;
     const bool more = kt + 1 < n_tiles;
@@ -921,7 +962,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_tr_kernel(const AttnArgs g)
         float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[r], c, -my_lse));
         if (MASK) {
           const int key = k0 + kt2 * 32 + (r >> 2) * 8 + 4 * h + (r & 3);
-          if (key > my_q) pv = 0.f;
+          if (key > seen) pv = 0.f;
         }
         dp_acc[r] = pv * (dp_acc[r] - my_delta);  // dS^T in place of dP^T
       }
@@ -936,12 +977,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_tr_kernel(const AttnArgs g)
 #pragma unroll
     for (int kt2 = 0; kt2 < 2; ++kt2) {
       const int sk0 = k0 + kt2 * 32;  // keys sk0 .. sk0 + 31 against queries wq0 .. wq0 + 31
-      if (!g.causal || sk0 + 31 <= wq0) subtile(std::false_type{}, kt2);
-      else if (sk0 <= wq0 + 31) subtile(std::true_type{}, kt2);
+      const bool whole = !RAG || sk0 + 31 <= last;
+      if (RAG && (sk0 > last || wq0 > last)) {}
+      else if (whole && (!g.causal || sk0 + 31 <= wq0)) subtile(std::false_type{}, kt2);
+      else if (!g.causal || sk0 <= wq0 + 31) subtile(std::true_type{}, kt2);
     }
     if (more) store_all(cur ^ 1);
     __syncthreads();
   }
+  if (RAG && my_q > last) return;
   uint16_t* DQ = (uint16_t*)g.dq.p + (int64_t)b * g.dq.sb + (int64_t)hh * g.dq.sh + (int64_t)my_q * g.dq.ss;
 #pragma unroll
   for (int d = 0; d < DT; ++d)
@@ -975,10 +1019,10 @@ static int attn_common(const nbk_attn_desc* d, AttnArgs* a) {
   NBK_REQUIRE(d != nullptr, "attention: null descriptor");
   NBK_REQUIRE(d->dtype == NBK_BF16, "attention: only bf16 is implemented (dtype %d)", d->dtype);
   NBK_REQUIRE(d->hd == 64 || d->hd == 128, "attention: head size %lld must be 64 or 128", (long long)d->hd);
-  NBK_REQUIRE(d->B > 0 && d->H > 0 && d->S > 0 && d->S % 128 == 0,
+  NBK_REQUIRE(d->B > 0 && d->H > 0 && d->S > 0 && (d->any_length || d->S % 128 == 0),
               "attention: B %lld, H %lld, S %lld (S must be a positive multiple of 128)",
               (long long)d->B, (long long)d->H, (long long)d->S);
-  NBK_REQUIRE(d->B * d->H <= 0x7fffffffLL && d->S / 128 <= 65535, "attention: extent beyond the grid limits");
+  NBK_REQUIRE(d->B * d->H <= 0x7fffffffLL && (d->S + 127) / 128 <= 65535, "attention: extent beyond the grid limits");
   a->B = (int32_t)d->B; a->H = (int32_t)d->H; a->S = (int32_t)d->S;
   a->causal = d->causal ? 1 : 0;
   a->scale = d->scale;
@@ -1004,17 +1048,19 @@ extern "C" int nbk_attention_fwd(const nbk_attn_desc* d, const nbk_attn_tensor* 
     return rc;
   NBK_REQUIRE(lse != nullptr, "attention: null lse");
   a.lse = (float*)lse;
-  const dim3 grid((unsigned)(d->B * d->H), (unsigned)(d->S / 128));
+  const dim3 grid((unsigned)(d->B * d->H), (unsigned)((d->S + 127) / 128));
   hipStream_t st = (hipStream_t)stream;
   // two stages of a row-major K and V tile each
   const size_t lds = 2 * 2 * 64 * (size_t)d->hd * 2;
-  if (d->hd == 64) {
-    if ((rc = attn_set_lds(attn_fwd_kernel<64>, lds))) return rc;
-    hipLaunchKernelGGL(attn_fwd_kernel<64>, grid, dim3(256), lds, st, a);
-  } else {
-    if ((rc = attn_set_lds(attn_fwd_kernel<128>, lds))) return rc;
-    hipLaunchKernelGGL(attn_fwd_kernel<128>, grid, dim3(256), lds, st, a);
-  }
+  const bool rag = d->S % 128 != 0;
+  auto launch = [&](auto kern) -> int {
+    const int lrc = attn_set_lds(kern, lds);
+    if (lrc == NBK_OK) hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, a);
+    return lrc;
+  };
+  rc = d->hd == 64 ? (rag ? launch(attn_fwd_kernel<64, true>) : launch(attn_fwd_kernel<64, false>))
+                   : (rag ? launch(attn_fwd_kernel<128, true>) : launch(attn_fwd_kernel<128, false>));
+  if (rc) return rc;
   return nbk_check_launch("attn_fwd_kernel");
 }
 
@@ -1028,23 +1074,31 @@ extern "C" int64_t nbk_attention_bwd_workspace(const nbk_attn_desc* d) {
 static int attn_bwd_launch(const nbk_attn_desc* d, AttnArgs& a, float* delta, hipStream_t st) {
   int rc;
   a.delta = delta;
-  const dim3 grid((unsigned)(d->B * d->H), (unsigned)(d->S / 128));
+  const dim3 grid((unsigned)(d->B * d->H), (unsigned)((d->S + 127) / 128));
+  auto launch = [&](auto q_kern, auto kv_kern, size_t lds_q, size_t lds_kv, int kv_lanes) -> int {
+    int lrc = attn_set_lds(q_kern, lds_q);
+    if (lrc == NBK_OK) lrc = attn_set_lds(kv_kern, lds_kv);
+    if (lrc != NBK_OK) return lrc;
+    // (the dQ kernel first: it leaves delta, the row sums of dO * O, for the dK / dV kernel)
+    hipLaunchKernelGGL(q_kern, grid, dim3(256), lds_q, st, a);
+    hipLaunchKernelGGL(kv_kern, grid, dim3(kv_lanes), lds_kv, st, a);
+    return NBK_OK;
+  };
+  const bool rag = d->S % 128 != 0;
   if (d->hd == 64) {
     // (the eight-wave dK / dV form was measured on this head size too: 70 against 68 us on the
     // transformer block's shape, so 64-wide heads keep the four-wave kernel, which fits twice on a CU)
-    // (the dQ kernel first: it leaves delta, the row sums of dO * O, for the dK / dV kernel)
     const size_t lds_kv = 2 * (2 * 64 * 64 * 2 + 2 * 64 * AT_TP * 2 + 2 * 64 * 4);
-    const size_t lds_qtr = 2 * (2 * 64 * 64 * 2);
-    if ((rc = attn_set_lds(attn_bwd_kv_kernel<64>, lds_kv))) return rc;
-    hipLaunchKernelGGL(attn_bwd_q_tr_kernel<64>, grid, dim3(256), lds_qtr, st, a);
-    hipLaunchKernelGGL(attn_bwd_kv_kernel<64>, grid, dim3(256), lds_kv, st, a);
+    const size_t lds_q = 2 * (2 * 64 * 64 * 2);
+    rc = rag ? launch(attn_bwd_q_tr_kernel<64, true>, attn_bwd_kv_kernel<64, true>, lds_q, lds_kv, 256)
+             : launch(attn_bwd_q_tr_kernel<64, false>, attn_bwd_kv_kernel<64, false>, lds_q, lds_kv, 256);
   } else {
-    const size_t lds_kv8 = 2 * (128 * 128 * 2) + 2 * (2 * 64 * 128 * 2 + 2 * 64 * 4);
-    const size_t lds_qtr = 2 * (2 * 64 * 128 * 2);
-    if ((rc = attn_set_lds(attn_bwd_kv8_kernel<128>, lds_kv8))) return rc;
-    hipLaunchKernelGGL(attn_bwd_q_tr_kernel<128>, grid, dim3(256), lds_qtr, st, a);
-    hipLaunchKernelGGL(attn_bwd_kv8_kernel<128>, grid, dim3(512), lds_kv8, st, a);
+    const size_t lds_kv = 2 * (128 * 128 * 2) + 2 * (2 * 64 * 128 * 2 + 2 * 64 * 4);
+    const size_t lds_q = 2 * (2 * 64 * 128 * 2);
+    rc = rag ? launch(attn_bwd_q_tr_kernel<128, true>, attn_bwd_kv8_kernel<128, true>, lds_q, lds_kv, 512)
+             : launch(attn_bwd_q_tr_kernel<128, false>, attn_bwd_kv8_kernel<128, false>, lds_q, lds_kv, 512);
   }
+  if (rc) return rc;
   return nbk_check_launch("attn_bwd kernels");
 }
 

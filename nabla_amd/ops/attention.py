@@ -27,7 +27,6 @@ from ..core.tensor import Tensor
 from .base import Operation
 
 _HEAD_SIZES = (64, 128)
-_SEQ_MULTIPLE = 128
 
 
 def fused_attention_applies(query: Tensor, key: Tensor, value: Tensor) -> bool:
@@ -39,7 +38,7 @@ def fused_attention_applies(query: Tensor, key: Tensor, value: Tensor) -> bool:
     if not (query.dtype is DType.bfloat16 and key.dtype is DType.bfloat16 and value.dtype is DType.bfloat16):
         return False
     b, h, s, hd = qs
-    return hd in _HEAD_SIZES and s % _SEQ_MULTIPLE == 0 and s > 0 and b * h <= 65535
+    return hd in _HEAD_SIZES and s > 0 and b * h <= 65535
 
 
 class FusedAttentionOp(Operation):
@@ -123,7 +122,7 @@ def fused_attention(query: Tensor, key: Tensor, value: Tensor, *, is_causal: boo
     if not fused_attention_applies(query, key, value):
         raise ValueError(
             "fused_attention covers bfloat16 [B, H, S, hd] tensors of one shape with hd in "
-            f"{_HEAD_SIZES} and S a multiple of {_SEQ_MULTIPLE}; got {tuple(query.shape)} "
+            f"{_HEAD_SIZES}; got {tuple(query.shape)} "
             f"{query.dtype}, {tuple(key.shape)} {key.dtype}, {tuple(value.shape)} {value.dtype}")
     if scale is None:
         scale = 1.0 / math.sqrt(int(query.shape[-1]))
