@@ -282,7 +282,7 @@ typedef struct nbk_gemm_desc {
    * bias gradient (the reduction of the cotangent to the bias' shape,
    * nabla/core/autograd/backward.py:31-54), taken from the B fragments the product has in
    * registers, so dy is read once.  bf16 operands, both row-contiguous (a_rs == b_cs == 1) and
-   * 16-byte aligned, K % 64 == 0, M % 8 == 0, N % 8 == 0, alpha 1, no bias / residual / activation;
+   * 16-byte aligned, M % 8 == 0, N % 8 == 0, alpha 1, no bias / residual / activation;
    * anything else is an error.  Row b of the sums belongs to batch index b of the launch, also with
    * two batch levels (b = outer * batch_inner + inner). */
   void* colsum;
@@ -301,7 +301,9 @@ typedef struct nbk_gemm_desc {
    * launch per pair, each adding itself to the result of the one before (plain products only:
    * no bias, residual, activation or alpha then). */
   int32_t n_terms;
-  int32_t reserved2;
+  /* 0, or the contraction length of the last batch member (of the last of every batch_inner members
+   * where there are two levels) in place of K: slices of one product along K need not divide it. */
+  int32_t k_last;
   nbk_gemm_term term[NBK_GEMM_MAX_TERMS];
 } nbk_gemm_desc;
 int nbk_gemm(const nbk_gemm_desc* d, void* stream);

@@ -184,6 +184,7 @@ class BoundPlan:
                     if rcs.dtype is not rc.dtype:
                         raise TypeError(f"matmul column sums are {rcs.dtype}, the product {rc.dtype}")
                     ptr_field(d, "colsum", rcs.buf, rcs.offset * rcs.dtype.size_in_bytes)
+                d.k_last = a.get("k_last", 0)
                 d.n_terms = 0
                 for ti, term in enumerate(a.get("terms") or ()):
                     ta, tb = term["a"], term["b"]

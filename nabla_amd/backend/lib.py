@@ -76,7 +76,7 @@ class GemmDesc(C.Structure):
         ("alpha", C.c_float), ("residual_op", C.c_int32),
         ("C_aux", C.c_void_p), ("aux_op", C.c_int32), ("reserved", C.c_int32),
         ("colsum", C.c_void_p),
-        ("n_terms", C.c_int32), ("reserved2", C.c_int32),
+        ("n_terms", C.c_int32), ("k_last", C.c_int32),
         ("term", GemmTerm * 4),
     ]
 

@@ -1912,7 +1912,7 @@ class Planner:
         if a_k_contiguous and N <= 32 and M >= 1024 and K % 64 == 0:
             return 1  # tall products with a few columns have a kernel that splits K by itself
         tiles = ((M + 127) // 128) * ((N + 127) // 128)
-        if rows_contiguous and 128 <= tiles <= 256 and K >= 4096 and K % 128 == 0:
+        if rows_contiguous and 128 <= tiles <= 256 and K >= 4096:
             # x^T dy with one workgroup per CU at most: every workgroup walks the same rows of
             # both operands at the same time, and on operands that come from memory (written
             # long before) the launch takes a third longer than on cached ones, whatever the
@@ -1920,8 +1920,20 @@ class Planner:
             # apart: 1024 x 4096 x 8192 113 -> 82 us, plus 10 us for the sum of the halves (four
             # slices: 67 us and 25)
             return 2
+        # The partial products and their sum cost 6 to 10 us, and a split product carries no
+        # epilogue.  Below 4096 the K loop of the 64 x 64 tile is as fast in one piece (512 x 512 x
+        # 1998: 12.4 us, 13.3 in two; 1800 x 1024 x 1024: 11.2 and 22) unless the launch has next to
+        # no workgroups, and so are 4096 deep ones with more than one such tile per CU (1800 x 1024
+        # x 4096: 35.7 and 36.5).  Others are split down to slices of 1024 (1000 x 1024 x 4096 34 ->
+        # 29 us in four), the longest and the smallest ones further (1024 x 1024 x 8192 65 -> 43 in
+        # eight, 256 x 256 x 4096 20 -> 13).
+        small = ((M + 63) // 64) * ((N + 63) // 64)
+        if (small > 32 and K < 4096) or (small > 256 and K < 8192):
+            return 1
+        least = 1024 if small > 32 and K < 8192 else 512
         ks = 1
-        while tiles * ks < 512 and tiles < 128 and K % (ks * 2 * 64) == 0 and K // (ks * 2) >= 512:
+        while tiles * ks < 512 and tiles < 128 and K // (ks * 2) >= least and \
+                (rows_contiguous or K % (ks * 2 * 64) == 0):
             ks *= 2
         return ks
 
@@ -1935,7 +1947,7 @@ class Planner:
             return None
         if not (pa[1] == 1 and pa[2] != 1 and pb[2] == 1 and pb[1] == N):
             return None
-        if M % 8 or N % 8 or M < 8 or N < 8 or K % (64 * ks) or K // ks <= 16:
+        if M % 8 or N % 8 or M < 8 or N < 8 or K // ks <= 16:
             return None
         if pa[2] % 8 or pa[2] >= 1 << 22 or N >= 1 << 22 or ra.offset % 8 or rb.offset % 8:
             return None
@@ -1970,15 +1982,16 @@ class Planner:
             self._emit(Step("gemm", [ra.buf, rb.buf] + self._epi_bufs(epi), writes,
                             dict(common, **epi, dst=dst, K=K, batch=1, a_bs=0, b_bs=0)))
             return
-        kc = K // ks
+        kc = -(-K // (64 * ks)) * 64  # (x^T dy: the last slice may be shorter)
+        k_last = K - (ks - 1) * kc if kc * ks != K else 0
         terminal = self._terminal(out)
         if terminal and not epi and self.group_siblings and \
-                self._join_sibling_product(ra, rb, common, kc, ks, key, dst):
+                self._join_sibling_product(ra, rb, common, K, ks, key, dst):
             return
         tmp = self._new_buf((ks, M, N), DType.float32)
         tref = ViewRef(tmp.id, 0, (ks, M, N), contiguous_strides((ks, M, N)), DType.float32)
         step = Step("gemm", [ra.buf, rb.buf], [tmp.id], dict(
-            common, dst=tref, K=kc, batch=ks, a_bs=kc * pa[2], b_bs=kc * pb[1]))
+            common, dst=tref, K=kc, k_last=k_last, k_all=K, batch=ks, a_bs=kc * pa[2], b_bs=kc * pb[1]))
         self._emit(step)
         red = Step("reduce_mid", [tmp.id], [dst.buf], dict(
             src=tref, dst=dst, outer=1, red=ks, inner=M * N, fn="sum"))
@@ -1987,7 +2000,7 @@ class Planner:
             # (more may join: _join_sibling_product)
             self._sibling_groups[id(step)] = [dict(off=rb.offset, key=key, reduce=red)]
 
-    def _join_sibling_product(self, ra: ViewRef, rb: ViewRef, common: dict, kc: int, ks: int, key,
+    def _join_sibling_product(self, ra: ViewRef, rb: ViewRef, common: dict, k_all: int, ks: int, key,
                               dst: ViewRef) -> bool:
         """A K-split product A^T B' whose left operand, shape and slices are those of a product
         among the launches just emitted (nothing but products since), with B' in the same buffer
@@ -2005,9 +2018,8 @@ class Planner:
                 continue
             h = st.attrs
             n = len(members)
-            ks_h = h["batch_inner"] if n > 1 else h["batch"]
             hb = h["b"]
-            same = (h["a"] == ra and h["M"] == M and h["N"] == N and h["K"] * ks_h == kc * ks and
+            same = (h["a"] == ra and h["M"] == M and h["N"] == N and h["k_all"] == k_all and
                     all(h[f] == common[f] for f in ("a_rs", "a_cs", "b_rs", "b_cs", "ldc", "alpha")) and
                     hb.buf == rb.buf and hb.dtype is rb.dtype and
                     (members[0]["key"] is not None) == (key is not None))
@@ -2026,16 +2038,17 @@ class Planner:
             # workgroups for two CUs, and fewer partial products go through memory (three
             # members of 64 tiles in the transformer block: 8, 4, 2 slices measured, two is best)
             tiles = -(-M // 128) * -(-N // 128) * (n + 1)
-            k_all, ks_new = kc * ks, 2
+            ks_new = 2
             while tiles * ks_new < 384 and ks_new < ks:
                 ks_new *= 2
-            ks = ks_new if (ks_new < ks and k_all % (ks_new * 64) == 0) else ks
-            kc = k_all // ks
+            ks = min(ks, ks_new)
+            kc = -(-k_all // (64 * ks)) * 64
+            k_last = k_all - (ks - 1) * kc if kc * ks != k_all else 0
             tmp = self.bufs[h["dst"].buf]
             tmp.numel = (n + 1) * ks * M * N
             tmp.shape = (n + 1, ks, M, N)
             h.pop("colsum_key", None)
-            h.update(K=kc, batch_inner=ks, a_bs2=kc * common["a_cs"], b_bs2=kc * common["b_rs"],
+            h.update(K=kc, k_last=k_last, batch_inner=ks, a_bs2=kc * common["a_cs"], b_bs2=kc * common["b_rs"],
                      c_bs2=M * N, a_bs=0, c_bs=ks * M * N)
             h.update(batch=(n + 1) * ks, b_bs=spacing,
                      b=ViewRef(hb.buf, order[0]["off"], hb.shape, hb.strides, hb.dtype),

@@ -2,7 +2,7 @@
 //
 // bf16 path (fp32 accumulate): v_mfma_f32_32x32x16_bf16.  A workgroup of four waves (2 x 2;
 // 128 x 128 tile) or eight (2 x 4; 256 x 256 tile) owns a BM x BN tile of C; K advances in
-// steps of 64 through two LDS buffers.
+// steps of 64 through two LDS buffers (64 x 64 tiles where the result is small).
 //   * an operand that is contiguous along K sits in LDS as [row][64 k], 128-byte rows whose
 //     eight 16-byte chunks are XOR-swizzled, so that the 16-byte fragment reads of the MFMA
 //     (32 consecutive rows, one chunk) are conflict-free without padding;
@@ -10,9 +10,10 @@
 //     backward products, and B of the forward product) sits in LDS k-major, [64 k][rows], and
 //     its MFMA fragments come out through the transposing read (ds_read_b64_tr_b16): the
 //     swap_axes of the backward GEMMs never touches memory or the vector ALU.
-// Two kernels share this layout idea: gemm_bf16_dl_kernel (aligned operands, K % 64 == 0) copies
-// global memory straight into LDS (global_load_lds_dwordx4); gemm_bf16_kernel takes every other
-// shape through guarded element-wise loads and registers.
+// Two kernels share this layout idea: gemm_bf16_dl_kernel (aligned operands, K % 64 == 0 or
+// both operands row-contiguous) copies global memory straight into LDS
+// (global_load_lds_dwordx4); gemm_bf16_kernel takes every other shape through guarded loads and
+// registers.
 // fp32 path: v_mfma_f32_32x32x2f32 with a 128 x 128 x 16 tile, operands kept
 // k-major in LDS.
 #include "nbk_common.h"
@@ -68,7 +69,15 @@ struct GemmArgs {
   struct Shallow { const void* A; const void* B; int64_t K, a_rs, a_cs, b_rs, b_cs; } shallow[2];
   struct Deep { const void* A; const void* B; int64_t K; } deep[2];
   int32_t n_shallow, n_deep;
+  int64_t k_last;        // contraction length of the last slice of a product split along K; 0: K
 };
+
+// Contraction length of this workgroup's batch member (the slice is the inner batch index where there
+// are two levels).
+__device__ __forceinline__ int64_t gemm_slice_k(const GemmArgs& g, int64_t bo, int64_t bi) {
+  const bool last = g.batch_inner > 1 ? bi == g.batch_inner - 1 : bo == (int64_t)gridDim.y - 1;
+  return g.k_last > 0 && last ? g.k_last : g.K;
+}
 
 __device__ __forceinline__ float gemm_act(float v, int act) {
   if (act == NBK_ACT_RELU) return fmaxf(v, 0.f);
@@ -122,10 +131,13 @@ __device__ __forceinline__ int swz(int row, int chunk) {
   return row * 8 + (chunk ^ (row & 7) ^ ((row >> 3) & 7));
 }
 
-// 16-byte guarded load of 8 consecutive bf16 along the unit-stride axis.
-__device__ __forceinline__ u32x4 ld8_bf16(const uint16_t* p, int64_t valid, bool vec) {
+// 16-byte guarded load of 8 consecutive bf16 along the unit-stride axis: one access, also where the
+// rows start at an odd element (global memory takes any alignment; eight 2-byte loads and their
+// packing bound every product with an odd row length, a vocabulary of no round size for one).
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+__device__ __forceinline__ u32x4 ld8_bf16(const uint16_t* p, int64_t valid) {
   u32x4 r = {0u, 0u, 0u, 0u};
-  if (valid >= 8 && vec) return *(const u32x4*)p;
+  if (valid >= 8) return *(const u32x4_any*)p;
   if (valid <= 0) return r;
   uint16_t t[8];
 #pragma unroll
@@ -190,7 +202,7 @@ struct TileLoader {
   u32x4 reg[NREG];
 
   __device__ __forceinline__ void load(const uint16_t* base, int64_t rs, int64_t cs, int64_t row0,
-                                       int64_t rows_total, int64_t k0, int64_t K, bool vec) {
+                                       int64_t rows_total, int64_t k0, int64_t K) {
     const int tid = threadIdx.x;
     if (KC) {
 #pragma unroll
@@ -198,7 +210,7 @@ struct TileLoader {
         const int t = tid + s * NT;
         const int row = t >> 3, c = t & 7;
         const int64_t gr = row0 + row, gk = k0 + c * 8;
-        if (gr < rows_total) reg[s] = ld8_bf16(base + gr * rs + gk, K - gk, vec);
+        if (gr < rows_total) reg[s] = ld8_bf16(base + gr * rs + gk, K - gk);
         else reg[s] = (u32x4){0u, 0u, 0u, 0u};
       }
     } else {
@@ -207,7 +219,7 @@ struct TileLoader {
         const int t = tid + s * NT;
         const int k = t / NC, c = t % NC;
         const int64_t gr = row0 + c * 8, gk = k0 + k;
-        if (gk < K) reg[s] = ld8_bf16(base + gk * cs + gr, rows_total - gr, vec);
+        if (gk < K) reg[s] = ld8_bf16(base + gk * cs + gr, rows_total - gr);
         else reg[s] = (u32x4){0u, 0u, 0u, 0u};
       }
     }
@@ -586,12 +598,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_kernel(const GemmArgs g) {
 
   TileLoader<BM, A_KC, NT> la;
   TileLoader<BN, B_KC, NT> lb;
-  const int64_t nk = (g.K + 63) / 64;
+  const int64_t K = gemm_slice_k(g, bo, bi);
+  const int64_t nk = (K + 63) / 64;
   // A is rows = m; for the loader a K-contiguous operand has (rs = row stride, k unit),
   // a row-contiguous one has (cs = k stride, row unit).
-  la.load(A, g.a_rs, g.a_cs, m0, g.M, 0, g.K, g.a_vec);
-  if constexpr (B_Q) lb.load_nf4((const uint8_t*)g.B, g.b_scales, g.b_block, nf4_table, g.b_cs, g.b_rs, n0, g.N, 0, g.K);
-  else lb.load(B, g.b_cs, g.b_rs, n0, g.N, 0, g.K, g.b_vec);
+  la.load(A, g.a_rs, g.a_cs, m0, g.M, 0, K);
+  if constexpr (B_Q) lb.load_nf4((const uint8_t*)g.B, g.b_scales, g.b_block, nf4_table, g.b_cs, g.b_rs, n0, g.N, 0, K);
+  else lb.load(B, g.b_cs, g.b_rs, n0, g.N, 0, K);
   la.store(gemm_lds);
   lb.store(gemm_lds + CA);
   __syncthreads();
@@ -687,9 +700,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_kernel(const GemmArgs g) {
   static_for<NFRAG>([&](auto r) { read_frag(std::integral_constant<int, 0>{}, r, gemm_lds, 0); });
   {
     const int64_t k1 = nk > 1 ? 64 : 0;  // a single-tile problem re-reads tile 0 (never stored)
-    la.load(A, g.a_rs, g.a_cs, m0, g.M, k1, g.K, g.a_vec);
-    if constexpr (B_Q) lb.load_nf4((const uint8_t*)g.B, g.b_scales, g.b_block, nf4_table, g.b_cs, g.b_rs, n0, g.N, k1, g.K);
-    else lb.load(B, g.b_cs, g.b_rs, n0, g.N, k1, g.K, g.b_vec);
+    la.load(A, g.a_rs, g.a_cs, m0, g.M, k1, K);
+    if constexpr (B_Q) lb.load_nf4((const uint8_t*)g.B, g.b_scales, g.b_block, nf4_table, g.b_cs, g.b_rs, n0, g.N, k1, K);
+    else lb.load(B, g.b_cs, g.b_rs, n0, g.N, k1, K);
   }
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
@@ -727,9 +740,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_kernel(const GemmArgs g) {
     // half of the MFMAs, barrier, first fragments of the next tile, the other half
     {
       const int64_t k2 = (kt + 2 < nk ? kt + 2 : nk - 1) * 64;
-      la.load(A, g.a_rs, g.a_cs, m0, g.M, k2, g.K, g.a_vec);
-      if constexpr (B_Q) lb.load_nf4((const uint8_t*)g.B, g.b_scales, g.b_block, nf4_table, g.b_cs, g.b_rs, n0, g.N, k2, g.K);
-      else lb.load(B, g.b_cs, g.b_rs, n0, g.N, k2, g.K, g.b_vec);
+      la.load(A, g.a_rs, g.a_cs, m0, g.M, k2, K);
+      if constexpr (B_Q) lb.load_nf4((const uint8_t*)g.B, g.b_scales, g.b_block, nf4_table, g.b_cs, g.b_rs, n0, g.N, k2, K);
+      else lb.load(B, g.b_cs, g.b_rs, n0, g.N, k2, K);
     }
     static_for<NMFMA / 2>([&](auto q) { mfma(S1{}, q); });
     {
@@ -801,8 +814,11 @@ __device__ __forceinline__ int dl_kc_xor(int row) {
 __device__ __forceinline__ int dl_seg_xor(int k) { return (k & 3) ^ (((k & 3) << 1) & 7); }
 // The 16x16x32 form reads k-rows k .. k + 3 and k + 8 .. k + 11 of one 32-byte segment in
 // half a wave: bit 3 of k joins the swizzle.
-template <bool MI16>
+// A k-row of 64 has four segments, two k-rows to a 256-byte window: bit 0 of k picks the half of the
+// window, and bits 1 and 3 tell the segments of a half apart.
+template <bool MI16, int ROWS>
 __device__ __forceinline__ int dl_seg_xor_of(int k) {
+  if constexpr (ROWS == 64) return ((k >> 1) & 1) | (((k >> 3) & 1) << 1);
   return MI16 ? dl_seg_xor(k) ^ ((k >> 3) & 1) : dl_seg_xor(k);
 }
 
@@ -815,6 +831,7 @@ struct DirectLoader {
   static constexpr int N = ROWS / (8 * NW);
   static constexpr int NC = ROWS / 8;
   static_assert(N >= 1 && N % 2 == 0, "instructions per wave");
+  static_assert(ROWS != 64 || MI16, "the swizzle of 64 rows is made for 16 x 16 x 32 fragments");
   int voff[N];         // byte offset of this lane's chunk from the tile's first element
   const char* base;    // operand + tile row offset (wave-uniform)
   int64_t kstep;       // bytes between consecutive K tiles (wave-uniform)
@@ -841,7 +858,7 @@ struct DirectLoader {
 #pragma unroll
       for (int j = 0; j < N; ++j) {
         const int l = (first + j) * 64 + lane;
-        const int k = l / NC, c = (l % NC) ^ (dl_seg_xor_of<MI16>(k) << 1);
+        const int k = l / NC, c = (l % NC) ^ (dl_seg_xor_of<MI16, ROWS>(k) << 1);
         const int64_t r = c * 8 < last ? c * 8 : last;
         voff[j] = (int)(k * cs * 2 + r * 2);
       }
@@ -868,7 +885,7 @@ struct DirectLoader {
       } else {
         const int64_t last = rows_total - 8 - row0;
         const int l = (first_ + j) * 64 + lane;
-        const int k = l / NC, c = (l % NC) ^ (dl_seg_xor_of<MI16>(k) << 1);
+        const int k = l / NC, c = (l % NC) ^ (dl_seg_xor_of<MI16, ROWS>(k) << 1);
         const int64_t r = c * 8 < last ? c * 8 : last;
         src = (const char*)(op + row0) + (k * cs * 2 + r * 2);
         there = k < kvalid;
@@ -949,11 +966,18 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g)
   // loop's are made), then A and B, then the deep pairs, which share the loop's lane offsets and
   // differ in the wave-uniform base only.  src_a(t) / src_b(t): where tile t starts in memory.
   // (tile numbers are 32-bit: the scalar unit compares those, 64-bit ones go through vector registers)
-  const int ns = g.n_shallow;
-  const int e0 = ns + (int)(g.K / 64);                                   // first tile past A and B
+  // Two row-contiguous operands take any K: what is left over a multiple of 64 (of this slice, where
+  // the product is split along K) is the first tile, like a shallow pair.
+  const int64_t K = gemm_slice_k(g, bo, bi);
+  const int k_over = !A_KC && !B_KC ? (int)(K & 63) : 0;
+  const int ns = k_over ? 1 : g.n_shallow;
+  const int e0 = ns + (int)(K / 64);                                     // first tile past A and B
   const int e1 = e0 + (g.n_deep > 0 ? (int)(g.deep[0].K / 64) : 0);      // ... past the first deep pair
   const int nk = e1 + (g.n_deep > 1 ? (int)(g.deep[1].K / 64) : 0);
-  if (ns > 0) {
+  if (k_over) {
+    LA::issue_tail(gemm_lds, A + (K - k_over) * g.a_cs, g.a_rs, g.a_cs, m0, g.M, k_over, wave, lane);
+    LB::issue_tail(gemm_lds + CA, B + (K - k_over) * g.b_rs, g.b_cs, g.b_rs, n0, g.N, k_over, wave, lane);
+  } else if (ns > 0) {
     const auto& t0 = g.shallow[0];
     LA::issue_tail(gemm_lds, (const uint16_t*)t0.A, t0.a_rs, t0.a_cs, m0, g.M, (int)t0.K, wave, lane);
     LB::issue_tail(gemm_lds + CA, (const uint16_t*)t0.B, t0.b_cs, t0.b_rs, n0, g.N, (int)t0.K, wave, lane);
@@ -1007,18 +1031,18 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g)
   int a_addr[TM], b_addr[TN];
   if constexpr (MI16) {
     const int p = lane & 15, q = lane >> 4;
-    const int kl = 8 * q + (p >> 2), sx = dl_seg_xor_of<true>(kl);
+    const int kl = 8 * q + (p >> 2), sxa = dl_seg_xor_of<true, BM>(kl), sxb = dl_seg_xor_of<true, BN>(kl);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int row = wm + i * 16 + p;
       if (A_KC) a_addr[i] = (row * 8 + (q ^ dl_kc_xor<true>(row))) * 16;
-      else a_addr[i] = kl * (BM * 2) + ((((wm >> 4) + i) ^ sx) * 32) + 8 * (p & 3);
+      else a_addr[i] = kl * (BM * 2) + ((((wm >> 4) + i) ^ sxa) * 32) + 8 * (p & 3);
     }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int row = wn + j * 16 + p;
       if (B_KC) b_addr[j] = (CA + row * 8 + (q ^ dl_kc_xor<true>(row))) * 16;
-      else b_addr[j] = CA * 16 + kl * (BN * 2) + ((((wn >> 4) + j) ^ sx) * 32) + 8 * (p & 3);
+      else b_addr[j] = CA * 16 + kl * (BN * 2) + ((((wn >> 4) + j) ^ sxb) * 32) + 8 * (p & 3);
     }
   } else {
     const int p = lane & 15, q = lane >> 4;
@@ -1487,6 +1511,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs g) {
   const float* A = (const float*)g.A + bo * g.a_bs + bi * g.a_bs2;
   const float* B = (const float*)g.B + bo * g.b_bs + bi * g.b_bs2;
   const int64_t c_off = bo * g.c_bs + bi * g.c_bs2;
+  const int64_t K = gemm_slice_k(g, bo, bi);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
   const int li = lane & 31, kg = lane >> 5;
@@ -1508,7 +1533,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs g) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int64_t gk = k0 + kk + e;
-        r[e] = (gr < rows_total && gk < g.K) ? P[gr * rs + gk] : 0.f;
+        r[e] = (gr < rows_total && gk < K) ? P[gr * rs + gk] : 0.f;
       }
     } else {
       // unit stride along rows: lane -> (k = tid/16, 8 consecutive rows)
@@ -1517,7 +1542,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs g) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int64_t gr = row0 + rr + e;
-        r[e] = (gr < rows_total && gk < g.K) ? P[gk * cs + gr] : 0.f;
+        r[e] = (gr < rows_total && gk < K) ? P[gk * cs + gr] : 0.f;
       }
     }
   };
@@ -1528,12 +1553,12 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs g) {
         const int row = tid >> 1, kk = (tid & 1) * 8;
         const int64_t gr = n0 + row, gk = k0 + kk;
         nf4_load8((const uint8_t*)g.B, g.b_scales, g.b_block, nf4_table, gr * g.b_cs + gk,
-                  gr < g.N ? g.K - gk : 0, r);
+                  gr < g.N ? K - gk : 0, r);
       } else {
         const int kk = tid >> 4, rr = (tid & 15) * 8;
         const int64_t gk = k0 + kk, gr = n0 + rr;
         nf4_load8((const uint8_t*)g.B, g.b_scales, g.b_block, nf4_table, gk * g.b_rs + gr,
-                  gk < g.K ? g.N - gr : 0, r);
+                  gk < K ? g.N - gr : 0, r);
       }
     } else {
       load_tile(B, g.b_cs, g.b_rs, n0, g.N, k0, B_KC, g.b_vec, r);
@@ -1551,7 +1576,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs g) {
     }
   };
 
-  const int64_t nk = (g.K + BK - 1) / BK;
+  const int64_t nk = (K + BK - 1) / BK;
   load_tile(A, g.a_rs, g.a_cs, m0, g.M, 0, A_KC, g.a_vec, ra);
   load_b(0, rb);
   store_tile(As[0], A_KC, ra);
@@ -1638,7 +1663,7 @@ __global__ __launch_bounds__(256) void gemm_f32_small_kernel(const GemmArgs g) {
   const bool m_ok = m < g.M, n_ok = n < g.N;
   const float* a_base = A_KC ? A + (m_ok ? m : 0) * g.a_rs : A + (m_ok ? m : 0);
   const float* b_base = B_KC ? B + (n_ok ? n : 0) * g.b_cs : B + (n_ok ? n : 0);
-  const int64_t K = g.K;
+  const int64_t K = gemm_slice_k(g, bo, bi);
   // k-steps of this wave: s = wave + 4 * i, covering k in [8 s, 8 s + 8)
   const int64_t n_steps = (K + 7) / 8;
   const int64_t my_steps = n_steps > wave ? (n_steps - wave + 3) / 4 : 0;
@@ -1858,6 +1883,8 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
               "gemm: residual_op %d", d->residual_op);
   a.res_mul = d->residual_op == NBK_RES_MUL;
   a.colsum = d->colsum;
+  NBK_REQUIRE(d->k_last >= 0 && (d->k_last == 0 || d->n_terms == 0), "gemm: k_last %d", d->k_last);
+  a.k_last = d->k_last;
   // K-contiguous when the stride along k is 1 (ties: a single row / column counts as K-contiguous)
   const bool akc = d->a_cs == 1;
   const bool bkc = d->b_rs == 1;
@@ -1883,7 +1910,7 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
   // (checked before any kernel is chosen: no path may take the product and drop the sums)
   NBK_REQUIRE(d->colsum == nullptr || (d->dtype_ab == NBK_BF16 && !akc && !bkc),
               "gemm: column sums need bf16 operands that are both row-contiguous (a_rs == b_cs == 1)");
-  if (!tail && d->dtype_ab == NBK_BF16 && d->N <= 32 && d->M >= 1024 && d->K >= 256 && d->K % 64 == 0 &&
+  if (!tail && d->k_last == 0 && d->dtype_ab == NBK_BF16 && d->N <= 32 && d->M >= 1024 && d->K >= 256 && d->K % 64 == 0 &&
       akc && a.a_vec && d->batch == 1 && d->bias == nullptr && d->residual == nullptr &&
       d->act == NBK_ACT_NONE && (bkc ? (bool)a.b_vec : (d->b_cs == 1 && d->N % 8 == 0 && a.b_vec))) {
     // 32 rows per workgroup, K split over its eight waves
@@ -1908,7 +1935,7 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
       return nbk_check_launch("gemm_skinny_n_kernel");
     }
   }
-  if (!tail && d->dtype_ab == NBK_BF16 && d->K <= 16 && akc && d->batch == 1 && d->N % 8 == 0 &&
+  if (!tail && d->k_last == 0 && d->dtype_ab == NBK_BF16 && d->K <= 16 && akc && d->batch == 1 && d->N % 8 == 0 &&
       d->ldc % 8 == 0 && ((uintptr_t)d->C & 15) == 0 && ((uintptr_t)d->residual & 15) == 0 &&
       (d->K == 16 ? a.a_vec : d->K == 8 && (d->a_rs % 8 == 0) && ((uintptr_t)d->A & 15) == 0)) {
     // (the vector path reads whole 16-byte pieces of A rows: K = 16 or 8)
@@ -1942,7 +1969,8 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
     // (the direct kernel keeps per-lane byte offsets within a tile in 32 bits: 256 rows or
     // 64 k-rows times the stride)
     const int64_t a_stride = akc ? d->a_rs : d->a_cs, b_stride = bkc ? d->b_cs : d->b_rs;
-    const bool fast = a.a_vec && a.b_vec && (d->K % 64 == 0) && (akc || d->M % 8 == 0) &&
+    const bool k_whole = d->K % 64 == 0 && d->k_last % 64 == 0;
+    const bool fast = a.a_vec && a.b_vec && (k_whole || (!akc && !bkc && !tail)) && (akc || d->M % 8 == 0) &&
                       (bkc || d->N % 8 == 0) && d->M >= 8 && d->N >= 8 &&
                       a_stride >= 0 && b_stride >= 0 && a_stride < (1 << 22) && b_stride < (1 << 22);
     if (tail) {
@@ -1992,12 +2020,20 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
         return rc;
       }
     }
+    // 64 x 64 tiles while two of them per CU hold the whole result: such a launch is bound by the
+    // latency of its K loop, not by the LDS reads a small tile repeats (a wave reads four fragments
+    // for four MFMAs, the 128 x 128 tile eight for sixteen).  Measured, 64 / 128: 1998 x 512 x 512
+    // 6.3 / 9.5 us, 512 x 512 x 1998 (x^T dy) 12.4 / 20.5, 1800 x 1024 x 1024 (464 small tiles) 11.2 /
+    // 14.4; past two per CU it turns: 1000 x 4096 x 1024 (1024 small tiles) 17.1 / 14.9.
+    constexpr int64_t SMALL_TILES = 512;
+    const int64_t small_tiles = ((d->M + 63) / 64) * ((d->N + 63) / 64) * d->batch;
     if (d->colsum != nullptr) {
       NBK_REQUIRE(fast && !akc && !bkc && d->bias == nullptr &&
                       d->residual == nullptr && d->act == NBK_ACT_NONE && d->alpha == 1.f,
                   "gemm: column sums go with a plain bf16 product of two row-contiguous, 16-byte "
-                  "aligned operands (K %% 64 == 0, M %% 8 == 0, N %% 8 == 0)");
-      return launch_bf16_dl_colsum<128, 128, 4>(a, d->batch, st);
+                  "aligned operands (M %% 8 == 0, N %% 8 == 0)");
+      return small_tiles <= SMALL_TILES ? launch_bf16_dl_colsum<64, 64, 4>(a, d->batch, st)
+                                        : launch_bf16_dl_colsum<128, 128, 4>(a, d->batch, st);
     }
     if (!fast) return launch_bf16<128, 128>(a, akc, bkc, d->batch, st);
     // 256 x 256 tiles run at about twice the rate of 128 x 128 ones per CU, one workgroup
@@ -2011,6 +2047,7 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
     // (eight waves on the big tile: 8-16 % faster than four on every shape measured)
     if (big_tiles * 10 >= rounds * cus * 6 && d->M >= 256 && d->N >= 256 && d->K > 128)
       return launch_bf16_dl<256, 256, 8, 1, true>(a, akc, bkc, d->batch, st);
+    if (small_tiles <= SMALL_TILES) return launch_bf16_dl<64, 64, 4, 1, true>(a, akc, bkc, d->batch, st);
     // (a 256 x 128 tile was measured and is no faster than 128 x 128 on mid-sized problems:
     // with one workgroup per CU a short K loop is bound by load latency, and two co-resident
     // 128 x 128 workgroups hide it better)

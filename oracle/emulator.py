@@ -302,8 +302,21 @@ def _gemm(a, mem):
     def mat(ref, bs, bs2, rs, cs, rows, cols):
         base = mem[ref.buf]
         return torch.as_strided(base, (bo, bi, rows, cols), (bs, bs2 if bi > 1 else 0, rs, cs), ref.offset)
-    A = mat(a["a"], a["a_bs"], a.get("a_bs2", 0), a["a_rs"], a["a_cs"], a["M"], a["K"]).float()
-    B = mat(a["b"], a["b_bs"], a.get("b_bs2", 0), a["b_rs"], a["b_cs"], a["K"], a["N"]).float()
+    def operand(ref, bs, bs2, rs, cs, rows, cols, k_axis):
+        k_last = a.get("k_last", 0)
+        if not k_last:
+            return mat(ref, bs, bs2, rs, cs, rows, cols).float()
+        full = torch.zeros((bo, bi, rows, cols))  # (the last slice of K is shorter: zeros behind it)
+        for zo in range(bo):
+            for zi in range(bi):
+                size = [rows, cols]
+                if (zi == bi - 1) if bi > 1 else (zo == bo - 1):
+                    size[k_axis] = k_last
+                at = ref.offset + zo * bs + (zi * bs2 if bi > 1 else 0)
+                full[zo, zi, :size[0], :size[1]] = torch.as_strided(mem[ref.buf], size, (rs, cs), at).float()
+        return full
+    A = operand(a["a"], a["a_bs"], a.get("a_bs2", 0), a["a_rs"], a["a_cs"], a["M"], a["K"], 1)
+    B = operand(a["b"], a["b_bs"], a.get("b_bs2", 0), a["b_rs"], a["b_cs"], a["K"], a["N"], 0)
     prod = torch.matmul(A.double(), B.double())
     for t in a.get("terms") or ():  # more operand pairs in the same accumulator (batch 1)
         At = torch.as_strided(mem[t["a"].buf], (a["M"], t["K"]), (t["a_rs"], t["a_cs"]), t["a"].offset)

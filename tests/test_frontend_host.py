@@ -1006,3 +1006,18 @@ def test_gelu_backward_recomputes_the_derivative_where_the_cotangent_is(emulator
     h = nb.grad(lambda t: nb.reduce_sum(nb.grad(lambda u: nb.reduce_sum(nb.gelu(u)))(t)))(T(x.astype(np.float32)))
     pdf = np.exp(-0.5 * x * x) / np.sqrt(2 * np.pi)
     np.testing.assert_allclose(h.numpy(), pdf * (2 - x * x), rtol=2e-4, atol=2e-5)
+
+
+def test_a_weight_gradient_over_unequal_slices(emulator):
+    """x^T dy over a number of rows that no split divides: the last slice is the shorter one."""
+    from nabla_amd.core import engine
+    rng = np.random.default_rng(8)
+    x, g = rng.integers(-3, 4, (1100, 16)).astype(np.float32), rng.integers(-3, 4, (1100, 24)).astype(np.float32)
+    bf = nb.DType.bfloat16
+    engine.clear_plan_cache()
+    got = nb.cast(nb.swap_axes(T(x, dtype=bf), 0, 1) @ T(g, dtype=bf), nb.DType.float32)
+    out = got.numpy()
+    st = [s.attrs for bp in engine._PLAN_CACHE.values() for s in bp.plan.steps if s.kind == "gemm"][0]
+    assert (st["batch"], st["K"], st["k_last"]) == (2, 576, 524)
+    np.testing.assert_array_equal(out, _bf16_round(x.T @ g))
+    engine.clear_plan_cache()
