@@ -18,6 +18,7 @@
 // k-major in LDS.
 #include "nbk_common.h"
 
+#include <type_traits>
 #include <utility>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -1492,26 +1493,21 @@ __global__ __launch_bounds__(SKN_WAVES * 64) void gemm_skinny_n_kernel(const Gem
   }
 }
 
-// ---------------------------------------------------------------------------- fp32
+// ------------------------------------------------------ fp32 against NF4-coded weights
 // 128 x 128 x 16 tile, LDS k-major ([k][rows], rows padded by 4 floats).
-template <bool A_KC, bool B_KC, bool B_Q = false>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs g) {
+template <bool B_KC>
+__global__ __launch_bounds__(256) void gemm_f32_nf4_kernel(const GemmArgs g) {
   constexpr int BM = 128, BN = 128, BK = 16, LD = 128 + 4;
   __shared__ float As[2][BK][LD];
   __shared__ float Bs[2][BK][LD];
-  __shared__ float nf4_table[B_Q ? 16 : 1];  // B_Q: B holds NF4 codes, g.b_scales the block scales
-  if (B_Q) {
-    if (threadIdx.x < 16) nf4_table[threadIdx.x] = nbk_nf4_levels[threadIdx.x];
-    __syncthreads();
-  }
+  __shared__ float nf4_table[16];  // (B holds NF4 codes, g.b_scales the block scales)
+  if (threadIdx.x < 16) nf4_table[threadIdx.x] = nbk_nf4_levels[threadIdx.x];
+  __syncthreads();
   int tm_i, tn_i;
   gemm_tile_coords(blockIdx.x, g.tiles_m, g.tiles_n, tm_i, tn_i);
   const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
-  const int64_t bo = (int64_t)blockIdx.y / g.batch_inner, bi = (int64_t)blockIdx.y % g.batch_inner;
-  const float* A = (const float*)g.A + bo * g.a_bs + bi * g.a_bs2;
-  const float* B = (const float*)g.B + bo * g.b_bs + bi * g.b_bs2;
-  const int64_t c_off = bo * g.c_bs + bi * g.c_bs2;
-  const int64_t K = gemm_slice_k(g, bo, bi);
+  const float* A = (const float*)g.A;
+  const int64_t K = g.K;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
   const int li = lane & 31, kg = lane >> 5;
@@ -1524,44 +1520,20 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs g) {
 
   // each lane stages 8 floats of A and 8 of B per k-tile (128*16 / 256)
   float ra[8], rb[8];
-  auto load_tile = [&](const float* P, int64_t rs, int64_t cs, int64_t row0, int64_t rows_total,
-                       int64_t k0, bool kc, bool vec, float* r) {
-    if (kc) {
-      // unit stride along k: lane -> (row = tid/2, 8 consecutive k)
-      const int row = tid >> 1, kk = (tid & 1) * 8;
-      const int64_t gr = row0 + row;
+  auto load_a = [&](int64_t k0, float* r) {
+    // lane -> (row = tid/2, 8 consecutive k)
+    const int64_t gr = m0 + (tid >> 1), gk = k0 + (tid & 1) * 8;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int64_t gk = k0 + kk + e;
-        r[e] = (gr < rows_total && gk < K) ? P[gr * rs + gk] : 0.f;
-      }
-    } else {
-      // unit stride along rows: lane -> (k = tid/16, 8 consecutive rows)
-      const int kk = tid >> 4, rr = (tid & 15) * 8;
-      const int64_t gk = k0 + kk;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int64_t gr = row0 + rr + e;
-        r[e] = (gr < rows_total && gk < K) ? P[gk * cs + gr] : 0.f;
-      }
-    }
+    for (int e = 0; e < 8; ++e) r[e] = (gr < g.M && gk + e < K) ? A[gr * g.a_rs + gk + e] : 0.f;
   };
   // B from NF4 codes: the same eight elements per lane, dequantised
   auto load_b = [&](int64_t k0, float* r) {
-    if constexpr (B_Q) {
-      if (B_KC) {
-        const int row = tid >> 1, kk = (tid & 1) * 8;
-        const int64_t gr = n0 + row, gk = k0 + kk;
-        nf4_load8((const uint8_t*)g.B, g.b_scales, g.b_block, nf4_table, gr * g.b_cs + gk,
-                  gr < g.N ? K - gk : 0, r);
-      } else {
-        const int kk = tid >> 4, rr = (tid & 15) * 8;
-        const int64_t gk = k0 + kk, gr = n0 + rr;
-        nf4_load8((const uint8_t*)g.B, g.b_scales, g.b_block, nf4_table, gk * g.b_rs + gr,
-                  gk < K ? g.N - gr : 0, r);
-      }
+    if (B_KC) {
+      const int64_t gr = n0 + (tid >> 1), gk = k0 + (tid & 1) * 8;
+      nf4_load8((const uint8_t*)g.B, g.b_scales, g.b_block, nf4_table, gr * g.b_cs + gk, gr < g.N ? K - gk : 0, r);
     } else {
-      load_tile(B, g.b_cs, g.b_rs, n0, g.N, k0, B_KC, g.b_vec, r);
+      const int64_t gk = k0 + (tid >> 4), gr = n0 + (tid & 15) * 8;
+      nf4_load8((const uint8_t*)g.B, g.b_scales, g.b_block, nf4_table, gk * g.b_rs + gr, gk < K ? g.N - gr : 0, r);
     }
   };
   auto store_tile = [&](float (*S)[LD], bool kc, const float* r) {
@@ -1577,16 +1549,16 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs g) {
   };
 
   const int64_t nk = (K + BK - 1) / BK;
-  load_tile(A, g.a_rs, g.a_cs, m0, g.M, 0, A_KC, g.a_vec, ra);
+  load_a(0, ra);
   load_b(0, rb);
-  store_tile(As[0], A_KC, ra);
+  store_tile(As[0], true, ra);
   store_tile(Bs[0], B_KC, rb);
   __syncthreads();
   for (int64_t kt = 0; kt < nk; ++kt) {
     const int cur = kt & 1;
     const bool more = kt + 1 < nk;
     if (more) {
-      load_tile(A, g.a_rs, g.a_cs, m0, g.M, (kt + 1) * BK, A_KC, g.a_vec, ra);
+      load_a((kt + 1) * BK, ra);
       load_b((kt + 1) * BK, rb);
     }
 #pragma unroll
@@ -1604,7 +1576,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs g) {
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
     }
     if (more) {
-      store_tile(As[cur ^ 1], A_KC, ra);
+      store_tile(As[cur ^ 1], true, ra);
       store_tile(Bs[cur ^ 1], B_KC, rb);
     }
     __syncthreads();
@@ -1616,116 +1588,191 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs g) {
     for (int j = 0; j < 2; ++j) {
       const int64_t col = n0 + wn + j * 32 + li;
       if (col >= g.N) continue;
-      float bv = g.bias ? ((const float*)g.bias)[col] : 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int64_t row = m0 + wm + i * 32 + (r >> 2) * 8 + kg * 4 + (r & 3);
-        if (row >= g.M) continue;
-        const int64_t idx = c_off + row * g.ldc + col;
-        float v, dv;
-        if (g.C2) {
-          gemm_act_pair<false>(acc[i][j][r] * g.alpha + bv, g.act, v, dv);
-          ((float*)g.C2)[idx] = dv;
-        } else {
-          v = gemm_act(acc[i][j][r] * g.alpha + bv, g.act);
-        }
-        if (g.residual) v = g.res_mul ? v * ((const float*)g.residual)[idx] : v + ((const float*)g.residual)[idx];
-        C[idx] = v;
+        if (row < g.M) C[row * g.ldc + col] = acc[i][j][r] * g.alpha;
       }
     }
 }
 
-// --------------------------------------------------------------- fp32, small problems
-// A product with only a handful of 128 x 128 tiles (the layers of a small MLP, a
-// classifier head) leaves most of the GPU idle and is bound by the latency of one
-// workgroup's K loop.  Here a workgroup owns a 32 x 32 tile of C, its four waves
-// split K between them (wave w takes k-steps w, w + 4, ...), operands go from global
-// memory straight to the MFMA registers in chunks of 8 k-steps that are all in
-// flight together while the previous chunk is multiplied, and the four partial
-// tiles meet in LDS.
-// Lane l of a v_mfma_f32_32x32x2f32 supplies A[row l % 32][k = l / 32] and
-// B[k = l / 32][col l % 32]; which two k values share an instruction is free as
-// long as A and B agree, so the lane with half h = l / 32 owns k = kb + 4h .. 4h + 3
-// of every 8-wide step and issues four instructions per step.
-template <bool A_KC, bool B_KC>
-__global__ __launch_bounds__(256) void gemm_f32_small_kernel(const GemmArgs g) {
-  constexpr int U = 8;  // k-steps (of 8) per chunk
-  __shared__ float part[4][32][33];
-  const int tn_i = blockIdx.x % g.tiles_n, tm_i = blockIdx.x / g.tiles_n;
-  const int64_t m0 = (int64_t)tm_i * 32, n0 = (int64_t)tn_i * 32;
+// --------------------------------------------------------------- fp32
+// Rows of one operand of a workgroup's K tile on their way from memory through registers to LDS, as
+// [row][k] with four floats of padding: a fragment is then one 16-byte LDS read of four k values of a
+// row, without bank conflicts for every pitch used (20, 36, 68 floats: 16 rows start on 16 different
+// groups of four banks).  The 16-byte chunks of a row are permuted by bits 4 and 5 of its number,
+// which spreads the transposed writes of a row-contiguous operand over all banks too.  Global
+// reads are 16-byte pieces at any 4-byte alignment.
+template <int N>
+using f32_piece = float __attribute__((ext_vector_type(N)));
+template <int N>
+using f32_piece_any = float __attribute__((ext_vector_type(N), aligned(4)));
+__device__ __forceinline__ int f32_at(int row, int chunk, int ld) { return row * ld + (chunk ^ (row >> 4 & 3)) * 4; }
+template <int ROWS, int BK, bool KC>
+struct F32Rows {
+  static constexpr int LD = BK + 4;
+  static constexpr int RB = ROWS >= 64 ? 4 : 2;  // row-contiguous operand: blocks of RB rows x 2 k
+  static constexpr int V = KC ? 4 : RB, Q = KC ? 1 : 2;  // a piece: Q accesses of V floats
+  static constexpr int PIECES = ROWS * BK / 256 / (V * Q);
+  static_assert(PIECES >= 1, "at least one piece per lane");
+  f32_piece<V> r[2][PIECES][Q];  // two K tiles in flight
+
+  __device__ static __forceinline__ void place(int p, int& row, int& kk) {
+    const int idx = (int)threadIdx.x + 256 * p;
+    if constexpr (KC) {
+      row = idx / (BK / 4);
+      kk = idx % (BK / 4) * 4;
+    } else {
+      row = idx % (ROWS / RB) * RB;
+      kk = idx / (ROWS / RB) * 2;
+    }
+  }
+  // `stride`: between rows (KC) or between k (row-contiguous).  Rows past the end repeat the last
+  // one (their results are not stored), k past the end reads as zero.
+  template <int SET>
+  __device__ __forceinline__ void load(const float* P, int64_t stride, int64_t row0, int64_t rows, int64_t k0, int64_t K) {
+    if (k0 + BK <= K && (KC || row0 + ROWS <= rows)) {
+#pragma unroll
+      for (int p = 0; p < PIECES; ++p) {
+        int row, kk;
+        place(p, row, kk);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          const float* src = KC ? P + min(row0 + row, rows - 1) * stride + k0 + kk : P + (k0 + kk + q) * stride + row0 + row;
+          r[SET][p][q] = *(const f32_piece_any<V>*)src;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int p = 0; p < PIECES; ++p) {
+        int row, kk;
+        place(p, row, kk);
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+#pragma unroll
+          for (int e = 0; e < V; ++e) {
+            const int64_t k = k0 + kk + (KC ? e : q), m = min(row0 + row + (KC ? 0 : e), rows - 1);
+            r[SET][p][q][e] = k < K ? P[KC ? m * stride + k : k * stride + m] : 0.f;
+          }
+      }
+    }
+  }
+  template <int SET>
+  __device__ __forceinline__ void store(float* S) {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      int row, kk;
+      place(p, row, kk);
+      // (the pieces stay as they were loaded until here: pairing two k of a row any earlier would
+      // wait for the loads right behind their request)
+#pragma unroll
+      for (int q = 0; q < Q; ++q) asm volatile("" : "+v"(r[SET][p][q]));
+      if constexpr (KC) {
+        *(f32_piece<4>*)(S + f32_at(row, kk >> 2, LD)) = r[SET][p][0];
+      } else {
+#pragma unroll
+        for (int e = 0; e < RB; ++e)
+          *(float2*)(S + f32_at(row + e, kk >> 2, LD) + (kk & 2)) = make_float2(r[SET][p][0][e], r[SET][p][1][e]);
+      }
+    }
+  }
+};
+
+// A workgroup of four waves owns a tile of WM IM x WN IN fragments of 32 x 32; WK waves share a
+// fragment and split every K tile of it (KS steps of 8 each), their sums meet in LDS at the end.
+// Bound by the fp32 matrix rate (157 TFLOP/s: 64 cycles an instruction, so that one 16-byte read per
+// operand for four of them costs nothing) where the tiles fill the chip, else by the length of a
+// workgroup's K loop: hence a choice of tiles down to 32 x 32.  Two K tiles are requested ahead: one
+// workgroup's 16 instructions a tile are shorter than a trip to memory.
+// Lane l of a v_mfma_f32_32x32x2f32 supplies A[row l % 32][k = l / 32] and B[k = l / 32][col l % 32];
+// which two k values share an instruction is free as long as A and B agree, so the lane with half
+// h = l / 32 owns k = 8 s + 4 h .. + 3 of step s and issues four instructions per step.  The smaller
+// tiles sum a product in four chains (waves x accumulators), the largest in one.
+// Before / after (guarded 128 x 128 tiles without loads ahead, or 32 x 32 ones straight from memory
+// below 33 of those): 512 x 2048 x 1024 as x^T dy 150 -> 43 us, 1024 x 2048 x 512 84 -> 32 (68
+// TFLOP/s), 32 x (256 x 64 x 256) 45 -> 10, 8192 x 4096 x 1024 947 -> 654 (105 TFLOP/s), 1024 x 512
+// x 512 14.4 -> 12.2, 128 x 256 x 784 16.4 -> 11.6.
+template <int WM, int WN, int WK, int IM, int IN, int KS, bool A_KC, bool B_KC>
+__global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs g) {
+  static_assert(WM * WN * WK == 4 && (WK == 1 || WK == 4), "four waves, together or apart");
+  constexpr int BM = 32 * WM * IM, BN = 32 * WN * IN, BK = 8 * KS * WK, LD = BK + 4;
+  constexpr int NA = IM * IN == 1 ? 4 / WK : 1;
+  __shared__ __align__(16) float lds[2 * (BM + BN) * LD];
+  static_assert(WK == 1 || 4 * 16 * 64 <= 2 * (BM + BN) * LD, "the partial sums fit");
+  int tm_i, tn_i;
+  gemm_tile_coords(blockIdx.x, g.tiles_m, g.tiles_n, tm_i, tn_i);
+  const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
   const int64_t bo = (int64_t)blockIdx.y / g.batch_inner, bi = (int64_t)blockIdx.y % g.batch_inner;
   const float* A = (const float*)g.A + bo * g.a_bs + bi * g.a_bs2;
   const float* B = (const float*)g.B + bo * g.b_bs + bi * g.b_bs2;
   const int64_t c_off = bo * g.c_bs + bi * g.c_bs2;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int li = lane & 31, h = lane >> 5;
-  const int64_t m = m0 + li, n = n0 + li;
-  const bool m_ok = m < g.M, n_ok = n < g.N;
-  const float* a_base = A_KC ? A + (m_ok ? m : 0) * g.a_rs : A + (m_ok ? m : 0);
-  const float* b_base = B_KC ? B + (n_ok ? n : 0) * g.b_cs : B + (n_ok ? n : 0);
   const int64_t K = gemm_slice_k(g, bo, bi);
-  // k-steps of this wave: s = wave + 4 * i, covering k in [8 s, 8 s + 8)
-  const int64_t n_steps = (K + 7) / 8;
-  const int64_t my_steps = n_steps > wave ? (n_steps - wave + 3) / 4 : 0;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wk = wave % WK, wn = wave / WK % WN * 32 * IN, wm = wave / (WK * WN) * 32 * IM;
+  const int li = lane & 31, h = lane >> 5;
+  const int64_t a_stride = A_KC ? g.a_rs : g.a_cs, b_stride = B_KC ? g.b_cs : g.b_rs;
 
-  auto fetch = [&](int64_t i, float* a, float* b) {
-    const int64_t kb = (wave + 4 * i) * 8 + 4 * h;
-    const bool in = i < my_steps;
-    if (A_KC) {
-      if (in && m_ok && g.a_vec && kb + 3 < K) {
-        const float4 v = *(const float4*)(a_base + kb);
-        a[0] = v.x; a[1] = v.y; a[2] = v.z; a[3] = v.w;
-      } else {
+  f32x16 acc[NA][IM][IN];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) a[j] = (in && m_ok && kb + j < K) ? a_base[kb + j] : 0.f;
-      }
-    } else {
+  for (int n = 0; n < NA; ++n)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) a[j] = (in && m_ok && kb + j < K) ? a_base[(kb + j) * g.a_cs] : 0.f;
-    }
-    if (B_KC) {
-      if (in && n_ok && g.b_vec && kb + 3 < K) {
-        const float4 v = *(const float4*)(b_base + kb);
-        b[0] = v.x; b[1] = v.y; b[2] = v.z; b[3] = v.w;
-      } else {
+    for (int i = 0; i < IM; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = (in && n_ok && kb + j < K) ? b_base[kb + j] : 0.f;
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = (in && n_ok && kb + j < K) ? b_base[(kb + j) * g.b_rs] : 0.f;
-    }
+      for (int j = 0; j < IN; ++j) acc[n][i][j] = (f32x16)(0.f);
+
+  F32Rows<BM, BK, A_KC> la;
+  F32Rows<BN, BK, B_KC> lb;
+  const int64_t nk = (K + BK - 1) / BK;
+  auto load = [&](auto set, int64_t kt) {
+    la.template load<set.value>(A, a_stride, m0, g.M, kt * BK, K);
+    lb.template load<set.value>(B, b_stride, n0, g.N, kt * BK, K);
   };
-
-  f32x16 acc = (f32x16)(0.f);
-  float ca[U][4], cb[U][4], na[U][4], nb[U][4];
+  auto store = [&](auto set) {
+    float* S = lds + set.value * (BM + BN) * LD;
+    la.template store<set.value>(S);
+    lb.template store<set.value>(S + BM * LD);
+  };
+  auto tile = [&](auto cur, auto next, int64_t kt) {
+    if (kt + 2 < nk) load(cur, kt + 2);  // (its registers went to LDS an iteration ago)
+    const float* As = lds + cur.value * (BM + BN) * LD;
+    const float* Bs = As + BM * LD;
 #pragma unroll
-  for (int u = 0; u < U; ++u) fetch(u, ca[u], cb[u]);
-  for (int64_t c0 = 0; c0 < my_steps; c0 += U) {
+    for (int s = 0; s < KS; ++s) {
+      f32x4 fa[IM], fb[IN];
 #pragma unroll
-    for (int u = 0; u < U; ++u) fetch(c0 + U + u, na[u], nb[u]);
+      for (int i = 0; i < IM; ++i) fa[i] = *(const f32x4*)(As + f32_at(wm + i * 32 + li, (wk * KS + s) * 2 + h, LD));
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+      for (int j = 0; j < IN; ++j) fb[j] = *(const f32x4*)(Bs + f32_at(wn + j * 32 + li, (wk * KS + s) * 2 + h, LD));
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ca[u][j], cb[u][j], acc, 0, 0, 0);
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+        for (int i = 0; i < IM; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) { ca[u][j] = na[u][j]; cb[u][j] = nb[u][j]; }
-  }
-  // D register r of lane (col li, half h) is row (r / 4) * 8 + h * 4 + r % 4
-#pragma unroll
-  for (int r = 0; r < 16; ++r) part[wave][(r >> 2) * 8 + h * 4 + (r & 3)][li] = acc[r];
+          for (int j = 0; j < IN; ++j)
+            acc[e % NA][i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][e], fb[j][e], acc[e % NA][i][j], 0, 0, 0);
+    }
+    if (kt + 1 < nk) store(next);
+    __syncthreads();
+  };
+  const std::integral_constant<int, 0> s0{};
+  const std::integral_constant<int, 1> s1{};
+  load(s0, 0);
+  if (nk > 1) load(s1, 1);
+  store(s0);
   __syncthreads();
+  for (int64_t kt = 0; kt < nk; kt += 2) {
+    tile(s0, s1, kt);
+    if (kt + 1 < nk) tile(s1, s0, kt + 1);
+  }
+
+  // D register r of lane (col li, half h) is row (r / 4) * 8 + h * 4 + r % 4
   float* C = (float*)g.C;
-  for (int e = threadIdx.x; e < 32 * 32; e += 256) {
-    const int r = e >> 5, c = e & 31;
-    const int64_t row = m0 + r, col = n0 + c;
-    if (row >= g.M || col >= g.N) continue;
-    float v = (part[0][r][c] + part[1][r][c]) + (part[2][r][c] + part[3][r][c]);
+  auto put = [&](int i, int j, int r, float sum) {
+    const int64_t row = m0 + wm + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3), col = n0 + wn + j * 32 + li;
+    if (row >= g.M || col >= g.N) return;
     const int64_t idx = c_off + row * g.ldc + col;
-    const float x = v * g.alpha + (g.bias ? ((const float*)g.bias)[col] : 0.f);
+    const float x = sum * g.alpha + (g.bias ? ((const float*)g.bias)[col] : 0.f);
+    float v;
     if (g.C2) {
       float dv;
       gemm_act_pair<false>(x, g.act, v, dv);
@@ -1735,10 +1782,33 @@ __global__ __launch_bounds__(256) void gemm_f32_small_kernel(const GemmArgs g) {
     }
     if (g.residual) v = g.res_mul ? v * ((const float*)g.residual)[idx] : v + ((const float*)g.residual)[idx];
     C[idx] = v;
+  };
+  auto chains = [&](int i, int j, int r) {
+    if constexpr (NA == 4) return (acc[0][i][j][r] + acc[1][i][j][r]) + (acc[2][i][j][r] + acc[3][i][j][r]);
+    else return acc[0][i][j][r];
+  };
+  if constexpr (WK == 1) {
+#pragma unroll
+    for (int i = 0; i < IM; ++i)
+#pragma unroll
+      for (int j = 0; j < IN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) put(i, j, r, chains(i, j, r));
+  } else {
+    // (every read of the last K tile lies before its barrier) each of the WK waves sums its share
+    // of the fragment's registers
+#pragma unroll
+    for (int r = 0; r < 16; ++r) lds[(wave * 16 + r) * 64 + lane] = chains(0, 0, r);
+    __syncthreads();
+    const float* part = lds + (wave - wk) * 16 * 64 + lane;
+#pragma unroll
+    for (int q = 0; q < 16 / WK; ++q) {
+      const int r = wk * (16 / WK) + q;
+      put(0, 0, r, (part[r * 64] + part[(16 + r) * 64]) + (part[(32 + r) * 64] + part[(48 + r) * 64]));
+    }
   }
 }
 
-// ------------------------------------------------------------------------- dispatch
 template <int BM, int BN, int NW = 4>
 static int launch_bf16(const GemmArgs& a, bool akc, bool bkc, int64_t batch, hipStream_t st) {
   GemmArgs g = a;
@@ -1834,6 +1904,22 @@ static int launch_bf16_dl_colsum(const GemmArgs& a, int64_t batch, hipStream_t s
   }
   hipLaunchKernelGGL(kern, grid, dim3(NW * 64), lds, st, g);
   return nbk_check_launch("gemm_bf16_dl_kernel (column sums)");
+}
+
+template <int WM, int WN, int WK, int IM, int IN, int KS>
+static int launch_f32(const GemmArgs& args, bool akc, bool bkc, int64_t batch, hipStream_t st) {
+  constexpr int BM = 32 * WM * IM, BN = 32 * WN * IN;
+  GemmArgs a = args;
+  const int64_t tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
+  NBK_REQUIRE(tiles_m * tiles_n <= 0x7fffffffLL, "gemm: launch too large");
+  a.tiles_m = (int)tiles_m;
+  a.tiles_n = (int)tiles_n;
+  const dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch);
+  if (akc && bkc) hipLaunchKernelGGL((gemm_f32_kernel<WM, WN, WK, IM, IN, KS, true, true>), grid, dim3(256), 0, st, a);
+  else if (akc) hipLaunchKernelGGL((gemm_f32_kernel<WM, WN, WK, IM, IN, KS, true, false>), grid, dim3(256), 0, st, a);
+  else if (bkc) hipLaunchKernelGGL((gemm_f32_kernel<WM, WN, WK, IM, IN, KS, false, true>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((gemm_f32_kernel<WM, WN, WK, IM, IN, KS, false, false>), grid, dim3(256), 0, st, a);
+  return nbk_check_launch("gemm_f32_kernel");
 }
 
 extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
@@ -2056,25 +2142,16 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
     return !(akc && bkc) ? launch_bf16_dl<128, 128, 4, 1, true>(a, akc, bkc, d->batch, st)
                          : launch_bf16_dl<128, 128, 4, 1, false>(a, akc, bkc, d->batch, st);
   }
-  a.tiles_m = (int)((d->M + 127) / 128);
-  a.tiles_n = (int)((d->N + 127) / 128);
-  if ((int64_t)a.tiles_m * a.tiles_n * d->batch <= 32) {
-    // too few big tiles to occupy the GPU: 32 x 32 tiles with K split inside the workgroup
-    a.tiles_m = (int)((d->M + 31) / 32);
-    a.tiles_n = (int)((d->N + 31) / 32);
-    dim3 sgrid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)d->batch);
-    if (akc && bkc) hipLaunchKernelGGL((gemm_f32_small_kernel<true, true>), sgrid, dim3(256), 0, st, a);
-    else if (akc) hipLaunchKernelGGL((gemm_f32_small_kernel<true, false>), sgrid, dim3(256), 0, st, a);
-    else if (bkc) hipLaunchKernelGGL((gemm_f32_small_kernel<false, true>), sgrid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((gemm_f32_small_kernel<false, false>), sgrid, dim3(256), 0, st, a);
-    return nbk_check_launch("gemm_f32_small_kernel");
-  }
-  dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)d->batch);
-  if (akc && bkc) hipLaunchKernelGGL((gemm_f32_kernel<true, true>), grid, dim3(256), 0, st, a);
-  else if (akc) hipLaunchKernelGGL((gemm_f32_kernel<true, false>), grid, dim3(256), 0, st, a);
-  else if (bkc) hipLaunchKernelGGL((gemm_f32_kernel<false, true>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((gemm_f32_kernel<false, false>), grid, dim3(256), 0, st, a);
-  return nbk_check_launch("gemm_f32_kernel");
+  // The largest tile that still gives every CU two workgroups: below that the K loop of one workgroup
+  // is what a launch waits for, and the more waves share a CU the less of it shows.  Measured, us on
+  // 128 x 128 / 64 x 64 / 32 x 32 tiles: 8192 x 4096 x 1024 (2048 large tiles) 654 / 746 / 841,
+  // 4096 x 1024 x 1024 (256; 1024 of 64) 120 / 107 / 115, 1024 x 2048 x 512 (512 of 64) 60 / 32 / 36,
+  // 512 x 2048 x 1024 as x^T dy (256 of 64) 118 / 46 / 43, 1024 x 512 x 2048 (128) 190 / 61 / 34,
+  // 128 x 256 x 784 (8) 80 / 28 / 12.
+  auto tiles = [&](int64_t edge) { return ((d->M + edge - 1) / edge) * ((d->N + edge - 1) / edge) * d->batch; };
+  if (tiles(128) >= 512) return launch_f32<2, 2, 1, 2, 2, 2>(a, akc, bkc, d->batch, st);
+  if (tiles(64) >= 512) return launch_f32<2, 2, 1, 1, 1, 4>(a, akc, bkc, d->batch, st);
+  return launch_f32<1, 1, 4, 1, 1, 2>(a, akc, bkc, d->batch, st);
 }
 
 // ------------------------------------------------------------------ NF4-coded weights
@@ -2110,9 +2187,9 @@ extern "C" int nbk_gemm_nf4(const nbk_gemm_nf4_desc* d, void* stream) {
   hipStream_t st = (hipStream_t)stream;
   const bool bkc = d->transpose_w != 0;
   if (d->dtype == NBK_F32) {
-    if (bkc) hipLaunchKernelGGL((gemm_f32_kernel<true, true, true>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((gemm_f32_kernel<true, false, true>), grid, dim3(256), 0, st, a);
-    return nbk_check_launch("gemm_f32_kernel (nf4)");
+    if (bkc) hipLaunchKernelGGL((gemm_f32_nf4_kernel<true>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((gemm_f32_nf4_kernel<false>), grid, dim3(256), 0, st, a);
+    return nbk_check_launch("gemm_f32_nf4_kernel");
   }
   const size_t pipe = 2 * (size_t)(TileGeom<128, true>::CHUNKS +
                                    (bkc ? TileGeom<128, true>::CHUNKS : TileGeom<128, false>::CHUNKS)) * 16;
