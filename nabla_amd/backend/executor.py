@@ -215,6 +215,10 @@ class BoundPlan:
                 d.transpose_w = 1 if a["transpose"] else 0
                 d.dtype = rx.dtype.abi
                 d.alpha = 1.0
+                ws = a.get("workspace")
+                if ws is not None:
+                    ptr_field(d, "workspace", ws.buf, 0)
+                    d.workspace_bytes = a["workspace_bytes"]
                 self.calls.append((L.nbk_gemm_nf4, [C.byref(d)], patches, d))
             elif k in ("conv2d", "conv2d_dgrad", "conv2d_wgrad"):
                 d = lib.ConvDesc()

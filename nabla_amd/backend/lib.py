@@ -87,6 +87,7 @@ class GemmNf4Desc(C.Structure):
         ("M", C.c_int64), ("w_rows", C.c_int64), ("w_cols", C.c_int64),
         ("lda", C.c_int64), ("ldc", C.c_int64),
         ("block", C.c_int32), ("transpose_w", C.c_int32), ("dtype", C.c_int32), ("alpha", C.c_float),
+        ("workspace", C.c_void_p), ("workspace_bytes", C.c_int64),
     ]
 
 

@@ -1459,10 +1459,18 @@ class Planner:
             x, codes, scales = (self._contig(i) for i in n.inputs)
             dst = self._alloc_value(out)
             kdim = n.inputs[0].shape[-1]
-            self._emit(Step("gemm_nf4", [x.buf, codes.buf, scales.buf], [dst.buf], dict(
-                x=x, codes=codes, scales=scales, dst=dst, M=_numel(n.inputs[0].shape[:-1]), K=kdim,
-                N=out.shape[-1], w_shape=n.attrs["w_shape"], block=n.attrs["block"],
-                transpose=n.attrs["transpose"])))
+            writes = [dst.buf]
+            attrs = dict(x=x, codes=codes, scales=scales, dst=dst, M=_numel(n.inputs[0].shape[:-1]), K=kdim,
+                         N=out.shape[-1], w_shape=n.attrs["w_shape"], block=n.attrs["block"],
+                         transpose=n.attrs["transpose"])
+            if kdim >= 128:
+                # room for the weight of this one product, decoded (the launch's rule: nbk_gemm_nf4)
+                shape = tuple(n.attrs["w_shape"])
+                wbuf = self._new_buf(shape, out.dtype)
+                attrs["workspace"] = ViewRef(wbuf.id, 0, shape, contiguous_strides(shape), out.dtype)
+                attrs["workspace_bytes"] = _numel(shape) * out.dtype.size_in_bytes
+                writes.append(wbuf.id)
+            self._emit(Step("gemm_nf4", [x.buf, codes.buf, scales.buf], writes, attrs))
         elif k in ("attention", "attention_bwd"):
             self._lower_attention(n)
         elif k in ("maxpool2d", "maxpool2d_bwd", "avgpool2d", "avgpool2d_bwd"):

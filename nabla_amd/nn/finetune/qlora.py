@@ -8,9 +8,9 @@ the sixteen NF4 levels (18-38) after division by that maximum (``indices``, one 
 the device.
 
 ``qlora_linear`` does not rebuild the dense weight where it can avoid it: with a bfloat16 or
-float32 compute type and a weight whose width is a multiple of 8 the codes are the B operand of
-the product itself -- the GEMM reads one byte per weight, looks the level up, applies the block
-scale and feeds the matrix cores (``matmul_nf4``).  Other cases dequantise first with a gather
+float32 compute type and a weight whose width is a multiple of 8 the product takes the codes
+(``matmul_nf4``: a short contraction looks the levels up while it multiplies, a longer one decodes
+the weight into scratch memory that the next launch reuses).  Other cases dequantise first with a gather
 and one row program.
 """
 from __future__ import annotations

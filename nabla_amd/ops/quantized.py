@@ -2,8 +2,8 @@
 
 ``dequantize_nf4`` followed by ``matmul`` (nabla/nn/finetune/qlora.py:77-113) builds the dense
 weight first: a gather, a row program and a tensor of the weight's full size, every step.
-``matmul_nf4`` is that pair as one op whose kernel takes the codes as the B operand of the
-product (one byte per weight from memory, level lookup and block scale on the way into LDS).  The
+``matmul_nf4`` is that pair as one op that takes the codes: a short contraction looks the levels up
+on the way into LDS, a longer one decodes the weight into scratch memory of that launch first.  The
 coded weight is data, not a parameter: the VJP returns the input gradient only, which is the same
 kernel on the transposed weight.
 """
