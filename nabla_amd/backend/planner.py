@@ -1946,6 +1946,15 @@ class Planner:
         return ks
 
     @staticmethod
+    def _slices(K: int, ks: int) -> tuple[int, int, int]:
+        """(slices, length of a slice, length of the last one) for ``K`` cut into about ``ks`` whole
+        numbers of 64; rounding a slice up can leave fewer of them (8200 in sixteen: fifteen of
+        576).  The last length is 0 where all are equal, and 1 to a slice's length - 1 otherwise."""
+        kc = -(-K // (64 * ks)) * 64
+        ks = -(-K // kc)
+        return ks, kc, K - (ks - 1) * kc if kc * ks != K else 0
+
+    @staticmethod
     def _colsum_key(ra: ViewRef, rb: ViewRef, pa, pb, M: int, N: int, K: int, ks: int, epi: dict):
         """What a deferred column sum must name to ride on this product (one launch, or ``ks``
         slices of K): the right operand is a whole row-major [K, N] bf16 matrix, the left one is
@@ -1979,6 +1988,8 @@ class Planner:
         common["alpha"] = epi.get("alpha", 1.0)
         if ks > 1 and set(epi) - {"alpha"}:
             ks = 1  # (only a scale survives the split: it goes on the partial products)
+        if ks > 1:
+            ks, kc, k_last = self._slices(K, ks)  # (x^T dy: the last slice may be shorter)
         key = self._colsum_key(ra, rb, pa, pb, M, N, K, ks, epi) if self.fold_column_sums else None
         if key is not None:
             common["colsum_key"] = key
@@ -1990,8 +2001,6 @@ class Planner:
             self._emit(Step("gemm", [ra.buf, rb.buf] + self._epi_bufs(epi), writes,
                             dict(common, **epi, dst=dst, K=K, batch=1, a_bs=0, b_bs=0)))
             return
-        kc = -(-K // (64 * ks)) * 64  # (x^T dy: the last slice may be shorter)
-        k_last = K - (ks - 1) * kc if kc * ks != K else 0
         terminal = self._terminal(out)
         if terminal and not epi and self.group_siblings and \
                 self._join_sibling_product(ra, rb, common, K, ks, key, dst):
@@ -2049,9 +2058,7 @@ class Planner:
             ks_new = 2
             while tiles * ks_new < 384 and ks_new < ks:
                 ks_new *= 2
-            ks = min(ks, ks_new)
-            kc = -(-k_all // (64 * ks)) * 64
-            k_last = k_all - (ks - 1) * kc if kc * ks != k_all else 0
+            ks, kc, k_last = self._slices(k_all, min(ks, ks_new))
             tmp = self.bufs[h["dst"].buf]
             tmp.numel = (n + 1) * ks * M * N
             tmp.shape = (n + 1, ks, M, N)
