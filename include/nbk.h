@@ -301,8 +301,9 @@ typedef struct nbk_gemm_desc {
    * launch per pair, each adding itself to the result of the one before (plain products only:
    * no bias, residual, activation or alpha then). */
   int32_t n_terms;
-  /* 0, or the contraction length of the last batch member (of the last of every batch_inner members
-   * where there are two levels) in place of K: slices of one product along K need not divide it. */
+  /* 0, or the contraction length (at most K) of the last batch member (of the last of every
+   * batch_inner members where there are two levels) in place of K: slices of one product along K need
+   * not divide it. */
   int32_t k_last;
   nbk_gemm_term term[NBK_GEMM_MAX_TERMS];
 } nbk_gemm_desc;

@@ -1969,7 +1969,9 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
               "gemm: residual_op %d", d->residual_op);
   a.res_mul = d->residual_op == NBK_RES_MUL;
   a.colsum = d->colsum;
-  NBK_REQUIRE(d->k_last >= 0 && (d->k_last == 0 || d->n_terms == 0), "gemm: k_last %d", d->k_last);
+  // (a slice longer than K would read behind both operands)
+  NBK_REQUIRE(d->k_last >= 0 && d->k_last <= d->K && (d->k_last == 0 || d->n_terms == 0),
+              "gemm: k_last %d (at most K = %lld, and 0 with more operand pairs)", d->k_last, (long long)d->K);
   a.k_last = d->k_last;
   // K-contiguous when the stride along k is 1 (ties: a single row / column counts as K-contiguous)
   const bool akc = d->a_cs == 1;

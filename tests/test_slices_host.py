@@ -68,3 +68,19 @@ def test_every_contraction_length():
                 n, kc, last = Planner._slices(K, ks)
                 assert kc % 64 == 0 and 2 <= n <= ks and (n - 1) * kc < K <= n * kc, (M, N, K)
                 assert last == (0 if n * kc == K else K - (n - 1) * kc), (M, N, K)
+
+
+def test_a_last_slice_longer_than_the_others_is_refused():
+    """On the host, before anything is launched: it would be read from behind the operands."""
+    import ctypes as C
+    from nabla_amd.backend import lib
+    L = lib.load()
+    for dtype, k_last, batch in [(1, 65, 4), (0, 65, 4), (1, 1 << 30, 1), (1, -1, 4)]:
+        d = lib.GemmDesc()
+        d.A = d.B = d.C = 4096
+        d.M = d.N = d.K = 64
+        d.a_rs, d.a_cs, d.b_rs, d.b_cs, d.ldc = 1, 64, 64, 1, 64
+        d.batch, d.batch_inner, d.a_bs, d.b_bs, d.c_bs = batch, 1, 4096, 4096, 4096
+        d.dtype_ab, d.dtype_c, d.alpha, d.k_last = dtype, 0, 1.0, k_last
+        with pytest.raises(ValueError, match="k_last"):
+            lib.check(L.nbk_gemm(C.byref(d), None))
