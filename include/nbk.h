@@ -54,7 +54,7 @@ int nbk_init(int device);
 const char* nbk_last_error(void);
 /* ABI version of this header; the ctypes shim refuses a mismatch. */
 int nbk_abi_version(void);
-#define NBK_ABI_VERSION 24
+#define NBK_ABI_VERSION 25
 
 /* ===================================================================== */
 /*  Row programs: fused elementwise chains + last-axis reductions         */

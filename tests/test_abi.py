@@ -209,3 +209,25 @@ def test_the_loss_program_over_long_bf16_rows_has_its_hand_scheduled_kernel(emul
     rp.C = vocab + 4      # not whole 16-byte pieces: the generated kernels take it
     assert L.nbk_rowprog_is_specialized(C.byref(rp)) == 1
     clear_plan_cache()
+
+
+#: what the structs of the header declare, by ABI number (comments and spacing aside)
+STRUCT_DIGESTS = {
+    24: "a3a2c6f668bffdc0",
+    25: "f1d532caffaaaacd",
+}
+
+
+def _struct_digest(header: str) -> str:
+    import hashlib
+    code = re.sub(r"/\*.*?\*/", " ", header, flags=re.S)
+    macros = re.findall(r"#define NBK_(?!ABI)\w+ \d+", code)
+    structs = re.findall(r"typedef struct nbk_\w+ \{.*?\} nbk_\w+;", code, flags=re.S)
+    return hashlib.sha256(" ".join(" ".join(macros + structs).split()).encode()).hexdigest()[:16]
+
+
+def test_a_changed_struct_has_a_new_abi_number():
+    """A binding made for one number passes structs of that number's layout: the library would
+    read behind a shorter one."""
+    from nabla_amd.backend import lib
+    assert STRUCT_DIGESTS[lib.ABI_VERSION] == _struct_digest(HEADER.read_text())
