@@ -586,7 +586,13 @@ class Decoder {
     while (pc < p_->n_ins && p_->ins[pc].op != NBK_OP_HALT) {
       const nbk_ins in = p_->ins[pc];
       if (in.op == NBK_OP_BODY) {
-        if (mode_ == RPVM_LOOP || level_ > 0) known_vec_.clear();
+        // (an input that a row starts with is one value in one register for the whole program: a
+        // second value on its slot would lose the register when the first is used up)
+        if (mode_ == RPVM_LOOP) known_vec_.clear();
+        else if (level_ > 0)
+          known_vec_.erase(std::remove_if(known_vec_.begin(), known_vec_.end(),
+                                          [&](int id) { return vals_[id].op != RPVM_LD; }),
+                           known_vec_.end());
         if (mode_ == RPVM_LOOP)
           for (int& v : vec) v = -1;  // (a chunk's values do not outlive it)
         const size_t begin = items_.size();
