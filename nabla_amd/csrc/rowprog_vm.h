@@ -26,7 +26,9 @@ enum rp_vm_op {
 #define RPVM_NONE 255      /* no result                                     */
 #define RPVM_SLOTS 8       /* inputs of a row or chunk requested at once: registers 0, 1, ... */
 #define RPVM_ROW_SLOTS 4   /* and scalars of a row                          */
-#define RPVM_MAX_INS 288
+/* Decoded instructions and one read ahead: a program's NBK_RP_MAX_INS and, where it is looped over, a
+   segment for the scalars behind every body (a third of them at most) and for those before the first. */
+#define RPVM_MAX_INS (NBK_RP_MAX_INS + NBK_RP_MAX_INS / 3 + 6)
 
 struct rp_vm_ins {
   uint8_t op, dst, a, b, c;

@@ -485,6 +485,7 @@ struct Val {
   int op = 0, a = -1, b = -1, c = -1, x = 0, y = 0;
   bool scalar = false, once = false, used = false;
   int reg = -1, last = -1;  // register, position of the last use
+  int own = -1;             // the register the program gave it (level 2)
 };
 enum ItemKind { DEF, STG, STR, ACCINIT, ACC, BODY_BEGIN, BODY_END };
 struct Item {
@@ -495,8 +496,9 @@ struct Item {
 
 class Decoder {
  public:
-  // `level` 0: values shared between phases; 1: vector values shared inside a phase only; 2: scalars
-  // in the program's own order too, which needs no more registers than the program was given.
+  // `level` 0: values shared between phases; 1: vector values shared inside a phase only; 2: the
+  // program as it stands, every value in the register it was given and every load in its place.  Level 2
+  // takes any program that is looped over its rows or has none to reduce.
   // At most `slots` inputs are requested ahead.
   Decoder(const nbk_rowprog* p, int mode, int file, int level, int slots)
       : p_(p), mode_(mode), file_(file), level_(level), max_slots_(slots) {}
@@ -531,6 +533,7 @@ class Decoder {
     return -1;
   }
   int define(const Val& v, bool shared) {
+    shared &= level_ < 2;
     if (shared) {
       const int got = find(v);
       if (got >= 0) return got;
@@ -569,10 +572,14 @@ class Decoder {
     for (int i = 0; i < p_->n_operands; ++i) op_written[i] = written(i);
     auto reg = [&](int r) {
       int& v = r < NBK_RP_NVEC ? vec[r] : scl[r - NBK_RP_NVEC];
-      if (v < 0) {  // read before it is written
+      if (v < 0) {  // read before it is written: zero
         Val z;
-        z.scalar = true; z.op = RPVM_IMM; z.x = NBK_RP_MAX_IMM;  // (the decoded program's own zero)
-        v = define(z, level_ < 2);
+        z.scalar = true; z.op = RPVM_IMM; z.x = NBK_RP_MAX_IMM;  // (the decoded program's own)
+        if (level_ == 2) z.own = r & (NBK_RP_NVEC - 1);
+        if (level_ == 2 && r < NBK_RP_NVEC) {  // (in the register itself: is it greater than itself?)
+          z.scalar = false; z.op = NBK_OP_GT; z.a = z.b = (int)vals_.size();
+        }
+        v = define(z, true);
       }
       return v;
     };
@@ -627,6 +634,7 @@ class Decoder {
             } else {
               operands(v, b);
             }
+            if (level_ == 2) v.own = b.dst;
             vec[b.dst] = define(v, shared);
           }
         }
@@ -648,7 +656,8 @@ class Decoder {
       }
       Val v;
       v.scalar = true;
-      bool shared = level_ < 2;
+      bool shared = true;
+      if (level_ == 2) v.own = in.dst - NBK_RP_NVEC;
       if (in.op == NBK_OP_IMM) {
         v.op = RPVM_IMM;
         v.x = in.a;
@@ -656,7 +665,7 @@ class Decoder {
       } else if (in.op == NBK_OP_LDR) {
         bool moves = op_written[in.a];
         for (int k = 0; k < p_->n_lead; ++k) moves |= p_->operand[in.a].lead_stride[k] != 0;
-        const int slot = moves && !op_written[in.a] ? row_slot_of(in.a) : -1;
+        const int slot = moves && !op_written[in.a] && level_ < 2 ? row_slot_of(in.a) : -1;
         v.op = slot >= 0 ? RPVM_LDS : RPVM_LDR;
         v.x = slot >= 0 ? slot : in.a;
         v.once = !moves;
@@ -724,8 +733,9 @@ class Decoder {
     bool vec_busy[RPVM_FILE_LARGE] = {}, scl_busy[NBK_RP_NSCL] = {};
     auto take = [&](Val& v) {
       bool* busy = v.scalar ? scl_busy : vec_busy;
-      const int n_regs = v.scalar ? NBK_RP_NSCL : file_;
-      for (int r = 0; r < n_regs; ++r)
+      const int r0 = v.own >= 0 ? v.own : 0;
+      const int r1 = v.own >= 0 ? v.own + 1 : v.scalar ? NBK_RP_NSCL : file_;
+      for (int r = r0; r < r1; ++r)
         if (!busy[r]) {
           busy[r] = true;
           v.reg = r;

@@ -3,7 +3,6 @@ executed on expressions instead of numbers: every store has to receive the same 
 the library decodes on the host."""
 import ctypes as C
 import random
-import re
 
 import pytest
 
@@ -12,7 +11,7 @@ from nabla_amd.backend import isa, lib
 FLAT, ROW, LOOP = 0, 1, 2  # rp_vm_mode
 (V_STG, V_STR, V_LD, V_LDG, V_LDS, V_LDR, V_COLIDX, V_RED, V_ACCINIT, V_ACC, V_IMM, V_LEADIDX, V_SEG) = range(1, 14)
 SCALAR, NONE, ROW_SLOTS = 32, 255, 4
-MAX_INS = int(re.search(r"RPVM_MAX_INS (\d+)", (lib.LIB_PATH.parent / "rowprog_vm.h").read_text())[1])
+MAX_INS = isa.MAX_INS + isa.MAX_INS // 3 + 6
 
 
 class VmIns(C.Structure):
@@ -204,6 +203,8 @@ def check(rp):
         if vm is not None:
             assert run_decoded(vm, m) == want, m
             assert run_decoded(vm, m, wave=False) == want, m
+    # (rows that no register file holds are walked in chunks: that form takes any program)
+    assert forms[modes[-1]] is not None
     return forms
 
 
@@ -240,8 +241,119 @@ def shared_inputs_program(rng):
     return program(ins, n_in + 3, rng.choice([1, 100, 1003]), True, range(n_in + 3))
 
 
+def random_program(rng):
+    """A valid program: bodies that read what they or the prologues wrote, reductions between
+    them, inputs read again, row scalars loaded twice, all registers in use."""
+    reduce, once = rng.random() < 0.75, rng.random() < 0.7  # (once: accumulators that rows in registers can have)
+    n_in, n_out = rng.randint(1, 14), rng.randint(1, 5)
+    n_vec, n_scl = rng.choice([4, 8, 12, 16, 16]), rng.choice([3, 8, 16])
+    moves = [i for i in range(n_in + n_out) if rng.random() < 0.7]
+    ops1 = [isa.UNARY[k] for k in ("neg", "exp", "relu")]
+    ops2 = [isa.BINARY[k] for k in ("add", "sub", "mul", "gt")]
+    scalars, ins, started = [], [], {}
+
+    def ew(regs, dst):
+        kind = rng.random()
+        if kind < 0.25:
+            return (rng.choice(ops1), dst, rng.choice(regs), 0, 0, 0)
+        if kind < 0.8:
+            return (rng.choice(ops2), dst, rng.choice(regs), rng.choice(regs), 0, 0)
+        return (rng.choice(sorted(TERNARY)), dst, *(rng.choice(regs) for _ in range(3)), 0)
+
+    for _ in range(rng.randint(1, 4)):
+        for _ in range(rng.randint(0, 2 + n_scl // 2)):
+            dst = isa.NVEC + rng.randrange(n_scl)
+            kind = rng.random()
+            if kind < 0.4:
+                ins.append((isa.LDR, dst, rng.randrange(n_in), 0, 0, 0))
+            elif kind < 0.6 or not scalars:
+                ins.append((isa.IMM, dst, rng.randrange(isa.MAX_IMM), 0, 0, 0))
+            elif kind < 0.7:
+                ins.append((isa.LEADIDX, dst, 0, rng.randint(0, 1), 0, 0))
+            elif kind < 0.75:
+                ins.append((isa.STR, n_in + rng.randrange(n_out), rng.choice(scalars), 0, 0, 0))
+                continue
+            else:
+                ins.append(ew(scalars, dst))
+            scalars.append(dst) if dst not in scalars else None
+        if reduce:
+            for k in range(isa.NACC):
+                if rng.random() < 0.6 and not (once and started.get(k, (0, 0))[1]):
+                    kind = rng.randrange(3)
+                    ins.append((isa.ACCINIT, k, kind, 0, 0, 0))
+                    started[k] = [kind, 0]
+        vecs, b = [], []
+        for _ in range(rng.randint(2, 30)):
+            dst = rng.randrange(n_vec)
+            kind = rng.random()
+            if kind < 0.4 or not vecs:
+                b.append((isa.LDG, dst, rng.randrange(n_in + (n_out if rng.random() < 0.1 else 0)), 0, 0, 0))
+            elif kind < 0.43:
+                b.append((isa.COLIDX, dst, rng.randint(0, 1), 0, 0, 0))
+            elif kind < 0.5:
+                b.append((isa.STG, n_in + rng.randrange(n_out), rng.choice(vecs + scalars), 0, 0, 0))
+                continue
+            elif kind < 0.6 and any(n == 0 or not once for _, n in started.values()):
+                k = rng.choice([k for k in sorted(started) if started[k][1] == 0 or not once])
+                b.append((isa.ACC, k, rng.choice(vecs), started[k][0], 0, 0))
+                started[k][1] += 1
+                continue
+            else:
+                b.append(ew(vecs + scalars, dst))
+            if dst not in vecs:
+                vecs.append(dst)
+        b.append((isa.STG, n_in + rng.randrange(n_out), rng.choice(vecs), 0, 0, 0))
+        ins += body(*b)
+        for k in sorted(started):
+            if started[k][1] and rng.random() < 0.8:
+                # (a second reduction of the same accumulator too, in a later phase)
+                dst = isa.NVEC + rng.randrange(n_scl)
+                ins.append((isa.RED, dst, k, started[k][0], 0, 0))
+                if dst not in scalars:
+                    scalars.append(dst)
+    ins += body((isa.LDG, 0, 0, 0, 0, 0), *[(isa.BINARY["add"], 0, 0, s, 0, 0) for s in scalars],
+                (isa.STG, n_in, 0, 0, 0, 0))
+    return program(ins, n_in + n_out, rng.choice([1, 3, 100, 1003, 5000]), reduce, moves)
+
+
+@pytest.mark.parametrize("seed", range(8))
+def test_random_programs(seed):
+    rng = random.Random(seed)
+    for _ in range(250):
+        check(random_program(rng))
+
+
 @pytest.mark.parametrize("seed", range(4))
 def test_inputs_read_again_in_a_later_phase(seed):
     rng = random.Random(seed)
     held = [check(shared_inputs_program(rng))[ROW] is not None for _ in range(150)]
     assert sum(held) > 75  # (rows in registers, the form that requests an input once for all phases)
+
+
+def test_all_scalars_alive_and_row_operands_loaded_twice():
+    """Sixteen scalars that every phase reads, the operands of a row among them, loaded again into
+    registers that are needed in between."""
+    rng = random.Random(1)
+    for n_row in range(1, 17):
+        S = isa.NVEC
+        ins = [(isa.LDR, S + k, k % n_row, 0, 0, 0) for k in range(16)]
+        for phase in range(3):
+            order = rng.sample(range(16), 16)
+            ins += [(isa.ACCINIT, 0, 0, 0, 0, 0)]
+            ins += body((isa.LDG, 0, 16, 0, 0, 0), *[(isa.BINARY["mul"], 0, 0, S + k, 0, 0) for k in order],
+                        (isa.ACC, 0, 0, 0, 0, 0), (isa.STG, 17, 0, 0, 0, 0))
+            ins += [(isa.RED, S + order[0], 0, 0, 0, 0)]
+            ins += [(isa.BINARY["add"], S + order[k], S + order[k], S + order[k - 1], 0, 0) for k in (1, 2)]
+            ins += [(isa.LDR, S + order[k], order[k] % n_row, 0, 0, 0) for k in (3, 4)]
+        check(program(ins, 18, 1003, True, range(18)))
+
+
+def test_the_longest_programs():
+    """As many instructions as a record holds, in the pattern whose looped form grows the most: a
+    scalar behind every body."""
+    for reduce in (False, True):
+        S = isa.NVEC
+        ins = [(isa.LDR, S + k, 0, 0, 0, 0) for k in range(1)]
+        while len(ins) + 4 <= isa.MAX_INS:
+            ins += body((isa.STG, 1, S, 0, 0, 0)) + [(isa.BINARY["add"], S, S, S, 0, 0)]
+        check(program(ins, 2, 100, reduce, [0, 1]))
