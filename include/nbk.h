@@ -122,7 +122,7 @@ enum nbk_rp_op {
   NBK_OP_LEADIDX = 8,  /* prologue: sreg dst <- index along leading dim a, as float (b = 0) or int32 (b = 1) */
   /* reductions over the row */
   NBK_OP_ACCINIT = 9,  /* prologue: acc dst <- identity of kind a              */
-  NBK_OP_ACC = 10,     /* body: acc dst <- combine(acc, vreg a), kind b        */
+  NBK_OP_ACC = 10,     /* body: acc dst <- combine(acc, vreg or sreg a), kind b */
   NBK_OP_RED = 11,     /* prologue: sreg dst <- block-reduce(acc a), kind b    */
   /* unary  dst <- f(a) */
   NBK_OP_MOV = 16, NBK_OP_NEG = 17, NBK_OP_RELU = 18, NBK_OP_EXP = 19,

@@ -867,11 +867,13 @@ class Decoder {
     }
     if (loop) end();
     if ((int)list.size() >= RPVM_MAX_INS) return false;
-    // reductions that stand together share one exchange between the wavefronts
+    // reductions that stand together share one exchange between the wavefronts (one over a scalar
+    // has its own: the scalar may be the result of its neighbour)
+    auto joins = [&](size_t k) { return list[k].op == RPVM_RED && list[k].a < RPVM_SCALAR; };
     for (size_t i = 0; i < list.size();) {
       size_t k = i + 1;
       if (list[i].op == RPVM_RED) {
-        while (k < list.size() && k - i < 4 && list[k].op == RPVM_RED) ++k;
+        while (k < list.size() && k - i < 4 && joins(i) && joins(k)) ++k;
         list[i].aux = (uint16_t)(k - i);
       }
       i = k;

@@ -295,7 +295,7 @@ def random_program(rng):
                 continue
             elif kind < 0.6 and any(n == 0 or not once for _, n in started.values()):
                 k = rng.choice([k for k in sorted(started) if started[k][1] == 0 or not once])
-                b.append((isa.ACC, k, rng.choice(vecs), started[k][0], 0, 0))
+                b.append((isa.ACC, k, rng.choice(vecs + vecs + scalars), started[k][0], 0, 0))
                 started[k][1] += 1
                 continue
             else:
@@ -357,3 +357,16 @@ def test_the_longest_programs():
         while len(ins) + 4 <= isa.MAX_INS:
             ins += body((isa.STG, 1, S, 0, 0, 0)) + [(isa.BINARY["add"], S, S, S, 0, 0)]
         check(program(ins, 2, 100, reduce, [0, 1]))
+
+
+@pytest.mark.parametrize("kinds", [(1, 0), (0, 0, 0), (2, 1, 0, 1)])
+def test_a_reduction_of_its_neighbours_result(kinds):
+    """Nothing but bodies stands between the reductions, and a body leaves nothing behind."""
+    S = isa.NVEC
+    ins = [(isa.ACCINIT, k, kind, 0, 0, 0) for k, kind in enumerate(kinds)]
+    ins += body((isa.LDG, 0, 0, 0, 0, 0), (isa.ACC, 0, 0, kinds[0], 0, 0)) + [(isa.RED, S, 0, kinds[0], 0, 0)]
+    for k in range(1, len(kinds)):
+        ins += body((isa.ACC, k, S + (k - 1) % 2, kinds[k], 0, 0)) + [(isa.RED, S + k % 2, k, kinds[k], 0, 0)]
+    last = S + (len(kinds) - 1) % 2
+    ins += body((isa.STG, 1, last, 0, 0, 0))
+    assert check(program(ins, 2, 1003, True, [0, 1]))[ROW] is not None
