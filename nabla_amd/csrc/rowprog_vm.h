@@ -20,8 +20,6 @@ enum rp_vm_op {
   RPVM_SEG          // the aux instructions behind it run once per chunk (b) or row; slots[c ..) are its inputs, a of them
 };
 
-#define RPVM_FILE_SMALL 16 /* vector registers of the two register files    */
-#define RPVM_FILE_LARGE 32
 #define RPVM_SCALAR 32     /* register numbers from here on are scalars     */
 #define RPVM_NONE 255      /* no result                                     */
 #define RPVM_SLOTS 8       /* inputs of a row or chunk requested at once: registers 0, 1, ... */
@@ -45,8 +43,7 @@ struct rp_vm {
   int32_t n_once, n_ins;
   int32_t n_slots, n_row_slots;
   int32_t lanes;     // lanes per row (power of two up to 32, or a multiple of 64)
-  int16_t file;      // vector registers it needs: RPVM_FILE_SMALL or RPVM_FILE_LARGE
-  int16_t rare;      // whether it calls one of the long functions (logarithm, erf, powers, ...)
+  int32_t rare;      // whether it calls one of the long functions (logarithm, erf, powers, ...)
   uint8_t slots[44]; // operand of every input slot (per segment in a looped program)
   uint8_t row_slots[RPVM_ROW_SLOTS], row_dst[RPVM_ROW_SLOTS];  // operands and registers of a row's scalars
   float imm[NBK_RP_MAX_IMM + 1];  // (and a zero)

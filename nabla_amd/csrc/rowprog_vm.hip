@@ -31,10 +31,6 @@
 enum { K_FLAT = 0, K_SUB = 1, K_ROW = 2, K_LOOP = 3 };
 
 typedef float vf16 __attribute__((ext_vector_type(16)));
-typedef float vf32 __attribute__((ext_vector_type(32)));
-template <int F> struct RpFile;
-template <> struct RpFile<16> { typedef vf16 vec; };
-template <> struct RpFile<32> { typedef vf32 vec; };
 typedef uint32_t rp_u4b __attribute__((ext_vector_type(4), aligned(1)));
 static_assert(NBK_RP_NSCL == 16, "the scalar file is a 16-wide vector");
 
@@ -211,10 +207,9 @@ struct RpInput {
   int back;
 };
 
-template <int K, int F, bool RARE>
-__global__ __launch_bounds__(K == K_ROW ? (F == 16 ? 1024 : 512) : K == K_LOOP ? 512 : 256, F == 16 ? (RARE ? 3 : 4) : 2)
+template <int K, bool RARE>
+__global__ __launch_bounds__(K == K_ROW ? 1024 : K == K_LOOP ? 512 : 256, RARE ? 3 : 4)
 void rp_vm_kernel(const rp_vm, uint32_t rows, uint32_t cpr, uint64_t total) {
-  typedef typename RpFile<F>::vec file;
   constexpr bool UNIFORM = K == K_ROW || K == K_LOOP;
   __shared__ float red_buf[128];
   const rp_prog P = (rp_prog)__builtin_amdgcn_kernarg_segment_ptr();  // (the first argument)
@@ -289,7 +284,7 @@ void rp_vm_kernel(const rp_vm, uint32_t rows, uint32_t cpr, uint64_t total) {
         const int64_t col = c0 + ((int64_t)cc << 2);
         const int64_t left = C - col;
         const int valid = !inside || left <= 0 ? 0 : left >= 4 ? 4 : (int)left;
-        file X, Y, Z, W;  // vector registers, by chunk component
+        vf16 X, Y, Z, W;  // vector registers, by chunk component
         {
           RpInput in[RPVM_SLOTS];
 #pragma unroll
@@ -444,7 +439,7 @@ void rp_vm_kernel(const rp_vm, uint32_t rows, uint32_t cpr, uint64_t total) {
           }
           // Every instruction writes both files, one without such a result what is there already: a
           // write under a branch makes the compiler copy the whole file (16 moves) around it.
-          const bool to_vec = in.dst < F;
+          const bool to_vec = in.dst < NBK_RP_NVEC;
           const float sv = r.x;
           if (!to_vec) r = make_float4(X[0], Y[0], Z[0], W[0]);
           const int d = to_vec ? in.dst : 0;
@@ -500,8 +495,8 @@ class Decoder {
   // program as it stands, every value in the register it was given and every load in its place.  Level 2
   // takes any program that is looped over its rows or has none to reduce.
   // At most `slots` inputs are requested ahead.
-  Decoder(const nbk_rowprog* p, int mode, int file, int level, int slots)
-      : p_(p), mode_(mode), file_(file), level_(level), max_slots_(slots) {}
+  Decoder(const nbk_rowprog* p, int mode, int level, int slots)
+      : p_(p), mode_(mode), level_(level), max_slots_(slots) {}
 
   // False if the mode or this level does not take the program.
   bool run(rp_vm* out) {
@@ -513,7 +508,7 @@ class Decoder {
 
  private:
   const nbk_rowprog* p_;
-  const int mode_, file_, level_, max_slots_;
+  const int mode_, level_, max_slots_;
   rp_vm* out_ = nullptr;
   std::vector<Val> vals_;
   std::vector<Item> items_;
@@ -730,11 +725,11 @@ class Decoder {
       if (it.kind == DEF && vals_[it.val].used && !vals_[it.val].once)
         sources(vals_[it.val], [&](int s) { use(s, i); });
     }
-    bool vec_busy[RPVM_FILE_LARGE] = {}, scl_busy[NBK_RP_NSCL] = {};
+    bool vec_busy[NBK_RP_NVEC] = {}, scl_busy[NBK_RP_NSCL] = {};
     auto take = [&](Val& v) {
       bool* busy = v.scalar ? scl_busy : vec_busy;
       const int r0 = v.own >= 0 ? v.own : 0;
-      const int r1 = v.own >= 0 ? v.own + 1 : v.scalar ? NBK_RP_NSCL : file_;
+      const int r1 = v.own >= 0 ? v.own + 1 : v.scalar ? NBK_RP_NSCL : NBK_RP_NVEC;
       for (int r = r0; r < r1; ++r)
         if (!busy[r]) {
           busy[r] = true;
@@ -879,7 +874,6 @@ class Decoder {
       i = k;
     }
     out_->n_ins = (int)list.size();
-    out_->file = file_;
     for (const rp_vm_ins& in : list) out_->rare |= is_rare(in.op);
     out_->n_slots = n_slots_;
     out_->n_row_slots = n_row_slots_;
@@ -944,22 +938,13 @@ int occupancy(const void* fn, int block, int* out) {
 }  // namespace
 
 bool rp_vm_decode(const nbk_rowprog* p, int mode, rp_vm* out) {
-  // From the fewest instructions to the fewest registers.  The large register file halves the
-  // wavefronts of a CU, so it has to save a quarter of the instructions against the small one
-  // without values shared between phases.
-  static const struct { int file, level, slots; } kTry[] = {
-      {RPVM_FILE_SMALL, 0, RPVM_SLOTS}, {RPVM_FILE_LARGE, 0, RPVM_SLOTS}, {RPVM_FILE_SMALL, 1, RPVM_SLOTS},
-      {RPVM_FILE_SMALL, 1, 4},          {RPVM_FILE_SMALL, 1, 0},          {RPVM_FILE_SMALL, 2, 0}};
-  bool found = false;
+  // From the fewest instructions to the fewest registers.
+  static const struct { int level, slots; } kTry[] = {{0, RPVM_SLOTS}, {1, RPVM_SLOTS}, {1, 4}, {1, 0}, {2, 0}};
   for (const auto& t : kTry) {
-    if (t.file == RPVM_FILE_LARGE && mode == RPVM_LOOP) continue;
-    rp_vm v = {};
-    if (!Decoder(p, mode, t.file, t.level, t.slots).run(&v)) continue;
-    if (!found || v.n_ins * 3 < out->n_ins * 4) *out = v;
-    found = true;
-    if (t.file == RPVM_FILE_SMALL) break;
+    *out = {};
+    if (Decoder(p, mode, t.level, t.slots).run(out)) return true;
   }
-  return found;
+  return false;
 }
 
 int rp_vm_launch(const nbk_rowprog* p, int64_t rows, hipStream_t stream) {
@@ -967,8 +952,7 @@ int rp_vm_launch(const nbk_rowprog* p, int64_t rows, hipStream_t stream) {
   int mode = p->has_reduce ? RPVM_ROW : RPVM_FLAT;
   std::shared_ptr<const rp_vm> d;
   if (mode == RPVM_FLAT || chunks <= 1024) d = decoded(p, mode);
-  // (with the large file 512 lanes fill a CU)
-  if (mode == RPVM_ROW && (!d || (d->file == RPVM_FILE_LARGE && chunks > 512))) {
+  if (mode == RPVM_ROW && !d) {
     mode = RPVM_LOOP;
     d = decoded(p, mode);
   }
@@ -979,10 +963,7 @@ int rp_vm_launch(const nbk_rowprog* p, int64_t rows, hipStream_t stream) {
   vm.n_lead = p->n_lead;
   for (int i = 0; i < p->n_imm; ++i) vm.imm[i] = p->imm[i];
   for (int i = 0; i < p->n_operands; ++i) vm.operand[i] = p->operand[i];
-#define RPVM_PICK(K)                                                        \
-  (d->file == RPVM_FILE_LARGE ? (const void*)rp_vm_kernel<K, 32, true>      \
-   : d->rare                  ? (const void*)rp_vm_kernel<K, 16, true>      \
-                              : (const void*)rp_vm_kernel<K, 16, false>)
+#define RPVM_PICK(K) (d->rare ? (const void*)rp_vm_kernel<K, true> : (const void*)rp_vm_kernel<K, false>)
   const void* fn;
   int block = 256;
   uint64_t groups = (uint64_t)rows;  // workgroups' worth of work
@@ -990,7 +971,7 @@ int rp_vm_launch(const nbk_rowprog* p, int64_t rows, hipStream_t stream) {
     fn = RPVM_PICK(K_FLAT);
     groups = ((uint64_t)rows * (uint64_t)chunks + 255) / 256;
   } else if (mode == RPVM_LOOP) {
-    fn = d->rare ? (const void*)rp_vm_kernel<K_LOOP, 16, true> : (const void*)rp_vm_kernel<K_LOOP, 16, false>;
+    fn = RPVM_PICK(K_LOOP);
     block = p->block;  // (the lanes of the generated kernels: sums associate as theirs do)
   } else if (chunks <= 32) {
     fn = RPVM_PICK(K_SUB);

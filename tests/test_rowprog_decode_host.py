@@ -21,7 +21,7 @@ class VmIns(C.Structure):
 class Vm(C.Structure):
     _fields_ = [("lead_dim", C.c_int64 * isa.MAX_LEAD), ("C", C.c_int64), ("n_lead", C.c_int32),
                 ("n_once", C.c_int32), ("n_ins", C.c_int32), ("n_slots", C.c_int32), ("n_row_slots", C.c_int32),
-                ("lanes", C.c_int32), ("file", C.c_int16), ("rare", C.c_int16), ("slots", C.c_uint8 * 44),
+                ("lanes", C.c_int32), ("rare", C.c_int32), ("slots", C.c_uint8 * 44),
                 ("row_slots", C.c_uint8 * ROW_SLOTS), ("row_dst", C.c_uint8 * ROW_SLOTS),
                 ("imm", C.c_float * (isa.MAX_IMM + 1)), ("operand", lib.Operand * isa.MAX_OPERANDS),
                 ("ins", VmIns * MAX_INS)]
@@ -111,7 +111,7 @@ def run_decoded(vm, mode, wave=True):
         return scl[r - SCALAR] if r >= SCALAR else vec[r]
 
     def put(dst, value):
-        if dst < vm.file:
+        if dst < isa.NVEC:
             vec[dst] = value
         elif dst != NONE:
             assert SCALAR <= dst < SCALAR + isa.NSCL
