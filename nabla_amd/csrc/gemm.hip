@@ -1692,8 +1692,12 @@ struct F32Rows {
 // below 33 of those): 512 x 2048 x 1024 as x^T dy 150 -> 43 us, 1024 x 2048 x 512 84 -> 32 (68
 // TFLOP/s), 32 x (256 x 64 x 256) 45 -> 10, 8192 x 4096 x 1024 947 -> 654 (105 TFLOP/s), 1024 x 512
 // x 512 14.4 -> 12.2, 128 x 256 x 784 16.4 -> 11.6.
+// Two workgroups have to fit a CU (four waves each: the second launch bound), which x^T dy missed by a
+// few registers while its accumulators stood in registers of their own: 8192 x 4096 x 1024 1014 -> 707
+// us, 7680 x 1920 x 64 90 -> 60, 4096 x 1024 x 1024 152 -> 104; with one row-contiguous operand 2 to 3 % less.
+// With none, two to five per cent more on contractions of 64 to 512: no bound there.
 template <int WM, int WN, int WK, int IM, int IN, int KS, bool A_KC, bool B_KC>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs g) {
+__global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(const GemmArgs g) {
   static_assert(WM * WN * WK == 4 && (WK == 1 || WK == 4), "four waves, together or apart");
   constexpr int BM = 32 * WM * IM, BN = 32 * WN * IN, BK = 8 * KS * WK, LD = BK + 4;
   constexpr int NA = IM * IN == 1 ? 4 / WK : 1;
