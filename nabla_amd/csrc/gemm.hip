@@ -1613,11 +1613,16 @@ struct F32Rows {
   static constexpr int LD = BK + 4;
   static constexpr int RB = ROWS >= 64 ? 4 : 2;  // row-contiguous operand: blocks of RB rows x 2 k
   static constexpr int V = KC ? 4 : RB, Q = KC ? 1 : 2;  // a piece: Q accesses of V floats
+  static constexpr int PAD = KC ? 0 : V - 1;  // LDS rows in front of the tile (place)
   static constexpr int PIECES = ROWS * BK / 256 / (V * Q);
   static_assert(PIECES >= 1, "at least one piece per lane");
   f32_piece<V> r[2][PIECES][Q];  // two K tiles in flight
 
-  __device__ static __forceinline__ void place(int p, int& row, int& kk) {
+  // Where a piece lies in the tile.  The pieces of a row-contiguous operand past its end lie where its
+  // last one does, which ends with the last row (and may begin before the tile): the edge of a
+  // result is loaded like the rest of it.  Element by element, the workgroups there took half as long
+  // again as the others: 79 x 150 x 1188 as x^T dy 29.0 us, 16.5 now, 576 x 248 x 2608 54.0 -> 29.9.
+  __device__ static __forceinline__ void place(int p, int64_t left, bool whole, int& row, int& kk) {
     const int idx = (int)threadIdx.x + 256 * p;
     if constexpr (KC) {
       row = idx / (BK / 4);
@@ -1625,44 +1630,49 @@ struct F32Rows {
     } else {
       row = idx % (ROWS / RB) * RB;
       kk = idx / (ROWS / RB) * 2;
+      if (whole) row = (int)min((int64_t)row, left - V);
     }
   }
-  // `stride`: between rows (KC) or between k (row-contiguous).  Rows past the end repeat the last
-  // one (their results are not stored), k past the end reads as zero.
+  // Whether the operand has rows for a whole piece.
+  __device__ static __forceinline__ bool pieces(int64_t rows) { return KC || rows >= V; }
+  // A K tile that lies inside K, in whole pieces.  `stride`: between rows (KC) or between k
+  // (row-contiguous).  Rows past the end repeat the last one or are left as they are in LDS (their results
+  // are not stored).
   template <int SET>
-  __device__ __forceinline__ void load(const float* P, int64_t stride, int64_t row0, int64_t rows, int64_t k0, int64_t K) {
-    if (k0 + BK <= K && (KC || row0 + ROWS <= rows)) {
-#pragma unroll
-      for (int p = 0; p < PIECES; ++p) {
-        int row, kk;
-        place(p, row, kk);
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-          const float* src = KC ? P + min(row0 + row, rows - 1) * stride + k0 + kk : P + (k0 + kk + q) * stride + row0 + row;
-          r[SET][p][q] = *(const f32_piece_any<V>*)src;
-        }
-      }
-    } else {
-#pragma unroll
-      for (int p = 0; p < PIECES; ++p) {
-        int row, kk;
-        place(p, row, kk);
-#pragma unroll
-        for (int q = 0; q < Q; ++q)
-#pragma unroll
-          for (int e = 0; e < V; ++e) {
-            const int64_t k = k0 + kk + (KC ? e : q), m = min(row0 + row + (KC ? 0 : e), rows - 1);
-            r[SET][p][q][e] = k < K ? P[KC ? m * stride + k : k * stride + m] : 0.f;
-          }
-      }
-    }
-  }
-  template <int SET>
-  __device__ __forceinline__ void store(float* S) {
+  __device__ __forceinline__ void load(const float* P, int64_t stride, int64_t row0, int64_t rows, int64_t k0) {
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
       int row, kk;
-      place(p, row, kk);
+      place(p, rows - row0, true, row, kk);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const float* src = KC ? P + min(row0 + row, rows - 1) * stride + k0 + kk : P + (k0 + kk + q) * stride + row0 + row;
+        r[SET][p][q] = *(const f32_piece_any<V>*)src;
+      }
+    }
+  }
+  // Any other K tile, element by element; k past the end reads as zero.
+  template <int SET>
+  __device__ __forceinline__ void load_each(const float* P, int64_t stride, int64_t row0, int64_t rows, int64_t k0, int64_t K) {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      int row, kk;
+      place(p, rows - row0, pieces(rows), row, kk);
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+          const int64_t k = k0 + kk + (KC ? e : q), m = min(row0 + row + (KC ? 0 : e), rows - 1);
+          r[SET][p][q][e] = k < K ? P[KC ? m * stride + k : k * stride + m] : 0.f;
+        }
+    }
+  }
+  template <int SET>
+  __device__ __forceinline__ void store(float* S, int64_t row0, int64_t rows) {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      int row, kk;
+      place(p, rows - row0, pieces(rows), row, kk);
       // (the pieces stay as they were loaded until here: pairing two k of a row any earlier would
       // wait for the loads right behind their request)
 #pragma unroll
@@ -1689,20 +1699,22 @@ struct F32Rows {
 // h = l / 32 owns k = 8 s + 4 h .. + 3 of step s and issues four instructions per step.  The smaller
 // tiles sum a product in four chains (waves x accumulators), the largest in one.
 // Before / after (guarded 128 x 128 tiles without loads ahead, or 32 x 32 ones straight from memory
-// below 33 of those): 512 x 2048 x 1024 as x^T dy 150 -> 43 us, 1024 x 2048 x 512 84 -> 32 (68
-// TFLOP/s), 32 x (256 x 64 x 256) 45 -> 10, 8192 x 4096 x 1024 947 -> 654 (105 TFLOP/s), 1024 x 512
-// x 512 14.4 -> 12.2, 128 x 256 x 784 16.4 -> 11.6.
+// below 33 of those): 512 x 2048 x 1024 as x^T dy 150 -> 39 us, 1024 x 2048 x 512 84 -> 28 (77
+// TFLOP/s), 32 x (256 x 64 x 256) 45 -> 10, 8192 x 4096 x 1024 946 -> 621 (111 TFLOP/s), 128 x 256 x
+// 784 15.5 -> 11.3.
 // Two workgroups have to fit a CU (four waves each: the second launch bound), which x^T dy missed by a
-// few registers while its accumulators stood in registers of their own: 8192 x 4096 x 1024 1014 -> 707
-// us, 7680 x 1920 x 64 90 -> 60, 4096 x 1024 x 1024 152 -> 104; with one row-contiguous operand 2 to 3 % less.
+// few registers while its accumulators stood in registers of their own: 8192 x 4096 x 1024 1014 -> 626
+// us, 7680 x 1920 x 64 90 -> 57, 4096 x 1024 x 1024 152 -> 94; with one row-contiguous operand 5 % less.
 // With none, two to five per cent more on contractions of 64 to 512: no bound there.
 template <int WM, int WN, int WK, int IM, int IN, int KS, bool A_KC, bool B_KC>
 __global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(const GemmArgs g) {
   static_assert(WM * WN * WK == 4 && (WK == 1 || WK == 4), "four waves, together or apart");
   constexpr int BM = 32 * WM * IM, BN = 32 * WN * IN, BK = 8 * KS * WK, LD = BK + 4;
   constexpr int NA = IM * IN == 1 ? 4 / WK : 1;
-  __shared__ __align__(16) float lds[2 * (BM + BN) * LD];
-  static_assert(WK == 1 || 4 * 16 * 64 <= 2 * (BM + BN) * LD, "the partial sums fit");
+  constexpr int A0 = F32Rows<BM, BK, A_KC>::PAD * LD, B0 = A0 + (BM + F32Rows<BN, BK, B_KC>::PAD) * LD;
+  constexpr int SET = B0 + BN * LD;  // (two of them)
+  __shared__ __align__(16) float lds[2 * SET];
+  static_assert(WK == 1 || 4 * 16 * 64 <= 2 * SET, "the partial sums fit");
   int tm_i, tn_i;
   gemm_tile_coords(blockIdx.x, g.tiles_m, g.tiles_n, tm_i, tn_i);
   const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
@@ -1727,19 +1739,27 @@ __global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(con
   F32Rows<BM, BK, A_KC> la;
   F32Rows<BN, BK, B_KC> lb;
   const int64_t nk = (K + BK - 1) / BK;
+  const bool pieces = la.pieces(g.M) && lb.pieces(g.N);
+  // (one branch for both operands: with a branch each, the second one's requests wait for the
+  // data of the first, 576 x 256 x 2608 40 us instead of 31)
   auto load = [&](auto set, int64_t kt) {
-    la.template load<set.value>(A, a_stride, m0, g.M, kt * BK, K);
-    lb.template load<set.value>(B, b_stride, n0, g.N, kt * BK, K);
+    if (pieces && (kt + 1) * BK <= K) {
+      la.template load<set.value>(A, a_stride, m0, g.M, kt * BK);
+      lb.template load<set.value>(B, b_stride, n0, g.N, kt * BK);
+    } else {
+      la.template load_each<set.value>(A, a_stride, m0, g.M, kt * BK, K);
+      lb.template load_each<set.value>(B, b_stride, n0, g.N, kt * BK, K);
+    }
   };
   auto store = [&](auto set) {
-    float* S = lds + set.value * (BM + BN) * LD;
-    la.template store<set.value>(S);
-    lb.template store<set.value>(S + BM * LD);
+    float* S = lds + set.value * SET;
+    la.template store<set.value>(S + A0, m0, g.M);
+    lb.template store<set.value>(S + B0, n0, g.N);
   };
   auto tile = [&](auto cur, auto next, int64_t kt) {
     if (kt + 2 < nk) load(cur, kt + 2);  // (its registers went to LDS an iteration ago)
-    const float* As = lds + cur.value * (BM + BN) * LD;
-    const float* Bs = As + BM * LD;
+    const float* As = lds + cur.value * SET + A0;
+    const float* Bs = lds + cur.value * SET + B0;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       f32x4 fa[IM], fb[IN];
@@ -2150,10 +2170,10 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
   }
   // The largest tile that still gives every CU two workgroups: below that the K loop of one workgroup
   // is what a launch waits for, and the more waves share a CU the less of it shows.  Measured, us on
-  // 128 x 128 / 64 x 64 / 32 x 32 tiles: 8192 x 4096 x 1024 (2048 large tiles) 654 / 746 / 841,
-  // 4096 x 1024 x 1024 (256; 1024 of 64) 120 / 107 / 115, 1024 x 2048 x 512 (512 of 64) 60 / 32 / 36,
-  // 512 x 2048 x 1024 as x^T dy (256 of 64) 118 / 46 / 43, 1024 x 512 x 2048 (128) 190 / 61 / 34,
-  // 128 x 256 x 784 (8) 80 / 28 / 12.
+  // 128 x 128 / 64 x 64 / 32 x 32 tiles: 8192 x 4096 x 1024 (2048 large tiles) 623 / 705 / 858,
+  // 4096 x 1024 x 1024 (256; 1024 of 64) 104 / 94 / 113, 1024 x 2048 x 512 (512 of 64) 56 / 29 / 35,
+  // 1024 x 512 x 2048 (128) 175 / 53 / 33, 128 x 256 x 784 (8) 72 / 25 / 11; as x^T dy the line would lie
+  // lower (512 x 2048 x 1024, 256 of 64: 93 / 32 / 39).
   auto tiles = [&](int64_t edge) { return ((d->M + edge - 1) / edge) * ((d->N + edge - 1) / edge) * d->batch; };
   if (tiles(128) >= 512) return launch_f32<2, 2, 1, 2, 2, 2>(a, akc, bkc, d->batch, st);
   if (tiles(64) >= 512) return launch_f32<2, 2, 1, 1, 1, 4>(a, akc, bkc, d->batch, st);
