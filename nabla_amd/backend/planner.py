@@ -1271,7 +1271,7 @@ class Planner:
         a, b = mm.inputs[:2]
         dt = a.dtype if a.dtype is b.dtype else DType.float32
         # (batched x @ W is one product with all the rows)
-        return self._split_k(_numel(m.shape[:-1]), m.shape[-1], a.shape[-1], dt) == 1
+        return self._split_k(_numel(m.shape[:-1]), m.shape[-1], a.shape[-1], dt, epilogue=True) == 1
 
     def build(self) -> Plan:
         nodes = self._live_nodes()
@@ -1912,9 +1912,10 @@ class Planner:
 
     @staticmethod
     def _split_k(M: int, N: int, K: int, dtype: DType, a_k_contiguous: bool = False,
-                 rows_contiguous: bool = False) -> int:
+                 rows_contiguous: bool = False, epilogue: bool = False) -> int:
         """Slices of the contraction axis for a product whose output has too few 128 x 128
-        tiles to occupy the GPU while K is long (weight gradients: K = batch x sequence)."""
+        tiles to occupy the GPU while K is long (weight gradients: K = batch x sequence).
+        ``epilogue``: what follows the product could be folded into it if it stays whole."""
         if dtype is not DType.bfloat16:
             return 1
         if a_k_contiguous and N <= 32 and M >= 1024 and K % 64 == 0:
@@ -1929,16 +1930,28 @@ class Planner:
             # slices: 67 us and 25)
             return 2
         # The partial products and their sum cost 6 to 10 us, and a split product carries no
-        # epilogue.  Below 4096 the K loop of the 64 x 64 tile is as fast in one piece (512 x 512 x
-        # 1998: 12.4 us, 13.3 in two; 1800 x 1024 x 1024: 11.2 and 22) unless the launch has next to
-        # no workgroups, and so are 4096 deep ones with more than one such tile per CU (1800 x 1024
-        # x 4096: 35.7 and 36.5).  Others are split down to slices of 1024 (1000 x 1024 x 4096 34 ->
-        # 29 us in four), the longest and the smallest ones further (1024 x 1024 x 8192 65 -> 43 in
-        # eight, 256 x 256 x 4096 20 -> 13).
+        # epilogue.  What a launch on few workgroups waits for is its K loop, on 64 x 64 tiles while
+        # there are at most two per CU.  Measured, us whole / in two / four / eight, the sum
+        # included, with eight products of one size in a step:
         small = ((M + 63) // 64) * ((N + 63) // 64)
-        if (small > 32 and K < 4096) or (small > 256 and K < 8192):
-            return 1
-        least = 1024 if small > 32 and K < 8192 else 512
+        if small > 256 and K < 8192:
+            return 1  # (1024 x 1536 x 2048 22 / 24 / 26, 1792 x 1024 x 4096 38 / 42 / 38 / 49)
+        if small > 32 and K < 4096:
+            # Up to about 512 workgroups with slices of 512 and more: 512 x 512 x 2048 21.7 / 16.0 /
+            # 14.7 / 15.3, 512 x 512 x 3072 29 / 19 / 15 / 15, 768 x 768 x 2048 21.7 / 17.0 / 16.9 / 19.5,
+            # 1024 x 1024 x 2048 22.0 / 18.5 / 21.1; at 1024 the two are even (512 x 512 x 1024 15.3 / 15.1).
+            # An epilogue of its own is another launch of 5 us, so one that can be folded keeps the
+            # product whole up to 2048.
+            if K <= (2048 if epilogue else 1024):
+                return 1
+            ks = 1
+            while small * ks * 2 <= 576 and K // (ks * 2) >= 512 and (rows_contiguous or K % (ks * 2 * 64) == 0):
+                ks *= 2
+            return ks
+        # Longer ones down to slices of 1024 (512 x 1024 x 4096 37 / 24 / 19 / 21, 1024 x 1024 x 6144
+        # 52 / 45 / 38 / 38), the longest and the smallest results to slices of 512 (512 x 512 x 4096
+        # 37 / 23 / 17 / 15, 256 x 256 x 4096 36 / 22 / 15 / 14, 1024 x 1024 x 8192 90 / 56 / 46 / 43).
+        least = 1024 if small > 64 and K < 8192 else 512
         ks = 1
         while tiles * ks < 512 and tiles < 128 and K // (ks * 2) >= least and \
                 (rows_contiguous or K % (ks * 2 * 64) == 0):

@@ -84,3 +84,22 @@ def test_a_last_slice_longer_than_the_others_is_refused():
         d.dtype_ab, d.dtype_c, d.alpha, d.k_last = dtype, 0, 1.0, k_last
         with pytest.raises(ValueError, match="k_last"):
             lib.check(L.nbk_gemm(C.byref(d), None))
+
+
+def test_few_workgroups_and_a_middling_contraction_are_split():
+    """Results of 33 to 256 tiles of 64 x 64 wait for one workgroup's loop over K: whole, 512 x 512 x
+    3072 takes twice what it takes in four slices.  What can be folded into the product outweighs
+    that up to 2048."""
+    from nabla_amd.backend.planner import Planner
+    for kind in (dict(rows_contiguous=True), dict(a_k_contiguous=True)):
+        def split(M, N, K, **kw):
+            return Planner._split_k(M, N, K, nb.DType.bfloat16, **kind, **kw)
+        assert split(512, 512, 1024) == 1
+        assert split(512, 512, 1536) == 2 and split(1024, 1024, 1536) == 2
+        assert split(512, 512, 2048) == 4 and split(512, 512, 3072) == 4
+        assert split(768, 768, 2048) == 4 and split(1024, 1024, 3072) == 2
+        assert split(512, 512, 4096) == 8 and split(512, 1024, 4096) == 4
+        assert split(1024, 1536, 2048) == 1 and split(1792, 1024, 4096) == 1
+        assert split(512, 512, 2048, epilogue=True) == 1 and split(512, 512, 3072, epilogue=True) == 4
+    assert Planner._split_k(512, 512, 1998, nb.DType.bfloat16, rows_contiguous=True) == 2
+    assert Planner._split_k(512, 512, 1998, nb.DType.bfloat16, a_k_contiguous=True) == 1
