@@ -2168,14 +2168,22 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
     return !(akc && bkc) ? launch_bf16_dl<128, 128, 4, 1, true>(a, akc, bkc, d->batch, st)
                          : launch_bf16_dl<128, 128, 4, 1, false>(a, akc, bkc, d->batch, st);
   }
-  // The largest tile that still gives every CU two workgroups: below that the K loop of one workgroup
-  // is what a launch waits for, and the more waves share a CU the less of it shows.  Measured, us on
-  // 128 x 128 / 64 x 64 / 32 x 32 tiles: 8192 x 4096 x 1024 (2048 large tiles) 623 / 705 / 858,
-  // 4096 x 1024 x 1024 (256; 1024 of 64) 104 / 94 / 113, 1024 x 2048 x 512 (512 of 64) 56 / 29 / 35,
-  // 1024 x 512 x 2048 (128) 175 / 53 / 33, 128 x 256 x 784 (8) 72 / 25 / 11; as x^T dy the line would lie
-  // lower (512 x 2048 x 1024, 256 of 64: 93 / 32 / 39).
+  // Two workgroups run on a CU at a time.  A round of 128 x 128 tiles does the work of four of 64 x 64
+  // in the time of four, or of 3.5 where K is long; so the larger tile is taken where it fills the
+  // chip and needs no more than that, its last round and what lies past the edges counted.  Short contractions are all
+  // prologue and epilogue, and the smaller tile overlaps them better.  Measured, us on 128 x 128 / 64 x 64:
+  // 8192 x 4096 x 1024 (2048 large tiles) 623 / 705, 8 x (1024 x 1024 x 1024) (512) 160 / 184, 5000 x 3000
+  // x 256 (960) 108 / 111; 3072 x 2944 x 1024 (552) 258 / 204, 64 x (333 x 333 x 64) (576) 56 / 40, 64 x
+  // (64 x 999 x 256) (512, half of them empty) 61 / 38, 4096 x 4096 x 64 (1024) 65 / 62.
+  // Below two small tiles per CU the K loop of one workgroup is what a launch waits for, and the
+  // more waves share a CU the less of it shows: on 64 x 64 / 32 x 32 tiles 1024 x 2048 x 512 (512 of 64)
+  // 29 / 35, 1024 x 512 x 2048 (128) 53 / 33, 128 x 256 x 784 (8) 25 / 11; as x^T dy the line would lie
+  // lower (512 x 2048 x 1024, 256 of 64: 32 / 39).
   auto tiles = [&](int64_t edge) { return ((d->M + edge - 1) / edge) * ((d->N + edge - 1) / edge) * d->batch; };
-  if (tiles(128) >= 512) return launch_f32<2, 2, 1, 2, 2, 2>(a, akc, bkc, d->batch, st);
+  const int64_t slots = 2 * (int64_t)nbk_num_cus();
+  auto rounds = [&](int64_t edge) { return (tiles(edge) + slots - 1) / slots; };
+  if (tiles(128) >= slots && d->K >= 256 && rounds(128) * 80 <= rounds(64) * (d->K >= 512 ? 23 : 20))
+    return launch_f32<2, 2, 1, 2, 2, 2>(a, akc, bkc, d->batch, st);
   if (tiles(64) >= 512) return launch_f32<2, 2, 1, 1, 1, 4>(a, akc, bkc, d->batch, st);
   return launch_f32<1, 1, 4, 1, 1, 2>(a, akc, bkc, d->batch, st);
 }

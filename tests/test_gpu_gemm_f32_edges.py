@@ -10,8 +10,8 @@ import torch
 pytestmark = pytest.mark.gpu
 
 SIZES = [(m, n, k) for m, n in [(1, 3), (2, 1), (3, 2), (4, 5), (5, 4), (33, 34), (35, 67), (63, 31)] for k in (3, 64, 131)]
-SIZES += [(1473, 1475, 35), (1474, 1474, 32)]  # 64 x 64 tiles
-SIZES += [(2817, 2945, 17), (2818, 2947, 16), (2819, 2946, 33)]  # 128 x 128 tiles
+SIZES += [(1473, 1475, 35), (1474, 1474, 32), (2817, 2945, 17), (2818, 2947, 16)]  # 64 x 64 tiles
+SIZES += [(3969, 1923, 257), (3970, 1922, 256), (3971, 1921, 290), (4096, 2048, 259)]  # 128 x 128 tiles
 
 
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])

@@ -56,7 +56,7 @@ def product(L, M, N, K, layout, batch=(1, 1), odd=0, epilogue=False):
 
 SIZES = [(1, 1, 1), (32, 32, 64), (33, 31, 65), (200, 32, 3), (129, 65, 784), (513, 700, 63), (1000, 513, 129),  # 32 x 32
          (2048, 1024, 96), (1477, 1477, 37),  # 64 x 64
-         (4096, 2048, 48), (4099, 2051, 17)]  # 128 x 128
+         (4096, 2048, 48), (4099, 2051, 17)]  # (more of them: 128 x 128 ones take contractions of 256 and more)
 
 
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
