@@ -2137,15 +2137,24 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
     // for four MFMAs, the 128 x 128 tile eight for sixteen).  Measured, 64 / 128: 1998 x 512 x 512
     // 6.3 / 9.5 us, 512 x 512 x 1998 (x^T dy) 12.4 / 20.5, 1800 x 1024 x 1024 (464 small tiles) 11.2 /
     // 14.4; past two per CU it turns: 1000 x 4096 x 1024 (1024 small tiles) 17.1 / 14.9.
-    constexpr int64_t SMALL_TILES = 512;
-    const int64_t small_tiles = ((d->M + 63) / 64) * ((d->N + 63) / 64) * d->batch;
+    // A batch of products of one large tile each is the exception from one small tile per CU on: the four
+    // small ones lie on different XCDs, and each fetches its part of the operands again.  It shows where
+    // a row-contiguous operand ends inside a tile, whose rows lie across cache lines (90 x (104 x 104 x
+    // 512) as x^T dy 14.0 / 10.4, x 128 7.1 / 6.3), and on long contractions (128 x (128 x 128 x 512)
+    // 13.5 / 12.1, x 128 7.2 / 7.5).
+    const bool ragged = (!akc && d->M % 64 != 0) || (!bkc && d->N % 64 != 0);
+    const int64_t tiles_64 = ((d->M + 63) / 64) * ((d->N + 63) / 64) * d->batch;
+    const bool one_each = d->batch > 1 && d->M <= 128 && d->N <= 128 && tiles_64 > 256 &&
+                          (d->M > 64 || d->N > 64) &&
+                          ((ragged && d->K >= 128) || (d->K >= 512 && d->M % 64 == 0 && d->N % 64 == 0));
+    const bool small = tiles_64 <= 512 && !one_each;
     if (d->colsum != nullptr) {
       NBK_REQUIRE(fast && !akc && !bkc && d->bias == nullptr &&
                       d->residual == nullptr && d->act == NBK_ACT_NONE && d->alpha == 1.f,
                   "gemm: column sums go with a plain bf16 product of two row-contiguous, 16-byte "
                   "aligned operands (M %% 8 == 0, N %% 8 == 0)");
-      return small_tiles <= SMALL_TILES ? launch_bf16_dl_colsum<64, 64, 4>(a, d->batch, st)
-                                        : launch_bf16_dl_colsum<128, 128, 4>(a, d->batch, st);
+      return small ? launch_bf16_dl_colsum<64, 64, 4>(a, d->batch, st)
+                   : launch_bf16_dl_colsum<128, 128, 4>(a, d->batch, st);
     }
     if (!fast) return launch_bf16<128, 128>(a, akc, bkc, d->batch, st);
     // 256 x 256 tiles run at about twice the rate of 128 x 128 ones per CU, one workgroup
@@ -2159,7 +2168,7 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
     // (eight waves on the big tile: 8-16 % faster than four on every shape measured)
     if (big_tiles * 10 >= rounds * cus * 6 && d->M >= 256 && d->N >= 256 && d->K > 128)
       return launch_bf16_dl<256, 256, 8, 1, true>(a, akc, bkc, d->batch, st);
-    if (small_tiles <= SMALL_TILES) return launch_bf16_dl<64, 64, 4, 1, true>(a, akc, bkc, d->batch, st);
+    if (small) return launch_bf16_dl<64, 64, 4, 1, true>(a, akc, bkc, d->batch, st);
     // (a 256 x 128 tile was measured and is no faster than 128 x 128 on mid-sized problems:
     // with one workgroup per CU a short K loop is bound by load latency, and two co-resident
     // 128 x 128 workgroups hide it better)
