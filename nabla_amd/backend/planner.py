@@ -1971,8 +1971,8 @@ class Planner:
     def _colsum_key(ra: ViewRef, rb: ViewRef, pa, pb, M: int, N: int, K: int, ks: int, epi: dict):
         """What a deferred column sum must name to ride on this product (one launch, or ``ks``
         slices of K): the right operand is a whole row-major [K, N] bf16 matrix, the left one is
-        row-contiguous too, and the launch is one that takes the 128 x 128 tile anyway (the
-        kernel that carries the sums), with the alignment its direct loads ask for."""
+        row-contiguous too, and the launch is one that takes the 64 x 64 or 128 x 128 tile anyway
+        (the kernels that carry the sums), with the alignment their direct loads ask for."""
         if epi or ra.dtype is not DType.bfloat16 or rb.dtype is not DType.bfloat16:
             return None
         if not (pa[1] == 1 and pa[2] != 1 and pb[2] == 1 and pb[1] == N):

@@ -1020,7 +1020,7 @@ static int attn_common(const nbk_attn_desc* d, AttnArgs* a) {
   NBK_REQUIRE(d->dtype == NBK_BF16, "attention: only bf16 is implemented (dtype %d)", d->dtype);
   NBK_REQUIRE(d->hd == 64 || d->hd == 128, "attention: head size %lld must be 64 or 128", (long long)d->hd);
   NBK_REQUIRE(d->B > 0 && d->H > 0 && d->S > 0 && (d->any_length || d->S % 128 == 0),
-              "attention: B %lld, H %lld, S %lld (S must be a positive multiple of 128)",
+              "attention: B %lld, H %lld, S %lld (all positive, and S a multiple of 128 unless any_length is set)",
               (long long)d->B, (long long)d->H, (long long)d->S);
   NBK_REQUIRE(d->B * d->H <= 0x7fffffffLL && (d->S + 127) / 128 <= 65535, "attention: extent beyond the grid limits");
   a->B = (int32_t)d->B; a->H = (int32_t)d->H; a->S = (int32_t)d->S;

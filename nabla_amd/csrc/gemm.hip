@@ -2134,9 +2134,9 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
     }
     // 64 x 64 tiles while two of them per CU hold the whole result: such a launch is bound by the
     // latency of its K loop, not by the LDS reads a small tile repeats (a wave reads four fragments
-    // for four MFMAs, the 128 x 128 tile eight for sixteen).  Measured, 64 / 128: 1998 x 512 x 512
-    // 6.3 / 9.5 us, 512 x 512 x 1998 (x^T dy) 12.4 / 20.5, 1800 x 1024 x 1024 (464 small tiles) 11.2 /
-    // 14.4; past two per CU it turns: 1000 x 4096 x 1024 (1024 small tiles) 17.1 / 14.9.
+    // for four MFMAs, the 128 x 128 tile eight for sixteen).  Measured on operands in the nearest cache,
+    // 64 / 128: 1998 x 512 x 512 6.3 / 9.5 us, 512 x 512 x 1998 (x^T dy) 12.4 / 20.5, 1800 x 1024 x 1024 (464
+    // small tiles) 11.2 / 14.4; past two per CU it turns: 1000 x 4096 x 1024 (1024 small tiles) 17.1 / 14.9.
     // A batch of products of one large tile each is the exception from one small tile per CU on: the four
     // small ones lie on different XCDs, and each fetches its part of the operands again.  It shows where
     // a row-contiguous operand ends inside a tile, whose rows lie across cache lines (90 x (104 x 104 x
@@ -2198,8 +2198,9 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
 }
 
 // ------------------------------------------------------------------ NF4-coded weights
-// A whole weight from its codes, eight per lane: bound by memory (one byte read and two or four
-// written per weight: 4 M bf16 weights 7.1 us, 1.8 TB/s with the launch).
+// A whole weight from its codes, eight per lane.  One byte is read and two or four are written per
+// weight, yet weights of a usual size take what a launch and one trip to memory and back take: 4 M
+// bf16 weights 7.1 us, 1.8 TB/s where a large copy reaches 7.0.
 template <typename T>
 __global__ __launch_bounds__(256) void nf4_decode_kernel(const uint8_t* codes, const float* scales, T* w,
                                                          uint32_t groups, uint32_t groups_per_block) {

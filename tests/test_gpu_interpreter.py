@@ -59,8 +59,7 @@ def test_rows_of_every_length(interpreted, cols, dtype):
 
 @pytest.mark.parametrize("n_inputs", [1, 6, 9, 12])
 def test_many_inputs_shared_by_two_phases(interpreted, n_inputs):
-    """More inputs than are requested ahead, each read before and after a reduction: the values
-    the phases share need the large register file, or are computed again."""
+    """More inputs than are requested ahead, each read before and after a reduction."""
     rows, cols = 130, 200
     rng = np.random.default_rng(n_inputs)
     xs = [tensor(rng.standard_normal((rows, cols)).astype(np.float32), "float32") for _ in range(n_inputs)]
