@@ -185,6 +185,8 @@ def program(ins, n_operands, cols, reduce, moves=()):
     for i in range(n_operands):
         rp.operand[i].ptr, rp.operand[i].col_stride, rp.operand[i].stage_slot = 4096, 1, -1
         rp.operand[i].lead_stride[0] = cols if i in moves else 0
+    for i in range(isa.MAX_IMM):
+        rp.imm[i] = i - isa.MAX_IMM // 2
     ins = ins + [(isa.HALT, 0, 0, 0, 0, 0)]
     assert len(ins) <= isa.MAX_INS
     rp.n_ins = len(ins)
@@ -241,15 +243,28 @@ def shared_inputs_program(rng):
     return program(ins, n_in + 3, rng.choice([1, 100, 1003]), True, range(n_in + 3))
 
 
-def random_program(rng):
+def inputs_and_stores(rp):
+    """Operands that the program loads, and those that it stores."""
+    loads, stores = set(), set()
+    for i in range(rp.n_ins):
+        n = rp.ins[i]
+        if n.op in (isa.LDG, isa.LDR):
+            loads.add(n.a)
+        elif n.op in (isa.STG, isa.STR):
+            stores.add(n.dst)
+    return loads, stores
+
+
+def random_program(rng, exact=False):
     """A valid program: bodies that read what they or the prologues wrote, reductions between
-    them, inputs read again, row scalars loaded twice, all registers in use."""
+    them, inputs read again, row scalars loaded twice, all registers in use.  ``exact``: operations that
+    keep whole numbers, no integer registers, and outputs that are only written."""
     reduce, once = rng.random() < 0.75, rng.random() < 0.7  # (once: accumulators that rows in registers can have)
     n_in, n_out = rng.randint(1, 14), rng.randint(1, 5)
     n_vec, n_scl = rng.choice([4, 8, 12, 16, 16]), rng.choice([3, 8, 16])
-    moves = [i for i in range(n_in + n_out) if rng.random() < 0.7]
-    ops1 = [isa.UNARY[k] for k in ("neg", "exp", "relu")]
-    ops2 = [isa.BINARY[k] for k in ("add", "sub", "mul", "gt")]
+    moves = [i for i in range(n_in + n_out) if rng.random() < 0.7 or exact and i >= n_in]
+    ops1 = [isa.UNARY[k] for k in ("neg", "abs" if exact else "exp", "relu")]
+    ops2 = [isa.BINARY[k] for k in (("gt", "sub", "gt") if exact else ("add", "sub", "mul", "gt"))]
     scalars, ins, started = [], [], {}
 
     def ew(regs, dst):
@@ -258,7 +273,7 @@ def random_program(rng):
             return (rng.choice(ops1), dst, rng.choice(regs), 0, 0, 0)
         if kind < 0.8:
             return (rng.choice(ops2), dst, rng.choice(regs), rng.choice(regs), 0, 0)
-        return (rng.choice(sorted(TERNARY)), dst, *(rng.choice(regs) for _ in range(3)), 0)
+        return (isa.TERNARY["where"] if exact else rng.choice(sorted(TERNARY)), dst, *(rng.choice(regs) for _ in range(3)), 0)
 
     for _ in range(rng.randint(1, 4)):
         for _ in range(rng.randint(0, 2 + n_scl // 2)):
@@ -269,7 +284,7 @@ def random_program(rng):
             elif kind < 0.6 or not scalars:
                 ins.append((isa.IMM, dst, rng.randrange(isa.MAX_IMM), 0, 0, 0))
             elif kind < 0.7:
-                ins.append((isa.LEADIDX, dst, 0, rng.randint(0, 1), 0, 0))
+                ins.append((isa.LEADIDX, dst, 0, 0 if exact else rng.randint(0, 1), 0, 0))
             elif kind < 0.75:
                 ins.append((isa.STR, n_in + rng.randrange(n_out), rng.choice(scalars), 0, 0, 0))
                 continue
@@ -279,7 +294,7 @@ def random_program(rng):
         if reduce:
             for k in range(isa.NACC):
                 if rng.random() < 0.6 and not (once and started.get(k, (0, 0))[1]):
-                    kind = rng.randrange(3)
+                    kind = rng.randrange(1 if exact else 0, 3)
                     ins.append((isa.ACCINIT, k, kind, 0, 0, 0))
                     started[k] = [kind, 0]
         vecs, b = [], []
@@ -287,9 +302,9 @@ def random_program(rng):
             dst = rng.randrange(n_vec)
             kind = rng.random()
             if kind < 0.4 or not vecs:
-                b.append((isa.LDG, dst, rng.randrange(n_in + (n_out if rng.random() < 0.1 else 0)), 0, 0, 0))
+                b.append((isa.LDG, dst, rng.randrange(n_in + (n_out if rng.random() < 0.1 and not exact else 0)), 0, 0, 0))
             elif kind < 0.43:
-                b.append((isa.COLIDX, dst, rng.randint(0, 1), 0, 0, 0))
+                b.append((isa.COLIDX, dst, 0 if exact else rng.randint(0, 1), 0, 0, 0))
             elif kind < 0.5:
                 b.append((isa.STG, n_in + rng.randrange(n_out), rng.choice(vecs + scalars), 0, 0, 0))
                 continue
