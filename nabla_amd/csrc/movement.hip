@@ -149,202 +149,177 @@ extern "C" int nbk_fill(void* dst, int32_t dtype, int64_t n, double value, void*
 }
 
 // ---- reduction over a middle axis ---------------------------------------------
-// in [outer, red, inner] -> out [outer, inner].  Lanes run along `inner`
-// (coalesced); each workgroup owns a 64-column strip and splits `red` over its
-// four waves, then combines the four partials through LDS.  (A long axis over few
-// columns is cut into slices by the caller: two launches, fp32 partials in between.)
+// in [outer, red, inner] -> out [outer, inner].  A workgroup of 256 lanes owns a strip of
+// `lx` (1 .. 256, a power of two) neighbouring pieces of the row and walks the reduced axis
+// 256 / lx rows abreast; the partial sums of a column meet across lanes, then in LDS.
+// What bounds it is how many workgroups there are: one CU takes rows from the other XCDs' results
+// at 15 to 35 GB/s whatever it keeps in flight (4 or 8 rows per lane measured the same), and
+// a wavefront that waits for one row after the other is pure latency.  So the strip is as narrow
+// as it takes to give every CU work (reduce_strip).  The earlier form had strips of 64 to 256
+// pieces and rows four abreast, and where the row was shorter most of its lanes idled; times in
+// us, before and after, behind a kernel that has just written the operand: 128x256 fp32 10.7 / 4.5,
+// 200x32 15.1 / 3.5, 27 x (74x512) bf16 15.1 / 5.4, 32 x (256x1024) bf16 65.7 / 14.1, 64x4096
+// fp32 17.7 / 3.3, 50 x (196x72) 16.2 / 5.7, the four halves of a split product 4x786432 11.0 / 9.3.
+// (A long axis over few columns is cut into slices by the caller: two launches, fp32 partials
+// in between.)
 __device__ __forceinline__ float red_comb(float a, float b, int kind) {
   return kind == NBK_RED_SUM ? a + b : (kind == NBK_RED_MAX ? fmaxf(a, b) : fminf(a, b));
 }
-__device__ __forceinline__ void reduce_mid_body(const void* __restrict__ in, void* __restrict__ out,
-                                                int dti, int dto, int64_t red, int64_t inner,
-                                                int kind, int64_t bx, int64_t o) {
-  __shared__ float part[4][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t col = bx * 64 + lane;
-  float acc = kind == NBK_RED_SUM ? 0.f : (kind == NBK_RED_MAX ? -INFINITY : INFINITY);
-  if (col < inner) {
-    const int64_t base = o * red * inner + col;
-    // four accumulators; sixteen loads in flight while the axis is long enough (a short axis
-    // over few columns is pure latency: every round trip saved shows), then four
-    float a0 = acc, a1 = acc, a2 = acc, a3 = acc;
-    int64_t r = w;
-    for (; r + 60 < red; r += 64) {
-      float v[16];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) v[q] = nbk_load_as_f32(in, base + (r + 4 * q) * inner, dti);
-#pragma unroll
-      for (int q = 0; q < 16; q += 4) {
-        a0 = red_comb(a0, v[q], kind); a1 = red_comb(a1, v[q + 1], kind);
-        a2 = red_comb(a2, v[q + 2], kind); a3 = red_comb(a3, v[q + 3], kind);
-      }
-    }
-    for (; r + 12 < red; r += 16) {
-      float v0 = nbk_load_as_f32(in, base + r * inner, dti);
-      float v1 = nbk_load_as_f32(in, base + (r + 4) * inner, dti);
-      float v2 = nbk_load_as_f32(in, base + (r + 8) * inner, dti);
-      float v3 = nbk_load_as_f32(in, base + (r + 12) * inner, dti);
-      a0 = red_comb(a0, v0, kind); a1 = red_comb(a1, v1, kind);
-      a2 = red_comb(a2, v2, kind); a3 = red_comb(a3, v3, kind);
-    }
-    for (; r < red; r += 4) a0 = red_comb(a0, nbk_load_as_f32(in, base + r * inner, dti), kind);
-    acc = red_comb(red_comb(a0, a1, kind), red_comb(a2, a3, kind), kind);
+// A piece of a row: 16 bytes where the rows allow it, else one element.
+struct RedF32x4 {
+  typedef uint4 raw;
+  static constexpr int N = 4;
+  static __device__ __forceinline__ void unpack(const uint4 u, int, float* v) {
+    v[0] = __uint_as_float(u.x); v[1] = __uint_as_float(u.y);
+    v[2] = __uint_as_float(u.z); v[3] = __uint_as_float(u.w);
   }
-  part[w][lane] = acc;
+  static __device__ __forceinline__ uint4 load(const void* p, int64_t i, int) { return ((const uint4*)p)[i]; }
+};
+struct RedBf16x8 {
+  typedef uint4 raw;
+  static constexpr int N = 8;
+  static __device__ __forceinline__ void unpack(const uint4 u, int, float* v) {
+    v[0] = __uint_as_float(u.x << 16); v[1] = __uint_as_float(u.x & 0xffff0000u);
+    v[2] = __uint_as_float(u.y << 16); v[3] = __uint_as_float(u.y & 0xffff0000u);
+    v[4] = __uint_as_float(u.z << 16); v[5] = __uint_as_float(u.z & 0xffff0000u);
+    v[6] = __uint_as_float(u.w << 16); v[7] = __uint_as_float(u.w & 0xffff0000u);
+  }
+  static __device__ __forceinline__ uint4 load(const void* p, int64_t i, int) { return ((const uint4*)p)[i]; }
+};
+struct RedF32 {
+  typedef float raw;
+  static constexpr int N = 1;
+  static __device__ __forceinline__ void unpack(const float u, int, float* v) { v[0] = u; }
+  static __device__ __forceinline__ float load(const void* p, int64_t i, int) { return ((const float*)p)[i]; }
+};
+struct RedBf16 {
+  typedef uint16_t raw;
+  static constexpr int N = 1;
+  static __device__ __forceinline__ void unpack(const uint16_t u, int, float* v) { v[0] = nbk_bf16_to_f32(u); }
+  static __device__ __forceinline__ uint16_t load(const void* p, int64_t i, int) { return ((const uint16_t*)p)[i]; }
+};
+struct RedAny {
+  typedef float raw;
+  static constexpr int N = 1;
+  static __device__ __forceinline__ void unpack(const float u, int, float* v) { v[0] = u; }
+  static __device__ __forceinline__ float load(const void* p, int64_t i, int dt) { return nbk_load_as_f32(p, i, dt); }
+};
+constexpr int RED_FLIGHT = 8;  // rows in flight per lane
+
+template <typename P>
+__device__ __forceinline__ void reduce_strip_body(const void* __restrict__ in, void* __restrict__ out,
+                                                  int dti, int dto, int64_t red, int64_t inner, int kind,
+                                                  int64_t bx, int64_t o, int lxs, float* part) {
+  constexpr int N = P::N;
+  const int LX = 1 << lxs, RY = 256 >> lxs;
+  const int64_t pieces = inner / N;
+  const int64_t at = bx * LX + (threadIdx.x & (LX - 1));
+  const int64_t base = o * red * pieces + (at < pieces ? at : pieces - 1);
+  const float ident = kind == NBK_RED_SUM ? 0.f : (kind == NBK_RED_MAX ? -INFINITY : INFINITY);
+  float acc[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) acc[e] = ident;
+  auto add = [&](const typename P::raw u) {
+    float v[N];
+    P::unpack(u, dti, v);
+#pragma unroll
+    for (int e = 0; e < N; ++e) acc[e] = red_comb(acc[e], v[e], kind);
+  };
+  const int64_t step = (int64_t)RY * pieces;
+  int64_t r = threadIdx.x >> lxs, i = base + r * pieces;
+#pragma unroll 1
+  for (; r + (RED_FLIGHT - 1) * RY < red; r += RED_FLIGHT * RY, i += RED_FLIGHT * step) {
+    typename P::raw u[RED_FLIGHT];
+#pragma unroll
+    for (int q = 0; q < RED_FLIGHT; ++q) u[q] = P::load(in, i + q * step, dti);
+#pragma unroll
+    for (int q = 0; q < RED_FLIGHT; ++q) add(u[q]);
+  }
+  if (r < red) {  // the rows left, requested together too
+    typename P::raw u[RED_FLIGHT - 1];
+#pragma unroll
+    for (int q = 0; q < RED_FLIGHT - 1; ++q) u[q] = P::load(in, r + q * RY < red ? i + q * step : i, dti);
+#pragma unroll
+    for (int q = 0; q < RED_FLIGHT - 1; ++q)
+      if (r + q * RY < red) add(u[q]);
+  }
+  if (RY == 1) {  // a column is one lane's: no partial sums to meet
+    if (at >= pieces) return;
+    const int64_t to = o * pieces + at;
+    const bool whole = N == 4 && ((uintptr_t)out & 15) == 0;
+    if (whole && dto == NBK_F32) {
+      ((float4*)out)[to] = make_float4(acc[0], acc[1 % N], acc[2 % N], acc[3 % N]);
+    } else if (whole && dto == NBK_BF16) {
+      ((uint2*)out)[to] = make_uint2((uint32_t)nbk_f32_to_bf16(acc[0]) | ((uint32_t)nbk_f32_to_bf16(acc[1 % N]) << 16),
+                                     (uint32_t)nbk_f32_to_bf16(acc[2 % N]) | ((uint32_t)nbk_f32_to_bf16(acc[3 % N]) << 16));
+    } else {
+#pragma unroll
+      for (int e = 0; e < N; ++e) nbk_store_from_f32(out, to * N + e, dto, acc[e]);
+    }
+    return;
+  }
+  for (int s = LX; s < 64; s <<= 1)  // rows that share a wavefront
+#pragma unroll
+    for (int e = 0; e < N; ++e) acc[e] = red_comb(acc[e], __shfl_xor(acc[e], s), kind);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lanes = LX < 64 ? LX : 64, across = LX >> 6 ? LX >> 6 : 1;
+  if (lane < lanes)
+#pragma unroll
+    for (int e = 0; e < N; ++e) part[wave * (64 * N) + lane * N + e] = acc[e];
   __syncthreads();
-  if (w == 0 && col < inner) {
-    float v = red_comb(red_comb(part[0][lane], part[1][lane], kind),
-                       red_comb(part[2][lane], part[3][lane], kind), kind);
+  const int cols = lanes * N;  // of one wavefront
+  for (int c = threadIdx.x; c < across * cols; c += 256) {
+    const int64_t col = bx * LX * N + c;
+    if (col >= inner) break;
+    const float* p = part + (c / cols) * (64 * N) + c % cols;
+    float v = p[0];
+    for (int k = across; k < 4; k += across) v = red_comb(v, p[k * (64 * N)], kind);
     nbk_store_from_f32(out, o * inner + col, dto, v);
   }
 }
-__global__ __launch_bounds__(256) void reduce_mid_kernel(const void* __restrict__ in,
-                                                         void* __restrict__ out, int dti, int dto,
-                                                         int64_t red, int64_t inner, int kind) {
-  reduce_mid_body(in, out, dti, dto, red, inner, kind, blockIdx.x, blockIdx.y);
+// How a reduction is laid out, a function of its own shape alone: the order of summation, and so
+// the result, does not depend on how reductions are grouped into launches.
+struct RedLayout {
+  int mode;  // 1: bf16 by 16 bytes, 2: fp32 by 16 bytes; by element 3: bf16, 4: fp32, 0: other types
+  int lxs;   // log2 of the strip's width in pieces
+  int64_t blocks_x;
+};
+// The strip: 256 pieces, halved while the launch has fewer than 1024 workgroups and there are rows
+// left to put abreast.  Down to 256 bytes of a row the narrower strip is never slower; below that
+// two workgroups share cache lines, which pays for launches that leave half of the chip idle (128
+// bytes from 512 workgroups down: 32 x (256x1024) bf16 16.3 -> 14.1 us; 64 bytes only with more
+// than eight rows per lane left: 64 x (1024x64) fp32 16.4 -> 12.2, but 27 x (74x512) bf16 5.4 -> 6.3).
+static RedLayout reduce_layout(const void* in, int dti, int64_t outer, int64_t red, int64_t inner) {
+  RedLayout L;
+  const bool aligned = ((uintptr_t)in & 15) == 0;
+  L.mode = dti == NBK_BF16 ? (aligned && inner % 8 == 0 ? 1 : 3) : dti == NBK_F32 ? (aligned && inner % 4 == 0 ? 2 : 4) : 0;
+  const int64_t pieces = inner / (L.mode == 1 ? 8 : L.mode == 2 ? 4 : 1);
+  int s = 0;
+  while (s < 8 && (1ll << s) < pieces) ++s;
+  const int whole = L.mode == 1 || L.mode == 2 ? 4 : 5;  // 256 bytes of a row (fp32 by element: 128)
+  // (a few long rows, the partial products of a GEMM split along K, are added in their order: a
+  // strip of 256 is as fast there, 4 x 65536 2.1 us)
+  const bool in_order = L.mode == 2 && red <= 8 && inner >= 65536;
+  for (; !in_order && s > 0 && (256 >> s) < red; --s) {
+    const int64_t blocks = outer * ((pieces + (1ll << s) - 1) >> s);
+    const bool narrower = s > whole ? blocks < 1024 : s == whole ? blocks < 512
+                        : s == whole - 1 && blocks < 256 && red * (1ll << s) > 8 * 256;
+    if (!narrower) break;
+  }
+  L.lxs = s;
+  L.blocks_x = (pieces + (1ll << s) - 1) >> s;
+  return L;
 }
-
-// Vector form: a lane owns VEC consecutive columns (16 bytes of input per row), a
-// workgroup 64 * VEC columns; its four waves take every fourth row and keep up to
-// sixteen row loads in flight each.  T is the input element (uint16_t = bf16, float).
-template <typename T, int VEC>
-__device__ __forceinline__ void reduce_mid_vec_body(const T* __restrict__ in, void* __restrict__ out,
-                                                    int dto, int64_t red, int64_t inner, int kind,
-                                                    int64_t bx, int64_t o, int wc) {
-  // The four waves stand wc (1, 2 or 4) side by side along the row and 4 / wc deep along the
-  // reduced axis: a wide row is read in long contiguous runs, and a short reduced axis (the
-  // partial sums of a split product) still keeps every wave busy.
-  __shared__ float part[4][64][VEC + 1];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wcid = w % wc, wr = w / wc, WR = 4 / wc;
-  const int64_t col = ((bx * wc + wcid) * 64 + lane) * VEC;
-  const float ident = kind == NBK_RED_SUM ? 0.f : (kind == NBK_RED_MAX ? -INFINITY : INFINITY);
-  float acc[VEC];
-#pragma unroll
-  for (int e = 0; e < VEC; ++e) acc[e] = ident;
-  if (col < inner) {
-    const T* base = in + o * red * inner + col;
-    auto unpack = [&](const uint4 u, float* v) {
-      if (sizeof(T) == 2) {
-        v[0] = __uint_as_float(u.x << 16); v[1] = __uint_as_float(u.x & 0xffff0000u);
-        v[2] = __uint_as_float(u.y << 16); v[3] = __uint_as_float(u.y & 0xffff0000u);
-        v[4 % VEC] = __uint_as_float(u.z << 16); v[5 % VEC] = __uint_as_float(u.z & 0xffff0000u);
-        v[6 % VEC] = __uint_as_float(u.w << 16); v[7 % VEC] = __uint_as_float(u.w & 0xffff0000u);
-      } else {
-        v[0] = __uint_as_float(u.x); v[1] = __uint_as_float(u.y);
-        v[2] = __uint_as_float(u.z); v[3] = __uint_as_float(u.w);
-      }
-    };
-    auto load = [&](int64_t r, float* v) { unpack(*(const uint4*)(base + r * inner), v); };
-    int64_t r = wr;
-    for (; r + 15 * WR < red; r += 16 * WR) {  // sixteen rows in flight, kept packed until added
-      uint4 raw[16];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) raw[q] = *(const uint4*)(base + (r + WR * q) * inner);
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        float v[VEC];
-        unpack(raw[q], v);
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) acc[e] = red_comb(acc[e], v[e], kind);
-      }
-    }
-    for (; r + 7 * WR < red; r += 8 * WR) {
-      float v[8][VEC];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) load(r + WR * q, v[q]);
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) acc[e] = red_comb(acc[e], v[q][e], kind);
-    }
-    for (; r < red; r += WR) {
-      float v[VEC];
-      load(r, v);
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) acc[e] = red_comb(acc[e], v[e], kind);
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < VEC; ++e) part[w][lane][e] = acc[e];
-  __syncthreads();
-  if (wr == 0 && col < inner) {
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      float v = part[wcid][lane][e];
-      for (int k = 1; k < WR; ++k) v = red_comb(v, part[k * wc + wcid][lane][e], kind);
-      nbk_store_from_f32(out, o * inner + col + e, dto, v);
-    }
-  }
-}
-// A few rows of a long fp32 row (the partial products of a GEMM split along K): one 16-byte piece
-// per lane and row, as above, is too little work per lane and leaves two loads in flight.  Here a
-// lane sums FEW_CPL pieces of the row, two rows of all of them requested at once, and stores
-// whole pieces.  Same order of summation as above (row 0 first), so the same results.
-constexpr int FEW_CPL = 4;
-__device__ __forceinline__ void reduce_few_rows_body(const float* __restrict__ in, void* __restrict__ out,
-                                                     int dto, int64_t red, int64_t inner, int kind,
-                                                     int64_t bx, int64_t o) {
-  const int64_t chunks = inner >> 2;
-  const float4* base = (const float4*)(in + o * red * inner);
-  const float ident = kind == NBK_RED_SUM ? 0.f : (kind == NBK_RED_MAX ? -INFINITY : INFINITY);
-  int64_t c[FEW_CPL];
-  float4 acc[FEW_CPL];
-#pragma unroll
-  for (int j = 0; j < FEW_CPL; ++j) {
-    c[j] = bx * (256 * FEW_CPL) + j * 256 + threadIdx.x;
-    acc[j] = make_float4(ident, ident, ident, ident);
-  }
-  auto add = [&](float4& a, const float4 v) {
-    a.x = red_comb(a.x, v.x, kind); a.y = red_comb(a.y, v.y, kind);
-    a.z = red_comb(a.z, v.z, kind); a.w = red_comb(a.w, v.w, kind);
-  };
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  int64_t r = 0;
-  for (; r + 1 < red; r += 2) {
-    float4 v0[FEW_CPL], v1[FEW_CPL];
-#pragma unroll
-    for (int j = 0; j < FEW_CPL; ++j) {
-      v0[j] = c[j] < chunks ? base[r * chunks + c[j]] : zero;
-      v1[j] = c[j] < chunks ? base[(r + 1) * chunks + c[j]] : zero;
-    }
-#pragma unroll
-    for (int j = 0; j < FEW_CPL; ++j) { add(acc[j], v0[j]); add(acc[j], v1[j]); }
-  }
-  if (r < red) {
-#pragma unroll
-    for (int j = 0; j < FEW_CPL; ++j) add(acc[j], c[j] < chunks ? base[r * chunks + c[j]] : zero);
-  }
-#pragma unroll
-  for (int j = 0; j < FEW_CPL; ++j) {
-    if (c[j] >= chunks) continue;
-    const int64_t at = o * chunks + c[j];  // in pieces of four elements
-    if (dto == NBK_F32) {
-      ((float4*)out)[at] = acc[j];
-    } else if (dto == NBK_BF16) {
-      uint2 u;
-      u.x = (uint32_t)nbk_f32_to_bf16(acc[j].x) | ((uint32_t)nbk_f32_to_bf16(acc[j].y) << 16);
-      u.y = (uint32_t)nbk_f32_to_bf16(acc[j].z) | ((uint32_t)nbk_f32_to_bf16(acc[j].w) << 16);
-      ((uint2*)out)[at] = u;
-    } else {
-      nbk_store_from_f32(out, at * 4 + 0, dto, acc[j].x); nbk_store_from_f32(out, at * 4 + 1, dto, acc[j].y);
-      nbk_store_from_f32(out, at * 4 + 2, dto, acc[j].z); nbk_store_from_f32(out, at * 4 + 3, dto, acc[j].w);
-    }
-  }
-}
-// what a reduction must look like for the body above
-static bool reduce_few_rows_fits(const void* in, const void* out, int dti, int64_t red, int64_t inner) {
-  return dti == NBK_F32 && red <= 8 && inner % 4 == 0 && inner >= 65536 &&
-         ((uintptr_t)in & 15) == 0 && ((uintptr_t)out & 15) == 0;
-}
-__global__ __launch_bounds__(256) void reduce_few_rows_kernel(const float* __restrict__ in,
-                                                              void* __restrict__ out, int dto, int64_t red,
-                                                              int64_t inner, int kind) {
-  reduce_few_rows_body(in, out, dto, red, inner, kind, blockIdx.x, blockIdx.y);
+template <typename P>
+__global__ __launch_bounds__(256) void reduce_strip_kernel(const void* __restrict__ in, void* __restrict__ out,
+                                                           int dti, int dto, int64_t red, int64_t inner, int kind,
+                                                           int lxs) {
+  __shared__ float part[4 * 64 * P::N];
+  reduce_strip_body<P>(in, out, dti, dto, red, inner, kind, blockIdx.x, blockIdx.y, lxs, part);
 }
 
 // Integer tensors: exact, with a 64-bit accumulator.  The same [outer, red, inner] layout and
-// strip of 64 columns per workgroup as above; the four waves split `red` and meet in LDS.
+// 64 columns per workgroup; the four waves split `red` and meet in LDS.
 __device__ __forceinline__ int64_t red_comb_i(int64_t a, int64_t b, int kind) {
   return kind == NBK_RED_SUM ? a + b : (kind == NBK_RED_MAX ? (a > b ? a : b) : (a < b ? a : b));
 }
@@ -374,14 +349,6 @@ __global__ __launch_bounds__(256) void reduce_mid_int_kernel(const void* __restr
   }
 }
 
-template <typename T, int VEC>
-__global__ __launch_bounds__(256) void reduce_mid_vec_kernel(const T* __restrict__ in,
-                                                             void* __restrict__ out, int dto,
-                                                             int64_t red, int64_t inner, int kind,
-                                                             int wc) {
-  reduce_mid_vec_body<T, VEC>(in, out, dto, red, inner, kind, blockIdx.x, blockIdx.y, wc);
-}
-
 // Several independent reductions in one launch (the column sums behind the bias and norm
 // gradients of a step are many, small and ready at the same time: one launch instead of one
 // each).  A workgroup finds its task from the running block counts and runs the same body.
@@ -389,31 +356,29 @@ struct ReduceBatchArgs {
   int32_t n;
   int32_t first_block[NBK_REDUCE_BATCH_MAX + 1];
   int32_t blocks_x[NBK_REDUCE_BATCH_MAX];
-  int32_t mode[NBK_REDUCE_BATCH_MAX];  // 0: element-wise, 1: bf16 x 8, 2: fp32 x 4, 3: few fp32 rows
-  int32_t wc[NBK_REDUCE_BATCH_MAX];    // waves side by side along the row (vector modes)
+  int16_t mode[NBK_REDUCE_BATCH_MAX];
+  int16_t lxs[NBK_REDUCE_BATCH_MAX];
   nbk_reduce_task t[NBK_REDUCE_BATCH_MAX];
 };
 
 __global__ __launch_bounds__(256) void reduce_batch_kernel(const ReduceBatchArgs B) {
+  __shared__ float part[4 * 64 * RedBf16x8::N];
   int i = 0;
   while (i + 1 < B.n && (int)blockIdx.x >= B.first_block[i + 1]) ++i;
   const nbk_reduce_task& t = B.t[i];
   const int lb = (int)blockIdx.x - B.first_block[i];
   const int64_t bx = lb % B.blocks_x[i], o = lb / B.blocks_x[i];
-  if (B.mode[i] == 1)
-    reduce_mid_vec_body<uint16_t, 8>((const uint16_t*)t.in, t.out, t.dtype_out, t.red, t.inner, t.kind, bx, o, B.wc[i]);
-  else if (B.mode[i] == 2)
-    reduce_mid_vec_body<float, 4>((const float*)t.in, t.out, t.dtype_out, t.red, t.inner, t.kind, bx, o, B.wc[i]);
-  else if (B.mode[i] == 3)
-    reduce_few_rows_body((const float*)t.in, t.out, t.dtype_out, t.red, t.inner, t.kind, bx, o);
-  else
-    reduce_mid_body(t.in, t.out, t.dtype_in, t.dtype_out, t.red, t.inner, t.kind, bx, o);
+#define REDUCE_STRIP(P)                                                                                           \
+  reduce_strip_body<P>(t.in, t.out, t.dtype_in, t.dtype_out, t.red, t.inner, t.kind, bx, o, B.lxs[i], part)
+  switch (B.mode[i]) {
+    case 1: REDUCE_STRIP(RedBf16x8); break;
+    case 2: REDUCE_STRIP(RedF32x4); break;
+    case 3: REDUCE_STRIP(RedBf16); break;
+    case 4: REDUCE_STRIP(RedF32); break;
+    default: REDUCE_STRIP(RedAny);
+  }
+#undef REDUCE_STRIP
 }
-
-// Waves side by side for a row of `chunks` 16-byte pieces: as many as the row fills.  (A
-// function of the row alone: the order of summation, and so the result, does not depend on
-// how reductions are grouped into launches.)
-static int reduce_waves_across(int64_t chunks) { return chunks >= 256 ? 4 : (chunks >= 128 ? 2 : 1); }
 
 static int reduce_mid_slab(const void* in, void* out, int32_t dti, int32_t dto, int64_t outer,
                            int64_t red, int64_t inner, int32_t kind, void* stream);
@@ -444,31 +409,20 @@ static int reduce_mid_slab(const void* in, void* out, int32_t dti, int32_t dto, 
                        dto, red, inner, kind);
     return nbk_check_launch("reduce_mid_int_kernel");
   }
-  const bool aligned = ((uintptr_t)in & 15) == 0;
-  if (reduce_few_rows_fits(in, out, dti, red, inner)) {
-    dim3 grid((unsigned)((inner / 4 + 256 * FEW_CPL - 1) / (256 * FEW_CPL)), (unsigned)outer);
-    hipLaunchKernelGGL(reduce_few_rows_kernel, grid, dim3(256), 0, (hipStream_t)stream, (const float*)in,
-                       out, dto, red, inner, kind);
-    return nbk_check_launch("reduce_few_rows_kernel");
+  const RedLayout L = reduce_layout(in, dti, outer, red, inner);
+  dim3 grid((unsigned)L.blocks_x, (unsigned)outer);
+#define REDUCE_STRIP(P)                                                                                          \
+  hipLaunchKernelGGL(reduce_strip_kernel<P>, grid, dim3(256), 0, (hipStream_t)stream, in, out, dti, dto, red, inner, \
+                     kind, L.lxs)
+  switch (L.mode) {
+    case 1: REDUCE_STRIP(RedBf16x8); break;
+    case 2: REDUCE_STRIP(RedF32x4); break;
+    case 3: REDUCE_STRIP(RedBf16); break;
+    case 4: REDUCE_STRIP(RedF32); break;
+    default: REDUCE_STRIP(RedAny);
   }
-  if (dti == NBK_BF16 && inner % 8 == 0 && aligned) {
-    const int wc = reduce_waves_across(inner / 8);
-    dim3 grid((unsigned)((inner / 8 + 64 * wc - 1) / (64 * wc)), (unsigned)outer);
-    hipLaunchKernelGGL((reduce_mid_vec_kernel<uint16_t, 8>), grid, dim3(256), 0, (hipStream_t)stream,
-                       (const uint16_t*)in, out, dto, red, inner, kind, wc);
-    return nbk_check_launch("reduce_mid_vec_kernel");
-  }
-  if (dti == NBK_F32 && inner % 4 == 0 && aligned) {
-    const int wc = reduce_waves_across(inner / 4);
-    dim3 grid((unsigned)((inner / 4 + 64 * wc - 1) / (64 * wc)), (unsigned)outer);
-    hipLaunchKernelGGL((reduce_mid_vec_kernel<float, 4>), grid, dim3(256), 0, (hipStream_t)stream,
-                       (const float*)in, out, dto, red, inner, kind, wc);
-    return nbk_check_launch("reduce_mid_vec_kernel");
-  }
-  dim3 grid((unsigned)((inner + 63) / 64), (unsigned)outer);
-  hipLaunchKernelGGL(reduce_mid_kernel, grid, dim3(256), 0, (hipStream_t)stream, in, out, dti, dto,
-                     red, inner, kind);
-  return nbk_check_launch("reduce_mid_kernel");
+#undef REDUCE_STRIP
+  return nbk_check_launch("reduce_strip_kernel");
 }
 
 extern "C" int nbk_reduce_mid_batch(const nbk_reduce_task* tasks, int32_t n, void* stream) {
@@ -506,20 +460,12 @@ extern "C" int nbk_reduce_mid_batch(const nbk_reduce_task* tasks, int32_t n, voi
       NBK_REQUIRE(t.kind >= NBK_RED_SUM && t.kind <= NBK_RED_MIN, "reduce_mid_batch: task %d: kind %d", base + i, t.kind);
       NBK_REQUIRE(nbk_dtype_size(t.dtype_in) > 0 && nbk_dtype_size(t.dtype_out) > 0,
                   "reduce_mid_batch: task %d: bad dtype", base + i);
-      const bool aligned = ((uintptr_t)t.in & 15) == 0;
-      int vec = 1;
-      B.mode[i] = 0;
-      if (t.dtype_in == NBK_BF16 && t.inner % 8 == 0 && aligned) { B.mode[i] = 1; vec = 8; }
-      else if (t.dtype_in == NBK_F32 && t.inner % 4 == 0 && aligned) { B.mode[i] = 2; vec = 4; }
-      B.wc[i] = vec > 1 ? reduce_waves_across(t.inner / vec) : 1;
-      int64_t bx = (t.inner / vec + 64 * B.wc[i] - 1) / (64 * B.wc[i]);
-      if (reduce_few_rows_fits(t.in, t.out, t.dtype_in, t.red, t.inner)) {
-        B.mode[i] = 3;
-        bx = (t.inner / 4 + 256 * FEW_CPL - 1) / (256 * FEW_CPL);
-      }
-      B.blocks_x[i] = (int32_t)bx;
+      const RedLayout L = reduce_layout(t.in, t.dtype_in, t.outer, t.red, t.inner);
+      B.mode[i] = (int16_t)L.mode;
+      B.lxs[i] = (int16_t)L.lxs;
+      B.blocks_x[i] = (int32_t)L.blocks_x;
       B.first_block[i] = (int32_t)blocks;
-      blocks += bx * t.outer;
+      blocks += L.blocks_x * t.outer;
       NBK_REQUIRE(blocks <= 0x7fffffffLL, "reduce_mid_batch: launch too large");
       B.t[i] = t;
     }
