@@ -6,8 +6,9 @@ for the five benchmark steps, this module turns the instruction stream into
 straight-line HIP (same skeleton: persistent workgroups, 16-byte coalesced
 chunks, LDS staging of rows that are read in several phases, wavefront-shuffle +
 LDS-tree reductions) and writes them to ``csrc/rowprog_spec_gen*.hip`` together
-with a lookup table keyed by a hash of the program.  ``nbk_rowprog_launch``
-hashes the program it is given and uses the specialised kernel when one exists.
+with a lookup table keyed by a hash of operand types and instructions.  ``nbk_rowprog_launch``
+hashes the program it is given and uses the specialised kernel when one exists: at any size
+and alignment, with any immediates (a mean's row length is one).
 
     python -m nabla_amd.backend.specialize          # regenerate the sources
 
@@ -51,11 +52,35 @@ def program_bytes(a: dict) -> bytes:
     return out
 
 
-def program_hash(a: dict) -> int:
+def _fnv(data: bytes) -> int:
     h = _FNV_OFFSET
-    for b in program_bytes(a):
+    for b in data:
         h = ((h ^ b) * _FNV_PRIME) & 0xFFFFFFFFFFFFFFFF
     return h
+
+
+def program_hash(a: dict) -> int:
+    return _fnv(program_bytes(a))
+
+
+def key_bytes(a: dict) -> bytes:
+    """What a compiled kernel depends on; must match rp_program_key() in csrc/rowprog.hip.
+    Immediates are read at run time, and a chunk is loaded whole at any alignment."""
+    out = struct.pack("<BB", 1 if a["has_reduce"] else 0, len(a["operands"]))
+    for o in a["operands"]:
+        out += struct.pack("<BB", o.dtype.abi, cs_class(o.col_stride))
+    for i in a["ins"]:
+        out += struct.pack("<BBBBBH", *i)
+    return out
+
+
+def program_key(a: dict) -> int:
+    return _fnv(key_bytes(a))
+
+
+def stage_sig(a: dict) -> int:
+    """Which operand is staged where; must match rp_stage_sig() in csrc/rowprog.hip."""
+    return sum(((o.stage_slot + 1) & 7) << (3 * i) for i, o in enumerate(a["operands"]))
 
 
 # ------------------------------------------------------------------------ codegen
@@ -115,7 +140,7 @@ def stage16_operand(a: dict) -> int | None:
             loads[i[2]] = loads.get(i[2], 0) + 1
     for k, n in sorted(loads.items()):
         o = a["operands"][k]
-        if n >= 2 and o.dtype.abi in (1, 2) and o.vec_ok and o.col_stride == 1 and not o.is_output:
+        if n >= 2 and o.dtype.abi in (1, 2) and o.col_stride == 1 and not o.is_output:
             return k
     return None
 
@@ -164,7 +189,7 @@ def generate_kernel(a: dict, name: str, cpt: int = 0, stage16: int | None = None
     # operand descriptors with the specialised fields folded to constants
     for k, o in enumerate(ops):
         w(f"  nbk_operand o{k} = P.operand[{k}]; o{k}.dtype = {o.dtype.abi}; "
-          f"o{k}.vec_ok = {1 if o.vec_ok else 0}; o{k}.stage_slot = {o.stage_slot};"
+          f"o{k}.stage_slot = {o.stage_slot};"
           + (f" o{k}.col_stride = {o.col_stride};" if o.col_stride in (0, 1) else ""))
     w("  const int64_t ld1 = P.lead_dim[1], ld2 = P.lead_dim[2], ld3 = P.lead_dim[3];")
     used_s = sorted({r for i in ins for r in (i[1], i[2], i[3], i[4]) if isa.NVEC <= r < 32})
@@ -209,7 +234,7 @@ def generate_kernel(a: dict, name: str, cpt: int = 0, stage16: int | None = None
                 w(ind + f"nldr{k} = rp_load1(o{k}.ptr, noff{k}, o{k}.dtype);")
             for k in inputs:
                 full_load = f"rp_load4(o{k}, noff{k}, colj[j], 4)"
-                if ops[k].dtype.abi == 0 and ops[k].vec_ok and ops[k].col_stride == 1:
+                if ops[k].dtype.abi == 0 and ops[k].col_stride == 1:
                     full_load = (f"(STREAM ? rp_load4_stream((const float*)o{k}.ptr + noff{k} + colj[j]) : "
                                  f"{full_load})")
                 w("#pragma unroll")
@@ -336,7 +361,7 @@ def generate_kernel(a: dict, name: str, cpt: int = 0, stage16: int | None = None
                 elif bop == isa.STG:
                     if resident:
                         od = ops[bd]
-                        if od.dtype.abi == 0 and od.vec_ok and od.col_stride == 1:
+                        if od.dtype.abi == 0 and od.col_stride == 1:
                             w(ind + f"if (FULL && STREAM) rp_store4_stream((float*)o{bd}.ptr + off{bd} + col, "
                               f"{_as_vec(bx)}); else")
                         w(ind + f"if (FULL || valid > 0) rp_store4(o{bd}, off{bd}, col, valid, {_as_vec(bx)});")
@@ -511,40 +536,55 @@ def collect_programs() -> dict[int, dict]:
     return programs
 
 
+def kernels_of(programs: dict[int, dict]) -> list[tuple[int, str, dict, dict]]:
+    """(key, name, program, the program that the generic form is made of) of every kernel: programs
+    of one key share theirs.  It goes by the hash of the first; the generic form is that of the
+    longest rows, the ones that the register-resident forms leave to it."""
+    by_key: dict[int, list] = {}
+    for h, a in programs.items():
+        by_key.setdefault(program_key(a), []).append((h, a))
+    out = []
+    for key, members in sorted(by_key.items()):
+        h, a = members[0]
+        out.append((key, f"rp_spec_{h:016x}", a, max((m for _, m in members), key=lambda m: m["C"])))
+    return out
+
+
 def write_sources(programs: dict[int, dict]) -> list[Path]:
     for old in CSRC.glob("rowprog_spec_gen*.hip"):
         old.unlink()
-    items = sorted(programs.items())
+    items = kernels_of(programs)
     files = []
     for fi in range(N_FILES):
         chunk = items[fi::N_FILES]
         src = [_PRELUDE]
-        for h, a in chunk:
+        for _, name, a, generic in chunk:
             src.append(f"// members: {' '.join(a.get('members', []))}")
-            src.append(generate_kernel(a, f"rp_spec_{h:016x}"))
+            src.append(generate_kernel(generic, name))
             for c in resident_variants(a):
-                src.append(generate_kernel(a, f"rp_spec_{h:016x}_c{c}", cpt=c))
-            if stage16_operand(a) is not None:
-                src.append(generate_kernel(a, f"rp_spec_{h:016x}_s16", stage16=stage16_operand(a)))
+                src.append(generate_kernel(a, f"{name}_c{c}", cpt=c))
+            if stage16_operand(generic) is not None:
+                src.append(generate_kernel(generic, f"{name}_s16", stage16=stage16_operand(generic)))
             src.append("")
         src.append(f"extern const rp_spec_entry rp_spec_table_{fi}[] = {{")
-        for h, a in chunk:
+        for key, name, a, generic in chunk:
             rv = resident_variants(a)
             flat = not a["has_reduce"]
-            ks = [f"(const void*)rp_spec_{h:016x}" + ("<false>" if flat else "")]
+            ks = [f"(const void*){name}" + ("<false>" if flat else "")]
             kf = ["nullptr"]
             kst = ["nullptr"]
             for c in (1, 2, 4, 8):
-                ks.append(f"(const void*)rp_spec_{h:016x}_c{c}<false, false>" if c in rv else "nullptr")
-                kf.append(f"(const void*)rp_spec_{h:016x}_c{c}<true, false>" if c in rv else "nullptr")
-                kst.append(f"(const void*)rp_spec_{h:016x}_c{c}<true, true>" if c in rv else "nullptr")
-            kflat = f"(const void*)rp_spec_{h:016x}<true>" if flat else "nullptr"
-            k16 = f"(const void*)rp_spec_{h:016x}_s16" if stage16_operand(a) is not None else "nullptr"
-            src.append(f"  {{0x{h:016x}ULL, {{{', '.join(ks)}}}, {{{', '.join(kf)}}}, "
-                       f"{{{', '.join(kst)}}}, {kflat}, {k16}, {1 if a['has_reduce'] else 0}}},")
+                ks.append(f"(const void*){name}_c{c}<false, false>" if c in rv else "nullptr")
+                kf.append(f"(const void*){name}_c{c}<true, false>" if c in rv else "nullptr")
+                kst.append(f"(const void*){name}_c{c}<true, true>" if c in rv else "nullptr")
+            kflat = f"(const void*){name}<true>" if flat else "nullptr"
+            k16 = f"(const void*){name}_s16" if stage16_operand(generic) is not None else "nullptr"
+            src.append(f"  {{0x{key:016x}ULL, {{{', '.join(ks)}}}, {{{', '.join(kf)}}}, "
+                       f"{{{', '.join(kst)}}}, {kflat}, {k16}, 0x{stage_sig(generic):x}ULL, "
+                       f"{1 if a['has_reduce'] else 0}}},")
         src.append("  {0ULL, {nullptr, nullptr, nullptr, nullptr, nullptr}, "
                    "{nullptr, nullptr, nullptr, nullptr, nullptr}, "
-                   "{nullptr, nullptr, nullptr, nullptr, nullptr}, nullptr, nullptr, 0}};")
+                   "{nullptr, nullptr, nullptr, nullptr, nullptr}, nullptr, nullptr, 0, 0}};")
         src.append(f"extern const int rp_spec_count_{fi} = {len(chunk)};")
         path = CSRC / f"rowprog_spec_gen{fi}.hip"
         path.write_text("\n".join(src) + "\n")
@@ -556,8 +596,8 @@ def main() -> None:
     programs = collect_programs()
     files = write_sources(programs)
     n_block = sum(1 for a in programs.values() if a["has_reduce"])
-    print(f"specialised {len(programs)} row programs ({n_block} with reductions) into "
-          f"{len(files)} files")
+    print(f"specialised {len(programs)} row programs ({n_block} with reductions) as "
+          f"{len(kernels_of(programs))} kernels into {len(files)} files")
 
 
 if __name__ == "__main__":

@@ -114,10 +114,10 @@ static int rp_validate(const nbk_rowprog* p) {
 }
 
 // ---- specialised kernels -------------------------------------------------------
-// FNV-1a over the canonical bytes of a program (same bytes as program_bytes() in
+// A program's name: FNV-1a over its canonical bytes (same bytes as program_bytes() in
 // nabla_amd/backend/specialize.py): header, per-operand (dtype, stride class,
 // vec_ok, stage slot), instructions, immediates.  Extents and addresses are not
-// part of it -- a specialised kernel serves every size.
+// part of it.
 static uint64_t rp_program_hash(const nbk_rowprog* p) {
   uint64_t h = 0xCBF29CE484222325ULL;
   auto eat = [&](const void* data, size_t n) {
@@ -145,6 +145,34 @@ static uint64_t rp_program_hash(const nbk_rowprog* p) {
   return h;
 }
 
+// What a compiled kernel is found by: the same without what it does not depend on.  A kernel reads
+// immediates from the program it is launched with (a row length that a mean divides by is one), takes
+// operands at any alignment, and only its generic form depends on what is staged (rp_stage_sig).
+// Same bytes as key_bytes() in nabla_amd/backend/specialize.py.
+static uint64_t rp_program_key(const nbk_rowprog* p) {
+  uint64_t h = 0xCBF29CE484222325ULL;
+  auto eat = [&](uint8_t b) { h = (h ^ b) * 0x100000001B3ULL; };
+  eat(p->has_reduce ? 1 : 0);
+  eat((uint8_t)p->n_operands);
+  for (int i = 0; i < p->n_operands; ++i) {
+    const nbk_operand& o = p->operand[i];
+    eat((uint8_t)o.dtype);
+    eat((uint8_t)(o.col_stride == 0 ? 0 : (o.col_stride == 1 ? 1 : 2)));
+  }
+  for (int i = 0; i < p->n_ins; ++i) {
+    const nbk_ins& in = p->ins[i];
+    for (uint8_t b : {in.op, in.dst, in.a, in.b, in.c, (uint8_t)(in.aux & 0xff), (uint8_t)(in.aux >> 8)}) eat(b);
+  }
+  return h;
+}
+// Which operand is staged where, three bits each.
+static uint64_t rp_stage_sig(const nbk_rowprog* p) {
+  uint64_t sig = 0;
+  for (int i = 0; i < p->n_operands; ++i) sig |= (uint64_t)((p->operand[i].stage_slot + 1) & 7) << (3 * i);
+  return sig;
+}
+static_assert(NBK_RP_MAX_OPERANDS * 3 <= 64 && NBK_RP_MAX_STAGE + 1 <= 7, "the signature of what is staged");
+
 struct RpSpec {
   const void* kernel[5];
   const void* kernel_full[5];
@@ -152,6 +180,7 @@ struct RpSpec {
   const void* kernel_flat;
   const void* kernel_stage16;
   const rp_hand_entry* hand;
+  uint64_t stage_sig;
   int block_mode;
   bool lds_attr_set;
   bool lds16_attr_set;
@@ -179,14 +208,15 @@ static RpSpec* rp_find_spec(uint64_t h) {
         e.kernel_flat = tabs[t][i].kernel_flat;
         e.kernel_stage16 = tabs[t][i].kernel_stage16;
         e.block_mode = tabs[t][i].block_mode;
+        e.stage_sig = tabs[t][i].stage_sig;
         e.lds_attr_set = false;
         e.lds16_attr_set = false;
         e.hand = nullptr;
-        (*g_specs)[tabs[t][i].hash] = e;
+        (*g_specs)[tabs[t][i].key] = e;
       }
     // (a hand-scheduled kernel stands beside generated ones, which take the launches it declines)
     for (int i = 0; i < rp_hand_count; ++i) {
-      auto it = g_specs->find(rp_hand_table[i].hash);
+      auto it = g_specs->find(rp_hand_table[i].key);
       if (it != g_specs->end()) it->second.hand = &rp_hand_table[i];
     }
   }
@@ -234,7 +264,7 @@ static bool rp_hand_disabled() {
 
 extern "C" int nbk_rowprog_is_specialized(const nbk_rowprog* prog) {
   if (rp_validate(prog) != NBK_OK || rp_specs_disabled()) return 0;
-  RpSpec* spec = rp_find_spec(rp_program_hash(prog));
+  RpSpec* spec = rp_find_spec(rp_program_key(prog));
   if (!spec) return 0;
   return (spec->hand && !rp_hand_disabled() && spec->hand->fits(prog)) ? 2 : 1;
 }
@@ -256,7 +286,7 @@ extern "C" int nbk_rowprog_launch(const nbk_rowprog* prog, void* stream) {
   }
   const nbk_rowprog* p = &norm;
   RpSpec* spec = (rp_specs_disabled() || prog->reserved == 1) ? nullptr
-                                                               : rp_find_spec(rp_program_hash(prog));
+                                                               : rp_find_spec(rp_program_key(prog));
   if (spec && spec->block_mode != (p->has_reduce ? 1 : 0)) spec = nullptr;
   hipStream_t st = (hipStream_t)stream;
   int64_t rows = 1;
@@ -333,13 +363,15 @@ extern "C" int nbk_rowprog_launch(const nbk_rowprog* prog, void* stream) {
                                 (size_t)c_pad * 2, st));
         return NBK_OK;
       }
-      if (lds > 32 * 1024 && !spec->lds_attr_set) {
-        NBK_HIP(hipFuncSetAttribute(spec->kernel[0], hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    64 * 1024));
-        spec->lds_attr_set = true;
+      if (spec->stage_sig == rp_stage_sig(p)) {
+        if (lds > 32 * 1024 && !spec->lds_attr_set) {
+          NBK_HIP(hipFuncSetAttribute(spec->kernel[0], hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      64 * 1024));
+          spec->lds_attr_set = true;
+        }
+        NBK_HIP(hipLaunchKernel(spec->kernel[0], dim3((unsigned)grid), dim3(block), args, lds, st));
+        return NBK_OK;
       }
-      NBK_HIP(hipLaunchKernel(spec->kernel[0], dim3((unsigned)grid), dim3(block), args, lds, st));
-      return NBK_OK;
     }
     return rp_vm_launch(p, rows, st);
   }

@@ -18,7 +18,7 @@ __device__ __forceinline__ float rp_identity(int kind) {
 // ---- chunk load / store ----------------------------------------------------
 // Streaming forms for launches whose operands exceed the last-level cache: the
 // non-temporal hint keeps lines that are touched once from displacing others.
-typedef float rp_vf4 __attribute__((ext_vector_type(4)));
+typedef float rp_vf4 __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ float4 rp_load4_stream(const float* p) {
   rp_vf4 v = __builtin_nontemporal_load((const rp_vf4*)p);
   return make_float4(v.x, v.y, v.z, v.w);

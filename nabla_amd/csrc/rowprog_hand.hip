@@ -1,6 +1,6 @@
 // Hand-scheduled kernels for row programs whose generated kernel is bound by the vector ALU and
 // not by memory.  Each one computes exactly what its program computes (same operands, same
-// results up to the rounding of a differently associated sum) and is attached, by the hash of
+// results up to the rounding of a differently associated sum) and is attached, by the key of
 // that program, to the entry the generated kernels have in the lookup table; where a launch does
 // not meet a kernel's conditions (row length, alignment) the generated forms run as before.
 //
@@ -170,7 +170,7 @@ template __global__ void rp_hand_xent_bf16_i64<true>(const nbk_rowprog, int64_t)
 // XE_PIECES of them per lane and enough of them to occupy the lanes (shorter rows are served
 // well by the generated register-resident forms), 16-byte aligned in both row-shaped operands.
 static bool xe_fits(const nbk_rowprog* p) {
-  if (p->n_operands != 5 || (p->C & 7) != 0 || p->C < 4096 ||
+  if (p->n_operands != 5 || p->n_imm != 0 || (p->C & 7) != 0 || p->C < 4096 ||
       p->C > (int64_t)XE_BLOCK * XE_PIECES * 8)
     return false;
   for (int i = 0; i < 5; i += 4) {
@@ -186,9 +186,9 @@ static bool xe_fits(const nbk_rowprog* p) {
 // The program comes in two orders: with the label mask of the gradient phase recomputed (the
 // planner does that for masks of 2^22 elements and more) or shared with the loss phase.
 extern const rp_hand_entry rp_hand_table[] = {
-    {0x32ead8892650fe1bULL, (const void*)rp_hand_xent_bf16_i64<false>,
+    {0x270c5246c3834b29ULL, (const void*)rp_hand_xent_bf16_i64<false>,
      (const void*)rp_hand_xent_bf16_i64<true>, XE_BLOCK, xe_fits},
-    {0xb23538fd6922ab4fULL, (const void*)rp_hand_xent_bf16_i64<false>,
+    {0xe0795b4558a5e5a9ULL, (const void*)rp_hand_xent_bf16_i64<false>,
      (const void*)rp_hand_xent_bf16_i64<true>, XE_BLOCK, xe_fits},
 };
 extern const int rp_hand_count = (int)(sizeof(rp_hand_table) / sizeof(rp_hand_table[0]));

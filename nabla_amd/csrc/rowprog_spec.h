@@ -1,12 +1,12 @@
 // Lookup table of ahead-of-time specialised row kernels.  The generated sources
 // rowprog_spec_gen<N>.hip each define one table; rowprog.hip searches them by the
-// hash of the program it is asked to launch.
+// key of the program it is asked to launch (operand types and instructions).
 #pragma once
 #include <stdint.h>
 #include "nbk.h"
 
 struct rp_spec_entry {
-  uint64_t hash;
+  uint64_t key;
   // [0]: generic form (any row length).  [1..4]: register-resident forms for
   // reduction programs whose lanes own exactly 1 / 2 / 4 / 8 chunks of a row;
   // nullptr where that form was not generated.  Reduction programs take (nbk_rowprog,
@@ -26,15 +26,16 @@ struct rp_spec_entry {
   // (2 bytes per element: a 32 000-element row and two workgroups fit a CU), and every phase
   // reading it from there; nullptr where not generated.
   const void* kernel_stage16;
+  uint64_t stage_sig;  // what kernel[0] finds staged in LDS: a program that differs there cannot run it
   int block_mode;
 };
 
-// A hand-scheduled kernel for one program (rowprog_hand.hip), attached by hash to that program's
+// A hand-scheduled kernel for one program (rowprog_hand.hip), attached by key to that program's
 // entry above.  Signature of a generated reduction kernel; launched with `block` lanes per row when
 // `fits(program)` holds, `kernel_stream` (non-temporal loads and stores) for launches that move
 // more than the last-level cache holds.
 struct rp_hand_entry {
-  uint64_t hash;
+  uint64_t key;
   const void* kernel;
   const void* kernel_stream;
   int block;
