@@ -2,7 +2,7 @@
 
 The interpreter in ``csrc/rowprog.hip`` runs any fused group, but it pays a
 decode cost per instruction.  For the row programs that the lowering pass emits
-for the five benchmark steps, this module turns the instruction stream into
+for the five benchmark steps and for steps made of the package's layers, this module turns the instruction stream into
 straight-line HIP (same skeleton: persistent workgroups, 16-byte coalesced
 chunks, LDS staging of rows that are read in several phases, wavefront-shuffle +
 LDS-tree reductions) and writes them to ``csrc/rowprog_spec_gen*.hip`` together
@@ -26,7 +26,7 @@ from . import isa
 from .planner import Plan
 
 CSRC = Path(__file__).resolve().parents[1] / "csrc"
-N_FILES = 4  # generated sources are split so that they compile in parallel
+N_FILES = 8  # generated sources are split so that they compile in parallel
 
 _FNV_OFFSET = 0xCBF29CE484222325
 _FNV_PRIME = 0x100000001B3
@@ -145,24 +145,24 @@ def stage16_operand(a: dict) -> int | None:
     return None
 
 
-def generate_kernel(a: dict, name: str, cpt: int = 0, stage16: int | None = None) -> str:
+def generate_kernel(a: dict, name: str, resident: bool = False, stage16: int | None = None) -> str:
     """HIP source of one specialised kernel for the row program ``a``.
 
-    ``cpt`` = 0: generic form, chunk loops with a run-time trip count, rows that
-    are read in several phases staged in LDS.  ``cpt`` > 0 (reduction programs
-    only): every lane owns exactly ``cpt`` chunks of the row; all inputs are
-    loaded once into registers with every load in flight together, the chunk
-    loops are fully unrolled, and arithmetic repeated in a later phase is
-    removed by the compiler's common-subexpression elimination."""
+    Generic form: chunk loops with a run-time trip count, rows that are read in
+    several phases staged in LDS.  ``resident`` (reduction programs only): every
+    lane owns exactly CPT chunks of the row; all inputs are loaded once into
+    registers with every load in flight together, the chunk loops are fully
+    unrolled, and arithmetic repeated in a later phase is removed by the
+    compiler's common-subexpression elimination."""
     ops = a["operands"]
     ins = a["ins"]
     block_mode = bool(a["has_reduce"])
-    resident = cpt > 0
     assert not resident or block_mode
     inputs = full_inputs(a)
-    # every stored tensor a 16-bit float: hardware transcendentals are accurate enough
+    # every stored tensor a 16-bit float: hardware transcendentals are accurate enough for the
+    # benchmark steps; elsewhere the functions are the interpreter's
     stored = {i[1] for i in ins if i[0] in (isa.STR, isa.STG)}
-    lowp = bool(stored) and all(ops[k].dtype.abi in (1, 2) for k in stored)
+    lowp = bool(stored) and all(ops[k].dtype.abi in (1, 2) for k in stored) and a.get("benchmark", True)
     L: list[str] = []
     w = L.append
     if block_mode:
@@ -170,9 +170,9 @@ def generate_kernel(a: dict, name: str, cpt: int = 0, stage16: int | None = None
         # more smaller ones) share a CU and one loads while the other computes
         occ = ""
         if resident:
-            # FULL: the row is exactly cpt chunks per lane, no lane or element is masked
+            # FULL: the row is exactly CPT chunks per lane, no lane or element is masked
             # STREAM: fp32 unit-stride operands are read and written with the non-temporal hint
-            w("template <bool FULL, bool STREAM>")
+            w("template <int CPT, bool FULL, bool STREAM>")
         w(f"__global__ __launch_bounds__(512) {occ}void {name}(const nbk_rowprog P, int64_t rows) {{")
         w("  __shared__ float red_buf[64];")
         w("  int red_phase = 0; (void)red_phase;")
@@ -206,9 +206,9 @@ def generate_kernel(a: dict, name: str, cpt: int = 0, stage16: int | None = None
         # Software pipeline over the rows of a persistent workgroup: the loads of the next
         # row are issued before the current row is computed and stored, so a row's load
         # latency overlaps the previous row's arithmetic and never queues behind its stores.
-        w(f"  int64_t colj[{cpt}]; int validj[{cpt}];")
+        w(f"  int64_t colj[CPT]; int validj[CPT];")
         w("#pragma unroll")
-        w(f"  for (int j = 0; j < {cpt}; ++j) {{")
+        w(f"  for (int j = 0; j < CPT; ++j) {{")
         w("    const int64_t ch = threadIdx.x + (int64_t)j * blockDim.x;")
         w("    colj[j] = ch << 2;")
         w("    const int64_t left = C - colj[j];")
@@ -219,7 +219,7 @@ def generate_kernel(a: dict, name: str, cpt: int = 0, stage16: int | None = None
         for k in hoisted:
             w(f"  float nldr{k} = 0.f;")
         for k in inputs:
-            w(f"  float4 n{k}[{cpt}];")
+            w(f"  float4 n{k}[CPT];")
 
         def fetch(row_expr: str, ind: str) -> None:
             w(ind + decomp.replace("ROW", row_expr).replace("LI", "nlead"))
@@ -238,18 +238,19 @@ def generate_kernel(a: dict, name: str, cpt: int = 0, stage16: int | None = None
                     full_load = (f"(STREAM ? rp_load4_stream((const float*)o{k}.ptr + noff{k} + colj[j]) : "
                                  f"{full_load})")
                 w("#pragma unroll")
-                w(ind + f"for (int j = 0; j < {cpt}; ++j) n{k}[j] = FULL ? {full_load} : "
+                w(ind + f"for (int j = 0; j < CPT; ++j) n{k}[j] = FULL ? {full_load} : "
                   f"(validj[j] > 0 ? rp_load4(o{k}, noff{k}, colj[j], validj[j]) : "
                   "make_float4(0.f, 0.f, 0.f, 0.f));")
 
         # the pipeline doubles the registers that hold inputs; past 8 float4 per lane that
         # costs more occupancy than the overlap returns
-        prefetch = cpt * max(1, len(inputs)) <= PREFETCH_MAX_REGS
-        if prefetch:
-            fetch("blockIdx.x", "  ")
+        w(f"  constexpr bool AHEAD = CPT * {max(1, len(inputs))} <= {PREFETCH_MAX_REGS};")
+        w("  auto fetch = [&](int64_t at) {")
+        fetch("at", "    ")
+        w("  };")
+        w("  if (AHEAD) fetch(blockIdx.x);")
         w("  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {")
-        if not prefetch:
-            fetch("row", "    ")
+        w("    if (!AHEAD) fetch(row);")
         w("    uint32_t lead_idx[4] = {nlead[0], nlead[1], nlead[2], nlead[3]};")
         w("    (void)lead_idx;")
         for k in range(len(ops)):
@@ -257,13 +258,10 @@ def generate_kernel(a: dict, name: str, cpt: int = 0, stage16: int | None = None
         for k in hoisted:
             w(f"    const float ldr{k} = nldr{k};")
         for k in inputs:
-            w(f"    float4 r{k}[{cpt}];")
+            w(f"    float4 r{k}[CPT];")
             w("#pragma unroll")
-            w(f"    for (int j = 0; j < {cpt}; ++j) r{k}[j] = n{k}[j];")
-        if prefetch:
-            w("    if (row + gridDim.x < rows) {")
-            fetch("row + gridDim.x", "      ")
-            w("    }")
+            w(f"    for (int j = 0; j < CPT; ++j) r{k}[j] = n{k}[j];")
+        w("    if (AHEAD && row + gridDim.x < rows) fetch(row + gridDim.x);")
     elif block_mode:
         w("  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {")
         # the host rejects launches of 2^31 rows or more, so 32-bit division is exact
@@ -332,7 +330,7 @@ def generate_kernel(a: dict, name: str, cpt: int = 0, stage16: int | None = None
             ind = "      " if block_mode else "    "
             if resident:
                 w("#pragma unroll")
-                w(f"    for (int j = 0; j < {cpt}; ++j) {{")
+                w(f"    for (int j = 0; j < CPT; ++j) {{")
                 w("      const int64_t col = colj[j];")
                 w("      const int valid = FULL ? 4 : validj[j];")
             elif block_mode:
@@ -420,7 +418,7 @@ def resident_variants(a: dict) -> list[int]:
 
 
 _PRELUDE = '''// GENERATED by nabla_amd/backend/specialize.py -- do not edit.
-// Straight-line versions of the row programs of the benchmark steps; the
+// Straight-line versions of the row programs of the benchmark steps and the package's layers; the
 // interpreter in rowprog.hip runs everything that is not listed here.
 #include "rowprog_device.h"
 #include "rowprog_spec.h"
@@ -429,8 +427,134 @@ extern __shared__ __align__(16) float rp_stage_lds[];
 '''
 
 
+def layer_steps():
+    """Steps made of the package's layers as programs use them: both float types, forward alone and
+    with gradients, dropout as the layers default to, plain gradients or AdamW in the step, masked
+    attention and full.  A few sizes each, because what fuses into a row program depends on which sums a
+    product takes over (a short product is split along K and leaves its bias to its reader)."""
+    import nabla_amd as nb
+    from nabla_amd import workloads as W
+    F = nb.nn.functional
+
+    def leaf(shape, dtype):
+        return nb.Tensor._from_torch(torch.empty(shape, dtype=dtype))
+
+    def leaves(shapes, dtype):
+        if isinstance(shapes, dict):
+            return {k: leaves(v, dtype) for k, v in shapes.items()}
+        if isinstance(shapes, list):
+            return [leaves(v, dtype) for v in shapes]
+        return leaf(shapes, dtype)
+
+    def ids(*shape):
+        return nb.Tensor._from_torch(torch.zeros(shape, dtype=torch.int64))
+
+    def train(loss, params, *rest, optimizer=False):
+        def run():
+            value, grads = nb.value_and_grad(loss)(params, *rest)
+            if not optimizer:
+                return value, grads
+            opt = nb.nn.optim.adamw_init(params)
+            opt["step"] = leaf((), torch.float32)
+            return (value, *nb.nn.optim.adamw_update(params, grads, opt, lr=1e-3, realize=False))
+        return run
+
+    def block(x, p, heads, causal, dropout):
+        b, s, d = x.shape
+
+        def split(t):
+            return nb.swap_axes(nb.reshape(t, (b, s, heads, d // heads)), 1, 2)
+
+        h = F.layer_norm(x, p["ln1_w"], p["ln1_b"])
+        q, k, v = (F.linear(h, p["w" + n], p.get("b" + n)) for n in "qkv")
+        a = F.scaled_dot_product_attention(split(q), split(k), split(v), dropout_p=dropout, is_causal=causal)
+        a = F.linear(nb.reshape(nb.swap_axes(a, 1, 2), (b, s, d)), p["wo"], p["bo"])
+        x = x + F.dropout(a, dropout)
+        h = F.layer_norm(x, p["ln2_w"], p["ln2_b"])
+        h = F.linear(nb.gelu(F.linear(h, p["w1"], p["b1"])), p["w2"], p["b2"])
+        return x + F.dropout(h, dropout)
+
+    for dtype in (torch.float32, torch.bfloat16):
+        for b, s, d, heads in ((1, 96, 256, 4), (2, 300, 512, 8), (4, 256, 512, 16), (8, 512, 1024, 16)):
+            p = leaves(W._block_shapes(d, 4 * d), dtype)
+            x = leaf((b, s, d), dtype)
+            for causal in (False, True):
+                for dropout in (0.0, 0.1):
+                    def loss(p, x, heads=heads, causal=causal, dropout=dropout):
+                        out = block(x, p, heads, causal, dropout)
+                        return nb.mean(out * out)
+                    yield train(loss, p, x)
+                    yield train(loss, p, x, optimizer=True)
+                    yield lambda p=p, x=x, a=(heads, causal, dropout): [block(x, p, *a)]
+        for b, s, d in ((1, 64, 512), (1, 420, 2048), (1, 1800, 1024), (2, 320, 512), (2, 1024, 2048)):
+            shapes = W.c5_shapes(layers=2, batch=b, seq=s, d=d, ff=4 * d, vocab=6400)
+            t = leaves({k: v for k, v in shapes.items() if k != "ids"}, dtype)
+            t["ids"] = ids(b, s)
+
+            def logits(t=t, d=d):
+                x = F.embedding(t["ids"], t["embed"])
+                for layer in t["layers"]:
+                    x = W.transformer_block(x, layer, d // 128)
+                return [F.layer_norm(x, t["lnf_w"], t["lnf_b"]) @ t["head"]]
+
+            yield logits
+            if dtype is torch.bfloat16:
+                yield lambda t=t, d=d: W.c5_step(t, d // 128)
+        for rows, cols in ((100, 250), (2048, 1024)):
+            xy = [leaf((rows, cols), dtype) for _ in range(2)]
+            yield lambda xy=xy: W.c2_step(*xy)
+            # operations by themselves, as eager evaluation runs them
+            unary = (nb.exp, nb.log, nb.sqrt, nb.rsqrt, nb.relu, nb.sigmoid, nb.silu, nb.tanh, nb.gelu, nb.abs, nb.neg)
+            rowwise = (nb.softmax, nb.logsoftmax, nb.reduce_sum, nb.reduce_max, nb.mean)
+            for op in (nb.add, nb.sub, nb.mul, nb.div):
+                yield lambda op=op, xy=xy: [op(*xy)]
+            for op in unary:
+                yield lambda op=op, xy=xy: [op(xy[0])]
+            for op in rowwise:
+                yield lambda op=op, xy=xy: [op(xy[0], axis=-1)]
+            weight, bias = leaf((cols,), dtype), leaf((cols,), dtype)
+            yield lambda xy=xy, w=weight, b=bias: [F.layer_norm(xy[0], w, b)]
+            labels = ids(rows)
+            yield lambda x=xy[0], labels=labels: nb.value_and_grad(
+                lambda z: F.cross_entropy_loss(z, labels))(x)
+        for tokens in (48, 1000, 4096):
+            codes = {"indices": nb.Tensor._from_torch(torch.zeros(512 * 2048, dtype=torch.uint8)),
+                     "scales": leaf((512 * 2048 // 64,), torch.float32), "original_numel": 512 * 2048,
+                     "padded_numel": 512 * 2048, "block_size": 64}
+            up, down = dict(codes, original_shape=(512, 2048)), dict(codes, original_shape=(2048, 512))
+            adapters = leaves({"up": {"A": (512, 8), "B": (8, 2048)}, "down": {"A": (2048, 8), "B": (8, 512)}}, dtype)
+
+            def loss(ad, x, up=up, down=down, dt=dtype):
+                def lin(x, w, a):
+                    return nb.nn.finetune.qlora_linear(x, w, a, alpha=16.0, compute_dtype=nb.DType.from_torch(dt))
+                out = x + lin(nb.gelu(lin(x, up, ad["up"])), down, ad["down"])
+                return nb.mean(out * out)
+
+            yield train(loss, adapters, leaf((tokens, 512), dtype))
+    for depth in (1, 2, 3, 4):
+        for batch in (32, 512):
+            sizes = [100] + [128] * depth + [10]
+            params = [(leaf((a, b), torch.float32), leaf((1, b), torch.float32)) for a, b in zip(sizes, sizes[1:])]
+
+            def loss(params, x, y):
+                for w, b in params[:-1]:
+                    x = nb.relu(x @ w + b)
+                return F.mse_loss(x @ params[-1][0] + params[-1][1], y)
+
+            args = leaf((batch, 100), torch.float32), leaf((batch, 10), torch.float32)
+            yield train(loss, params, *args)
+            yield train(loss, params, *args, optimizer=True)
+    for batch, hw, c, classes in ((1, 16, (1, 24, 40, 72), 7), (50, 28, (3, 16, 64, 128), 10)):
+        shapes = W.c4_shapes(batch, hw, c, classes)
+        t = leaves({k: v for k, v in shapes.items() if k != "labels"}, torch.float32)
+        t["labels"] = ids(batch)
+        yield lambda t=t: W.c4_step(t)
+        yield lambda t=t: [W.c4_logits(t, t["img"])]
+
+
 def collect_programs() -> dict[int, dict]:
-    """Plan the five benchmark steps at full size and return {hash: rowprog attrs}."""
+    """Plan the five benchmark steps at full size and the steps of the package's layers
+    (``layer_steps``); {hash: rowprog attrs}."""
     import nabla_amd as nb
     from nabla_amd import config
     from nabla_amd import workloads as W
@@ -522,7 +646,9 @@ def collect_programs() -> dict[int, dict]:
         jobs.append(with_flags(jobs[2], FOLD_PRODUCT_SUMS=False))
         jobs.append(with_flags(jobs[0], FOLD_RELU=False))
         jobs.append(with_flags(jobs[3], FOLD_RELU=False))
-        for job in jobs:
+        n_benchmark = len(jobs)
+        jobs.extend(layer_steps())
+        for i, job in enumerate(jobs):
             clear_plan_cache()
             res = job()
             flat = [x for x in nb.tree_leaves(res) if isinstance(x, nb.Tensor)]
@@ -530,7 +656,7 @@ def collect_programs() -> dict[int, dict]:
             for bound in _PLAN_CACHE.values():
                 for st in bound.plan.steps:
                     if st.kind == "rowprog":
-                        programs.setdefault(program_hash(st.attrs), st.attrs)
+                        programs.setdefault(program_hash(st.attrs), dict(st.attrs, benchmark=i < n_benchmark))
     finally:
         executor.set_executor(prev)
     return programs
@@ -539,14 +665,15 @@ def collect_programs() -> dict[int, dict]:
 def kernels_of(programs: dict[int, dict]) -> list[tuple[int, str, dict, dict]]:
     """(key, name, program, the program that the generic form is made of) of every kernel: programs
     of one key share theirs.  It goes by the hash of the first; the generic form is that of the
-    longest rows, the ones that the register-resident forms leave to it."""
+    longest rows, the ones that the register-resident forms leave to it (with the functions of the first)."""
     by_key: dict[int, list] = {}
     for h, a in programs.items():
         by_key.setdefault(program_key(a), []).append((h, a))
     out = []
     for key, members in sorted(by_key.items()):
         h, a = members[0]
-        out.append((key, f"rp_spec_{h:016x}", a, max((m for _, m in members), key=lambda m: m["C"])))
+        generic = max((m for _, m in members), key=lambda m: m["C"])
+        out.append((key, f"rp_spec_{h:016x}", a, dict(generic, benchmark=a.get("benchmark", True))))
     return out
 
 
@@ -561,8 +688,8 @@ def write_sources(programs: dict[int, dict]) -> list[Path]:
         for _, name, a, generic in chunk:
             src.append(f"// members: {' '.join(a.get('members', []))}")
             src.append(generate_kernel(generic, name))
-            for c in resident_variants(a):
-                src.append(generate_kernel(a, f"{name}_c{c}", cpt=c))
+            if resident_variants(a):
+                src.append(generate_kernel(a, f"{name}_c", resident=True))
             if stage16_operand(generic) is not None:
                 src.append(generate_kernel(generic, f"{name}_s16", stage16=stage16_operand(generic)))
             src.append("")
@@ -574,9 +701,9 @@ def write_sources(programs: dict[int, dict]) -> list[Path]:
             kf = ["nullptr"]
             kst = ["nullptr"]
             for c in (1, 2, 4, 8):
-                ks.append(f"(const void*){name}_c{c}<false, false>" if c in rv else "nullptr")
-                kf.append(f"(const void*){name}_c{c}<true, false>" if c in rv else "nullptr")
-                kst.append(f"(const void*){name}_c{c}<true, true>" if c in rv else "nullptr")
+                ks.append(f"(const void*){name}_c<{c}, false, false>" if c in rv else "nullptr")
+                kf.append(f"(const void*){name}_c<{c}, true, false>" if c in rv else "nullptr")
+                kst.append(f"(const void*){name}_c<{c}, true, true>" if c in rv else "nullptr")
             kflat = f"(const void*){name}<true>" if flat else "nullptr"
             k16 = f"(const void*){name}_s16" if stage16_operand(generic) is not None else "nullptr"
             src.append(f"  {{0x{key:016x}ULL, {{{', '.join(ks)}}}, {{{', '.join(kf)}}}, "

@@ -192,10 +192,12 @@ static RpSpec* rp_find_spec(uint64_t h) {
   std::lock_guard<std::mutex> lk(g_spec_mu);
   if (!g_specs) {
     g_specs = new std::unordered_map<uint64_t, RpSpec>();
-    const rp_spec_entry* tabs[NBK_RP_SPEC_FILES] = {rp_spec_table_0, rp_spec_table_1,
-                                                   rp_spec_table_2, rp_spec_table_3};
-    const int counts[NBK_RP_SPEC_FILES] = {rp_spec_count_0, rp_spec_count_1, rp_spec_count_2,
-                                           rp_spec_count_3};
+#define RP_TABLE(I) rp_spec_table_##I,
+#define RP_COUNT(I) rp_spec_count_##I,
+    const rp_spec_entry* tabs[NBK_RP_SPEC_FILES] = {NBK_RP_SPEC_EACH(RP_TABLE)};
+    const int counts[NBK_RP_SPEC_FILES] = {NBK_RP_SPEC_EACH(RP_COUNT)};
+#undef RP_TABLE
+#undef RP_COUNT
     for (int t = 0; t < NBK_RP_SPEC_FILES; ++t)
       for (int i = 0; i < counts[t]; ++i)
       {

@@ -167,10 +167,10 @@ template __global__ void rp_hand_xent_bf16_i64<true>(const nbk_rowprog, int64_t)
 
 #ifndef __HIP_DEVICE_COMPILE__
 // What a launch must meet for the kernel above: rows of whole 16-byte pieces, at most
-// XE_PIECES of them per lane and enough of them to occupy the lanes (shorter rows are served
-// well by the generated register-resident forms), 16-byte aligned in both row-shaped operands.
+// XE_PIECES of them per lane and enough of them to occupy the lanes (rows short enough to be
+// staged as fp32 are served well by the generated register-resident forms), 16-byte aligned in both row-shaped operands.
 static bool xe_fits(const nbk_rowprog* p) {
-  if (p->n_operands != 5 || p->n_imm != 0 || (p->C & 7) != 0 || p->C < 4096 ||
+  if (p->n_operands != 5 || p->n_imm != 0 || p->n_stage != 0 || (p->C & 7) != 0 || p->C < 4096 ||
       p->C > (int64_t)XE_BLOCK * XE_PIECES * 8)
     return false;
   for (int i = 0; i < 5; i += 4) {

@@ -44,9 +44,9 @@ struct rp_hand_entry {
 extern const rp_hand_entry rp_hand_table[];
 extern const int rp_hand_count;
 
-#define NBK_RP_SPEC_FILES 4
-extern const rp_spec_entry rp_spec_table_0[];
-extern const rp_spec_entry rp_spec_table_1[];
-extern const rp_spec_entry rp_spec_table_2[];
-extern const rp_spec_entry rp_spec_table_3[];
-extern const int rp_spec_count_0, rp_spec_count_1, rp_spec_count_2, rp_spec_count_3;
+#define NBK_RP_SPEC_FILES 8
+#define NBK_RP_SPEC_EACH(F) F(0) F(1) F(2) F(3) F(4) F(5) F(6) F(7)
+#define NBK_RP_SPEC_DECLARE(I)                       \
+  extern const rp_spec_entry rp_spec_table_##I[];    \
+  extern const int rp_spec_count_##I;
+NBK_RP_SPEC_EACH(NBK_RP_SPEC_DECLARE)
