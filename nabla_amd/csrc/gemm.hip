@@ -923,8 +923,10 @@ struct DirectLoader {
 // x^T dy, which reads dy anyway): the waves that hold the first block row of the first tile row
 // multiply a fragment of ones into one more accumulator per block column, from the B fragments
 // that are in registers for the product -- no byte is read twice.
-template <int BM, int BN, bool A_KC, bool B_KC, int EPI, int NW, int KSS, bool MI16, bool COLSUM = false>
+// STAGES: tile buffers (a power of two).  With more than two a copy has STAGES - 1 tiles' time to land.
+template <int BM, int BN, bool A_KC, bool B_KC, int EPI, int NW, int KSS, bool MI16, bool COLSUM = false, int STAGES = 2>
 __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g) {
+  static_assert((STAGES & (STAGES - 1)) == 0, "tile t is in buffer t % STAGES");
   constexpr int WGN = NW / 2;
   constexpr int WM = BM / 2, WN = BN / WGN;  // wave tile
   constexpr int FM = MI16 ? 16 : 32;          // rows / columns of an MFMA block
@@ -1162,37 +1164,65 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g)
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     __builtin_amdgcn_sched_barrier(0);
   };
+  // ... but for its youngest IN_FLIGHT copies (no fence: the compiler waits for every copy in front of one)
+  auto tile_barrier_behind = [&](auto in_flight) {
+    constexpr int V = decltype(in_flight)::value;
+    static_assert(V < 64, "vmcnt has six bits");
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(V) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
 
-  // Two tile buffers.  Tile kt + 1 is on its way while tile kt is multiplied; the barrier that
+  // Tiles kt + 1 .. kt + STAGES - 1 are on their way while tile kt is multiplied; the barrier that
   // ends tile kt (in the middle of its last step, whose fragments are in registers by then)
-  // frees its buffer for tile kt + 2, whose copies are started right behind that barrier and
-  // have the whole of tile kt + 1 to land.
-  tile_barrier();
-  static_for<NFRAG>([&](auto r) { read_frag(S0{}, r, gemm_lds, 0); });
-  if (nk > 1 && ns < 2) {
-    const char* sa = GEMM_SRC_A(1);
-    const char* sb = GEMM_SRC_B(1);
-    static_for<LA::N>([&](auto j) { la.template issue_one<decltype(j)::value>(gemm_lds + TILE_CHUNKS, sa); });
-    static_for<LB::N>([&](auto j) { lb.template issue_one<decltype(j)::value>(gemm_lds + TILE_CHUNKS + CA, sb); });
+  // frees its buffer for tile kt + STAGES, whose copies are started right behind that barrier.
+  // A wave's copies land in the order of their requests and every tile past the first ones takes NL of
+  // them, so that tile kt + 1 is there when no more than those of the STAGES - 2 behind it are missing.
+  constexpr int NL = LA::N + LB::N;
+#define GEMM_COPY_TILE(t, to)                                                                            \
+  do {                                                                                                   \
+    const char* sa = GEMM_SRC_A(t);                                                                      \
+    const char* sb = GEMM_SRC_B(t);                                                                      \
+    static_for<LA::N>([&](auto j) { la.template issue_one<decltype(j)::value>((to), sa); });             \
+    static_for<LB::N>([&](auto j) { lb.template issue_one<decltype(j)::value>((to) + CA, sb); });        \
+  } while (0)
+  if constexpr (STAGES > 2) {
+    if (nk > 1) {
+      // (past the last tile: that one again, so that the count holds)
+#pragma unroll
+      for (int t = 1; t < STAGES; ++t) {
+        const int src = t < nk ? t : nk - 1;
+        if (t >= ns) GEMM_COPY_TILE(src, gemm_lds + t * TILE_CHUNKS);
+      }
+    }
+    // (a shallow tile takes fewer copies)
+    if (ns > 0 || nk == 1) tile_barrier();
+    else tile_barrier_behind(std::integral_constant<int, (STAGES - 1) * NL>{});
+    static_for<NFRAG>([&](auto r) { read_frag(S0{}, r, gemm_lds, 0); });
+  } else {
+    tile_barrier();
+    static_for<NFRAG>([&](auto r) { read_frag(S0{}, r, gemm_lds, 0); });
+    if (nk > 1 && ns < 2) GEMM_COPY_TILE(1, gemm_lds + TILE_CHUNKS);
   }
   for (int kt = 0; kt + 1 < nk; ++kt) {
-    u32x4* cur = gemm_lds + (kt & 1) * TILE_CHUNKS;
-    const u32x4* nxt = gemm_lds + ((kt + 1) & 1) * TILE_CHUNKS;
+    u32x4* cur = gemm_lds + (kt & (STAGES - 1)) * TILE_CHUNKS;
+    const u32x4* nxt = gemm_lds + ((kt + 1) & (STAGES - 1)) * TILE_CHUNKS;
     static_for<NSTEP - 1>([&](auto st) {
       constexpr int ST = decltype(st)::value;
       stage(std::integral_constant<int, ST & 1>{}, cur, ST + 1);
     });
     frags_ready(S1{});  // the last step (NSTEP is even) is on set 1
     static_for<NMFMA / 2>([&](auto q) { mfma(S1{}, q); });
-    tile_barrier();
+    if constexpr (STAGES > 2) tile_barrier_behind(std::integral_constant<int, (STAGES - 2) * NL>{});
+    else tile_barrier();
     {
-      // Behind the barrier: the first fragments of tile kt + 1, the copies of tile kt + 2 and
+      // Behind the barrier: the first fragments of tile kt + 1, the copies of tile kt + STAGES and
       // the second half of the MFMAs, dealt out evenly and pinned in this order (the copies
       // and the reads both touch LDS, so the scheduler would otherwise leave the MFMAs last).
-      // (the last pass has no tile kt + 2: it fetches tile nk - 1 again, into a buffer that
+      // (past the last tile: it fetches tile nk - 1 again, into a buffer that
       // is not read any more, which keeps this block free of branches)
-      constexpr int NL = LA::N + LB::N, H = NMFMA / 2;
-      const int k2 = kt + 2 < nk ? kt + 2 : nk - 1;
+      constexpr int H = NMFMA / 2;
+      const int k2 = kt + STAGES < nk ? kt + STAGES : nk - 1;
       const char* src_a2 = GEMM_SRC_A(k2);
       const char* src_b2 = GEMM_SRC_B(k2);
       static_for<H>([&](auto q) {
@@ -1216,7 +1246,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g)
     colsum_step(S1{});
   }
   {
-    const u32x4* cur = gemm_lds + ((nk - 1) & 1) * TILE_CHUNKS;
+    const u32x4* cur = gemm_lds + ((nk - 1) & (STAGES - 1)) * TILE_CHUNKS;
     static_for<NSTEP - 1>([&](auto st) {
       constexpr int ST = decltype(st)::value;
       stage(std::integral_constant<int, ST & 1>{}, cur, ST + 1);
@@ -1242,6 +1272,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g)
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): no copy may land in a slab
   __syncthreads();  // the epilogue reuses the tile buffers as per-wave slabs
   gemm_epilogue<TM, TN, WN, true, EPI>(acc, g, m0, n0, wm, wn, c_off, wave, lane);
+#undef GEMM_COPY_TILE
 #undef GEMM_SRC_A
 #undef GEMM_SRC_B
 }
@@ -1873,19 +1904,21 @@ static int launch_bf16(const GemmArgs& a, bool akc, bool bkc, int64_t batch, hip
   return nbk_check_launch("gemm_bf16_kernel");
 }
 
-template <int BM, int BN, int NW, int KSS, bool MI16>
+// MI16: whether two K-contiguous operands are multiplied with the 16 x 16 x 32 instruction (the other
+// layouts always are).
+template <int BM, int BN, int NW, int KSS, bool MI16, int STAGES = 2>
 static int launch_bf16_dl(const GemmArgs& a, bool akc, bool bkc, int64_t batch, hipStream_t st) {
   GemmArgs g = a;
   g.tiles_m = (int)((a.M + BM - 1) / BM);
   g.tiles_n = (int)((a.N + BN - 1) / BN);
   dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)batch);
-  const size_t pipe = 2 * (size_t)(BM + BN) * 8 * 16;
+  const size_t pipe = STAGES * (size_t)(BM + BN) * 8 * 16;
   const size_t slabs = NW * 32 * (size_t)(BN / (NW / 2) + 4) * sizeof(float);
   const size_t lds = pipe > slabs ? pipe : slabs;
   const int epi = (a.residual != nullptr || a.act != NBK_ACT_NONE) ? 2 : (a.bias != nullptr ? 1 : 0);
 #define NBK_LAUNCH_DL(AK, BK_, EP)                                                            \
   do {                                                                                        \
-    auto kern = gemm_bf16_dl_kernel<BM, BN, AK, BK_, EP, NW, KSS, MI16>;                      \
+    auto kern = gemm_bf16_dl_kernel<BM, BN, AK, BK_, EP, NW, KSS, MI16 || !(AK && BK_), false, STAGES>; \
     static bool attr_set = false; /* idempotent, so a race only repeats the call */          \
     if (!attr_set) {                                                                          \
       NBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, \
@@ -1911,16 +1944,16 @@ static int launch_bf16_dl(const GemmArgs& a, bool akc, bool bkc, int64_t batch, 
 
 // The same launch with the column sums of B as a second result (both operands row-contiguous,
 // no epilogue: the weight gradient x^T dy beside the bias gradient).
-template <int BM, int BN, int NW>
+template <int BM, int BN, int NW, int STAGES = 2>
 static int launch_bf16_dl_colsum(const GemmArgs& a, int64_t batch, hipStream_t st) {
   GemmArgs g = a;
   g.tiles_m = (int)((a.M + BM - 1) / BM);
   g.tiles_n = (int)((a.N + BN - 1) / BN);
   dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)batch);
-  const size_t pipe = 2 * (size_t)(BM + BN) * 8 * 16;
+  const size_t pipe = STAGES * (size_t)(BM + BN) * 8 * 16;
   const size_t slabs = NW * 32 * (size_t)(BN / (NW / 2) + 4) * sizeof(float);
   const size_t lds = pipe > slabs ? pipe : slabs;
-  auto kern = gemm_bf16_dl_kernel<BM, BN, false, false, 0, NW, 1, true, true>;
+  auto kern = gemm_bf16_dl_kernel<BM, BN, false, false, 0, NW, 1, true, true, STAGES>;
   static bool attr_set = false; /* idempotent, so a race only repeats the call */
   if (!attr_set) {
     NBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -2148,34 +2181,49 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
                           (d->M > 64 || d->N > 64) &&
                           ((ragged && d->K >= 128) || (d->K >= 512 && d->M % 64 == 0 && d->N % 64 == 0));
     const bool small = tiles_64 <= 512 && !one_each;
+    // Four tile buffers where a launch leaves the LDS for them: a copy requested one tile ahead takes
+    // longer than the tile's few instructions, and a K loop of one workgroup per CU waited for every
+    // one.  Two against four buffers, us: 64 x 64 tiles 1024 x 1024 x 1024 12.0 / 9.0 (nn), 11.8 / 8.2 (xT
+    // dy), 520 x 520 x 768 9.8 / 7.7, 1000 x 1024 x 4096 34.5 / 21.6; on short contractions the requests in
+    // front of the loop cost more (1024 x 1024 x 512 5.7 / 5.8, x 256 4.7 / 4.9).  Two small tiles per CU are
+    // one of 64 x 128 with its four buffers: 1800 x 1024 x 1024 13.0 / 11.4, x 512 8.9 / 8.6, x 384 7.65 / 7.73.
+    // 128 x 128 tiles, where all run at once: 1800 x 2048 x 1024 17.7 / 15.3, x 384 10.9 / 10.5, x 256 9.3 / 9.3.
+    const int64_t cus = nbk_num_cus();
+    const bool deep = d->K > 512;
+    const bool wide = tiles_64 > cus && d->K >= 512 && d->N > 64;
+    const bool one_round = ((d->M + 127) / 128) * ((d->N + 127) / 128) * d->batch <= cus && d->K > 256;
     if (d->colsum != nullptr) {
       NBK_REQUIRE(fast && !akc && !bkc && d->bias == nullptr &&
                       d->residual == nullptr && d->act == NBK_ACT_NONE && d->alpha == 1.f,
                   "gemm: column sums go with a plain bf16 product of two row-contiguous, 16-byte "
                   "aligned operands (M %% 8 == 0, N %% 8 == 0)");
-      return small ? launch_bf16_dl_colsum<64, 64, 4>(a, d->batch, st)
-                   : launch_bf16_dl_colsum<128, 128, 4>(a, d->batch, st);
+      if (small && wide) return launch_bf16_dl_colsum<64, 128, 4, 4>(a, d->batch, st);
+      if (small) return deep ? launch_bf16_dl_colsum<64, 64, 4, 4>(a, d->batch, st)
+                             : launch_bf16_dl_colsum<64, 64, 4>(a, d->batch, st);
+      return one_round ? launch_bf16_dl_colsum<128, 128, 4, 4>(a, d->batch, st)
+                       : launch_bf16_dl_colsum<128, 128, 4>(a, d->batch, st);
     }
     if (!fast) return launch_bf16<128, 128>(a, akc, bkc, d->batch, st);
     // 256 x 256 tiles run at about twice the rate of 128 x 128 ones per CU, one workgroup
     // per CU at a time: take them when the rounds of workgroups they need are at least
     // 60 % full (256 tiles on 256 CUs is the ideal case, 128 or 300 tiles are not).
     const int64_t big_tiles = ((d->M + 255) / 256) * ((d->N + 255) / 256) * d->batch;
-    const int64_t cus = nbk_num_cus();
     const int64_t rounds = (big_tiles + cus - 1) / cus;
     // (a K loop of one or two iterations is all prologue and epilogue: there two co-resident
     // 128 x 128 workgroups per CU overlap better than one 256 x 256)
     // (eight waves on the big tile: 8-16 % faster than four on every shape measured)
     if (big_tiles * 10 >= rounds * cus * 6 && d->M >= 256 && d->N >= 256 && d->K > 128)
       return launch_bf16_dl<256, 256, 8, 1, true>(a, akc, bkc, d->batch, st);
-    if (small) return launch_bf16_dl<64, 64, 4, 1, true>(a, akc, bkc, d->batch, st);
+    if (small && wide) return launch_bf16_dl<64, 128, 4, 1, true, 4>(a, akc, bkc, d->batch, st);
+    if (small) return deep ? launch_bf16_dl<64, 64, 4, 1, true, 4>(a, akc, bkc, d->batch, st)
+                           : launch_bf16_dl<64, 64, 4, 1, true>(a, akc, bkc, d->batch, st);
     // (a 256 x 128 tile was measured and is no faster than 128 x 128 on mid-sized problems:
     // with one workgroup per CU a short K loop is bound by load latency, and two co-resident
     // 128 x 128 workgroups hide it better)
     // (the 16 x 16 x 32 instruction is 3-8 % faster on every shape and layout of the big tile; on
     // this one it gains 4-9 % with a row-contiguous operand and loses 5-10 % with two K-contiguous)
-    return !(akc && bkc) ? launch_bf16_dl<128, 128, 4, 1, true>(a, akc, bkc, d->batch, st)
-                         : launch_bf16_dl<128, 128, 4, 1, false>(a, akc, bkc, d->batch, st);
+    return one_round ? launch_bf16_dl<128, 128, 4, 1, false, 4>(a, akc, bkc, d->batch, st)
+                     : launch_bf16_dl<128, 128, 4, 1, false>(a, akc, bkc, d->batch, st);
   }
   // Two workgroups run on a CU at a time.  A round of 128 x 128 tiles does the work of four of 64 x 64
   // in the time of four, or of 3.5 where K is long; so the larger tile is taken where it fills the
