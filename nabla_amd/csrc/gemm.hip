@@ -17,6 +17,7 @@
 // fp32 path: v_mfma_f32_32x32x2f32 with a 128 x 128 x 16 tile, operands kept
 // k-major in LDS.
 #include "nbk_common.h"
+#include "split_f32.h"
 
 #include <type_traits>
 #include <utility>
@@ -1642,7 +1643,7 @@ __device__ __forceinline__ int f32_at(int row, int chunk, int ld) { return row *
 template <int ROWS, int BK, bool KC>
 struct F32Rows {
   static constexpr int LD = BK + 4;
-  static constexpr int RB = ROWS >= 64 ? 4 : 2;  // row-contiguous operand: blocks of RB rows x 2 k
+  static constexpr int RB = 2;  // row-contiguous operand: blocks of RB rows x 2 k
   static constexpr int V = KC ? 4 : RB, Q = KC ? 1 : 2;  // a piece: Q accesses of V floats
   static constexpr int PAD = KC ? 0 : V - 1;  // LDS rows in front of the tile (place)
   static constexpr int PIECES = ROWS * BK / 256 / (V * Q);
@@ -1719,33 +1720,22 @@ struct F32Rows {
   }
 };
 
-// A workgroup of four waves owns a tile of WM IM x WN IN fragments of 32 x 32; WK waves share a
-// fragment and split every K tile of it (KS steps of 8 each), their sums meet in LDS at the end.
-// Bound by the fp32 matrix rate (157 TFLOP/s: 64 cycles an instruction, so that one 16-byte read per
-// operand for four of them costs nothing) where the tiles fill the chip, else by the length of a
-// workgroup's K loop: hence a choice of tiles down to 32 x 32.  Two K tiles are requested ahead: one
-// workgroup's 16 instructions a tile are shorter than a trip to memory.
+// Small results: a workgroup of four waves owns a tile of 32 x 32 and splits every K tile of 64 (two steps of
+// 8 each); their sums meet in LDS at the end.  Bound by the length of a workgroup's K loop: two K tiles
+// are requested ahead, one workgroup's 8 instructions a wave and tile are shorter than a trip to memory.
 // Lane l of a v_mfma_f32_32x32x2f32 supplies A[row l % 32][k = l / 32] and B[k = l / 32][col l % 32];
 // which two k values share an instruction is free as long as A and B agree, so the lane with half
-// h = l / 32 owns k = 8 s + 4 h .. + 3 of step s and issues four instructions per step.  The smaller
-// tiles sum a product in four chains (waves x accumulators), the largest in one.
-// Before / after (guarded 128 x 128 tiles without loads ahead, or 32 x 32 ones straight from memory
-// below 33 of those): 512 x 2048 x 1024 as x^T dy 150 -> 39 us, 1024 x 2048 x 512 84 -> 28 (77
-// TFLOP/s), 32 x (256 x 64 x 256) 45 -> 10, 8192 x 4096 x 1024 946 -> 621 (111 TFLOP/s), 128 x 256 x
-// 784 15.5 -> 11.3.
-// Two workgroups have to fit a CU (four waves each: the second launch bound), which x^T dy missed by a
-// few registers while its accumulators stood in registers of their own: 8192 x 4096 x 1024 1014 -> 626
-// us, 7680 x 1920 x 64 90 -> 57, 4096 x 1024 x 1024 152 -> 94; with one row-contiguous operand 5 % less.
-// With none, two to five per cent more on contractions of 64 to 512: no bound there.
-template <int WM, int WN, int WK, int IM, int IN, int KS, bool A_KC, bool B_KC>
+// h = l / 32 owns k = 8 s + 4 h .. + 3 of step s and issues four instructions per step.  us: 1024 x 512 x 512
+// 12.9, 32 x (256 x 64 x 256) 9.6, 128 x 256 x 784 11.2.  Two workgroups have to fit a CU (four waves
+// each: the second launch bound); with no row-contiguous operand that costs two to five per cent more on
+// contractions of 64 to 512: no bound there.
+template <bool A_KC, bool B_KC>
 __global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(const GemmArgs g) {
-  static_assert(WM * WN * WK == 4 && (WK == 1 || WK == 4), "four waves, together or apart");
-  constexpr int BM = 32 * WM * IM, BN = 32 * WN * IN, BK = 8 * KS * WK, LD = BK + 4;
-  constexpr int NA = IM * IN == 1 ? 4 / WK : 1;
+  constexpr int BM = 32, BN = 32, WK = 4, KS = 2, BK = 8 * KS * WK, LD = BK + 4;
   constexpr int A0 = F32Rows<BM, BK, A_KC>::PAD * LD, B0 = A0 + (BM + F32Rows<BN, BK, B_KC>::PAD) * LD;
   constexpr int SET = B0 + BN * LD;  // (two of them)
   __shared__ __align__(16) float lds[2 * SET];
-  static_assert(WK == 1 || 4 * 16 * 64 <= 2 * SET, "the partial sums fit");
+  static_assert(4 * 16 * 64 <= 2 * SET, "the partial sums fit");
   int tm_i, tn_i;
   gemm_tile_coords(blockIdx.x, g.tiles_m, g.tiles_n, tm_i, tn_i);
   const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
@@ -1755,17 +1745,10 @@ __global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(con
   const int64_t c_off = bo * g.c_bs + bi * g.c_bs2;
   const int64_t K = gemm_slice_k(g, bo, bi);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wk = wave % WK, wn = wave / WK % WN * 32 * IN, wm = wave / (WK * WN) * 32 * IM;
   const int li = lane & 31, h = lane >> 5;
   const int64_t a_stride = A_KC ? g.a_rs : g.a_cs, b_stride = B_KC ? g.b_cs : g.b_rs;
 
-  f32x16 acc[NA][IM][IN];
-#pragma unroll
-  for (int n = 0; n < NA; ++n)
-#pragma unroll
-    for (int i = 0; i < IM; ++i)
-#pragma unroll
-      for (int j = 0; j < IN; ++j) acc[n][i][j] = (f32x16)(0.f);
+  f32x16 acc = (f32x16)(0.f);
 
   F32Rows<BM, BK, A_KC> la;
   F32Rows<BN, BK, B_KC> lb;
@@ -1793,18 +1776,10 @@ __global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(con
     const float* Bs = lds + cur.value * SET + B0;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      f32x4 fa[IM], fb[IN];
+      const f32x4 fa = *(const f32x4*)(As + f32_at(li, (wave * KS + s) * 2 + h, LD));
+      const f32x4 fb = *(const f32x4*)(Bs + f32_at(li, (wave * KS + s) * 2 + h, LD));
 #pragma unroll
-      for (int i = 0; i < IM; ++i) fa[i] = *(const f32x4*)(As + f32_at(wm + i * 32 + li, (wk * KS + s) * 2 + h, LD));
-#pragma unroll
-      for (int j = 0; j < IN; ++j) fb[j] = *(const f32x4*)(Bs + f32_at(wn + j * 32 + li, (wk * KS + s) * 2 + h, LD));
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int i = 0; i < IM; ++i)
-#pragma unroll
-          for (int j = 0; j < IN; ++j)
-            acc[e % NA][i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][e], fb[j][e], acc[e % NA][i][j], 0, 0, 0);
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], acc, 0, 0, 0);
     }
     if (kt + 1 < nk) store(next);
     __syncthreads();
@@ -1822,8 +1797,8 @@ __global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(con
 
   // D register r of lane (col li, half h) is row (r / 4) * 8 + h * 4 + r % 4
   float* C = (float*)g.C;
-  auto put = [&](int i, int j, int r, float sum) {
-    const int64_t row = m0 + wm + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3), col = n0 + wn + j * 32 + li;
+  auto put = [&](int r, float sum) {
+    const int64_t row = m0 + (r >> 2) * 8 + h * 4 + (r & 3), col = n0 + li;
     if (row >= g.M || col >= g.N) return;
     const int64_t idx = c_off + row * g.ldc + col;
     const float x = sum * g.alpha + (g.bias ? ((const float*)g.bias)[col] : 0.f);
@@ -1838,30 +1813,198 @@ __global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(con
     if (g.residual) v = g.res_mul ? v * ((const float*)g.residual)[idx] : v + ((const float*)g.residual)[idx];
     C[idx] = v;
   };
-  auto chains = [&](int i, int j, int r) {
-    if constexpr (NA == 4) return (acc[0][i][j][r] + acc[1][i][j][r]) + (acc[2][i][j][r] + acc[3][i][j][r]);
-    else return acc[0][i][j][r];
-  };
-  if constexpr (WK == 1) {
+  // (every read of the last K tile lies before its barrier) each wave sums its share of the registers
 #pragma unroll
-    for (int i = 0; i < IM; ++i)
+  for (int r = 0; r < 16; ++r) lds[(wave * 16 + r) * 64 + lane] = acc[r];
+  __syncthreads();
+  const float* part = lds + lane;
 #pragma unroll
-      for (int j = 0; j < IN; ++j)
+  for (int q = 0; q < 4; ++q) {
+    const int r = wave * 4 + q;
+    put(r, (part[r * 64] + part[(16 + r) * 64]) + (part[(32 + r) * 64] + part[(48 + r) * 64]));
+  }
+}
+
+// --------------------------------------------------------------- fp32 out of bf16 parts
+// One operand's rows of a workgroup's K tile on their way through registers: a lane takes pieces of 8
+// consecutive k of a row, which it splits when they have landed (split_f32.h).
+template <int ROWS, int NT, bool KC>
+struct SplitRows {
+  static constexpr int PIECES = ROWS * 4 / NT;
+  static_assert(PIECES >= 1 && PIECES * NT == ROWS * 4, "whole pieces per lane");
+  const float* at[PIECES];  // the piece's first element in the next K tile
+  int64_t stride, left;     // between k of a row-contiguous operand; k from the next tile's first to the end
+  float r[2][KC ? 1 : PIECES][8];  // two K tiles in flight, of either form
+  sp_f4 r4[2][KC ? PIECES : 1][2];
+  __device__ __forceinline__ static void place(int p, int& row, int& c) {
+    const int idx = (int)threadIdx.x + NT * p;
+    row = KC ? idx >> 2 : idx % ROWS;
+    c = KC ? idx & 3 : idx / ROWS;
+  }
+  // (rows past the end repeat the last one: their results are not stored)
+  __device__ __forceinline__ void init(const float* P, int64_t stride_, int64_t row0, int64_t rows, int64_t K) {
+    stride = stride_;
+    left = K;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) put(i, j, r, chains(i, j, r));
-  } else {
-    // (every read of the last K tile lies before its barrier) each of the WK waves sums its share
-    // of the fragment's registers
-#pragma unroll
-    for (int r = 0; r < 16; ++r) lds[(wave * 16 + r) * 64 + lane] = chains(0, 0, r);
-    __syncthreads();
-    const float* part = lds + (wave - wk) * 16 * 64 + lane;
-#pragma unroll
-    for (int q = 0; q < 16 / WK; ++q) {
-      const int r = wk * (16 / WK) + q;
-      put(0, 0, r, (part[r * 64] + part[(16 + r) * 64]) + (part[(32 + r) * 64] + part[(48 + r) * 64]));
+    for (int p = 0; p < PIECES; ++p) {
+      int row, c;
+      place(p, row, c);
+      const int64_t m = min(row0 + row, rows - 1);
+      at[p] = KC ? P + m * stride + c * 8 : P + (c * 8) * stride + m;
     }
   }
+  // Whether the next K tile lies inside K (one branch for both operands: with a branch each, the second
+  // one's requests wait for the data of the first).
+  __device__ __forceinline__ bool whole() const { return left >= SPLIT_BK; }
+  template <int SET>
+  __device__ __forceinline__ void load() {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      if constexpr (KC) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) r4[SET][p][h] = *(const sp_f4_any*)(at[p] + 4 * h);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r[SET][p][e] = at[p][e * stride];
+      }
+    }
+    next();
+  }
+  // The last tile of a contraction that is no multiple of 32.
+  template <int SET>
+  __device__ __forceinline__ void load_tail() {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      int row, c;
+      place(p, row, c);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x = c * 8 + e < left ? at[p][KC ? e : e * stride] : 0.f;
+        if constexpr (KC) r4[SET][p][e >> 2][e & 3] = x;
+        else r[SET][p][e] = x;
+      }
+    }
+    next();
+  }
+  __device__ __forceinline__ void next() {
+    left -= SPLIT_BK;
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) at[p] += KC ? (int64_t)SPLIT_BK : SPLIT_BK * stride;
+  }
+  template <int SET>
+  __device__ __forceinline__ void store(sp_u4* tile) {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      int row, c;
+      place(p, row, c);
+      float x[8];
+      // (the numbers stay as they were loaded until here: split any earlier, they would be waited for
+      // right behind their request)
+      if constexpr (KC) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) asm volatile("" : "+v"(r4[SET][p][h]));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(r[SET][p][e]));
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = KC ? r4[SET][p][e >> 2][e & 3] : r[SET][p][e];
+      split_store<ROWS>(tile, row, c, x);
+    }
+  }
+};
+
+// One element of a product in float32, for sums that are not finite.
+__device__ __attribute__((noinline)) float split_dot(const float* a, int64_t a_cs, const float* b, int64_t b_rs, int64_t K) {
+  float s = 0.f;
+  for (int64_t k = 0; k < K; ++k) s = fmaf(a[k * a_cs], b[k * b_rs], s);
+  return s;
+}
+
+// C = A B of float32 numbers: tiles of BM x BN, NWM x NWN waves, two K tiles of 32 in LDS.
+template <int BM, int BN, int NWM, int NWN, int NM, bool A_KC, bool B_KC, bool FULL>
+__global__ __launch_bounds__(NWM * NWN * 64) void gemm_f32_split_kernel(const GemmArgs g) {
+  constexpr int NT = NWM * NWN * 64, WM = BM / NWM, WN = BN / NWN, TM = WM / 16, TN = WN / 16;
+  constexpr int TILE = (BM + BN) * 12;  // 16-byte chunks: three parts of four chunks a row
+  extern __shared__ __align__(16) u32x4 gemm_lds[];
+  sp_u4* lds = (sp_u4*)gemm_lds;
+  int tm_i, tn_i;
+  gemm_tile_coords(blockIdx.x, g.tiles_m, g.tiles_n, tm_i, tn_i);
+  const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
+  const int64_t bo = (int64_t)blockIdx.y / g.batch_inner, bi = (int64_t)blockIdx.y % g.batch_inner;
+  const float* A = (const float*)g.A + bo * g.a_bs + bi * g.a_bs2;
+  const float* B = (const float*)g.B + bo * g.b_bs + bi * g.b_bs2;
+  const int64_t c_off = bo * g.c_bs + bi * g.c_bs2;
+  const int64_t K = gemm_slice_k(g, bo, bi);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / NWN * WM, wn = wave % NWN * WN;
+  SplitRows<BM, NT, A_KC> la;
+  SplitRows<BN, NT, B_KC> lb;
+  la.init(A, A_KC ? g.a_rs : g.a_cs, m0, g.M, K);
+  lb.init(B, B_KC ? g.b_cs : g.b_rs, n0, g.N, K);
+  SplitAcc<TM, TN, NM> acc;
+  acc.zero();
+  const int nk = (int)((K + SPLIT_BK - 1) / SPLIT_BK);
+#define SPLIT_LOAD(SET)                                                  \
+  do {                                                                   \
+    if (la.whole()) { la.template load<SET>(); lb.template load<SET>(); } \
+    else { la.template load_tail<SET>(); lb.template load_tail<SET>(); }  \
+  } while (0)
+#define SPLIT_STORE(SET) do { la.template store<SET>(lds + SET * TILE); lb.template store<SET>(lds + SET * TILE + BM * 12); } while (0)
+  // tile kt, with tile kt + 2 requested and tile kt + 1 split into the other buffer meanwhile
+#define SPLIT_TILE(SET, REQUEST, MORE)                                                                   \
+  do {                                                                                                   \
+    REQUEST;                                                                                             \
+    acc.template multiply<BM, BN, SET>(lds + SET * TILE, lds + SET * TILE + BM * 12, wm, wn, lane);      \
+    if (MORE) SPLIT_STORE((1 - SET));                                                                    \
+    __syncthreads();                                                                                     \
+  } while (0)
+  SPLIT_LOAD(0);
+  if (nk > 1) SPLIT_LOAD(1);
+  SPLIT_STORE(0);
+  __syncthreads();
+  int kt = 0;
+  // (while the requests are whole tiles they stand in no branch: behind one, the compiler waits for the
+  // youngest request before it lets the splitting have the older ones)
+  for (; kt + 3 < (int)(K / SPLIT_BK); kt += 2) {
+    SPLIT_TILE(0, (la.template load<0>(), lb.template load<0>()), true);
+    SPLIT_TILE(1, (la.template load<1>(), lb.template load<1>()), true);
+  }
+  for (; kt < nk; ++kt) {
+    SPLIT_TILE(0, if (kt + 2 < nk) SPLIT_LOAD(0), kt + 1 < nk);
+    if (++kt < nk) SPLIT_TILE(1, if (kt + 2 < nk) SPLIT_LOAD(1), kt + 1 < nk);
+  }
+#undef SPLIT_TILE
+#undef SPLIT_STORE
+#undef SPLIT_LOAD
+  float* C = (float*)g.C;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int64_t col = n0 + wn + j * 16 + (lane & 15);
+      if (col >= g.N) continue;
+      const float bias = g.bias ? ((const float*)g.bias)[col] : 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t row = m0 + wm + i * 16 + (lane >> 4) * 4 + r;
+        if (row >= g.M) continue;
+        float sum = acc.sum(i, j, r);
+        if (!(fabsf(sum) < INFINITY)) sum = split_dot(A + row * g.a_rs, g.a_cs, B + col * g.b_cs, g.b_rs, K);
+        const int64_t idx = c_off + row * g.ldc + col;
+        const float x = sum * g.alpha + bias;
+        float v;
+        if (FULL && g.C2) {
+          float dv;
+          gemm_act_pair<false>(x, g.act, v, dv);
+          ((float*)g.C2)[idx] = dv;
+        } else {
+          v = FULL ? gemm_act(x, g.act) : g.act == NBK_ACT_RELU ? fmaxf(x, 0.f) : x;
+        }
+        if (FULL && g.residual) v = g.res_mul ? v * ((const float*)g.residual)[idx] : v + ((const float*)g.residual)[idx];
+        C[idx] = v;
+      }
+    }
 }
 
 template <int BM, int BN, int NW = 4>
@@ -1963,20 +2106,52 @@ static int launch_bf16_dl_colsum(const GemmArgs& a, int64_t batch, hipStream_t s
   return nbk_check_launch("gemm_bf16_dl_kernel (column sums)");
 }
 
-template <int WM, int WN, int WK, int IM, int IN, int KS>
 static int launch_f32(const GemmArgs& args, bool akc, bool bkc, int64_t batch, hipStream_t st) {
-  constexpr int BM = 32 * WM * IM, BN = 32 * WN * IN;
+  GemmArgs a = args;
+  const int64_t tiles_m = (a.M + 31) / 32, tiles_n = (a.N + 31) / 32;
+  NBK_REQUIRE(tiles_m * tiles_n <= 0x7fffffffLL, "gemm: launch too large");
+  a.tiles_m = (int)tiles_m;
+  a.tiles_n = (int)tiles_n;
+  const dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch);
+  if (akc && bkc) hipLaunchKernelGGL((gemm_f32_kernel<true, true>), grid, dim3(256), 0, st, a);
+  else if (akc) hipLaunchKernelGGL((gemm_f32_kernel<true, false>), grid, dim3(256), 0, st, a);
+  else if (bkc) hipLaunchKernelGGL((gemm_f32_kernel<false, true>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((gemm_f32_kernel<false, false>), grid, dim3(256), 0, st, a);
+  return nbk_check_launch("gemm_f32_kernel");
+}
+
+template <int BM, int BN, int NWM, int NWN, int NM>
+static int launch_f32_split(const GemmArgs& args, bool akc, bool bkc, int64_t batch, hipStream_t st) {
   GemmArgs a = args;
   const int64_t tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
   NBK_REQUIRE(tiles_m * tiles_n <= 0x7fffffffLL, "gemm: launch too large");
   a.tiles_m = (int)tiles_m;
   a.tiles_n = (int)tiles_n;
   const dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch);
-  if (akc && bkc) hipLaunchKernelGGL((gemm_f32_kernel<WM, WN, WK, IM, IN, KS, true, true>), grid, dim3(256), 0, st, a);
-  else if (akc) hipLaunchKernelGGL((gemm_f32_kernel<WM, WN, WK, IM, IN, KS, true, false>), grid, dim3(256), 0, st, a);
-  else if (bkc) hipLaunchKernelGGL((gemm_f32_kernel<WM, WN, WK, IM, IN, KS, false, true>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((gemm_f32_kernel<WM, WN, WK, IM, IN, KS, false, false>), grid, dim3(256), 0, st, a);
-  return nbk_check_launch("gemm_f32_kernel");
+  const size_t lds = 2 * (size_t)(BM + BN) * 12 * 16;
+  const bool full = a.C2 || a.residual || a.act == NBK_ACT_GELU;
+#define NBK_LAUNCH_SPLIT(AK, BK_, F)                                                                     \
+  do {                                                                                                   \
+    auto kern = gemm_f32_split_kernel<BM, BN, NWM, NWN, NM, AK, BK_, F>;                                 \
+    static bool attr_set = false; /* idempotent, so a race only repeats the call */                     \
+    if (!attr_set) {                                                                                     \
+      NBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
+      attr_set = true;                                                                                   \
+    }                                                                                                    \
+    hipLaunchKernelGGL(kern, grid, dim3(NWM * NWN * 64), lds, st, a);                                    \
+  } while (0)
+#define NBK_LAUNCH_SPLIT2(AK, BK_)                                 \
+  do {                                                             \
+    if (full) NBK_LAUNCH_SPLIT(AK, BK_, true);                     \
+    else NBK_LAUNCH_SPLIT(AK, BK_, false);                         \
+  } while (0)
+  if (akc && bkc) NBK_LAUNCH_SPLIT2(true, true);
+  else if (akc) NBK_LAUNCH_SPLIT2(true, false);
+  else if (bkc) NBK_LAUNCH_SPLIT2(false, true);
+  else NBK_LAUNCH_SPLIT2(false, false);
+#undef NBK_LAUNCH_SPLIT2
+#undef NBK_LAUNCH_SPLIT
+  return nbk_check_launch("gemm_f32_split_kernel");
 }
 
 extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
@@ -2225,24 +2400,19 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
     return one_round ? launch_bf16_dl<128, 128, 4, 1, false, 4>(a, akc, bkc, d->batch, st)
                      : launch_bf16_dl<128, 128, 4, 1, false>(a, akc, bkc, d->batch, st);
   }
-  // Two workgroups run on a CU at a time.  A round of 128 x 128 tiles does the work of four of 64 x 64
-  // in the time of four, or of 3.5 where K is long; so the larger tile is taken where it fills the
-  // chip and needs no more than that, its last round and what lies past the edges counted.  Short contractions are all
-  // prologue and epilogue, and the smaller tile overlaps them better.  Measured, us on 128 x 128 / 64 x 64:
-  // 8192 x 4096 x 1024 (2048 large tiles) 623 / 705, 8 x (1024 x 1024 x 1024) (512) 160 / 184, 5000 x 3000
-  // x 256 (960) 108 / 111; 3072 x 2944 x 1024 (552) 258 / 204, 64 x (333 x 333 x 64) (576) 56 / 40, 64 x
-  // (64 x 999 x 256) (512, half of them empty) 61 / 38, 4096 x 4096 x 64 (1024) 65 / 62.
-  // Below two small tiles per CU the K loop of one workgroup is what a launch waits for, and the
-  // more waves share a CU the less of it shows: on 64 x 64 / 32 x 32 tiles 1024 x 2048 x 512 (512 of 64)
-  // 29 / 35, 1024 x 512 x 2048 (128) 53 / 33, 128 x 256 x 784 (8) 25 / 11; as x^T dy the line would lie
-  // lower (512 x 2048 x 1024, 256 of 64: 32 / 39).
+  // Out of bf16 parts where a launch gives most CUs a tile of 64 x 64; below that the K loop of one workgroup
+  // is what a launch waits for, and four waves that share a fragment of 32 x 32 on the float32
+  // instruction have the shorter one.  us, 32 x 32 / 64 x 64 out of parts: 1024 x 512 x 512 (128 tiles of 64)
+  // 12.9 / 15.9, 512 x 2048 x 1024 (256) 34 / 27 and as x^T dy 40 / 27, 1024 x 1024 x 200 (256) 15.1 / 10.3.
+  // 128 x 128 tiles run one to a CU, two of 64 x 64 do; a round of the former does the work of two of the
+  // latter in 1.7 of one's time: 4096 x 4096 x 1024 (4 rounds / 8) 197 / 251, 4096 x 1024 x 64 (1 / 2) 12.4 /
+  // 14.2, 64 x (333 x 333 x 64) (3 / 5) 33 / 29, 2048 x 1024 x 1024 (1 / 1) 44 / 39.
   auto tiles = [&](int64_t edge) { return ((d->M + edge - 1) / edge) * ((d->N + edge - 1) / edge) * d->batch; };
-  const int64_t slots = 2 * (int64_t)nbk_num_cus();
-  auto rounds = [&](int64_t edge) { return (tiles(edge) + slots - 1) / slots; };
-  if (tiles(128) >= slots && d->K >= 256 && rounds(128) * 80 <= rounds(64) * (d->K >= 512 ? 23 : 20))
-    return launch_f32<2, 2, 1, 2, 2, 2>(a, akc, bkc, d->batch, st);
-  if (tiles(64) >= 512) return launch_f32<2, 2, 1, 1, 1, 4>(a, akc, bkc, d->batch, st);
-  return launch_f32<1, 1, 4, 1, 1, 2>(a, akc, bkc, d->batch, st);
+  const int64_t cus = nbk_num_cus(), t64 = tiles(64);
+  if (t64 * 4 < cus * 3) return launch_f32(a, akc, bkc, d->batch, st);
+  const int64_t rounds_64 = (t64 + 2 * cus - 1) / (2 * cus), rounds_128 = (tiles(128) + cus - 1) / cus;
+  if (rounds_128 * 17 <= rounds_64 * 10) return launch_f32_split<128, 128, 2, 4, 2>(a, akc, bkc, d->batch, st);
+  return launch_f32_split<64, 64, 2, 2, 2>(a, akc, bkc, d->batch, st);
 }
 
 // ------------------------------------------------------------------ NF4-coded weights

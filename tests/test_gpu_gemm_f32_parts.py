@@ -1,0 +1,68 @@
+"""float32 products out of bf16 parts: every layout at the edges of both tiles and of a K tile of 32, slices,
+epilogues, against float64; numbers that have no parts (infinities, NaN, beyond the largest bf16)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def product(a, b, layout, alpha=1.0, **fields):
+    from nabla_amd.backend import lib
+    M, K = a.shape
+    N = b.shape[1]
+    ad = torch.tensor(np.ascontiguousarray(a.T if layout[0] == "t" else a)).cuda()
+    bd = torch.tensor(np.ascontiguousarray(b.T if layout[1] == "t" else b)).cuda()
+    out = torch.full((M, N), float("nan"), device="cuda")
+    d = lib.GemmDesc()
+    d.A, d.B, d.C = ad.data_ptr(), bd.data_ptr(), out.data_ptr()
+    d.M, d.N, d.K = M, N, K
+    d.a_rs, d.a_cs = (1, M) if layout[0] == "t" else (K, 1)
+    d.b_rs, d.b_cs = (1, K) if layout[1] == "t" else (N, 1)
+    d.ldc, d.batch, d.batch_inner, d.dtype_ab, d.dtype_c, d.alpha = N, 1, 1, 0, 0, alpha
+    for name, value in fields.items():
+        setattr(d, name, value)
+    lib.check(lib.load().nbk_gemm(C.byref(d), C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    return out.cpu().numpy()
+
+
+# A sum is rounded once per K tile of 32 and accumulator (2^-24 of what has been summed, at most the sum of
+# magnitudes) and once in each of the five small products; what the six leave out is 2^-25 of a product.
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("M,N,K", [(1025, 769, 31), (897, 1024, 64), (1100, 1200, 65), (1024, 1000, 129),   # 64 x 64
+                                   (2047, 2050, 95), (2100, 1990, 160), (4097, 1921, 33)])                 # 128 x 128
+def test_against_float64(hip, layout, M, N, K):
+    rng = np.random.default_rng(K)
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((M, K), (K, N)))
+    bias = rng.standard_normal(N).astype(np.float32)
+    bd = torch.tensor(bias).cuda()
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    want, size = a64 @ b64, np.abs(a64) @ np.abs(b64)
+    tol = (-(-K // 32) + 4) * 2.0 ** -24 * size + 2.0 ** -23 * np.abs(want)
+    assert (np.abs(product(a, b, layout) - want) <= tol).all()
+    got = product(a, b, layout, alpha=0.5, bias=bd.data_ptr(), act=1)  # relu
+    want = np.maximum(0.5 * want + bias, 0.0)
+    assert (np.abs(got - want) <= tol + 2.0 ** -23 * (np.abs(want) + np.abs(bias))).all()
+
+
+@pytest.mark.parametrize("M,N", [(1024, 1024), (2048, 2048)])
+def test_numbers_without_parts(hip, M, N):
+    K = 70
+    rng = np.random.default_rng(0)
+    a, b = (rng.uniform(0.5, 1.0, s).astype(np.float32) for s in ((M, K), (K, N)))
+    a[3, 5], a[70, 69], b[11, 20] = np.inf, -np.inf, np.nan
+    a[9, 1], b[1, 30] = np.inf, 0.0                     # (infinity times zero)
+    a[M - 1, 0], b[0, N - 1] = 3.4e38, 1e-30             # rounds to infinity as a bf16
+    a[40, :] = 1e37                                      # a sum beyond the largest float32
+    want = np.zeros((M, N), np.float32)
+    with np.errstate(all="ignore"):
+        for k in range(K):
+            want += a[:, k:k + 1] * b[k:k + 1]
+    got = product(a, b, "nn")
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+    np.testing.assert_array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)]))
+    ok = np.isfinite(want)
+    assert (np.abs(got[ok] - want[ok]) <= 1e-5 * np.abs(want[ok])).all()
