@@ -1,6 +1,5 @@
 // conv2d (NHWC x RSCK) forward, input gradient and filter gradient as implicit
-// GEMMs on v_mfma_f32_32x32x2f32.  No im2col buffer is materialised: the tile
-// loaders gather straight from the image.
+// GEMMs.  No im2col buffer is materialised: the tile loaders gather straight from the image.
 //
 //   forward : M = N*Ho*Wo   Ng = Cout   K = R*S*Cin   (k = (r, s, c), c fastest)
 //             A[m,k] = x[n, ho*sh-pt+r, wo*sw-pl+s, c]      B[k,j] = w[r,s,c,j]
@@ -10,16 +9,18 @@
 //             A[m,k] = x[n, ho*sh-pt+r, wo*sw-pl+s, c]      B[k,j] = dy[n,ho,wo,j]
 // Out-of-image taps read zero, which is the zero padding of the reference op.
 //
-// Address arithmetic is kept out of the K loop: a lane owns one output pixel
-// (forward, dgrad) or one run of 8 filter rows (wgrad) for the whole tile and
-// decomposes it once; with channel counts that are multiples of 16 (8 for wgrad)
-// a 16-wide K step lies inside one filter tap, the tap is uniform across the
-// workgroup, and every lane fetches 8 consecutive channels as two 16-byte loads
-// (FAST).  Other channel counts take the element-wise gather.
+// Forward and dgrad multiply out of bf16 parts (split_f32.h), the filter gradient on the float32
+// instruction.  Address arithmetic is kept out of the K loop: a lane decomposes its pixels or filter
+// rows once and steps through the taps.
 // wgrad contracts over every output pixel of the batch while its result is tiny,
 // so it is split along K over blockIdx.z into a workspace and summed by a second
 // kernel in a fixed order (no atomics: results do not depend on scheduling).
+//
+// us, before (float32 instruction, channel counts that are no multiple of 16 gathered one by one) / now:
+// 64 x 32 x 32, 64 -> 128 channels forward 98 / 79, dgrad 107 / 83; 64 x 16 x 16, 128 -> 256 107 / 67, 138 / 80;
+// 50 x 28 x 28, 24 -> 40 44 / 25, 96 / 23; 50 x 14 x 14, 40 -> 72 48 / 22, 123 / 22; 5 x 13 x 13, 24 -> 40 31 / 12, 71 / 15.
 #include "nbk_common.h"
+#include "split_f32.h"
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -129,15 +130,14 @@ __device__ __forceinline__ void conv_ld8(const float* p, bool ok, float* r) {
   r[4] = v1.x; r[5] = v1.y; r[6] = v1.z; r[7] = v1.w;
 }
 
+// Filter gradient on the float32 instruction, channel counts that are multiples of 8.
 // NJ: 32-column MFMA tiles per wave along the output's channel axis: 2 for a 128 x 128
 // workgroup tile, 1 for 128 x 64 (channel counts up to 64 would waste half of the wider tile).
-template <int MODE, bool FAST, int NJ>
-__global__ __launch_bounds__(256) void conv_kernel(const ConvArgs g) {
+template <int NJ>
+__global__ __launch_bounds__(256) void conv_wgrad_kernel(const ConvArgs g) {
   // Tiles sit in LDS k-major, [k][128 rows], with the rows of k-row k rotated by 32 places when
   // (k ^ k / 8) is odd.  The two halves of a wave read k-rows 2 ks and 2 ks + 1 of one MFMA
-  // step, and the two lanes of a pixel store k-rows e and 8 + e: either way the halves land
-  // 32 banks apart (a padded pitch of 132 serves the stores only: 77-87 % of the LDS cycles of
-  // these kernels were bank conflicts).
+  // step, and either way the halves land 32 banks apart.
   constexpr int BK = 16, LD = 128, BN = 64 * NJ;
   __shared__ float As[2][BK][LD];
   __shared__ float Bs[2][BK][LD];
@@ -158,173 +158,48 @@ __global__ __launch_bounds__(256) void conv_kernel(const ConvArgs g) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = (f32x16)(0.f);
 
-  // ---- per-lane constants of the A gather ----
-  // forward / dgrad: the lane's pixel; wgrad: the lane's first filter row and, as running
-  // state, the pixel of its K column.
-  const int a_row = tid >> 1, a_kk = (tid & 1) * 8;  // fwd / dgrad: pixel row, 8 k
-  const int w_kk = tid >> 4, w_rr = (tid & 15) * 8;  // wgrad: pixel column, 8 filter rows
-  int p_n = 0, p_y = 0, p_x = 0;
-  bool p_ok = false;
-  int f_r = 0, f_s = 0, f_c = 0;
-  bool f_ok = false;
-  if (MODE == CONV_WGRAD) {
-    const int64_t m = m0 + w_rr;
-    f_ok = m < g.M;
-    const int mm = f_ok ? (int)m : 0;
-    f_c = mm % (int)d.Cin;
-    const int rs = mm / (int)d.Cin;
-    f_s = rs % (int)d.S;
-    f_r = rs / (int)d.S;
-    const int64_t px = k_begin + w_kk;  // < 2^31 (checked on the host)
-    p_x = (int)(px % d.Wo);
-    const int t = (int)(px / d.Wo);
-    p_y = t % (int)d.Ho;
-    p_n = t / (int)d.Ho;
-  } else {
-    const int64_t m = m0 + a_row;
-    p_ok = m < g.M;
-    const int mm = p_ok ? (int)m : 0;
-    const int wd = MODE == CONV_FWD ? (int)d.Wo : (int)d.W;
-    const int hd = MODE == CONV_FWD ? (int)d.Ho : (int)d.H;
-    p_x = mm % wd;
-    const int t = mm / wd;
-    p_y = t % hd;
-    p_n = t / hd;
-  }
+  // the lane's first filter row and, as running state, the pixel of its K column
+  const int w_kk = tid >> 4, w_rr = (tid & 15) * 8;  // pixel column, 8 filter rows
+  const int64_t m = m0 + w_rr;
+  const bool f_ok = m < g.M;
+  const int mm = f_ok ? (int)m : 0;
+  const int f_c = mm % (int)d.Cin, rs = mm / (int)d.Cin;
+  const int f_s = rs % (int)d.S, f_r = rs / (int)d.S;
+  const int64_t px = k_begin + w_kk;  // < 2^31 (checked on the host)
+  int p_x = (int)(px % d.Wo);
+  const int t = (int)(px / d.Wo);
+  int p_y = t % (int)d.Ho, p_n = t / (int)d.Ho;
 
   float ra[8], rb[8];
-  const bool unit_stride = d.stride_h == 1 && d.stride_w == 1;
-  // forward / dgrad, FAST: the filter tap (t_r, t_s) and the first channel t_c of the K step
-  // that is loaded next (uniform; kept as running counters: a 64-bit division per K step and
-  // operand otherwise)
-  int t_r = 0, t_s = 0, t_c = 0;
-  if (FAST && MODE != CONV_WGRAD) {
-    const int ck = MODE == CONV_FWD ? (int)d.Cin : (int)d.Cout;
-    const int tap = (int)(k_begin / ck);
-    t_c = (int)(k_begin - (int64_t)tap * ck);
-    t_r = tap / (int)d.S;
-    t_s = tap - t_r * (int)d.S;
-  }
-  // forward: row, column and number of the lane's input pixel at tap (0, 0); dgrad with unit
-  // stride: the same for its output pixel
-  int q_h0 = 0, q_w0 = 0, q_pix0 = 0;
-  if (MODE == CONV_FWD) {
-    q_h0 = p_y * d.stride_h - d.pad_t;
-    q_w0 = p_x * d.stride_w - d.pad_l;
-    q_pix0 = (p_n * (int)d.H + q_h0) * (int)d.W + q_w0;
-  } else if (MODE == CONV_DGRAD) {
-    q_h0 = p_y + d.pad_t;
-    q_w0 = p_x + d.pad_l;
-    q_pix0 = (p_n * (int)d.Ho + q_h0) * (int)d.Wo + q_w0;
-  }
-  auto next_tap = [&]() {
-    if (FAST && MODE != CONV_WGRAD) {
-      const int ck = MODE == CONV_FWD ? (int)d.Cin : (int)d.Cout;
-      t_c += BK;
-      if (t_c >= ck) {
-        t_c -= ck;
-        if (++t_s == (int)d.S) { t_s = 0; ++t_r; }
-      }
+  auto load = [&](int64_t k0) {
+    // pixel (p_n, p_y, p_x) is column k0 + w_kk; taps of rows m0 + w_rr .. + 7
+    const int64_t k = k0 + w_kk, j = n0 + w_rr;
+    const int h = p_y * d.stride_h - d.pad_t + f_r, w = p_x * d.stride_w - d.pad_l + f_s;
+    const bool ok = f_ok && k < k_end && h >= 0 && h < d.H && w >= 0 && w < d.W;
+    conv_ld8(g.a + (((int64_t)p_n * d.H + h) * d.W + w) * d.Cin + f_c, ok, ra);
+    // advance the pixel by one K step
+    p_x += BK;
+    while (p_x >= d.Wo) {
+      p_x -= (int)d.Wo;
+      if (++p_y >= d.Ho) { p_y = 0; ++p_n; }
     }
+    conv_ld8(g.b + k * d.Cout + j, k < k_end && j < g.Ng, rb);  // dy, [K, Cout] row-major
   };
-  auto load_a = [&](int64_t k0) {
-    if (MODE == CONV_WGRAD) {
-      // pixel (p_n, p_y, p_x) is column k0 + w_kk; taps of rows m0 + w_rr .. + 7
-      const bool k_ok = k0 + w_kk < k_end;
-      if (FAST) {
-        const int h = p_y * d.stride_h - d.pad_t + f_r, w = p_x * d.stride_w - d.pad_l + f_s;
-        const bool ok = f_ok && k_ok && h >= 0 && h < d.H && w >= 0 && w < d.W;
-        conv_ld8(g.a + (((int64_t)p_n * d.H + h) * d.W + w) * d.Cin + f_c, ok, ra);
-      } else {
+  auto store = [&](int buf) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ra[e] = conv_load_a<MODE>(g, m0 + w_rr + e, k0 + w_kk, k_end);
-      }
-      // advance the pixel by one K step
-      p_x += BK;
-      while (p_x >= d.Wo) {
-        p_x -= (int)d.Wo;
-        if (++p_y >= d.Ho) { p_y = 0; ++p_n; }
-      }
-    } else if (FAST) {
-      const int c0 = t_c + a_kk, r = t_r, s = t_s;
-      if (MODE == CONV_FWD) {
-        // (the lane's pixel at tap (0, 0) is a constant of the lane; the tap adds a uniform
-        // number of pixels; pixel numbers fit 32 bits, checked on the host)
-        const int h = q_h0 + r, w = q_w0 + s;
-        const bool ok = p_ok && h >= 0 && h < d.H && w >= 0 && w < d.W;
-        conv_ld8(g.a + (int64_t)(q_pix0 + r * (int)d.W + s) * d.Cin + c0, ok, ra);
-      } else if (unit_stride) {
-        const int ho = q_h0 - r, wo = q_w0 - s;
-        const bool ok = p_ok && ho >= 0 && wo >= 0 && ho < d.Ho && wo < d.Wo;
-        conv_ld8(g.a + (int64_t)(q_pix0 - r * (int)d.Wo - s) * d.Cout + c0, ok, ra);
-      } else {  // (two integer divisions per lane and K step)
-        const int hn = p_y + d.pad_t - r, wn = p_x + d.pad_l - s;
-        const int ho = hn / d.stride_h, wo = wn / d.stride_w;
-        const bool ok = p_ok && hn >= 0 && wn >= 0 && ho * d.stride_h == hn &&
-                        wo * d.stride_w == wn && ho < d.Ho && wo < d.Wo;
-        conv_ld8(g.a + (((int64_t)p_n * d.Ho + ho) * d.Wo + wo) * d.Cout + c0, ok, ra);
-      }
-    } else {
+    for (int e = 0; e < 8; ++e) As[buf][w_kk][rot(w_kk, w_rr) + e] = ra[e];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) ra[e] = conv_load_a<MODE>(g, m0 + a_row, k0 + a_kk + e, k_end);
-    }
-  };
-  auto store_a = [&](float (*S)[LD]) {
-    if (MODE == CONV_WGRAD) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) S[w_kk][rot(w_kk, w_rr) + e] = ra[e];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) S[a_kk + e][rot(a_kk + e, a_row)] = ra[e];
-    }
-  };
-  auto load_b = [&](int64_t k0) {
-    if (MODE == CONV_DGRAD) {
-      // w[r, s, j, co]: contiguous along k = co for a fixed input channel j
-      const int64_t j = n0 + a_row;
-      if (FAST) {
-        const int tap = t_r * (int)d.S + t_s, co = t_c + a_kk;
-        conv_ld8(g.b + ((int64_t)tap * d.Cin + j) * d.Cout + co, j < g.Ng, rb);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) rb[e] = conv_load_b<MODE>(g, k0 + a_kk + e, j, k_end);
-      }
-    } else {
-      // [K, Cout] row-major: w for the forward product, dy for wgrad
-      const int64_t k = k0 + w_kk, j = n0 + w_rr;
-      if (FAST) {
-        conv_ld8(g.b + k * d.Cout + j, k < k_end && j < g.Ng, rb);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) rb[e] = conv_load_b<MODE>(g, k, j + e, k_end);
-      }
-    }
-  };
-  auto store_b = [&](float (*S)[LD]) {
-    if (MODE == CONV_DGRAD) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) S[a_kk + e][rot(a_kk + e, a_row)] = rb[e];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) S[w_kk][rot(w_kk, w_rr) + e] = rb[e];
-    }
+    for (int e = 0; e < 8; ++e) Bs[buf][w_kk][rot(w_kk, w_rr) + e] = rb[e];
   };
 
   const int64_t nk = (k_end - k_begin + BK - 1) / BK;
-  load_a(k_begin);
-  load_b(k_begin);
-  next_tap();
-  store_a(As[0]);
-  store_b(Bs[0]);
+  load(k_begin);
+  store(0);
   __syncthreads();
   for (int64_t kt = 0; kt < nk; ++kt) {
     const int cur = kt & 1;
     const bool more = kt + 1 < nk;
-    if (more) {
-      load_a(k_begin + (kt + 1) * BK);
-      load_b(k_begin + (kt + 1) * BK);
-      next_tap();
-    }
+    if (more) load(k_begin + (kt + 1) * BK);
 #pragma unroll
     for (int ks = 0; ks < BK / 2; ++ks) {
       const int k = ks * 2 + kg;
@@ -339,10 +214,7 @@ __global__ __launch_bounds__(256) void conv_kernel(const ConvArgs g) {
         for (int j = 0; j < NJ; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
     }
-    if (more) {
-      store_a(As[cur ^ 1]);
-      store_b(Bs[cur ^ 1]);
-    }
+    if (more) store(cur ^ 1);
     __syncthreads();
   }
 #pragma unroll
@@ -350,16 +222,262 @@ __global__ __launch_bounds__(256) void conv_kernel(const ConvArgs g) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       const int64_t col = n0 + wn + j * 32 + li;
-      const bool col_ok = col < g.Ng;
-      const float bv = (g.bias && col_ok) ? g.bias[col] : 0.f;
-      const bool relu = MODE == CONV_FWD && d.act == NBK_ACT_RELU;
+      if (col >= g.Ng) continue;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int64_t row = m0 + wm + i * 32 + (r >> 2) * 8 + kg * 4 + (r & 3);
-        const float v = acc[i][j][r] + bv;
-        if (col_ok && row < g.M) out[row * g.Ng + col] = relu ? fmaxf(v, 0.f) : v;
+        if (row < g.M) out[row * g.Ng + col] = acc[i][j][r];
       }
     }
+}
+
+// ---- out of bf16 parts (split_f32.h) --------------------------------------------------------
+// Tiles of BM x BN on NWM x NWN waves, K tiles of 32 in two LDS buffers.  A lane takes pieces of 8
+// consecutive k of a row: forward and dgrad, 8 channels of a pixel at one tap (channel counts that are
+// multiples of 8: FAST), each piece with its own tap; wgrad, one filter row at 8 pixels.  The pieces of the
+// next tile but one are requested before a tile is multiplied and split behind it.
+// The launch's K loop is the sum of its matrix instructions and of what it costs to gather and to split
+// (5.5 instructions a number), which the two waves of a SIMD cover for each other only in part.
+template <int MODE, bool FAST, int ROWS, int NT, bool IS_A>
+struct ConvRows {
+  static constexpr int PIECES = ROWS * 4 > NT ? ROWS * 4 / NT : 1;
+  static_assert(PIECES == 1 || PIECES * NT == ROWS * 4, "whole pieces per lane");
+  // (a tile of fewer pieces than lanes: the lanes behind them request the first number of the tensor)
+  static __device__ __forceinline__ bool mine() { return ROWS * 4 >= NT || (int)threadIdx.x < ROWS * 4; }
+  // whether a piece's 8 numbers stand side by side in memory
+  static constexpr bool WHOLE = FAST && MODE != CONV_WGRAD && (IS_A || MODE == CONV_DGRAD);
+  int row[PIECES], c[PIECES];
+  // forward / dgrad: pixel at tap (0, 0) of an A piece; wgrad: the tap's offset from a pixel
+  int q_h[PIECES], q_w[PIECES], q_pix[PIECES], ch[PIECES];
+  bool ok[PIECES];
+  int t_r[PIECES], t_s[PIECES], t_c[PIECES];  // the next K tile's tap and first channel; wgrad: pixel (n, y, x)
+  float r[2][PIECES][8];
+
+  __device__ __forceinline__ void init(const ConvArgs& g, int64_t row0, int64_t k_begin) {
+    const nbk_conv_desc& d = g.d;
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      const int idx = (int)threadIdx.x + NT * p;
+      row[p] = WHOLE ? idx >> 2 : idx % ROWS;
+      c[p] = WHOLE ? idx & 3 : idx / ROWS;
+      const int64_t m = row0 + row[p];
+      const int k = (int)k_begin + c[p] * 8;
+      ok[p] = mine() && m < (IS_A ? g.M : g.Ng);
+      const int mm = ok[p] ? (int)m : 0;
+      if (MODE == CONV_WGRAD) {
+        if (IS_A) {
+          int s;
+          const int rs = g.by_cin.divmod(mm, ch[p]);
+          const int rr = g.by_s.divmod(rs, s);
+          q_h[p] = rr - d.pad_t;
+          q_w[p] = s - d.pad_l;
+          const int t = g.by_wo.divmod(k, t_c[p]);
+          t_r[p] = g.by_ho.divmod(t, t_s[p]);
+        }
+      } else {
+        const ConvDiv& by = MODE == CONV_FWD ? g.by_cin : g.by_cout;
+        const int tap = by.divmod(k, t_c[p]);
+        t_r[p] = g.by_s.divmod(tap, t_s[p]);
+        if (IS_A) {
+          int x, y;
+          const int t = (MODE == CONV_FWD ? g.by_wo : g.by_w).divmod(mm, x);
+          const int n = (MODE == CONV_FWD ? g.by_ho : g.by_h).divmod(t, y);
+          if (MODE == CONV_FWD) {
+            q_h[p] = y * d.stride_h - d.pad_t;
+            q_w[p] = x * d.stride_w - d.pad_l;
+            q_pix[p] = (n * (int)d.H + q_h[p]) * (int)d.W + q_w[p];
+          } else {
+            q_h[p] = y + d.pad_t;
+            q_w[p] = x + d.pad_l;
+            q_pix[p] = n;
+          }
+        }
+      }
+    }
+  }
+  // Forward / dgrad: where channel `chan` of piece p's pixel lies at tap (r, s), and whether it is inside.
+  __device__ __forceinline__ bool where(const nbk_conv_desc& d, int p, int r, int s, int chan, int64_t& at) const {
+    if (MODE == CONV_FWD) {
+      const int h = q_h[p] + r, w = q_w[p] + s;
+      at = (int64_t)(q_pix[p] + r * (int)d.W + s) * d.Cin + chan;
+      return h >= 0 && h < d.H && w >= 0 && w < d.W;
+    }
+    const int hn = q_h[p] - r, wn = q_w[p] - s;
+    int ho = hn, wo = wn;
+    bool in = hn >= 0 && wn >= 0;
+    if (d.stride_h != 1 || d.stride_w != 1) {
+      ho = hn / d.stride_h;
+      wo = wn / d.stride_w;
+      in = in && ho * d.stride_h == hn && wo * d.stride_w == wn;
+    }
+    at = (int64_t)((q_pix[p] * (int)d.Ho + ho) * (int)d.Wo + wo) * d.Cout + chan;
+    return in && ho < d.Ho && wo < d.Wo;
+  }
+  // K tile at k0 into set SET; the pieces move on to the next.
+  template <int SET>
+  __device__ __forceinline__ void load(const ConvArgs& g, int64_t row0, int64_t k0, int64_t k_end) {
+    const nbk_conv_desc& d = g.d;
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      const int64_t k = k0 + c[p] * 8, m = row0 + row[p];
+      float* x = r[SET][p];
+      if constexpr (!FAST && !IS_A) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = ok[p] ? conv_load_b<MODE>(g, k + e, m, k_end) : 0.f;
+      } else if constexpr (!FAST) {  // every number has a tap of its own
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          int chan, s;
+          const int tap = (MODE == CONV_FWD ? g.by_cin : g.by_cout).divmod((int)k + e, chan);
+          const int rr = g.by_s.divmod(tap, s);
+          int64_t at;
+          const bool in = ok[p] && k + e < k_end && where(d, p, rr, s, chan, at);
+          const float v = g.a[in ? at : 0];
+          x[e] = in ? v : 0.f;
+        }
+      } else if constexpr (MODE == CONV_WGRAD && IS_A) {
+        // 8 pixels in a row of the output, or across its end
+        int n = t_r[p], y = t_s[p], w = t_c[p];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int ih = y * d.stride_h + q_h[p], iw = w * d.stride_w + q_w[p];
+          const bool in = ok[p] && k + e < k_end && ih >= 0 && ih < d.H && iw >= 0 && iw < d.W;
+          const int64_t at = in ? (int64_t)((n * (int)d.H + ih) * (int)d.W + iw) * d.Cin + ch[p] : 0;
+          const float v = g.a[at];
+          x[e] = in ? v : 0.f;
+          if (++w == d.Wo) {
+            w = 0;
+            if (++y == d.Ho) { y = 0; ++n; }
+          }
+        }
+      } else if constexpr (WHOLE) {
+        bool in = ok[p] && k < k_end;
+        int64_t at;
+        if (!IS_A) {  // dgrad: w[r, s, j, co]
+          at = ((int64_t)(t_r[p] * (int)d.S + t_s[p]) * d.Cin + m) * d.Cout + t_c[p];
+        } else {
+          in = in && where(d, p, t_r[p], t_s[p], t_c[p], at);
+        }
+        // (what lies outside reads the first numbers of the tensor: no branch around the request)
+        const float* src = (IS_A ? g.a : g.b) + (in ? at : 0);
+        const sp_f4 v0 = *(const sp_f4_any*)src, v1 = *(const sp_f4_any*)(src + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[e] = in ? v0[e] : 0.f;
+          x[4 + e] = in ? v1[e] : 0.f;
+        }
+      } else {  // [K, Cout] row-major: w for the forward product, dy for wgrad
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const bool in = ok[p] && k + e < k_end;
+          const float v = g.b[in ? (k + e) * d.Cout + m : 0];
+          x[e] = in ? v : 0.f;
+        }
+      }
+      if constexpr (FAST && MODE == CONV_WGRAD && IS_A) {
+        t_c[p] += SPLIT_BK;
+        while (t_c[p] >= d.Wo) {
+          t_c[p] -= (int)d.Wo;
+          if (++t_s[p] >= d.Ho) { t_s[p] = 0; ++t_r[p]; }
+        }
+      } else if constexpr (WHOLE) {
+        const int ck = MODE == CONV_FWD ? (int)d.Cin : (int)d.Cout;
+        t_c[p] += SPLIT_BK;
+        while (t_c[p] >= ck) {
+          t_c[p] -= ck;
+          if (++t_s[p] == (int)d.S) { t_s[p] = 0; ++t_r[p]; }
+        }
+      }
+    }
+  }
+  template <int SET>
+  __device__ __forceinline__ void store(sp_u4* tile) {
+    if (mine())
+#pragma unroll
+      for (int p = 0; p < PIECES; ++p) split_store<ROWS>(tile, row[p], c[p], r[SET][p]);
+  }
+};
+
+template <int MODE, bool FAST, int BM, int BN, int NWM, int NWN>
+__global__ __launch_bounds__(NWM * NWN * 64) void conv_split_kernel(const ConvArgs g) {
+  constexpr int NT = NWM * NWN * 64, WM = BM / NWM, WN = BN / NWN, TM = WM / 16, TN = WN / 16;
+  constexpr int TILE = (BM + BN) * 12;
+  extern __shared__ __align__(16) sp_u4 conv_lds[];
+  const int tm_i = blockIdx.x % g.tiles_m, tn_i = blockIdx.x / g.tiles_m;
+  const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
+  const int64_t k_begin = (int64_t)blockIdx.z * g.k_per_split;
+  const int64_t k_end = min(g.K, k_begin + g.k_per_split);
+  float* out = g.out + (g.splits > 1 ? (int64_t)blockIdx.z * g.M * g.Ng : 0);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / NWN * WM, wn = wave % NWN * WN;
+  ConvRows<MODE, FAST, BM, NT, true> la;
+  ConvRows<MODE, FAST, BN, NT, false> lb;
+  la.init(g, m0, k_begin);
+  lb.init(g, n0, k_begin);
+  SplitAcc<TM, TN, 2> acc;
+  acc.zero();
+  const int nk = (int)((k_end - k_begin + SPLIT_BK - 1) / SPLIT_BK);
+#define CONV_LOAD(SET, T)                                                  \
+  do {                                                                     \
+    const int64_t k0 = k_begin + (int64_t)(T) * SPLIT_BK;                  \
+    la.template load<SET>(g, m0, k0, k_end);                               \
+    lb.template load<SET>(g, n0, k0, k_end);                               \
+  } while (0)
+#define CONV_STORE(SET)                                                    \
+  do {                                                                     \
+    la.template store<SET>(conv_lds + SET * TILE);                         \
+    lb.template store<SET>(conv_lds + SET * TILE + BM * 12);               \
+  } while (0)
+#define CONV_MULTIPLY(SET) acc.template multiply<BM, BN, SET>(conv_lds + SET * TILE, conv_lds + SET * TILE + BM * 12, wm, wn, lane)
+  CONV_LOAD(0, 0);
+  CONV_LOAD(1, 1);  // (past the end: zeros)
+  CONV_STORE(0);
+  __syncthreads();
+  int kt = 0;
+  for (; kt + 1 < nk; kt += 2) {
+    CONV_LOAD(0, kt + 2);
+    CONV_MULTIPLY(0);
+    CONV_STORE(1);
+    __syncthreads();
+    CONV_LOAD(1, kt + 3);
+    CONV_MULTIPLY(1);
+    CONV_STORE(0);
+    __syncthreads();
+  }
+  if (kt < nk) CONV_MULTIPLY(0);
+#undef CONV_MULTIPLY
+#undef CONV_STORE
+#undef CONV_LOAD
+  const bool relu = MODE == CONV_FWD && g.d.act == NBK_ACT_RELU;
+  uint32_t again = 0;  // sums that are not finite: computed again in float32
+  static_assert(TM * TN * 4 <= 32, "a bit for each of a lane's results");
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int64_t col = n0 + wn + j * 16 + (lane & 15);
+      if (col >= g.Ng) continue;
+      const float bias = g.bias ? g.bias[col] : 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t row = m0 + wm + i * 16 + (lane >> 4) * 4 + r;
+        if (row >= g.M) continue;
+        const float sum = acc.sum(i, j, r);
+        if (!(fabsf(sum) < INFINITY)) again |= 1u << ((i * TN + j) * 4 + r);
+        out[row * g.Ng + col] = relu ? fmaxf(sum + bias, 0.f) : sum + bias;
+      }
+    }
+  while (again) {
+    const int at = __ffs(again) - 1;
+    again &= again - 1;
+    const int64_t col = n0 + wn + (at >> 2) % TN * 16 + (lane & 15);
+    const int64_t row = m0 + wm + (at >> 2) / TN * 16 + (lane >> 4) * 4 + (at & 3);
+    float sum = 0.f;
+    for (int64_t k = k_begin; k < k_end; ++k)
+      sum = fmaf(conv_load_a<MODE>(g, row, k, k_end), conv_load_b<MODE>(g, k, col, k_end), sum);
+    sum += g.bias ? g.bias[col] : 0.f;
+    out[row * g.Ng + col] = relu ? fmaxf(sum, 0.f) : sum;
+  }
 }
 
 // out[i] = sum over z of partial[z][i]; eight slices are in flight per lane and the order
@@ -402,11 +520,47 @@ static int conv_check(const nbk_conv_desc* d) {
 
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-template <int MODE>
-static int conv_launch(ConvArgs& a, bool fast, hipStream_t st) {
+template <int MODE, bool FAST, int BM, int BN, int NWM, int NWN>
+static int conv_launch_tile(ConvArgs& a, hipStream_t st) {
+  a.tiles_m = (int)((a.M + BM - 1) / BM);
+  a.tiles_n = (int)((a.Ng + BN - 1) / BN);
+  const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n;
+  NBK_REQUIRE(blocks <= 0x7fffffffLL, "conv2d: launch too large");
+  const size_t lds = 2 * (size_t)(BM + BN) * 12 * 16;
+  auto kern = conv_split_kernel<MODE, FAST, BM, BN, NWM, NWN>;
+  static bool attr_set = false; /* idempotent, so a race only repeats the call */
+  if (!attr_set) {
+    NBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, 1, (unsigned)a.splits), dim3(NWM * NWN * 64), lds, st, a);
+  return nbk_check_launch("conv_split_kernel");
+}
+// Forward and dgrad.  128 x 128 tiles run one to a CU and two of 64 x 64 do; a round of the former does the work of
+// two of the latter in 1.7 of one's time.  us, 128 x 128 / 64 x 64: 64 x 32 x 32, 64 -> 128 channels, 79 / 108; 64 x 16
+// x 16, 128 -> 256, 67 / 100, its input gradient (128 columns: 128 tiles) 108 / 80; 90 x 20 x 20, 56 -> 120 72 / 71.
+// Up to 32 channels of results, tiles of 128 x 32 from one per CU on: 50 x 28 x 28, 1 -> 24 9.1 against 11.0,
+// input gradient of 24 -> 40 23 against 29; below that 1 x 32 x 32, 16 -> 32 12.0 against 10.3.
+// (128 x 64 tiles: 5 % less than 64 x 64 at best.)
+template <int MODE, bool FAST>
+static int conv_launch(ConvArgs& a, hipStream_t st) {
+  a.set_divisors();
+  const int64_t cus = nbk_num_cus(), m128 = (a.M + 127) / 128;
+  const int64_t t64 = ((a.M + 63) / 64) * ((a.Ng + 63) / 64);
+  if (a.Ng <= 32 && m128 >= cus) return conv_launch_tile<MODE, FAST, 128, 32, 4, 1>(a, st);
+  const int64_t rounds_128 = (m128 * ((a.Ng + 127) / 128) + cus - 1) / cus, rounds_64 = (t64 + 2 * cus - 1) / (2 * cus);
+  if (rounds_128 * 17 <= rounds_64 * 10) return conv_launch_tile<MODE, FAST, 128, 128, 2, 4>(a, st);
+  return conv_launch_tile<MODE, FAST, 64, 64, 2, 2>(a, st);
+}
+
+// The filter gradient of channel counts that are multiples of 8 stays on the float32 instruction: its pieces
+// of 8 k are 8 pixels, whose gather costs more than the instruction saves (64 x 32 x 32, 64 -> 128 channels 139
+// us against 112).  Others gather number by number there, too (3 -> 64 44 against 51, 1 -> 24 of 50 x 28 x 28 34 against 39).
+static int conv_launch_wgrad(ConvArgs& a, bool fast, hipStream_t st) {
+  a.set_divisors();
+  if (!fast) return conv_launch_tile<CONV_WGRAD, true, 64, 64, 2, 2>(a, st);
   // the narrow workgroup tile when the last 128-wide column tile would be at most half full,
   // or when the wide tiling gives fewer workgroups than the GPU has CUs
-  a.set_divisors();
   const int64_t wide = ((a.M + 127) / 128) * ((a.Ng + 127) / 128) * a.splits;
   const bool narrow = (a.Ng - 1) % 128 < 64 || wide < nbk_num_cus();
   const int bn = narrow ? 64 : 128;
@@ -415,11 +569,9 @@ static int conv_launch(ConvArgs& a, bool fast, hipStream_t st) {
   const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n;
   NBK_REQUIRE(blocks <= 0x7fffffffLL, "conv2d: launch too large");
   const dim3 grid((unsigned)blocks, 1, (unsigned)a.splits);
-  if (fast && narrow) hipLaunchKernelGGL((conv_kernel<MODE, true, 1>), grid, dim3(256), 0, st, a);
-  else if (fast) hipLaunchKernelGGL((conv_kernel<MODE, true, 2>), grid, dim3(256), 0, st, a);
-  else if (narrow) hipLaunchKernelGGL((conv_kernel<MODE, false, 1>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((conv_kernel<MODE, false, 2>), grid, dim3(256), 0, st, a);
-  return nbk_check_launch("conv_kernel");
+  if (narrow) hipLaunchKernelGGL((conv_wgrad_kernel<1>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((conv_wgrad_kernel<2>), grid, dim3(256), 0, st, a);
+  return nbk_check_launch("conv_wgrad_kernel");
 }
 
 extern "C" int nbk_conv2d_fwd(const nbk_conv_desc* d, const void* x, const void* w,
@@ -432,8 +584,8 @@ extern "C" int nbk_conv2d_fwd(const nbk_conv_desc* d, const void* x, const void*
   a.a = (const float*)x; a.b = (const float*)w; a.bias = (const float*)bias; a.out = (float*)y;
   a.M = d->N * d->Ho * d->Wo; a.Ng = d->Cout; a.K = d->R * d->S * d->Cin;
   a.splits = 1; a.k_per_split = (a.K + 15) / 16 * 16;
-  const bool fast = d->Cin % 16 == 0 && d->Cout % 8 == 0 && aligned16(x) && aligned16(w);
-  return conv_launch<CONV_FWD>(a, fast, (hipStream_t)stream);
+  return d->Cin % 8 == 0 ? conv_launch<CONV_FWD, true>(a, (hipStream_t)stream)
+                         : conv_launch<CONV_FWD, false>(a, (hipStream_t)stream);
 }
 
 extern "C" int nbk_conv2d_dgrad(const nbk_conv_desc* d, const void* dy, const void* w, void* dx,
@@ -447,8 +599,8 @@ extern "C" int nbk_conv2d_dgrad(const nbk_conv_desc* d, const void* dy, const vo
   a.a = (const float*)dy; a.b = (const float*)w; a.bias = nullptr; a.out = (float*)dx;
   a.M = d->N * d->H * d->W; a.Ng = d->Cin; a.K = d->R * d->S * d->Cout;
   a.splits = 1; a.k_per_split = (a.K + 15) / 16 * 16;
-  const bool fast = d->Cout % 16 == 0 && aligned16(dy) && aligned16(w);
-  return conv_launch<CONV_DGRAD>(a, fast, (hipStream_t)stream);
+  return d->Cout % 8 == 0 ? conv_launch<CONV_DGRAD, true>(a, (hipStream_t)stream)
+                          : conv_launch<CONV_DGRAD, false>(a, (hipStream_t)stream);
 }
 
 // K split of the filter-gradient product: as many workgroups as the GPU holds at once (two per
@@ -499,7 +651,7 @@ extern "C" int nbk_conv2d_wgrad(const nbk_conv_desc* d, const void* x, const voi
   a.k_per_split = kps;
   if (splits > 1) a.out = (float*)workspace;
   const bool fast = d->Cin % 8 == 0 && d->Cout % 8 == 0 && aligned16(x) && aligned16(dy);
-  rc = conv_launch<CONV_WGRAD>(a, fast, (hipStream_t)stream);
+  rc = conv_launch_wgrad(a, fast, (hipStream_t)stream);
   if (rc || splits == 1) return rc;
   const int64_t n = a.M * a.Ng;
   int64_t blocks = (n + 255) / 256;
