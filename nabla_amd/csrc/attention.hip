@@ -10,7 +10,7 @@
 // of 128 nothing else exists (RAG = false).  For any other S (RAG = true) the rows past the end
 // are read from row S - 1 (an address inside the tensor, finite values), walked rows past the end
 // get probability zero in the tile that holds them, owned ones are not stored, and a wave
-// without an owned row inside skips the arithmetic.  B1 H8 S1800 hd128, causal: 44 us; as batched
+// without an owned row inside skips the arithmetic.  B1 H8 S1800 hd128, causal: 33 us; as batched
 // products around a softmax program (which wrote the scores three times) it took 260 us, and a
 // training step of a B6 S333 H8 hd64 block 756 us where it takes 566 with these kernels.
 //
@@ -222,7 +222,7 @@ __device__ __forceinline__ at_bf16x8 at_tr_pair(const unsigned char* lo, const u
 
 
 // ------------------------------------------------------------------------------ forward
-// Grid: (B * H, S / 128).  Wave w owns queries q0 + 32w .. + 31 (one per lane pair).
+// Grid: (B * H, S / (32 QW)).  Wave w owns queries q0 + 32w .. + 31 (one per lane pair).
 //
 // The softmax runs in base 2 on t = score * scale * log2(e).  The running maximum m of a
 // row is only raised when some row of the wave has outgrown it by more than AT_SLACK (a
@@ -232,21 +232,26 @@ constexpr float AT_SLACK = 8.0f;
 constexpr float AT_LOG2E = 1.4426950408889634f;
 constexpr float AT_LN2 = 0.6931471805599453f;
 
-template <int HD, bool RAG>
-__global__ __launch_bounds__(256, HD == 64 ? (RAG ? 3 : 4) : 2) void attn_fwd_kernel(const AttnArgs g) {
+// PARTS: groups of QW waves that own the same 32 QW queries and take every PARTS-th key tile each, with
+// tile buffers, maxima, sums and accumulators of their own, which meet in LDS at the end.  A wave's tile is
+// a chain of latencies, and a launch with few workgroups waits for the one with the most tiles: B1 H8
+// S1800 hd128, causal (120 workgroups of 128 queries, up to 29 tiles) 45 us in one part.
+template <int HD, bool RAG, int PARTS, int QW>
+__global__ __launch_bounds__(64 * QW * PARTS, PARTS > 1 ? 1 : HD == 64 ? (RAG ? 3 : 4) : 2) void attn_fwd_kernel(const AttnArgs g) {
   constexpr int KSTEPS = HD / 16, DT = HD / 32, NCH = HD / 8;
   constexpr int TILE = 64 * HD * 2, STAGE = 2 * TILE;
   extern __shared__ __align__(16) unsigned char at_lds[];
-  auto k_tile = [&](int buf) { return (at_u32x4*)(at_lds + buf * STAGE); };
-  auto v_tile = [&](int buf) { return (at_u32x4*)(at_lds + buf * STAGE + TILE); };
+  const int part = PARTS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * QW)) : 0;
+  auto k_tile = [&](int buf) { return (at_u32x4*)(at_lds + (part * 2 + buf) * STAGE); };
+  auto v_tile = [&](int buf) { return (at_u32x4*)(at_lds + (part * 2 + buf) * STAGE + TILE); };
 
   // Grid (B * H, tiles): workgroups are handed out along x first, so every (batch, head) runs
   // its longest causal rows before any runs a shorter one, and the tail of the launch consists
   // of the shortest workgroups.
   const int bh = blockIdx.x, b = bh / g.H, hh = bh % g.H;
   const int qt = (int)gridDim.y - 1 - (int)blockIdx.y;
-  const int q0 = qt * 128;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 31, h = lane >> 5;
+  const int q0 = qt * (32 * QW);
+  const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & (QW - 1), li = lane & 31, h = lane >> 5;
   const uint16_t* Q = g.q.p + (int64_t)b * g.q.sb + (int64_t)hh * g.q.sh;
   const uint16_t* K = g.k.p + (int64_t)b * g.k.sb + (int64_t)hh * g.k.sh;
   const uint16_t* V = g.v.p + (int64_t)b * g.v.sb + (int64_t)hh * g.v.sh;
@@ -277,11 +282,11 @@ __global__ __launch_bounds__(256, HD == 64 ? (RAG ? 3 : 4) : 2) void attn_fwd_ke
   float l_r = 0.f;
 
   const int all_tiles = RAG ? (g.S + 63) / 64 : g.S / 64;
-  const int n_tiles = !g.causal ? all_tiles : RAG ? min((q0 + 128) / 64, all_tiles) : (q0 + 128) / 64;
+  const int n_tiles = !g.causal ? all_tiles : RAG ? min((q0 + 32 * QW) / 64, all_tiles) : (q0 + 32 * QW) / 64;
   // K and V tiles go from memory into LDS without passing through registers: a wave instruction
   // deposits 64 x 16 bytes in a row (four rows of a 128-wide tile, eight of a 64-wide one), so
   // the swizzle is applied to the address each lane fetches from.
-  constexpr int PER_WAVE = 64 * NCH / 64 / 4;  // instructions per wave and tile
+  constexpr int PER_WAVE = 64 * NCH / 64 / QW;  // instructions per wave and tile
   int src_off_k[PER_WAVE], src_off_v[PER_WAVE];  // element offsets of this lane's chunks in a tile
 #pragma unroll
   for (int j = 0; j < PER_WAVE; ++j) {
@@ -337,12 +342,13 @@ __global__ __launch_bounds__(256, HD == 64 ? (RAG ? 3 : 4) : 2) void attn_fwd_ke
     return at_tr_pair(base + tr_lo + ((tr_x_lo ^ (dd << 2)) << 4), base + tr_hi + ((tr_x_hi ^ (dd << 2)) << 4));
   };
   const int seen = g.causal ? (RAG ? min(my_q, last) : my_q) : last;  // the last key this lane's query sees
-  request(0, 0);
+  if (PARTS == 1 || part < n_tiles) request(part, 0);
   tile_barrier();
-  for (int kt = 0; kt < n_tiles; ++kt) {
-    const int cur = kt & 1;
-    const bool more = kt + 1 < n_tiles;
-    if (more) request(kt + 1, cur ^ 1);
+  // (every part walks as many rounds: the barriers are the workgroup's)
+  for (int round = 0; round * PARTS < n_tiles; ++round) {
+    const int cur = round & 1, kt = round * PARTS + part;
+    const bool more = kt + PARTS < n_tiles;
+    if (more) request(kt + PARTS, cur ^ 1);
     const at_u32x4* Ks = k_tile(cur);
     const at_u32x4* Vs = v_tile(cur);
     const int k0 = kt * 64;
@@ -408,10 +414,41 @@ __global__ __launch_bounds__(256, HD == 64 ? (RAG ? 3 : 4) : 2) void attn_fwd_ke
     };
     // keys of this tile against the wave's queries: all visible, some, or none
     const bool whole = !RAG || k0 + 63 <= last;
-    if (RAG && wq0 > last) {}
+    if ((RAG && wq0 > last) || (PARTS > 1 && kt >= n_tiles)) {}
     else if (whole && (!g.causal || k0 + 63 <= wq0)) tile(std::false_type{});
     else if (!g.causal || k0 <= wq0 + 31) tile(std::true_type{});
     tile_barrier();
+  }
+  if constexpr (PARTS > 1) {
+    // the other parts' rows through the tile buffers, which are free behind the last barrier
+    constexpr int NR = DT * 16 + 3;
+    float* rows = (float*)at_lds + wave * 64 + lane;
+    if (part > 0) {
+      float* mine = rows + (part - 1) * NR * (64 * QW);
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mine[(d * 16 + r) * (64 * QW)] = o_acc[d][r];
+      mine[DT * 16 * (64 * QW)] = m_i;
+      mine[(DT * 16 + 1) * (64 * QW)] = l_i;
+      mine[(DT * 16 + 2) * (64 * QW)] = l_r;
+    }
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll
+    for (int q = 0; q < PARTS - 1; ++q) {
+      const float* other = rows + q * NR * (64 * QW);
+      const float m_o = other[DT * 16 * (64 * QW)], m_new = fmaxf(m_i, m_o);
+      // (a part without a key that this query sees still has its first maximum: its factor is zero)
+      const float mine = __builtin_amdgcn_exp2f(m_i - m_new), theirs = __builtin_amdgcn_exp2f(m_o - m_new);
+      m_i = m_new;
+      l_i = l_i * mine + other[(DT * 16 + 1) * (64 * QW)] * theirs;
+      l_r = l_r * mine + other[(DT * 16 + 2) * (64 * QW)] * theirs;
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o_acc[d][r] = o_acc[d][r] * mine + other[(d * 16 + r) * (64 * QW)] * theirs;
+    }
   }
   l_i += at_xhalf(l_i);
   l_r += at_xhalf(l_r);
@@ -1048,18 +1085,29 @@ extern "C" int nbk_attention_fwd(const nbk_attn_desc* d, const nbk_attn_tensor* 
     return rc;
   NBK_REQUIRE(lse != nullptr, "attention: null lse");
   a.lse = (float*)lse;
-  const dim3 grid((unsigned)(d->B * d->H), (unsigned)((d->S + 127) / 128));
   hipStream_t st = (hipStream_t)stream;
-  // two stages of a row-major K and V tile each
-  const size_t lds = 2 * 2 * 64 * (size_t)d->hd * 2;
   const bool rag = d->S % 128 != 0;
-  auto launch = [&](auto kern) -> int {
+  auto launch = [&](auto kern, int parts, int waves) -> int {
+    const dim3 grid((unsigned)(d->B * d->H), (unsigned)((d->S + 32 * waves - 1) / (32 * waves)));
+    // two stages of a row-major K and V tile each
+    const size_t lds = (size_t)parts * 2 * 2 * 64 * (size_t)d->hd * 2;
     const int lrc = attn_set_lds(kern, lds);
-    if (lrc == NBK_OK) hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, a);
+    if (lrc == NBK_OK) hipLaunchKernelGGL(kern, grid, dim3(64 * waves * parts), lds, st, a);
     return lrc;
   };
-  rc = d->hd == 64 ? (rag ? launch(attn_fwd_kernel<64, true>) : launch(attn_fwd_kernel<64, false>))
-                   : (rag ? launch(attn_fwd_kernel<128, true>) : launch(attn_fwd_kernel<128, false>));
+#define ATTN_FWD(PARTS, QW)                                                                                          \
+  (d->hd == 64 ? (rag ? launch(attn_fwd_kernel<64, true, PARTS, QW>, PARTS, QW) : launch(attn_fwd_kernel<64, false, PARTS, QW>, PARTS, QW)) \
+               : (rag ? launch(attn_fwd_kernel<128, true, PARTS, QW>, PARTS, QW) : launch(attn_fwd_kernel<128, false, PARTS, QW>, PARTS, QW)))
+  // 64 queries in two parts while that gives no CU a second workgroup (with causal 64-wide heads, whose workgroups
+  // end at different times, a third), then 128 in two parts while a CU holds no more than two of those and a part
+  // has three tiles, else 128 in one.  us, one part of 128 / two of 128 / two of 64: B1 H8 S1800 hd128 causal 45 /
+  // 38 / 33, B1 H16 S1024 hd64 causal 20 / 17 / 14.5, B2 21 / 18 / 17, B1 H4 S256 8.5 / 8.7 / 7.2, B3 H8 S700 hd64 16.1
+  // / 14.7 / 16.8, B2 H16 S2048 hd128 causal 58 / 56 / 82, B8 H16 S1024 hd64 causal 38 / 47 / 48.
+  const int64_t heads = d->B * d->H, cus = nbk_num_cus(), g64 = heads * ((d->S + 63) / 64), g128 = heads * ((d->S + 127) / 128);
+  if (g64 <= cus * (d->hd == 64 && d->causal ? 2 : 1)) rc = ATTN_FWD(2, 2);
+  else if (g128 <= 2 * cus && d->S > 320) rc = ATTN_FWD(2, 4);
+  else rc = ATTN_FWD(1, 4);
+#undef ATTN_FWD
   if (rc) return rc;
   return nbk_check_launch("attn_fwd_kernel");
 }
