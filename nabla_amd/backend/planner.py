@@ -632,6 +632,8 @@ class Planner:
             return
         if step.kind == "copy" and _numel(step.attrs["src"].shape) == 0:
             return
+        if not self._waiting_bufs.isdisjoint(step.reads):
+            self._flush_reduces(waiting_only=True)
         idx = len(self.steps)
         for r in step.reads:
             b = self.bufs[r]
@@ -1281,7 +1283,12 @@ class Planner:
         self.skip_nodes: set[int] = set()  # reductions folded into an earlier one
         self.n_split = 0                   # fusion groups cut in two at lowering time
         self._materialized: dict = {}
-        self._deferred_reduces: list[list[Step]] = [[], []]  # first-stage / second-stage tasks
+        # reductions that wait to go out together, as first-stage and second-stage tasks: those whose
+        # results only leave the plan, until its end; the others until a step reads one of them
+        self._deferred_reduces: list[list[Step]] = [[], []]
+        self._waiting_reduces: list[list[Step]] = [[], []]
+        self._waiting_bufs: set[int] = set()
+        self._waiting_bytes = 0
         self.users: dict[int, list[ir.Node]] = {}
         for n in nodes:
             for i in n.inputs:
@@ -1552,28 +1559,58 @@ class Planner:
                 return False
         return True
 
+    # What a waiting reduction reads stays in memory until it goes out.  One launch less is worth
+    # 4 us, the time a pass over 16 to 20 MB takes: reductions over more gain nothing that counts
+    # by waiting, and all that wait together hold at most this much.
+    MAX_WAITING_BYTES = 128 << 20
+
     def _emit_reduce(self, step: Step, stage: int, terminal: bool) -> None:
-        """A reduction whose result only leaves the plan waits for the end of the plan, where all
-        such reductions go out together (one launch per stage instead of one each)."""
+        """A reduction waits for the end of the plan, where its result only leaves it, or for the
+        first step that reads its result (in a step with an optimizer that is one launch behind the
+        whole backward pass): all that wait go out together, one launch per stage instead of one each."""
+        if not self._waiting_bufs.isdisjoint(step.reads) and stage == 0:
+            self._flush_reduces(waiting_only=True)
         if terminal:
             self._deferred_reduces[stage].append(step)
-        else:
-            self._emit(step)
+            return
+        if self._waiting_bufs.isdisjoint(step.reads):  # (a second stage stays with its first)
+            held = self.bufs[step.reads[0]].nbytes
+            if self._waiting_bytes + held > self.MAX_WAITING_BYTES:
+                self._flush_reduces(waiting_only=True)
+            self._waiting_bytes += held
+        self._waiting_reduces[stage].append(step)
+        self._waiting_bufs.update(step.writes)
 
-    def _fold_column_sums(self) -> None:
+    def _reads_waiting(self, nodes: list[ir.Node]) -> bool:
+        """True if one of the nodes reads, directly or through views, the result of a reduction
+        that waits."""
+        todo, seen = [i for n in nodes for i in n.inputs], set()
+        while todo and self._waiting_bufs:
+            v = todo.pop()
+            if v.id in seen:
+                continue
+            seen.add(v.id)
+            at = self.loc.get(v.id)
+            if at is None:
+                todo.extend(v.node.inputs)
+            elif isinstance(at, ViewRef) and at.buf in self._waiting_bufs:
+                return True
+        return False
+
+    def _fold_column_sums(self, tasks: list[list[Step]]) -> None:
         """Deferred column sums whose matrix is the right operand of a product that was emitted
         with room for them (``colsum_key`` on both) become a result of that product's launch:
         the matrix is read once.  A product split along K leaves one row of partial sums per
         slice, which the second stage adds up as it would have the first stage's."""
         hosts = {}  # key -> (step, member of a joined launch)
         for idx, st in enumerate(self.steps):
-            if st.kind != "gemm":
+            if st.kind != "gemm" or (st.attrs.get("colsum") is not None and "colsum_keys" not in st.attrs):
                 continue
             keys = st.attrs.get("colsum_keys") or [st.attrs.get("colsum_key")]
             for member, key in enumerate(keys):
                 if key is not None and key not in hosts:
                     hosts[key] = (idx, member)
-        first, second = self._deferred_reduces
+        first, second = tasks
         for task in list(first):
             key = task.attrs.get("colsum_key")
             idx, member = hosts.pop(key, (None, 0)) if key is not None else (None, 0)
@@ -1605,17 +1642,21 @@ class Planner:
             b = self.bufs[target.buf]
             b.first, b.last = min(b.first, idx), max(b.last, idx)
 
-    def _flush_reduces(self) -> None:
+    def _flush_reduces(self, waiting_only: bool = False) -> None:
+        groups, self._waiting_reduces = self._waiting_reduces, [[], []]
+        self._waiting_bufs, self._waiting_bytes = set(), 0
+        if not waiting_only:
+            groups = [w + d for w, d in zip(groups, self._deferred_reduces)]
+            self._deferred_reduces = [[], []]
         if self.fold_column_sums:
-            self._fold_column_sums()
-        for tasks in self._deferred_reduces:
+            self._fold_column_sums(groups)
+        for tasks in groups:
             if len(tasks) == 1:
                 self._emit(tasks[0])
             elif tasks:
                 self._emit(Step("reduce_batch", [r for t in tasks for r in t.reads],
                                 [w for t in tasks for w in t.writes],
                                 dict(tasks=[t.attrs for t in tasks])))
-        self._deferred_reduces = [[], []]
 
     def _lower_reduce_mid(self, n: ir.Node) -> None:
         if n.pos in self.skip_nodes:
@@ -1687,7 +1728,7 @@ class Planner:
         # the column sums of a matrix that a product also reads as its row-contiguous right
         # operand (a bias gradient beside the weight gradient) can ride on that product
         fold = {}
-        if (terminal and self.fold_column_sums and kind == "sum" and outer == 1 and
+        if (self.fold_column_sums and kind == "sum" and outer == 1 and
                 x.dtype is DType.bfloat16 and out.dtype is DType.bfloat16):
             fold = dict(colsum_key=(src.buf, src.offset, red, inner))
         if split > 1:
@@ -2050,7 +2091,7 @@ class Planner:
             h = st.attrs
             n = len(members)
             hb = h["b"]
-            same = (h["a"] == ra and h["M"] == M and h["N"] == N and h["k_all"] == k_all and
+            same = (h.get("colsum") is None and h["a"] == ra and h["M"] == M and h["N"] == N and h["k_all"] == k_all and
                     all(h[f] == common[f] for f in ("a_rs", "a_cs", "b_rs", "b_cs", "ldc", "alpha")) and
                     hb.buf == rb.buf and hb.dtype is rb.dtype and
                     (members[0]["key"] is not None) == (key is not None))
@@ -2062,8 +2103,8 @@ class Planner:
             if spacing <= 0 or spacing % 8 or any(
                     order[j + 1]["off"] - order[j]["off"] != spacing for j in range(n)):
                 continue
-            # nothing emitted since may write what this member reads
-            if any(w in (ra.buf, rb.buf) for later in self.steps[idx + 1:] for w in later.writes):
+            # nothing emitted since, or still waiting, may write what this member reads
+            if not self._waiting_bufs.isdisjoint((ra.buf, rb.buf)) or any(w in (ra.buf, rb.buf) for later in self.steps[idx + 1:] for w in later.writes):
                 return False
             # the launch has the tiles of all its members: fewer slices of K give it three
             # workgroups for two CUs, and fewer partial products go through memory (three
@@ -2199,6 +2240,8 @@ class Planner:
         """One row program for the group; a group that exceeds a limit of the row-program
         format (operands, registers, instructions) is cut in two in program order, the values
         that cross the cut go through memory, and each half is lowered on its own."""
+        if self._reads_waiting(g.nodes):
+            self._flush_reduces(waiting_only=True)  # (not inside the trial: it may be taken back)
         snap = (len(self.bufs), dict(self.loc), dict(self._out_pending), dict(self._out_done),
                 len(self.steps), dict(self._materialized))
         try:
