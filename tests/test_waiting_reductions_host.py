@@ -61,8 +61,8 @@ def test_bias_gradients_that_an_update_reads(emulator, monkeypatch, rows, dtype)
         np.testing.assert_allclose(a, c, rtol=tol, atol=tol)
 
 
-def test_a_fused_group_that_is_cut_in_two(emulator, monkeypatch):
-    """More operands than one row program holds, among them results of waiting reductions."""
+def test_fused_groups_that_read_waiting_results(emulator, monkeypatch):
+    """A chain over more results than one row program takes."""
     rng = np.random.default_rng(0)
     mats = [rng.standard_normal((7, 5, 48)) for _ in range(30)]
 
