@@ -10,6 +10,9 @@ from __future__ import annotations
 
 from typing import Any
 
+from ..ops.binary import add
+from ..ops.creation import zeros_like
+from ..ops.reduction import reduce_sum
 from .pytree import tree_leaves
 from .tensor import BatchedTensor, Tensor, TensorImpl
 from .tracing import OpNode, Trace
@@ -17,8 +20,6 @@ from .tracing import OpNode, Trace
 
 def _reduce_to_shape(cot: Tensor, target_shape: tuple[int, ...]) -> Tensor:
     """Undo broadcasting: sum the cotangent down to the primal's shape."""
-    from ..ops.reduction import reduce_sum
-
     cot_shape = tuple(cot.shape)
     if len(cot_shape) > len(target_shape):
         diff = len(cot_shape) - len(target_shape)
@@ -31,8 +32,6 @@ def _reduce_to_shape(cot: Tensor, target_shape: tuple[int, ...]) -> Tensor:
 
 
 def _accumulate_cotangent(cot_map: dict, target: TensorImpl, cot: Tensor) -> None:
-    from ..ops.binary import add
-
     existing = cot_map.get(target)
     cot_map[target] = add(existing, cot) if existing is not None else cot
 
@@ -79,7 +78,6 @@ class BackwardEngine:
             elif o in self.cotangent_map:
                 cots.append(self.cotangent_map[o])
             else:
-                from ..ops.creation import zeros_like
                 cots.append(zeros_like(Tensor(impl=o)))
         # ops emitted by a VJP rule are part of the differentiable graph only
         # when a higher-order derivative is asked for
@@ -107,7 +105,6 @@ class BackwardEngine:
             _accumulate_cotangent(self.cotangent_map, arg, c)
 
     def _finalize(self) -> dict:
-        from ..ops.creation import zeros_like
         grads: dict[Tensor, Tensor] = {}
         for inp in tree_leaves(self.trace.inputs):
             if not isinstance(inp, Tensor):
@@ -133,7 +130,6 @@ def backward(output: Tensor, gradient: Tensor | None = None, *, retain_graph: bo
              create_graph: bool = False) -> None:
     """PyTorch-style: accumulate into ``.grad`` of every ``requires_grad`` leaf and
     realize all gradients as one batch (backward.py:380-460)."""
-    from ..ops.binary import add
     from ..ops.creation import ones_like
     from .tensor import realize_all
 

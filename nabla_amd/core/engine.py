@@ -47,6 +47,9 @@ def clear_plan_cache() -> None:
 
 def _freeze(x: Any):
     """Hashable form of an op's kwargs."""
+    t = type(x)
+    if t is int or t is str or t is bool or t is float or x is None:
+        return x
     if isinstance(x, dict):
         return tuple(sorted((k, _freeze(v)) for k, v in x.items()))
     if isinstance(x, (list, tuple)):

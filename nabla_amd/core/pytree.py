@@ -17,25 +17,35 @@ def register_pytree_node(cls: type, flatten_fn: Callable, unflatten_fn: Callable
 
 
 class PyTreeDef:
-    __slots__ = ("kind", "aux", "children", "num_leaves")
+    __slots__ = ("kind", "aux", "children", "num_leaves", "_flat_key", "_hash")
 
     def __init__(self, kind: Any, aux: Any, children: tuple, num_leaves: int):
         self.kind = kind
         self.aux = aux
         self.children = children
         self.num_leaves = num_leaves
+        self._flat_key = self._hash = None
 
     def _key(self):
-        return (self.kind, self.aux, self.children)
+        """Nested tuples down to the leaves, made once: compared and hashed without a call of
+        Python code per node (a compiled step hashes its arguments' structure at every call)."""
+        k = self._flat_key
+        if k is None:
+            k = self._flat_key = (self.kind, self.aux, tuple([c._key() for c in self.children]))
+        return k
 
     def __eq__(self, other):
         return isinstance(other, PyTreeDef) and self._key() == other._key()
 
     def __hash__(self):
-        try:
-            return hash(self._key())
-        except TypeError:
-            return hash((self.kind, repr(self.aux), self.children))
+        h = self._hash
+        if h is None:
+            try:
+                h = hash(self._key())
+            except TypeError:  # (an auxiliary value that has no hash)
+                h = hash((self.kind, repr(self.aux), self.children))
+            self._hash = h
+        return h
 
     def __repr__(self):
         if self.kind is _K_LEAF:
@@ -46,73 +56,69 @@ class PyTreeDef:
 _K_LEAF = "leaf"
 _K_NONE = "none"
 _LEAF_DEF = PyTreeDef(_K_LEAF, None, (), 1)
+_NONE_DEF = PyTreeDef(_K_NONE, None, (), 0)
+
+
+_TENSOR: type | None = None  # (core.tensor's class; that module comes later)
 
 
 def is_tensor(x: Any) -> bool:
-    from .tensor import Tensor
+    global _TENSOR
+    if _TENSOR is None:
+        from .tensor import Tensor
+        _TENSOR = Tensor
+    return isinstance(x, _TENSOR)
 
-    return isinstance(x, Tensor)
+
+def _flatten_into(node, leaves: list, is_leaf) -> PyTreeDef:
+    if is_leaf is not None and is_leaf(node):
+        leaves.append(node)
+        return _LEAF_DEF
+    if node is None:
+        return _NONE_DEF
+    t = type(node)
+    if t in _REGISTRY:
+        children, aux = _REGISTRY[t][0](node)
+    elif t is list or t is tuple:
+        children, aux = node, None
+    elif isinstance(node, tuple) and hasattr(node, "_fields"):  # namedtuple
+        children, aux = node, None
+    elif t is dict:
+        aux = tuple(sorted(node, key=repr))
+        children = [node[k] for k in aux]
+    else:
+        leaves.append(node)
+        return _LEAF_DEF
+    n = len(leaves)
+    defs = tuple([_flatten_into(c, leaves, is_leaf) for c in children])
+    return PyTreeDef(t, aux, defs, len(leaves) - n)
 
 
 def tree_flatten(tree: Any, is_leaf: Callable[[Any], bool] | None = None):
     leaves: list[Any] = []
+    return leaves, _flatten_into(tree, leaves, is_leaf)
 
-    def go(node) -> PyTreeDef:
-        if is_leaf is not None and is_leaf(node):
-            leaves.append(node)
-            return _LEAF_DEF
-        if node is None:
-            return PyTreeDef(_K_NONE, None, (), 0)
-        t = type(node)
-        if t in _REGISTRY:
-            children, aux = _REGISTRY[t][0](node)
-            defs = tuple(go(c) for c in children)
-            return PyTreeDef(t, aux, defs, sum(d.num_leaves for d in defs))
-        if t is list or t is tuple:
-            defs = tuple(go(c) for c in node)
-            return PyTreeDef(t, None, defs, sum(d.num_leaves for d in defs))
-        if isinstance(node, tuple) and hasattr(node, "_fields"):  # namedtuple
-            defs = tuple(go(c) for c in node)
-            return PyTreeDef(t, None, defs, sum(d.num_leaves for d in defs))
-        if t is dict:
-            keys = tuple(sorted(node.keys(), key=repr))
-            defs = tuple(go(node[k]) for k in keys)
-            return PyTreeDef(dict, keys, defs, sum(d.num_leaves for d in defs))
-        leaves.append(node)
-        return _LEAF_DEF
 
-    try:
-        treedef = go(tree)
-    finally:
-        # the closure refers to itself: unless that is undone it lives, and `leaves` with it,
-        # until the cycle collector runs (device memory of dropped tensors would wait for that)
-        go = None
-    return leaves, treedef
+def _unflatten_from(d: PyTreeDef, it) -> Any:
+    kind = d.kind
+    if kind is _K_LEAF:
+        return next(it)
+    if kind is _K_NONE:
+        return None
+    kids = [_unflatten_from(c, it) for c in d.children]
+    if kind is list:
+        return kids
+    if kind is tuple:
+        return tuple(kids)
+    if kind is dict:
+        return dict(zip(d.aux, kids))
+    if kind in _REGISTRY:
+        return _REGISTRY[kind][1](d.aux, kids)
+    return kind(*kids)  # namedtuple
 
 
 def tree_unflatten(treedef: PyTreeDef, leaves) -> Any:
-    it = iter(leaves)
-
-    def go(d: PyTreeDef):
-        if d.kind is _K_LEAF:
-            return next(it)
-        if d.kind is _K_NONE:
-            return None
-        kids = [go(c) for c in d.children]
-        if d.kind is list:
-            return kids
-        if d.kind is tuple:
-            return tuple(kids)
-        if d.kind is dict:
-            return dict(zip(d.aux, kids))
-        if d.kind in _REGISTRY:
-            return _REGISTRY[d.kind][1](d.aux, kids)
-        return d.kind(*kids)  # namedtuple
-
-    try:
-        return go(treedef)
-    finally:
-        go = None  # (self-referential closure holding `leaves`, as in tree_flatten)
+    return _unflatten_from(treedef, iter(leaves))
 
 
 def tree_leaves(tree: Any, is_leaf=None) -> list:

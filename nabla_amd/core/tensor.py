@@ -455,12 +455,23 @@ def _ensure_tensor(value: Any, like: Tensor) -> Tensor:
     return Tensor.constant(value, device=like.device)
 
 
+_OPS = None
+
+
+def _ops_package():
+    """``nabla_amd.ops``, which is built on this module."""
+    global _OPS
+    if _OPS is None:
+        from .. import ops
+        _OPS = ops
+    return _OPS
+
+
 # ---- generated methods (api.py:1405-1483) -------------------------------------
 def _bind() -> None:
     def binary(op_name: str, reverse: bool):
         def method(self, other):
-            from .. import ops
-            fn = getattr(ops, op_name)
+            fn = getattr(_ops_package(), op_name)
             other_t = _ensure_tensor(other, self)
             return fn(other_t, self) if reverse else fn(self, other_t)
         return method

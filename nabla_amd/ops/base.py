@@ -20,6 +20,7 @@ from typing import Any
 
 from .. import config
 from ..core.dtype import DType, promote
+from ..core.engine import GRAPH, _freeze
 from ..core.pytree import PyTreeDef, _K_LEAF
 from ..core.tensor import BatchedTensor, Tensor, TensorImpl
 from ..core.tracing import OpNode
@@ -44,7 +45,6 @@ def ensure_tensor(x: Any, like: Tensor | None = None) -> Tensor:
 def _freeze_kwargs(kwargs: dict | None):
     if not kwargs:
         return ()
-    from ..core.engine import _freeze
     return _freeze(kwargs)
 
 
@@ -107,7 +107,6 @@ class Operation(ABC):
             outs.append(Tensor(impl=impl))
         self._setup_output_refs(outs, args, kwargs)
         if config.EAGER_MAX_GRAPH and not config.TRACING:
-            from ..core.engine import GRAPH
             GRAPH.evaluate(*outs)
         return outs
 
@@ -158,8 +157,6 @@ class BinaryOperation(Operation):
         return [tuple(x.shape)], [dtype], [x.device]
 
     def __call__(self, args: OpArgs, kwargs: OpKwargs) -> OpResult:
-        from . import view as view_ops
-
         x, y = args[0], args[1]
         if not isinstance(x, Tensor):
             x = ensure_tensor(x, y if isinstance(y, Tensor) else None)
@@ -224,3 +221,6 @@ class CreationOperation(Operation):
 
     def vjp_rule(self, primals, cotangents, outputs, kwargs):
         return []
+
+
+from . import view as view_ops  # noqa: E402  (itself built on the classes above)

@@ -10,6 +10,7 @@ from __future__ import annotations
 from ..backend import ir
 from ..core.dtype import promote
 from ..core.tensor import Tensor
+from . import view as view_ops
 from .base import BinaryOperation, Operation, ensure_tensor
 
 
@@ -123,8 +124,6 @@ class MatmulOp(Operation):
         return [ir.matmul(ir.cast(a, dt), ir.cast(b, dt))]
 
     def __call__(self, args, kwargs):
-        from . import view as view_ops
-
         x = ensure_tensor(args[0])
         y = ensure_tensor(args[1])
         x1d, y1d = len(x.shape) == 1, len(y.shape) == 1
@@ -152,10 +151,9 @@ class MatmulOp(Operation):
 
     def vjp_rule(self, primals, cotangents, outputs, kwargs):
         # dX = G @ W^T ; dW = X^T @ G  (binary.py:303-314)
-        from .view import swap_axes
         x, y = primals
         g = cotangents[0]
-        return [matmul(g, swap_axes(y, -2, -1)), matmul(swap_axes(x, -2, -1), g)]
+        return [matmul(g, view_ops.swap_axes(y, -2, -1)), matmul(view_ops.swap_axes(x, -2, -1), g)]
 
     def jvp_rule(self, primals, tangents, outputs, kwargs):
         x, y = primals

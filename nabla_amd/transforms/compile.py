@@ -137,12 +137,14 @@ class CompiledFunction:
 
     # ---- keys ---------------------------------------------------------------
     def _tensor_signature(self, t: Tensor, arg_idx: int):
+        if not self.dynamic_dims:
+            return (tuple(t.shape), t.dtype._name_, None)
         shape: list = list(t.shape)
         if arg_idx in self.dynamic_dims:
             for dim_idx, sym in self.dynamic_dims[arg_idx].items():
                 if dim_idx < len(shape):
                     shape[dim_idx] = f"${sym}"
-        return (tuple(shape), str(t.dtype), None)
+        return (tuple(shape), t.dtype._name_, None)
 
     def _build_keys(self, flat: list):
         sigs, statics, concrete = [], [], []
