@@ -1,0 +1,66 @@
+"""Convolutions out of bf16 parts: forward, input and filter gradient at the edges of their tiles (128 x 128,
+64 x 64, 128 x 32) and of a K tile, in pieces of eight channels and number by number, against float64;
+numbers that have no parts."""
+import numpy as np
+import pytest
+import torch
+
+import nabla_amd as nb
+
+pytestmark = pytest.mark.gpu
+
+
+def ours(x, w, g, pad, stride):
+    def loss(a, b):
+        return nb.reduce_sum(nb.conv2d(a, b, stride=(stride, stride), padding=(pad,) * 4) * T(g))
+    T = nb.Tensor.constant
+    y = nb.conv2d(T(x), T(w), stride=(stride, stride), padding=(pad,) * 4).numpy()
+    return [y] + [t.numpy() for t in nb.grad(loss, argnums=(0, 1))(T(x), T(w))]
+
+
+def reference(x, w, g, pad, stride):
+    """The three results in float64."""
+    tx = torch.tensor(x, dtype=torch.float64).permute(0, 3, 1, 2).requires_grad_()
+    tw = torch.tensor(w, dtype=torch.float64).permute(3, 2, 0, 1).requires_grad_()
+    y = torch.nn.functional.conv2d(tx, tw, padding=pad, stride=stride)
+    dx, dw = torch.autograd.grad(y, (tx, tw), torch.tensor(g, dtype=torch.float64).permute(0, 3, 1, 2))
+    return [y.detach().permute(0, 2, 3, 1).numpy(), dx.permute(0, 2, 3, 1).numpy(), dw.permute(2, 3, 1, 0).numpy()]
+
+
+@pytest.mark.parametrize("n,hw,cin,cout,r,pad,stride", [
+    (33, 32, 8, 32, 3, 1, 1), (37, 31, 5, 31, 3, 1, 1),      # results of up to 32 channels: 128 x 32
+    (32, 33, 64, 130, 3, 1, 1), (41, 29, 20, 128, 3, 0, 1),  # 128 x 128
+    (2, 9, 24, 65, 3, 1, 2), (3, 8, 7, 64, 1, 0, 1),         # 64 x 64, a K tile and less
+    (1, 5, 1, 1, 3, 1, 1), (3, 12, 16, 40, 5, 2, 1)])
+def test_against_float64(hip, n, hw, cin, cout, r, pad, stride):
+    rng = np.random.default_rng(cin)
+    ho = (hw + 2 * pad - r) // stride + 1
+    x = rng.standard_normal((n, hw, hw, cin)).astype(np.float32)
+    w = rng.standard_normal((r, r, cin, cout)).astype(np.float32)
+    g = rng.standard_normal((n, ho, ho, cout)).astype(np.float32)
+    got = ours(x, w, g, pad, stride)
+    want = reference(x, w, g, pad, stride)
+    size = reference(np.abs(x), np.abs(w), np.abs(g), pad, stride)
+    # a sum is rounded once per K tile of 32 and accumulator (2^-24 of the sum of magnitudes at most) and once in
+    # each small product; the filter gradient on the float32 instruction once per two numbers
+    # of a slice of K, in the worst case
+    for a, c, s, terms in zip(got, want, size, (r * r * cin / 32, r * r * cout / 32, n * ho * ho / 2)):
+        assert (np.abs(a - c) <= (terms + 6) * 2.0 ** -24 * s + 2.0 ** -23 * np.abs(c)).all()
+
+
+@pytest.mark.parametrize("n,hw,cin,cout", [(33, 32, 8, 32), (32, 32, 8, 128), (2, 9, 7, 65)])
+def test_numbers_without_parts(hip, n, hw, cin, cout):
+    rng = np.random.default_rng(0)
+    x = rng.uniform(0.5, 1.0, (n, hw, hw, cin)).astype(np.float32)
+    w = rng.uniform(0.5, 1.0, (3, 3, cin, cout)).astype(np.float32)
+    x[0, 1, 1, 0], x[n - 1, 4, 7, 3], x[0, 5, 5, 1] = np.inf, np.nan, 3.4e38  # (the last: infinity as a bf16)
+    w[0, 0, 0, 3], w[1, 1, 1, 2] = 0.0, 1e-30                                # (infinity times zero)
+    got = nb.conv2d(nb.Tensor.constant(x), nb.Tensor.constant(w), padding=(1, 1, 1, 1)).numpy()
+    want = torch.nn.functional.conv2d(torch.tensor(x).double().permute(0, 3, 1, 2),
+                                      torch.tensor(w).double().permute(3, 2, 0, 1), padding=1)
+    want = want.permute(0, 2, 3, 1).numpy()
+    over = np.abs(want) > 3.5e38
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    assert np.isinf(got[over]).all()
+    ok = np.abs(want) < 3.3e38
+    assert (np.abs(got[ok] - want[ok]) <= 1e-5 * np.abs(want[ok])).all()
