@@ -480,22 +480,41 @@ __global__ __launch_bounds__(NWM * NWN * 64) void conv_split_kernel(const ConvAr
   }
 }
 
-// out[i] = sum over z of partial[z][i]; eight slices are in flight per lane and the order
-// of the additions is fixed, so the result does not depend on scheduling.
-__global__ __launch_bounds__(256) void conv_sum_partials(const float* partial, float* out,
-                                                         int64_t n, int splits) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    float s = 0.f;
-    int z = 0;
-    for (; z + 8 <= splits; z += 8) {
+// out[i] = sum over z of partial[z][i].  Eight loads in flight are a trip to memory, and a lane that adds every
+// slice of a small filter by itself makes one trip behind the other on a few CUs; so ZG lanes share a sum,
+// each with every ZG-th slice, and meet in LDS.  The order of the additions is fixed: the result
+// does not depend on scheduling.
+template <int ZG>
+__global__ __launch_bounds__(256) void conv_sum_partials(const float* partial, float* out, int64_t n, int splits) {
+  constexpr int COLS = 256 / ZG;
+  __shared__ float part[ZG][COLS];
+  const int col = (int)threadIdx.x % COLS, zg = (int)threadIdx.x / COLS;
+  const int64_t i = (int64_t)blockIdx.x * COLS + col;
+  float s = 0.f;
+  if (i < n) {
+    int z = zg;
+    for (; z + 7 * ZG < splits; z += 8 * ZG) {
       float v[8];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) v[q] = partial[(int64_t)(z + q) * n + i];
+      for (int q = 0; q < 8; ++q) v[q] = partial[(int64_t)(z + q * ZG) * n + i];
       s += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
     }
-    for (; z < splits; ++z) s += partial[(int64_t)z * n + i];
-    out[i] = s;
+    for (; z < splits; z += ZG) s += partial[(int64_t)z * n + i];
   }
+  if constexpr (ZG > 1) {
+    part[zg][col] = s;
+    __syncthreads();
+    if (zg > 0) return;
+    float v[ZG];
+#pragma unroll
+    for (int q = 0; q < ZG; ++q) v[q] = part[q][col];
+#pragma unroll
+    for (int w = ZG / 2; w > 0; w /= 2)
+#pragma unroll
+      for (int q = 0; q < w; ++q) v[q] += v[q + w];
+    s = v[0];
+  }
+  if (i < n) out[i] = s;
 }
 
 static int conv_check(const nbk_conv_desc* d) {
@@ -654,9 +673,15 @@ extern "C" int nbk_conv2d_wgrad(const nbk_conv_desc* d, const void* x, const voi
   rc = conv_launch_wgrad(a, fast, (hipStream_t)stream);
   if (rc || splits == 1) return rc;
   const int64_t n = a.M * a.Ng;
-  int64_t blocks = (n + 255) / 256;
-  if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(conv_sum_partials, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
-                     (const float*)workspace, (float*)dw, n, splits);
+  auto sum = [&](auto kern, int cols) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)((n + cols - 1) / cols)), dim3(256), 0, (hipStream_t)stream,
+                       (const float*)workspace, (float*)dw, n, splits);
+  };
+  // (the fewer results, the fewer lanes to add them.  us with the product, one lane a sum / these: 64 x 32 x 32, 3 -> 64
+  // channels (1728 results, 512 slices) 43 / 23, 50 x 28 x 28, 1 -> 24 35 / 17.6, 50 x 14 x 14, 24 -> 40 17.7 / 14.9; by four
+  // 50 x 14 x 14, 40 -> 72 29.4 / 26.8, 64 x 32 x 32, 64 -> 128 109 / 107; 128 -> 256 is the same either way)
+  if (n <= 64 * (int64_t)nbk_num_cus()) sum(conv_sum_partials<16>, 16);
+  else if (n <= 512 * (int64_t)nbk_num_cus()) sum(conv_sum_partials<4>, 64);
+  else sum(conv_sum_partials<1>, 256);
   return nbk_check_launch("conv_sum_partials");
 }
