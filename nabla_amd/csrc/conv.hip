@@ -231,6 +231,82 @@ __global__ __launch_bounds__(256) void conv_wgrad_kernel(const ConvArgs g) {
     }
 }
 
+// Filter gradient of up to 32 filter rows (a first layer: 3 x 3 taps of one or three channels), any channel counts and
+// alignment.  All of it is reading dy once, so nothing is staged: a lane is one filter row, its tap fixed for the
+// launch, and what an MFMA step wants of x and of dy it loads itself, STEPS of them in flight.  The eight half waves of a
+// workgroup take an eighth of its slice of pixels each (which pixels share an instruction is free as long as both
+// operands agree), and the waves' sums meet in LDS.
+// us with the sum of the slices (2 to 5), the kernels for any number of rows / this one: 64 x 32 x 32, 3 -> 64 channels
+// 22.9 / 13.1 (dy once: 2.4), 96 x 40 x 40 38 / 24, 50 x 28 x 28, 1 -> 24 17.5 / 11.3, 2 x 14 x 14, 3 -> 16 12.9 / 7.7; one
+// tap, 64 x 32 x 32, 32 -> 64 20.3 / 13.5, 8 -> 512 80 / 44, 50 x 14 x 14, 16 -> 40 12.1 / 10.7.  Error against float64 0.41 to
+// 0.6 of what one chain a slice has (3 -> 64 2.5e-7 -> 1.2e-7).
+template <int NB>
+__global__ __launch_bounds__(256) void conv_wgrad_few_kernel(const ConvArgs g) {
+  constexpr int STEPS = 16;
+  __shared__ float part[4][NB * 16][64];
+  const nbk_conv_desc& d = g.d;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 31, h = lane >> 5;
+  const int64_t n0 = (int64_t)blockIdx.x * (32 * NB);
+  const int64_t k_begin = (int64_t)blockIdx.z * g.k_per_split, k_end = min(g.K, k_begin + g.k_per_split);
+  const int run = (int)((k_end - k_begin + 7) / 8);
+  const int64_t first = k_begin + (int64_t)(wave * 2 + h) * run;
+  int left = (int)max((int64_t)0, min((int64_t)run, k_end - first));
+  const int px = left > 0 ? (int)first : 0;  // < 2^31 (checked on the host)
+  // (filter rows and columns past the end repeat the last one: their results are not stored)
+  int f_c, f_s, x, y;
+  const int f_rs = g.by_cin.divmod(min(li, (int)g.M - 1), f_c);
+  const int q_h = g.by_s.divmod(f_rs, f_s) - d.pad_t, q_w = f_s - d.pad_l;
+  const int t = g.by_wo.divmod(px, x);
+  int n = g.by_ho.divmod(t, y);
+  const float* b[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) b[j] = g.b + (int64_t)px * d.Cout + min(n0 + j * 32 + li, g.Ng - 1);
+  f32x16 acc[2][NB];  // (two chains a wave: half the roundings in a row)
+#pragma unroll
+  for (int j = 0; j < NB; ++j) acc[0][j] = acc[1][j] = (f32x16)(0.f);
+  for (int t0 = 0; t0 < run; t0 += STEPS) {
+    float fa[STEPS], fb[NB][STEPS];
+#pragma unroll
+    for (int e = 0; e < STEPS; ++e) {
+      const bool live = left > 0;
+      const int ih = y * d.stride_h + q_h, iw = x * d.stride_w + q_w;
+      const bool in = live && ih >= 0 && ih < d.H && iw >= 0 && iw < d.W;
+      const float v = g.a[in ? (int64_t)((n * (int)d.H + ih) * (int)d.W + iw) * d.Cin + f_c : 0];
+      fa[e] = in ? v : 0.f;
+      --left;
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const float w = *b[j];
+        fb[j][e] = live ? w : 0.f;
+        b[j] += left > 0 ? d.Cout : 0;  // (the last pixel again)
+      }
+      if (++x == d.Wo) {
+        x = 0;
+        if (++y == d.Ho) { y = 0; ++n; }
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < STEPS; ++e)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        acc[e & 1][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[j][e], acc[e & 1][j], 0, 0, 0);
+  }
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) part[wave][j * 16 + r][lane] = acc[0][j][r] + acc[1][j][r];
+  __syncthreads();
+  // D register r of lane (column li, half h) is row (r / 4) * 8 + h * 4 + r % 4; a wave sums its share of the registers
+  float* out = g.out + (g.splits > 1 ? (int64_t)blockIdx.z * g.M * g.Ng : 0);
+#pragma unroll
+  for (int q = 0; q < NB * 4; ++q) {
+    const int at = wave * (NB * 4) + q, r = at & 15;
+    const int64_t row = (r >> 2) * 8 + h * 4 + (r & 3), col = n0 + (at >> 4) * 32 + li;
+    const float sum = (part[0][at][lane] + part[1][at][lane]) + (part[2][at][lane] + part[3][at][lane]);
+    if (row < g.M && col < g.Ng) out[row * g.Ng + col] = sum;
+  }
+}
+
 // ---- out of bf16 parts (split_f32.h) --------------------------------------------------------
 // Tiles of BM x BN on NWM x NWN waves, K tiles of 32 in two LDS buffers.  A lane takes pieces of 8
 // consecutive k of a row: forward and dgrad, 8 channels of a pixel at one tap (channel counts that are
@@ -574,9 +650,17 @@ static int conv_launch(ConvArgs& a, hipStream_t st) {
 
 // The filter gradient of channel counts that are multiples of 8 stays on the float32 instruction: its pieces
 // of 8 k are 8 pixels, whose gather costs more than the instruction saves (64 x 32 x 32, 64 -> 128 channels 139
-// us against 112).  Others gather number by number there, too (3 -> 64 44 against 51, 1 -> 24 of 50 x 28 x 28 34 against 39).
+// us against 112).  Others gather number by number there, too (before the sum of slices took many lanes 3 -> 64 44 against 51).
 static int conv_launch_wgrad(ConvArgs& a, bool fast, hipStream_t st) {
   a.set_divisors();
+  if (a.M <= 32) {  // one block of 32 filter rows: faster at every size above
+    const int64_t nb = a.Ng <= 32 ? 1 : 2, columns = (a.Ng + 32 * nb - 1) / (32 * nb);
+    NBK_REQUIRE(columns <= 0x7fffffffLL, "conv2d: launch too large");
+    const dim3 grid((unsigned)columns, 1, (unsigned)a.splits);
+    if (nb == 1) hipLaunchKernelGGL((conv_wgrad_few_kernel<1>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((conv_wgrad_few_kernel<2>), grid, dim3(256), 0, st, a);
+    return nbk_check_launch("conv_wgrad_few_kernel");
+  }
   if (!fast) return conv_launch_tile<CONV_WGRAD, true, 64, 64, 2, 2>(a, st);
   // the narrow workgroup tile when the last 128-wide column tile would be at most half full,
   // or when the wide tiling gives fewer workgroups than the GPU has CUs
