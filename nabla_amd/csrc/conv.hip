@@ -9,8 +9,8 @@
 //             A[m,k] = x[n, ho*sh-pt+r, wo*sw-pl+s, c]      B[k,j] = dy[n,ho,wo,j]
 // Out-of-image taps read zero, which is the zero padding of the reference op.
 //
-// Forward and dgrad multiply out of bf16 parts (split_f32.h), the filter gradient on the float32
-// instruction.  Address arithmetic is kept out of the K loop: a lane decomposes its pixels or filter
+// Forward and dgrad multiply out of bf16 parts (split_f32.h), the filter gradient and filters of
+// a few numbers on the float32 instruction.  Address arithmetic is kept out of the K loop: a lane decomposes its pixels or filter
 // rows once and steps through the taps.
 // wgrad contracts over every output pixel of the batch while its result is tiny,
 // so it is split along K over blockIdx.z into a workspace and summed by a second
@@ -304,6 +304,73 @@ __global__ __launch_bounds__(256) void conv_wgrad_few_kernel(const ConvArgs g) {
     const int64_t row = (r >> 2) * 8 + h * 4 + (r & 3), col = n0 + (at >> 4) * 32 + li;
     const float sum = (part[0][at][lane] + part[1][at][lane]) + (part[2][at][lane] + part[3][at][lane]);
     if (row < g.M && col < g.Ng) out[row * g.Ng + col] = sum;
+  }
+}
+
+// Forward of filters with up to 2 STEPS numbers a channel of the result (a first layer), any channel counts and
+// alignment: as above, nothing is staged.  A lane is a pixel and knows the taps of the numbers that it supplies (k = 2 e + h
+// of step e); the filter stays in registers while a wave goes from block to block of 32 pixels.
+// us, the former tiles on the float32 instruction / tiles out of bf16 parts / this kernel: 64 x 32 x 32, 3 -> 64 channels
+// 14.2 / 15.6 / 10.4, 96 x 40 x 40 24 / 32 / 19, 1 -> 64 19 / 32 / 14, 50 x 28 x 28, 1 -> 24 9.7 / 9.5 / 5.3, 5 x 5 taps
+// 64 x 30 x 30, 1 -> 32 12.4 / 10.6 / 7.4; one tap 64 x 32 x 32, 32 -> 64 11.8 / 13.4 / 10.7, 8 -> 512 52 / 69 / 33.  Bound by the
+// result's writes where it is large (3 -> 64: 2.4 us of them).  Error against float64 0.78 to 0.93 of one chain's.
+template <int NB, int STEPS>
+__global__ __launch_bounds__(256, 2) void conv_fwd_few_kernel(const ConvArgs g) {
+  const nbk_conv_desc& d = g.d;
+  const int lane = threadIdx.x & 63, li = lane & 31, h = lane >> 5;
+  const int64_t n0 = (int64_t)blockIdx.y * (32 * NB);
+  float fb[NB][STEPS];
+  int off[STEPS], tap[STEPS];
+#pragma unroll
+  for (int e = 0; e < STEPS; ++e) {
+    const int k = 2 * e + h;
+    const bool ok = k < g.K;
+    int c, s;
+    const int r = g.by_s.divmod(g.by_cin.divmod(ok ? k : 0, c), s);
+    off[e] = ok ? (r * (int)d.W + s) * (int)d.Cin + c : -1;
+    tap[e] = r << 8 | s;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const float v = g.b[(ok ? k : 0) * d.Cout + min(n0 + j * 32 + li, g.Ng - 1)];
+      fb[j][e] = ok ? v : 0.f;
+    }
+  }
+  float bias[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) bias[j] = g.bias ? g.bias[min(n0 + j * 32 + li, g.Ng - 1)] : 0.f;
+  const bool relu = d.act == NBK_ACT_RELU;
+  const int64_t step = (int64_t)gridDim.x * 128;
+  for (int64_t m0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 32; m0 < g.M; m0 += step) {
+    // (pixels past the end repeat the last one: their results are not stored)
+    int x, y;
+    const int t = g.by_wo.divmod((int)min(m0 + li, g.M - 1), x);
+    const int n = g.by_ho.divmod(t, y);
+    const int h0 = y * d.stride_h - d.pad_t, w0 = x * d.stride_w - d.pad_l;
+    const int64_t base = (((int64_t)n * d.H + h0) * d.W + w0) * d.Cin;
+    float fa[STEPS];
+#pragma unroll
+    for (int e = 0; e < STEPS; ++e) {
+      const int ih = h0 + (tap[e] >> 8), iw = w0 + (tap[e] & 255);
+      const bool in = off[e] >= 0 && ih >= 0 && ih < d.H && iw >= 0 && iw < d.W;
+      const float v = g.a[in ? base + off[e] : 0];
+      fa[e] = in ? v : 0.f;
+    }
+    f32x16 acc[2][NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[0][j] = acc[1][j] = (f32x16)(0.f);
+#pragma unroll
+    for (int e = 0; e < STEPS; ++e)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        acc[e & 1][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[j][e], acc[e & 1][j], 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int64_t row = m0 + (r >> 2) * 8 + h * 4 + (r & 3), col = n0 + j * 32 + li;
+        const float v = acc[0][j][r] + acc[1][j][r] + bias[j];
+        if (row < g.M && col < g.Ng) g.out[row * g.Ng + col] = relu ? fmaxf(v, 0.f) : v;
+      }
   }
 }
 
@@ -677,6 +744,14 @@ static int conv_launch_wgrad(ConvArgs& a, bool fast, hipStream_t st) {
   return nbk_check_launch("conv_wgrad_kernel");
 }
 
+template <int NB, int STEPS>
+static int conv_launch_fwd_few(const ConvArgs& a, hipStream_t st) {
+  const int64_t blocks = (a.M + 127) / 128, most = 4 * (int64_t)nbk_num_cus();
+  const dim3 grid((unsigned)(blocks < most ? blocks : most), (unsigned)((a.Ng + 32 * NB - 1) / (32 * NB)));
+  hipLaunchKernelGGL((conv_fwd_few_kernel<NB, STEPS>), grid, dim3(256), 0, st, a);
+  return nbk_check_launch("conv_fwd_few_kernel");
+}
+
 extern "C" int nbk_conv2d_fwd(const nbk_conv_desc* d, const void* x, const void* w,
                               const void* bias, void* y, void* stream) {
   int rc = conv_check(d);
@@ -687,6 +762,14 @@ extern "C" int nbk_conv2d_fwd(const nbk_conv_desc* d, const void* x, const void*
   a.a = (const float*)x; a.b = (const float*)w; a.bias = (const float*)bias; a.out = (float*)y;
   a.M = d->N * d->Ho * d->Wo; a.Ng = d->Cout; a.K = d->R * d->S * d->Cin;
   a.splits = 1; a.k_per_split = (a.K + 15) / 16 * 16;
+  // (offsets inside a filter stand in 32 bits, the launch's second axis ends at 65535)
+  // sixteen steps are what the registers hold; faster at every size above
+  if (a.K <= 32 && d->R * d->W * d->Cin < 0x7fffffffLL && d->Cout <= 65535 * 32) {
+    a.set_divisors();
+    hipStream_t st = (hipStream_t)stream;
+    if (a.Ng <= 32) return a.K <= 16 ? conv_launch_fwd_few<1, 8>(a, st) : conv_launch_fwd_few<1, 16>(a, st);
+    return a.K <= 16 ? conv_launch_fwd_few<2, 8>(a, st) : conv_launch_fwd_few<2, 16>(a, st);
+  }
   return d->Cin % 8 == 0 ? conv_launch<CONV_FWD, true>(a, (hipStream_t)stream)
                          : conv_launch<CONV_FWD, false>(a, (hipStream_t)stream);
 }
