@@ -184,14 +184,16 @@ typedef struct nbk_rowprog {
 int nbk_rowprog_launch(const nbk_rowprog* prog, void* stream);
 /* 1 if the library carries a straight-line (ahead-of-time specialised) kernel
  * for this program, 2 if it also carries a hand-scheduled kernel that this launch
- * (row length, alignment) would take, 0 if the interpreter will run it.  Results
- * are the same to rounding either way; NBK_ROWPROG_INTERPRET=1 forces the
- * interpreter, NBK_ROWPROG_HAND=0 the generated kernels. */
+ * (row length, alignment) would take, 3 if the program is one of those that have a
+ * kernel with approximate functions of their own (16-bit results), 0 if the interpreter
+ * will run it.  Results are the same to rounding either way; NBK_ROWPROG_INTERPRET=1
+ * forces the interpreter, NBK_ROWPROG_HAND=0 the generated kernels. */
 int nbk_rowprog_is_specialized(const nbk_rowprog* prog);
 /* The 64-bit hash (FNV-1a over header, operand classes, instructions, immediates; pointers,
- * strides and extents excluded) by which a program finds its specialised kernel.  That
- * kernel's name ends in the hash in hex, so a profile can be matched to the program it is
- * for.  0 for an invalid program. */
+ * strides and extents excluded) of a program.  Kernels are found by operand types and
+ * instructions alone and those with approximate functions by this hash; a kernel's name
+ * holds, in hex, the hash of the program it was generated from, so a profile can be
+ * matched to it.  0 for an invalid program. */
 uint64_t nbk_rowprog_hash(const nbk_rowprog* prog);
 
 /* ===================================================================== */

@@ -8,7 +8,8 @@ chunks, LDS staging of rows that are read in several phases, wavefront-shuffle +
 LDS-tree reductions) and writes them to ``csrc/rowprog_spec_gen*.hip`` together
 with a lookup table keyed by a hash of operand types and instructions.  ``nbk_rowprog_launch``
 hashes the program it is given and uses the specialised kernel when one exists: at any size
-and alignment, with any immediates (a mean's row length is one).
+and alignment, with any immediates (a mean's row length is one).  Eleven programs of the bf16 benchmark
+steps have a second kernel each with approximate functions, found by the hash of the whole program.
 
     python -m nabla_amd.backend.specialize          # regenerate the sources
 
@@ -145,6 +146,19 @@ def stage16_operand(a: dict) -> int | None:
     return None
 
 
+# what rp_unary_lowp and rp_binary_lowp (csrc/rowprog_device.h) compute otherwise than the interpreter
+_APPROXIMATED = {"exp", "log", "sqrt", "rsqrt", "erf", "gelu", "dgelu", "sigmoid", "div"}
+
+
+def takes_approximations(a: dict) -> bool:
+    """A program of the benchmark steps with one of these functions and 16-bit floats for results,
+    beside whose rounding the hardware's functions and the short GELU are accurate enough."""
+    stored = {i[1] for i in a["ins"] if i[0] in (isa.STR, isa.STG)}
+    return (a.get("benchmark", False) and bool(stored) and
+            all(a["operands"][k].dtype.abi in (1, 2) for k in stored) and
+            any(isa.EW_NAME.get(i[0]) in _APPROXIMATED for i in a["ins"]))
+
+
 def generate_kernel(a: dict, name: str, resident: bool = False, stage16: int | None = None) -> str:
     """HIP source of one specialised kernel for the row program ``a``.
 
@@ -159,10 +173,7 @@ def generate_kernel(a: dict, name: str, resident: bool = False, stage16: int | N
     block_mode = bool(a["has_reduce"])
     assert not resident or block_mode
     inputs = full_inputs(a)
-    # every stored tensor a 16-bit float: hardware transcendentals are accurate enough for the
-    # benchmark steps; elsewhere the functions are the interpreter's
-    stored = {i[1] for i in ins if i[0] in (isa.STR, isa.STG)}
-    lowp = bool(stored) and all(ops[k].dtype.abi in (1, 2) for k in stored) and a.get("benchmark", True)
+    lowp = "approx_hash" in a
     L: list[str] = []
     w = L.append
     if block_mode:
@@ -664,16 +675,21 @@ def collect_programs() -> dict[int, dict]:
 
 def kernels_of(programs: dict[int, dict]) -> list[tuple[int, str, dict, dict]]:
     """(key, name, program, the program that the generic form is made of) of every kernel: programs
-    of one key share theirs.  It goes by the hash of the first; the generic form is that of the
-    longest rows, the ones that the register-resident forms leave to it (with the functions of the first)."""
+    of one key share theirs, which computes what the interpreter computes.  It goes by the hash of the
+    first; the generic form is that of the longest rows, the ones that the register-resident forms leave
+    to it.  A program that takes approximations has, beside that, kernels of its own, found by its hash:
+    another program of the same instructions has made no such choice."""
     by_key: dict[int, list] = {}
     for h, a in programs.items():
         by_key.setdefault(program_key(a), []).append((h, a))
     out = []
     for key, members in sorted(by_key.items()):
         h, a = members[0]
-        generic = max((m for _, m in members), key=lambda m: m["C"])
-        out.append((key, f"rp_spec_{h:016x}", a, dict(generic, benchmark=a.get("benchmark", True))))
+        out.append((key, f"rp_spec_{h:016x}", a, max((m for _, m in members), key=lambda m: m["C"])))
+    for h, a in sorted(programs.items()):
+        if takes_approximations(a):
+            a = dict(a, approx_hash=h)
+            out.append((program_key(a), f"rp_spec_{h:016x}_approx", a, a))
     return out
 
 
@@ -708,10 +724,10 @@ def write_sources(programs: dict[int, dict]) -> list[Path]:
             k16 = f"(const void*){name}_s16" if stage16_operand(generic) is not None else "nullptr"
             src.append(f"  {{0x{key:016x}ULL, {{{', '.join(ks)}}}, {{{', '.join(kf)}}}, "
                        f"{{{', '.join(kst)}}}, {kflat}, {k16}, 0x{stage_sig(generic):x}ULL, "
-                       f"{1 if a['has_reduce'] else 0}}},")
+                       f"{1 if a['has_reduce'] else 0}, 0x{a.get('approx_hash', 0):x}ULL}},")
         src.append("  {0ULL, {nullptr, nullptr, nullptr, nullptr, nullptr}, "
                    "{nullptr, nullptr, nullptr, nullptr, nullptr}, "
-                   "{nullptr, nullptr, nullptr, nullptr, nullptr}, nullptr, nullptr, 0, 0}};")
+                   "{nullptr, nullptr, nullptr, nullptr, nullptr}, nullptr, nullptr, 0, 0, 0}};")
         src.append(f"extern const int rp_spec_count_{fi} = {len(chunk)};")
         path = CSRC / f"rowprog_spec_gen{fi}.hip"
         path.write_text("\n".join(src) + "\n")

@@ -147,7 +147,8 @@ static uint64_t rp_program_hash(const nbk_rowprog* p) {
 
 // What a compiled kernel is found by: the same without what it does not depend on.  A kernel reads
 // immediates from the program it is launched with (a row length that a mean divides by is one), takes
-// operands at any alignment, and only its generic form depends on what is staged (rp_stage_sig).
+// operands at any alignment, and only its generic form depends on what is staged (rp_stage_sig).  (Kernels with
+// approximate functions are found by the whole hash above: they serve the programs they were chosen for.)
 // Same bytes as key_bytes() in nabla_amd/backend/specialize.py.
 static uint64_t rp_program_key(const nbk_rowprog* p) {
   uint64_t h = 0xCBF29CE484222325ULL;
@@ -182,15 +183,20 @@ struct RpSpec {
   const rp_hand_entry* hand;
   uint64_t stage_sig;
   int block_mode;
+  bool has_approx;  // g_approx holds kernels for a program of this key
+  bool approximate;
   bool lds_attr_set;
   bool lds16_attr_set;
 };
 static std::mutex g_spec_mu;
-static std::unordered_map<uint64_t, RpSpec>* g_specs = nullptr;
+static std::unordered_map<uint64_t, RpSpec>* g_specs = nullptr;   // by key
+static std::unordered_map<uint64_t, RpSpec>* g_approx = nullptr;  // by hash: the chosen programs alone
 
-static RpSpec* rp_find_spec(uint64_t h) {
+static RpSpec* rp_find_spec(const nbk_rowprog* p) {
+  const uint64_t key = rp_program_key(p);
   std::lock_guard<std::mutex> lk(g_spec_mu);
   if (!g_specs) {
+    g_approx = new std::unordered_map<uint64_t, RpSpec>();
     g_specs = new std::unordered_map<uint64_t, RpSpec>();
 #define RP_TABLE(I) rp_spec_table_##I,
 #define RP_COUNT(I) rp_spec_count_##I,
@@ -214,16 +220,27 @@ static RpSpec* rp_find_spec(uint64_t h) {
         e.lds_attr_set = false;
         e.lds16_attr_set = false;
         e.hand = nullptr;
-        (*g_specs)[tabs[t][i].key] = e;
+        e.has_approx = false;
+        e.approximate = tabs[t][i].approx_hash != 0;
+        if (tabs[t][i].approx_hash) (*g_approx)[tabs[t][i].approx_hash] = e;
+        else (*g_specs)[tabs[t][i].key] = e;
       }
+    for (int t = 0; t < NBK_RP_SPEC_FILES; ++t)
+      for (int i = 0; i < counts[t]; ++i)
+        if (tabs[t][i].approx_hash) g_specs->at(tabs[t][i].key).has_approx = true;
     // (a hand-scheduled kernel stands beside generated ones, which take the launches it declines)
     for (int i = 0; i < rp_hand_count; ++i) {
       auto it = g_specs->find(rp_hand_table[i].key);
       if (it != g_specs->end()) it->second.hand = &rp_hand_table[i];
     }
   }
-  auto it = g_specs->find(h);
-  return it == g_specs->end() ? nullptr : &it->second;
+  auto it = g_specs->find(key);
+  if (it == g_specs->end()) return nullptr;
+  if (it->second.has_approx) {
+    auto a = g_approx->find(rp_program_hash(p));
+    if (a != g_approx->end()) return &a->second;
+  }
+  return &it->second;
 }
 
 // Resident workgroups per CU of a kernel at a block size (no dynamic LDS); cached.
@@ -266,9 +283,9 @@ static bool rp_hand_disabled() {
 
 extern "C" int nbk_rowprog_is_specialized(const nbk_rowprog* prog) {
   if (rp_validate(prog) != NBK_OK || rp_specs_disabled()) return 0;
-  RpSpec* spec = rp_find_spec(rp_program_key(prog));
+  RpSpec* spec = rp_find_spec(prog);
   if (!spec) return 0;
-  return (spec->hand && !rp_hand_disabled() && spec->hand->fits(prog)) ? 2 : 1;
+  return (spec->hand && !rp_hand_disabled() && spec->hand->fits(prog)) ? 2 : spec->approximate ? 3 : 1;
 }
 
 extern "C" uint64_t nbk_rowprog_hash(const nbk_rowprog* prog) {
@@ -288,7 +305,7 @@ extern "C" int nbk_rowprog_launch(const nbk_rowprog* prog, void* stream) {
   }
   const nbk_rowprog* p = &norm;
   RpSpec* spec = (rp_specs_disabled() || prog->reserved == 1) ? nullptr
-                                                               : rp_find_spec(rp_program_key(prog));
+                                                               : rp_find_spec(prog);
   if (spec && spec->block_mode != (p->has_reduce ? 1 : 0)) spec = nullptr;
   hipStream_t st = (hipStream_t)stream;
   int64_t rows = 1;

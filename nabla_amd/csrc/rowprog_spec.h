@@ -28,6 +28,9 @@ struct rp_spec_entry {
   const void* kernel_stage16;
   uint64_t stage_sig;  // what kernel[0] finds staged in LDS: a program that differs there cannot run it
   int block_mode;
+  // 0, or the hash of the one program of this key that these kernels are for: they compute
+  // rp_unary_lowp and rp_binary_lowp, which a benchmark step takes and no other program chose
+  uint64_t approx_hash;
 };
 
 // A hand-scheduled kernel for one program (rowprog_hand.hip), attached by key to that program's

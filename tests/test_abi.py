@@ -146,6 +146,30 @@ def test_generated_kernels_cover_every_row_program_of_the_benchmark_steps():
     assert not missing, "row programs without a specialised kernel: " + "; ".join(missing)
 
 
+def test_approximate_functions_stay_with_the_programs_they_were_chosen_for():
+    """Another program of the same instructions (rows at another alignment, another length to
+    divide by) runs the kernel whose functions are the interpreter's."""
+    from nabla_amd.backend import lib, specialize
+    L = lib.load()
+    chosen = 0
+    for a in specialize.collect_programs().values():
+        rp = _program_record(a)
+        kind = L.nbk_rowprog_is_specialized(C.byref(rp))
+        assert (kind == 3) == specialize.takes_approximations(a)
+        if kind != 3:
+            continue
+        chosen += 1
+        if rp.n_imm:
+            was, rp.imm[0] = rp.imm[0], rp.imm[0] * 1.5
+            assert L.nbk_rowprog_is_specialized(C.byref(rp)) == 1
+            rp.imm[0] = was
+        if any(o.vec_ok for o in a["operands"]):
+            for i in range(rp.n_operands):
+                rp.operand[i].vec_ok = 0
+            assert L.nbk_rowprog_is_specialized(C.byref(rp)) == 1
+    assert chosen >= 8
+
+
 def test_the_committed_traffic_counters_belong_to_the_kernel_the_stress_step_runs():
     """`bench.py` reports the HBM traffic of the stress step from `profiles/hbm_traffic_c2.json`,
     which names the kernel (by program hash) whose counters it holds.  A planner or op change

@@ -82,3 +82,40 @@ def test_against_the_interpreter(hip, programs, cols):
             compared += 1
         assert rows >= 1
     assert compared >= 30
+
+
+def test_functions_are_the_interpreters(hip, programs):
+    """Programs without reductions at an alignment that no benchmark step has: bit for bit."""
+    L = lib.load()
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    rng = np.random.default_rng(0)
+    n, compared = 4099, 0
+    for a in programs:
+        rp = _program_record(a)
+        if rp.has_reduce or any(o.col_stride == 0 or not o.dtype.is_float() for o in a["operands"]):
+            continue
+        rp.n_lead, rp.C = 1, n
+        rp.lead_dim[0] = 1
+        written = {i[1] for i in a["ins"] if i[0] in (isa.STG, isa.STR)}
+        keep, outs = [], []
+        for i, o in enumerate(a["operands"]):
+            x = (torch.tensor(rng.standard_normal(n + 1)) * 3).to(o.dtype.to_torch()).cuda()
+            keep.append(x)
+            od = rp.operand[i]
+            od.vec_ok, od.ptr, od.col_stride = 0, x.data_ptr() + x.element_size(), 1
+            for k in range(4):
+                od.lead_stride[k] = 0
+            if i in written:
+                outs.append(x)
+        results = []
+        for rp.reserved in (0, 1):
+            for x in outs:
+                x.zero_()
+            assert rp.reserved or L.nbk_rowprog_is_specialized(C.byref(rp)) == 1
+            lib.check(L.nbk_rowprog_launch(C.byref(rp), st))
+            results.append([x.clone() for x in outs])
+        for got, want in zip(*results):
+            same = (got == want) | (got.isnan() & want.isnan())
+            assert same.all(), f"{specialize.program_hash(a):016x} ({' '.join(a['members'])[:60]})"
+        compared += 1
+    assert compared >= 40
