@@ -11,10 +11,13 @@
 // = 16384 8.2e-7 / 5.9e-7; the float32 instruction in one chain 5.9e-7 / 4.4e-7 and 2.2e-6 / 1.7e-6, in
 // four 2.9e-7 / 1.2e-7 and 1.2e-6 / 4.4e-7.  (All six in one accumulator: as the one chain.)
 //   A number that is not finite, or rounds to infinity as a bf16, has no such parts and its sums come out
-// as NaN: whoever stores a sum that is not finite computes it again (split_dot).  Numbers below
-// 2^-109 lose the digits of x3 that a bf16 no longer holds.
+// as NaN: a wave with a sum that is not finite runs its tile again on the float32 instruction (SplitAcc::again)
+// and stores those of it that the parts did not give.  Numbers below 2^-109 lose the digits of x3 that a bf16 no
+// longer holds.
 #pragma once
 #include "nbk_common.h"
+
+#include <type_traits>
 
 typedef uint32_t sp_u4 __attribute__((ext_vector_type(4)));
 typedef float sp_f2 __attribute__((ext_vector_type(2)));
@@ -74,6 +77,51 @@ struct SplitAcc {
     float s = main[0][i][j][r];
     if constexpr (NM == 2) s += main[1][i][j][r];
     return s + small[i][j][r];
+  }
+  // All of K on the float32 instruction, operands straight from memory: a(i, k, inside) and b(j, k, inside) are the
+  // lane's row (lane % 16) of block i and its column of block j, zero past the end of K unless `inside` says
+  // that k is not.  A step is 16 k, four consecutive ones a lane.
+  template <class A, class B>
+  __device__ __forceinline__ void again(int64_t k_begin, int64_t k_end, int lane, A a, B b) {
+    zero();
+    float fa[2][TM][4], fb[2][TN][4];  // (the next step's numbers are on their way)
+    auto load = [&](auto set, int64_t k0) {
+      const int64_t k = k0 + (lane >> 4) * 4;
+      auto all = [&](auto inside) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll
+          for (int i = 0; i < TM; ++i) fa[set.value][i][e] = a(i, k + e, inside);
+#pragma unroll
+          for (int j = 0; j < TN; ++j) fb[set.value][j][e] = b(j, k + e, inside);
+        }
+      };
+      if (k0 + 16 <= k_end) all(std::true_type{});
+      else all(std::false_type{});
+    };
+    auto multiply = [&](auto set) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            main[e % NM][i][j] =
+                __builtin_amdgcn_mfma_f32_16x16x4f32(fa[set.value][i][e], fb[set.value][j][e], main[e % NM][i][j], 0, 0, 0);
+    };
+    load(std::integral_constant<int, 0>{}, k_begin);
+#pragma unroll 1
+    for (int64_t k0 = k_begin; k0 < k_end; k0 += 32) {  // (past the end: zeros)
+      load(std::integral_constant<int, 1>{}, k0 + 16);
+      multiply(std::integral_constant<int, 0>{});
+      load(std::integral_constant<int, 0>{}, k0 + 32);
+      multiply(std::integral_constant<int, 1>{});
+    }
+  }
+  __device__ __forceinline__ float sum_again(int i, int j, int r) const {
+    float s = main[0][i][j][r];
+    if constexpr (NM == 2) s += main[1][i][j][r];
+    return s;
   }
   // One K tile; wm, wn: the wave's first row and column in the workgroup's tile.
   template <int BM, int BN, int SET>

@@ -64,3 +64,26 @@ def test_numbers_without_parts(hip, n, hw, cin, cout):
     assert np.isinf(got[over]).all()
     ok = np.abs(want) < 3.3e38
     assert (np.abs(got[ok] - want[ok]) <= 1e-5 * np.abs(want[ok])).all()
+
+
+@pytest.mark.parametrize("cin,cout", [(64, 128), (20, 40)])
+def test_numbers_without_parts_cost_one_more_pass(hip, cin, cout):
+    """Images of NaN throughout: every wave runs its tile again on the float32 instruction and gathers number by
+    number (one result after the other took 43 to 130 times as long)."""
+    from nabla_amd.backend import lib
+    from test_gpu_gemm_f32_parts import seconds
+    d = lib.ConvDesc()
+    d.N, d.H, d.W, d.Cin, d.R, d.S, d.Cout, d.Ho, d.Wo = 32, 32, 32, cin, 3, 3, cout, 32, 32
+    d.stride_h = d.stride_w = d.pad_t = d.pad_b = d.pad_l = d.pad_r = 1
+    w = torch.ones((3, 3, cin, cout), device="cuda")
+    st = lib.C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ptr = lambda t: lib.C.c_void_p(t.data_ptr())
+    L = lib.load()
+    for run, ci, co in ((lambda x, y: L.nbk_conv2d_fwd(lib.C.byref(d), ptr(x), ptr(w), None, ptr(y), st), cin, cout),
+                        (lambda x, y: L.nbk_conv2d_dgrad(lib.C.byref(d), ptr(x), ptr(w), ptr(y), st), cout, cin)):
+        times = []
+        for value in (1.0, float("nan")):
+            x, y = torch.full((32, 32, 32, ci), value, device="cuda"), torch.empty((32, 32, 32, co), device="cuda")
+            times.append(seconds(lambda: lib.check(run(x, y))))
+            assert torch.isnan(y).all() == (value != value)
+        assert times[1] <= 10 * times[0]

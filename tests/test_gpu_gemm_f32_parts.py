@@ -66,3 +66,35 @@ def test_numbers_without_parts(hip, M, N):
     np.testing.assert_array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)]))
     ok = np.isfinite(want)
     assert (np.abs(got[ok] - want[ok]) <= 1e-5 * np.abs(want[ok])).all()
+
+
+def seconds(f, n=20):
+    f()
+    a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    a.record()
+    for _ in range(n):
+        f()
+    b.record()
+    b.synchronize()
+    return a.elapsed_time(b)
+
+
+@pytest.mark.parametrize("layout", ["nn", "tn"])
+def test_numbers_without_parts_cost_one_more_pass(hip, layout):
+    """A product of NaN throughout: every wave runs its tile again on the float32 instruction, which has a
+    third of the rate (one result after the other took 46 times as long)."""
+    from nabla_amd.backend import lib
+    n = 1024
+    out = torch.empty((n, n), device="cuda")
+    times = []
+    for value in (1.0, float("nan")):
+        x = torch.full((n, n), value, device="cuda")
+        d = lib.GemmDesc()
+        d.A, d.B, d.C = x.data_ptr(), x.data_ptr(), out.data_ptr()
+        d.M, d.N, d.K = n, n, n
+        d.a_rs, d.a_cs = (1, n) if layout[0] == "t" else (n, 1)
+        d.b_rs, d.b_cs, d.ldc, d.batch, d.batch_inner, d.alpha = n, 1, n, 1, 1, 1.0
+        st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        times.append(seconds(lambda: lib.check(lib.load().nbk_gemm(C.byref(d), st))))
+        assert torch.isnan(out).all() == (value != value)
+    assert times[1] <= 8 * times[0]
