@@ -49,6 +49,17 @@ def test_against_float64(hip, n, hw, cin, cout, r, pad, stride):
 
 
 @pytest.mark.parametrize("n,hw,cin,cout", [(33, 32, 8, 32), (32, 32, 8, 128), (2, 9, 7, 65)])
+def test_small_numbers(hip, n, hw, cin, cout):
+    """Images and cotangents of a few digits of the smallest float32 kind, filters as much larger."""
+    rng = np.random.default_rng(0)
+    x, w, g = (np.ldexp(rng.standard_normal(s), e).astype(np.float32) for s, e in (
+        ((n, hw, hw, cin), -130), ((3, 3, cin, cout), 70), ((n, hw, hw, cout), -120)))
+    for a, c, s in list(zip(ours(x, w, g, 1, 1), reference(x, w, g, 1, 1),
+                            reference(np.abs(x), np.abs(w), np.abs(g), 1, 1)))[:2]:
+        assert (np.abs(a - c) <= (9 * max(cin, cout) / 32 + 6) * 2.0 ** -24 * s + 2.0 ** -23 * np.abs(c)).all()
+
+
+@pytest.mark.parametrize("n,hw,cin,cout", [(33, 32, 8, 32), (32, 32, 8, 128), (2, 9, 7, 65)])
 def test_numbers_without_parts(hip, n, hw, cin, cout):
     rng = np.random.default_rng(0)
     x = rng.uniform(0.5, 1.0, (n, hw, hw, cin)).astype(np.float32)

@@ -48,6 +48,22 @@ def test_against_float64(hip, layout, M, N, K):
 
 
 @pytest.mark.parametrize("M,N", [(1024, 1024), (2048, 2048)])
+@pytest.mark.parametrize("e,f", [(-30, 40), (-112, 60), (-126, 70), (-140, 80), (-145, 100), (40, 50), (100, -100),
+                                 (120, -30), (-70, -60)])
+def test_numbers_of_every_size(hip, M, N, e, f):
+    """Operands about 2^e and 2^f, down to the smallest float32 and up to sums near the largest."""
+    K = 70
+    rng = np.random.default_rng(K)
+    a, b = (np.ldexp(rng.standard_normal(s), x).astype(np.float32) for s, x in (((M, K), e), ((K, N), f)))
+    for x, y in ((a, b), (b.T, a.T)):
+        x64, y64 = x.astype(np.float64), y.astype(np.float64)
+        want, size = x64 @ y64, np.abs(x64) @ np.abs(y64)
+        # as above, for numbers whose last digit may be 2^-149 (the sum is one of float32 numbers itself)
+        tol = (-(-K // 32) + 4) * 2.0 ** -24 * size + 2.0 ** -23 * np.abs(want) + K * 2.0 ** -149
+        assert (np.abs(product(np.ascontiguousarray(x), np.ascontiguousarray(y), "nn") - want) <= tol).all()
+
+
+@pytest.mark.parametrize("M,N", [(1024, 1024), (2048, 2048)])
 def test_numbers_without_parts(hip, M, N):
     K = 70
     rng = np.random.default_rng(0)
