@@ -1560,8 +1560,8 @@ class Planner:
         return True
 
     # What a waiting reduction reads stays in memory until it goes out.  One launch less is worth
-    # 4 us, the time a pass over 16 to 20 MB takes: reductions over more gain nothing that counts
-    # by waiting, and all that wait together hold at most this much.
+    # 4 us, the time a pass over 16 to 20 MB takes: a reduction over more than this gains nothing that
+    # counts and goes out at once, and all that wait for a reader hold at most this much together.
     MAX_WAITING_BYTES = 128 << 20
 
     def _emit_reduce(self, step: Step, stage: int, terminal: bool) -> None:
@@ -1575,6 +1575,9 @@ class Planner:
             return
         if self._waiting_bufs.isdisjoint(step.reads):  # (a second stage stays with its first)
             held = self.bufs[step.reads[0]].nbytes
+            if held > self.MAX_WAITING_BYTES:
+                self._emit(step)
+                return
             if self._waiting_bytes + held > self.MAX_WAITING_BYTES:
                 self._flush_reduces(waiting_only=True)
             self._waiting_bytes += held

@@ -77,3 +77,58 @@ def test_fused_groups_that_read_waiting_results(emulator, monkeypatch):
     (got, n), (want, n_alone) = both_ways(monkeypatch, make)
     assert n < n_alone
     np.testing.assert_array_equal(got[0], want[0])
+
+
+def test_sources_above_the_limit_do_not_wait(emulator, monkeypatch):
+    """x @ w, its column sums, and six products before a step reads them: a source larger than the limit is
+    reduced behind the product that writes it, and its memory is free for the next one."""
+    rng = np.random.default_rng(0)
+    w = [rng.standard_normal((256, 256)) for _ in range(7)]
+    x = rng.standard_normal((512, 256))
+
+    def make():
+        def f(x, *w):
+            x = x @ w[0]
+            total = nb.reduce_sum(x, axis=0)
+            for m in w[1:]:
+                x = x @ m
+            return [total + x]
+        return nb.compile(f)(T(x), *[T(m) for m in w])
+
+    plans = {}
+    for limit in (Planner.MAX_WAITING_BYTES, x.nbytes // 2 - 1, -1):  # (x is float64: half of it in float32)
+        monkeypatch.setattr(Planner, "MAX_WAITING_BYTES", limit)
+        engine.clear_plan_cache()
+        got = make()[0].numpy()
+        (plan,) = [bp.plan for bp in engine._PLAN_CACHE.values()]
+        kinds = [s.kind for s in plan.steps]
+        plans[limit] = (kinds.index("reduce_mid"), plan.arena_bytes, got)
+    engine.clear_plan_cache()
+    (at_wait, arena_wait, want), (at, arena, got), (at_never, arena_never, _) = plans.values()
+    assert at_wait == 6 and at == at_never == 1
+    assert arena == arena_never < arena_wait
+    np.testing.assert_array_equal(got, want)
+
+
+def test_all_that_wait_together_stay_below_the_limit(emulator, monkeypatch):
+    """Three sources at the limit wait for their reader; where two fit, the third sends the first two out."""
+    rng = np.random.default_rng(0)
+    x = rng.standard_normal((64, 128))
+    w = [rng.standard_normal((128, 128)) for _ in range(4)]
+
+    def make():
+        def f(x, *w):
+            sums = 0.0
+            for m in w[:3]:
+                x = x @ m
+                sums = nb.sin(sums + nb.reduce_sum(x, axis=0))
+            return [sums + x @ w[3]]
+        return nb.compile(f)(T(x), *[T(m) for m in w])
+
+    for fit, launches in ((3, ["reduce_batch"]), (2, ["reduce_batch", "reduce_mid"])):
+        monkeypatch.setattr(Planner, "MAX_WAITING_BYTES", fit * 64 * 128 * 4)
+        engine.clear_plan_cache()
+        make()
+        (plan,) = [bp.plan for bp in engine._PLAN_CACHE.values()]
+        engine.clear_plan_cache()
+        assert [s.kind for s in plan.steps if s.kind.startswith("reduce")] == launches
