@@ -380,8 +380,8 @@ __global__ __launch_bounds__(256) void reduce_batch_kernel(const ReduceBatchArgs
 #undef REDUCE_STRIP
 }
 
-static int reduce_mid_slab(const void* in, void* out, int32_t dti, int32_t dto, int64_t outer,
-                           int64_t red, int64_t inner, int32_t kind, void* stream);
+static int reduce_mid_slab(const RedLayout& L, const void* in, void* out, int32_t dti, int32_t dto,
+                           int64_t outer, int64_t red, int64_t inner, int32_t kind, void* stream);
 
 extern "C" int nbk_reduce_mid(const void* in, void* out, int32_t dti, int32_t dto, int64_t outer,
                               int64_t red, int64_t inner, int32_t kind, void* stream) {
@@ -389,11 +389,13 @@ extern "C" int nbk_reduce_mid(const void* in, void* out, int32_t dti, int32_t dt
   NBK_REQUIRE(outer > 0 && red > 0 && inner > 0, "reduce_mid: empty extent");
   NBK_REQUIRE(kind >= NBK_RED_SUM && kind <= NBK_RED_MIN, "reduce_mid: kind %d", kind);
   NBK_REQUIRE(nbk_dtype_size(dti) > 0 && nbk_dtype_size(dto) > 0, "reduce_mid: bad dtype");
-  // `outer` rides on the grid's second dimension (65535 at most): longer ones go in slabs
+  // `outer` rides on the grid's second dimension (65535 at most): longer ones go in slabs, all of
+  // them laid out as the whole is
   const int64_t kSlab = 65535;
+  const RedLayout L = reduce_layout(in, dti, outer, red, inner);
   for (int64_t o0 = 0; o0 < outer; o0 += kSlab) {
     const int64_t n = outer - o0 < kSlab ? outer - o0 : kSlab;
-    const int rc = reduce_mid_slab((const char*)in + o0 * red * inner * nbk_dtype_size(dti),
+    const int rc = reduce_mid_slab(L, (const char*)in + o0 * red * inner * nbk_dtype_size(dti),
                                    (char*)out + o0 * inner * nbk_dtype_size(dto), dti, dto, n, red,
                                    inner, kind, stream);
     if (rc != NBK_OK) return rc;
@@ -401,15 +403,14 @@ extern "C" int nbk_reduce_mid(const void* in, void* out, int32_t dti, int32_t dt
   return NBK_OK;
 }
 
-static int reduce_mid_slab(const void* in, void* out, int32_t dti, int32_t dto, int64_t outer,
-                           int64_t red, int64_t inner, int32_t kind, void* stream) {
+static int reduce_mid_slab(const RedLayout& L, const void* in, void* out, int32_t dti, int32_t dto,
+                           int64_t outer, int64_t red, int64_t inner, int32_t kind, void* stream) {
   if (dti == NBK_I32 || dti == NBK_I64) {
     dim3 grid((unsigned)((inner + 63) / 64), (unsigned)outer);
     hipLaunchKernelGGL(reduce_mid_int_kernel, grid, dim3(256), 0, (hipStream_t)stream, in, out, dti,
                        dto, red, inner, kind);
     return nbk_check_launch("reduce_mid_int_kernel");
   }
-  const RedLayout L = reduce_layout(in, dti, outer, red, inner);
   dim3 grid((unsigned)L.blocks_x, (unsigned)outer);
 #define REDUCE_STRIP(P)                                                                                          \
   hipLaunchKernelGGL(reduce_strip_kernel<P>, grid, dim3(256), 0, (hipStream_t)stream, in, out, dti, dto, red, inner, \

@@ -35,3 +35,25 @@ def test_strips(hip, dtype, outer, red, inner):
             got = out.cpu().numpy()
             np.testing.assert_array_equal(got[shift:-1].reshape(outer, inner), want.astype(np.float32))
             assert got[-1] == 7.5 and (shift == 0 or got[0] == 7.5)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("outer,red,inner", [(65535 + 100, 24, 33), (65535 + 40, 40, 64), (600, 70, 33)])
+def test_one_order_of_additions(hip, dtype, outer, red, inner):
+    """Alone or in a launch with others, and past the 65535 members that one launch's grid holds: the same bits, and
+    members of the same numbers the same results."""
+    from nabla_amd.backend import lib
+    L = lib.load()
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    code, tdt = TYPES[dtype]
+    one = torch.randn((1, red, inner), generator=torch.Generator().manual_seed(0)).to(tdt).cuda()
+    x = one.expand(outer, red, inner).contiguous()
+    alone, batched = (torch.empty((outer, inner), device="cuda") for _ in range(2))
+    lib.check(L.nbk_reduce_mid(C.c_void_p(x.data_ptr()), C.c_void_p(alone.data_ptr()), code, 0, outer, red, inner, 0, st))
+    task = lib.ReduceTask()
+    task.in_, task.out = x.data_ptr(), batched.data_ptr()
+    task.dtype_in, task.dtype_out, task.kind = code, 0, 0
+    task.outer, task.red, task.inner = outer, red, inner
+    lib.check(L.nbk_reduce_mid_batch(C.byref(task), 1, st))
+    assert torch.equal(alone, batched)
+    assert torch.equal(alone, alone[:1].expand(outer, inner))
