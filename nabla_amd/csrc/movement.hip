@@ -160,6 +160,8 @@ extern "C" int nbk_fill(void* dst, int32_t dtype, int64_t n, double value, void*
 // us, before and after, behind a kernel that has just written the operand: 128x256 fp32 10.7 / 4.5,
 // 200x32 15.1 / 3.5, 27 x (74x512) bf16 15.1 / 5.4, 32 x (256x1024) bf16 65.7 / 14.1, 64x4096
 // fp32 17.7 / 3.3, 50 x (196x72) 16.2 / 5.7, the four halves of a split product 4x786432 11.0 / 9.3.
+// (These, and the lines in reduce_layout, from before the combining function was a template's; by themselves in
+// a row 32 x (256x1024) bf16 8.0 / 3.8 since then.)
 // (A long axis over few columns is cut into slices by the caller: two launches, fp32 partials
 // in between.)
 __device__ __forceinline__ float red_comb(float a, float b, int kind) {
@@ -206,9 +208,9 @@ struct RedAny {
 };
 constexpr int RED_FLIGHT = 8;  // rows in flight per lane
 
-template <typename P>
-__device__ __forceinline__ void reduce_strip_body(const void* __restrict__ in, void* __restrict__ out,
-                                                  int dti, int dto, int64_t red, int64_t inner, int kind,
+template <typename P, int kind>
+__device__ __forceinline__ void reduce_strip_kind(const void* __restrict__ in, void* __restrict__ out,
+                                                  int dti, int dto, int64_t red, int64_t inner,
                                                   int64_t bx, int64_t o, int lxs, float* part) {
   constexpr int N = P::N;
   const int LX = 1 << lxs, RY = 256 >> lxs;
@@ -216,14 +218,21 @@ __device__ __forceinline__ void reduce_strip_body(const void* __restrict__ in, v
   const int64_t at = bx * LX + (threadIdx.x & (LX - 1));
   const int64_t base = o * red * pieces + (at < pieces ? at : pieces - 1);
   const float ident = kind == NBK_RED_SUM ? 0.f : (kind == NBK_RED_MAX ? -INFINITY : INFINITY);
-  float acc[N];
+  // CHAINS sums of a lane's rows side by side, T rows at a time: where no rows stand abreast, one sum
+  // would be rounded once a row.  Error against float64 of uniform numbers, one sum / these: 64 x (1024x4099)
+  // fp32 4.2e-7 / 5.0e-8, 1024 x (12x1000) 5.4e-8 / 4.0e-8.  (Less than eight rows are added in their order.)
+  constexpr int CHAINS = N == 1 ? 8 : 2, T = RED_FLIGHT / CHAINS;
+  static_assert(T == 1 || T == 4, "a sum of one row or of four");
+  float acc[CHAINS][N];
 #pragma unroll
-  for (int e = 0; e < N; ++e) acc[e] = ident;
-  auto add = [&](const typename P::raw u) {
+  for (int c = 0; c < CHAINS; ++c)
+#pragma unroll
+    for (int e = 0; e < N; ++e) acc[c][e] = ident;
+  auto add = [&](int c, const typename P::raw u) {
     float v[N];
     P::unpack(u, dti, v);
 #pragma unroll
-    for (int e = 0; e < N; ++e) acc[e] = red_comb(acc[e], v[e], kind);
+    for (int e = 0; e < N; ++e) acc[c][e] = red_comb(acc[c][e], v[e], kind);
   };
   const int64_t step = (int64_t)RY * pieces;
   int64_t r = threadIdx.x >> lxs, i = base + r * pieces;
@@ -233,39 +242,62 @@ __device__ __forceinline__ void reduce_strip_body(const void* __restrict__ in, v
 #pragma unroll
     for (int q = 0; q < RED_FLIGHT; ++q) u[q] = P::load(in, i + q * step, dti);
 #pragma unroll
-    for (int q = 0; q < RED_FLIGHT; ++q) add(u[q]);
+    for (int c = 0; c < CHAINS; ++c) {
+      float v[T][N];
+#pragma unroll
+      for (int q = 0; q < T; ++q) P::unpack(u[c * T + q], dti, v[q]);
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        float x = v[0][e];
+        if constexpr (T == 4) x = red_comb(red_comb(x, v[1][e], kind), red_comb(v[2][e], v[3][e], kind), kind);
+        acc[c][e] = red_comb(acc[c][e], x, kind);
+      }
+    }
   }
   if (r < red) {  // the rows left, requested together too
     typename P::raw u[RED_FLIGHT - 1];
 #pragma unroll
     for (int q = 0; q < RED_FLIGHT - 1; ++q) u[q] = P::load(in, r + q * RY < red ? i + q * step : i, dti);
+    if (N > 1 && red < RED_FLIGHT) {
 #pragma unroll
-    for (int q = 0; q < RED_FLIGHT - 1; ++q)
-      if (r + q * RY < red) add(u[q]);
+      for (int q = 0; q < RED_FLIGHT - 1; ++q)
+        if (r + q * RY < red) add(0, u[q]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < RED_FLIGHT - 1; ++q)
+        if (r + q * RY < red) add(q % CHAINS, u[q]);
+    }
   }
+#pragma unroll
+  for (int w = CHAINS / 2; w > 0; w /= 2)
+#pragma unroll
+    for (int c = 0; c < w; ++c)
+#pragma unroll
+      for (int e = 0; e < N; ++e) acc[c][e] = red_comb(acc[c][e], acc[c + w][e], kind);
+  float(&sum)[N] = acc[0];
   if (RY == 1) {  // a column is one lane's: no partial sums to meet
     if (at >= pieces) return;
     const int64_t to = o * pieces + at;
     const bool whole = N == 4 && ((uintptr_t)out & 15) == 0;
     if (whole && dto == NBK_F32) {
-      ((float4*)out)[to] = make_float4(acc[0], acc[1 % N], acc[2 % N], acc[3 % N]);
+      ((float4*)out)[to] = make_float4(sum[0], sum[1 % N], sum[2 % N], sum[3 % N]);
     } else if (whole && dto == NBK_BF16) {
-      ((uint2*)out)[to] = make_uint2((uint32_t)nbk_f32_to_bf16(acc[0]) | ((uint32_t)nbk_f32_to_bf16(acc[1 % N]) << 16),
-                                     (uint32_t)nbk_f32_to_bf16(acc[2 % N]) | ((uint32_t)nbk_f32_to_bf16(acc[3 % N]) << 16));
+      ((uint2*)out)[to] = make_uint2((uint32_t)nbk_f32_to_bf16(sum[0]) | ((uint32_t)nbk_f32_to_bf16(sum[1 % N]) << 16),
+                                     (uint32_t)nbk_f32_to_bf16(sum[2 % N]) | ((uint32_t)nbk_f32_to_bf16(sum[3 % N]) << 16));
     } else {
 #pragma unroll
-      for (int e = 0; e < N; ++e) nbk_store_from_f32(out, to * N + e, dto, acc[e]);
+      for (int e = 0; e < N; ++e) nbk_store_from_f32(out, to * N + e, dto, sum[e]);
     }
     return;
   }
   for (int s = LX; s < 64; s <<= 1)  // rows that share a wavefront
 #pragma unroll
-    for (int e = 0; e < N; ++e) acc[e] = red_comb(acc[e], __shfl_xor(acc[e], s), kind);
+    for (int e = 0; e < N; ++e) sum[e] = red_comb(sum[e], __shfl_xor(sum[e], s), kind);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lanes = LX < 64 ? LX : 64, across = LX >> 6 ? LX >> 6 : 1;
   if (lane < lanes)
 #pragma unroll
-    for (int e = 0; e < N; ++e) part[wave * (64 * N) + lane * N + e] = acc[e];
+    for (int e = 0; e < N; ++e) part[wave * (64 * N) + lane * N + e] = sum[e];
   __syncthreads();
   const int cols = lanes * N;  // of one wavefront
   for (int c = threadIdx.x; c < across * cols; c += 256) {
@@ -276,6 +308,18 @@ __device__ __forceinline__ void reduce_strip_body(const void* __restrict__ in, v
     for (int k = across; k < 4; k += across) v = red_comb(v, p[k * (64 * N)], kind);
     nbk_store_from_f32(out, o * inner + col, dto, v);
   }
+}
+// (a function chosen anew for every number was two thirds of the instructions: us, 2 x (3287x2624) bf16 27.4 / 12.7,
+// 33 x (7479x56) 53 / 13.3, 42 x (105x4664) 16.6 / 11.0)
+template <typename P>
+__device__ __forceinline__ void reduce_strip_body(const void* __restrict__ in, void* __restrict__ out,
+                                                  int dti, int dto, int64_t red, int64_t inner, int kind,
+                                                  int64_t bx, int64_t o, int lxs, float* part) {
+#define REDUCE_KIND(K) reduce_strip_kind<P, K>(in, out, dti, dto, red, inner, bx, o, lxs, part)
+  if (kind == NBK_RED_SUM) REDUCE_KIND(NBK_RED_SUM);
+  else if (kind == NBK_RED_MAX) REDUCE_KIND(NBK_RED_MAX);
+  else REDUCE_KIND(NBK_RED_MIN);
+#undef REDUCE_KIND
 }
 // How a reduction is laid out, a function of its own shape alone: the order of summation, and so
 // the result, does not depend on how reductions are grouped into launches.
@@ -294,8 +338,10 @@ static RedLayout reduce_layout(const void* in, int dti, int64_t outer, int64_t r
   const bool aligned = ((uintptr_t)in & 15) == 0;
   L.mode = dti == NBK_BF16 ? (aligned && inner % 8 == 0 ? 1 : 3) : dti == NBK_F32 ? (aligned && inner % 4 == 0 ? 2 : 4) : 0;
   const int64_t pieces = inner / (L.mode == 1 ? 8 : L.mode == 2 ? 4 : 1);
+  // (by element, two rows abreast at least: sixteen chains with the eight of a lane)
+  const int widest = (L.mode == 1 || L.mode == 2 || red <= RED_FLIGHT) ? 8 : 7;
   int s = 0;
-  while (s < 8 && (1ll << s) < pieces) ++s;
+  while (s < widest && (1ll << s) < pieces) ++s;
   const int whole = L.mode == 1 || L.mode == 2 ? 4 : 5;  // 256 bytes of a row (fp32 by element: 128)
   // (a few long rows, the partial products of a GEMM split along K, are added in their order: a
   // strip of 256 is as fast there, 4 x 65536 2.1 us)

@@ -57,3 +57,23 @@ def test_one_order_of_additions(hip, dtype, outer, red, inner):
     lib.check(L.nbk_reduce_mid_batch(C.byref(task), 1, st))
     assert torch.equal(alone, batched)
     assert torch.equal(alone, alone[:1].expand(outer, inner))
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("outer,red,inner", [(64, 1024, 4099), (1024, 12, 1000), (8, 1000, 30011), (1030, 130, 1024),
+                                             (3, 2000, 20), (1, 4096, 64)])
+def test_long_axes_are_not_one_chain(hip, dtype, outer, red, inner):
+    """Sums of uniform numbers against float64.  A sum of n equal shares in one chain is rounded once a share, at
+    about half of its value on the average: sqrt(n) / 3 of 2^-24 of it.  In sixteen chains, or in two that take
+    four numbers at a time, the longest axis here keeps below 2^-23; one chain has 10 * 2^-24."""
+    from nabla_amd.backend import lib
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    code, tdt = TYPES[dtype]
+    x = torch.rand((outer, red, inner), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda").to(tdt)
+    out = torch.empty((outer, inner), device="cuda")
+    lib.check(lib.load().nbk_reduce_mid(C.c_void_p(x.data_ptr()), C.c_void_p(out.data_ptr()), code, 0, outer, red, inner, 0, st))
+    off = size = 0.0
+    for got, rows in zip(out, x):
+        want = rows.sum(0, dtype=torch.float64)
+        off, size = off + ((got - want) ** 2).sum(), size + (want ** 2).sum()
+    assert (off / size) ** 0.5 <= 2.0 ** -23
