@@ -220,7 +220,7 @@ __device__ __forceinline__ void reduce_strip_kind(const void* __restrict__ in, v
   const float ident = kind == NBK_RED_SUM ? 0.f : (kind == NBK_RED_MAX ? -INFINITY : INFINITY);
   // CHAINS sums of a lane's rows side by side, T rows at a time: where no rows stand abreast, one sum
   // would be rounded once a row.  Error against float64 of uniform numbers, one sum / these: 64 x (1024x4099)
-  // fp32 4.2e-7 / 5.0e-8, 1024 x (12x1000) 5.4e-8 / 4.0e-8.  (Less than eight rows are added in their order.)
+  // fp32 4.2e-7 / 5.0e-8, 1024 x (12x1000) 5.4e-8 / 4.0e-8.  (Up to eight rows are added in their order.)
   constexpr int CHAINS = N == 1 ? 8 : 2, T = RED_FLIGHT / CHAINS;
   static_assert(T == 1 || T == 4, "a sum of one row or of four");
   float acc[CHAINS][N];
@@ -241,16 +241,21 @@ __device__ __forceinline__ void reduce_strip_kind(const void* __restrict__ in, v
     typename P::raw u[RED_FLIGHT];
 #pragma unroll
     for (int q = 0; q < RED_FLIGHT; ++q) u[q] = P::load(in, i + q * step, dti);
+    if (N > 1 && red == RED_FLIGHT) {
 #pragma unroll
-    for (int c = 0; c < CHAINS; ++c) {
-      float v[T][N];
+      for (int q = 0; q < RED_FLIGHT; ++q) add(0, u[q]);
+    } else {
 #pragma unroll
-      for (int q = 0; q < T; ++q) P::unpack(u[c * T + q], dti, v[q]);
+      for (int c = 0; c < CHAINS; ++c) {
+        float v[T][N];
 #pragma unroll
-      for (int e = 0; e < N; ++e) {
-        float x = v[0][e];
-        if constexpr (T == 4) x = red_comb(red_comb(x, v[1][e], kind), red_comb(v[2][e], v[3][e], kind), kind);
-        acc[c][e] = red_comb(acc[c][e], x, kind);
+        for (int q = 0; q < T; ++q) P::unpack(u[c * T + q], dti, v[q]);
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+          float x = v[0][e];
+          if constexpr (T == 4) x = red_comb(red_comb(x, v[1][e], kind), red_comb(v[2][e], v[3][e], kind), kind);
+          acc[c][e] = red_comb(acc[c][e], x, kind);
+        }
       }
     }
   }
