@@ -627,6 +627,33 @@ __global__ __launch_bounds__(NWM * NWN * 64) void conv_split_kernel(const ConvAr
   }
 }
 
+// Results of one product each (the input gradient of one output channel and one tap, the filter gradient of one pixel):
+// rounded once, where the six products of the parts would be rounded together.  A wave has 16 rows, a lane a column.  us,
+// 64 x 32 x 32, 128 -> 1 channels: 8.2, out of parts 27 (its writes: 4.8).
+template <int MODE>
+__global__ __launch_bounds__(256) void conv_outer_kernel(const ConvArgs g) {
+  constexpr int ROWS = 16;
+  const int lane = threadIdx.x & 63;
+  const int64_t m0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * ROWS;
+  const float x = conv_load_a<MODE>(g, m0 + (lane & (ROWS - 1)), 0, 1);
+  for (int64_t n = lane; n - lane < g.Ng; n += 64) {
+    const float w = conv_load_b<MODE>(g, 0, n, 1);
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      const float xr = __shfl(x, r);
+      if (m0 + r < g.M && n < g.Ng) g.out[(m0 + r) * g.Ng + n] = xr * w;
+    }
+  }
+}
+template <int MODE>
+static int conv_launch_outer(ConvArgs& a, hipStream_t st) {
+  a.set_divisors();
+  const int64_t blocks = (a.M + 63) / 64;
+  NBK_REQUIRE(blocks <= 0x7fffffffLL, "conv2d: launch too large");
+  hipLaunchKernelGGL(conv_outer_kernel<MODE>, dim3((unsigned)blocks), dim3(256), 0, st, a);
+  return nbk_check_launch("conv_outer_kernel");
+}
+
 // out[i] = sum over z of partial[z][i].  Eight loads in flight are a trip to memory, and a lane that adds every
 // slice of a small filter by itself makes one trip behind the other on a few CUs; so ZG lanes share a sum,
 // each with every ZG-th slice, and meet in LDS.  The order of the additions is fixed: the result
@@ -723,6 +750,7 @@ static int conv_launch(ConvArgs& a, hipStream_t st) {
 // of 8 k are 8 pixels, whose gather costs more than the instruction saves (64 x 32 x 32, 64 -> 128 channels 139
 // us against 112).  Others gather number by number there, too (before the sum of slices took many lanes 3 -> 64 44 against 51).
 static int conv_launch_wgrad(ConvArgs& a, bool fast, hipStream_t st) {
+  if (a.K == 1) return conv_launch_outer<CONV_WGRAD>(a, st);
   a.set_divisors();
   if (a.M <= 32) {  // one block of 32 filter rows: faster at every size above
     const int64_t nb = a.Ng <= 32 ? 1 : 2, columns = (a.Ng + 32 * nb - 1) / (32 * nb);
@@ -789,6 +817,7 @@ extern "C" int nbk_conv2d_dgrad(const nbk_conv_desc* d, const void* dy, const vo
   a.a = (const float*)dy; a.b = (const float*)w; a.bias = nullptr; a.out = (float*)dx;
   a.M = d->N * d->H * d->W; a.Ng = d->Cin; a.K = d->R * d->S * d->Cout;
   a.splits = 1; a.k_per_split = (a.K + 15) / 16 * 16;
+  if (a.K == 1) return conv_launch_outer<CONV_DGRAD>(a, (hipStream_t)stream);
   return d->Cout % 8 == 0 ? conv_launch<CONV_DGRAD, true>(a, (hipStream_t)stream)
                           : conv_launch<CONV_DGRAD, false>(a, (hipStream_t)stream);
 }

@@ -2008,11 +2008,25 @@ __global__ __launch_bounds__(NWM * NWN * 64) void gemm_f32_split_kernel(const Ge
     return left;
   };
   static_assert(TM * TN * 4 <= 32, "a bit for each of a lane's results");
+  // (a contraction of one number is a product, rounded once: six rounded together are up to 0.78 of the last place off)
+  const bool one = K == 1;
   const uint32_t left = store([&](int i, int j, int r) { return acc.sum(i, j, r); },
-                              [](float s, uint32_t) { return fabsf(s) < INFINITY; });
+                              [&](float s, uint32_t) { return fabsf(s) < INFINITY && !one; });
   // (us, numbers that have parts / one infinity / NaN throughout: 1024 x 1024 x 1024 25 / 52 / 55, 4096 x 4096 x 1024
   // 193 / 336 / 585, where the float32 instruction alone takes 37 and 313; a lane at a time 1660 and 13700 at last)
-  if (__any(left != 0)) {
+  if (one) {
+    static_assert(WM <= 64, "a row for each lane");
+    const float x = A[min(m0 + wm + min(lane, WM - 1), g.M - 1) * g.a_rs];
+    float y[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) y[j] = B[min(n0 + wn + j * 16 + (lane & 15), g.N - 1) * g.b_cs];
+    float mine[TM][4];  // (shuffled here: the lanes past an edge leave `store`)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mine[i][r] = __shfl(x, i * 16 + (lane >> 4) * 4 + r);
+    store([&](int i, int j, int r) { return mine[i][r] * y[j]; }, [](float, uint32_t) { return true; });
+  } else if (__any(left != 0)) {
     const float* pa[TM];
     const float* pb[TN];
 #pragma unroll

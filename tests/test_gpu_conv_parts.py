@@ -48,6 +48,17 @@ def test_against_float64(hip, n, hw, cin, cout, r, pad, stride):
         assert (np.abs(a - c) <= (terms + 6) * 2.0 ** -24 * s + 2.0 ** -23 * np.abs(c)).all()
 
 
+@pytest.mark.parametrize("n,hw,cin", [(33, 32, 8), (32, 32, 128), (2, 9, 65)])
+def test_a_result_of_one_product_is_rounded_once(hip, n, hw, cin):
+    """Input gradients of one output channel and one tap; filter gradients of one pixel."""
+    rng = np.random.default_rng(cin)
+    x, g = (rng.standard_normal((n, hw, hw, c)).astype(np.float32) for c in (cin, 1))
+    w = rng.standard_normal((1, 1, cin, 1)).astype(np.float32)
+    np.testing.assert_array_equal(ours(x, w, g, 0, 1)[1], g * w[0, 0, :, 0])
+    x, w, g = (rng.standard_normal(s).astype(np.float32) for s in ((1, 1, 1, cin), (1, 1, cin, 37), (1, 1, 1, 37)))
+    np.testing.assert_array_equal(ours(x, w, g, 0, 1)[2][0, 0], x[0, 0, 0][:, None] * g[0, 0, 0])
+
+
 @pytest.mark.parametrize("n,hw,cin,cout", [(33, 32, 8, 32), (32, 32, 8, 128), (2, 9, 7, 65)])
 def test_small_numbers(hip, n, hw, cin, cout):
     """Images and cotangents of a few digits of the smallest float32 kind, filters as much larger."""

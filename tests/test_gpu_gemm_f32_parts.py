@@ -63,6 +63,17 @@ def test_numbers_of_every_size(hip, M, N, e, f):
         assert (np.abs(product(np.ascontiguousarray(x), np.ascontiguousarray(y), "nn") - want) <= tol).all()
 
 
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("M,N", [(1024, 1024), (2048, 2048), (1025, 897)])
+def test_a_contraction_of_one_number_is_rounded_once(hip, M, N, layout):
+    rng = np.random.default_rng(M)
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((M, 1), (1, N)))
+    np.testing.assert_array_equal(product(a, b, layout), a * b)
+    bias = rng.standard_normal(N).astype(np.float32)
+    bd = torch.tensor(bias).cuda()
+    np.testing.assert_array_equal(product(a, b, layout, bias=bd.data_ptr(), act=1), np.maximum(a * b + bias, 0))
+
+
 @pytest.mark.parametrize("M,N", [(1024, 1024), (2048, 2048)])
 def test_numbers_without_parts(hip, M, N):
     K = 70
