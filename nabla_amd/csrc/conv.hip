@@ -58,10 +58,11 @@ struct ConvArgs {
   int64_t M, Ng, K;
   int64_t k_per_split;  // multiple of 16
   int32_t tiles_m, tiles_n, splits;
-  ConvDiv by_cin, by_cout, by_s, by_w, by_h, by_wo, by_ho;
+  ConvDiv by_cin, by_cout, by_s, by_w, by_h, by_wo, by_ho, by_sh, by_sw;
   __host__ void set_divisors() {
     by_cin.set(d.Cin); by_cout.set(d.Cout); by_s.set(d.S);
     by_w.set(d.W); by_h.set(d.H); by_wo.set(d.Wo); by_ho.set(d.Ho);
+    by_sh.set(d.stride_h); by_sw.set(d.stride_w);
   }
 };
 
@@ -91,9 +92,10 @@ __device__ __forceinline__ float conv_load_a(const ConvArgs& g, int64_t m64, int
     const int t = g.by_w.divmod(m, w);
     const int n = g.by_h.divmod(t, h);
     const int hn = h + d.pad_t - r, wn = w + d.pad_l - s;
-    if (hn < 0 || wn < 0 || hn % d.stride_h != 0 || wn % d.stride_w != 0) return 0.f;
-    const int ho = hn / d.stride_h, wo = wn / d.stride_w;
-    if (ho >= Ho || wo >= Wo) return 0.f;
+    if (hn < 0 || wn < 0) return 0.f;
+    int between_h, between_w;
+    const int ho = g.by_sh.divmod(hn, between_h), wo = g.by_sw.divmod(wn, between_w);
+    if (between_h != 0 || between_w != 0 || ho >= Ho || wo >= Wo) return 0.f;
     return g.a[(int64_t)((n * Ho + ho) * Wo + wo) * Cout + co];
   } else {
     int c, s, wo, ho;
@@ -439,7 +441,8 @@ struct ConvRows {
     }
   }
   // Forward / dgrad: where channel `chan` of piece p's pixel lies at tap (r, s), and whether it is inside.
-  __device__ __forceinline__ bool where(const nbk_conv_desc& d, int p, int r, int s, int chan, int64_t& at) const {
+  __device__ __forceinline__ bool where(const ConvArgs& g, int p, int r, int s, int chan, int64_t& at) const {
+    const nbk_conv_desc& d = g.d;
     if (MODE == CONV_FWD) {
       const int h = q_h[p] + r, w = q_w[p] + s;
       at = (int64_t)(q_pix[p] + r * (int)d.W + s) * d.Cin + chan;
@@ -449,9 +452,10 @@ struct ConvRows {
     int ho = hn, wo = wn;
     bool in = hn >= 0 && wn >= 0;
     if (d.stride_h != 1 || d.stride_w != 1) {
-      ho = hn / d.stride_h;
-      wo = wn / d.stride_w;
-      in = in && ho * d.stride_h == hn && wo * d.stride_w == wn;
+      int between_h, between_w;
+      ho = g.by_sh.divmod(max(hn, 0), between_h);
+      wo = g.by_sw.divmod(max(wn, 0), between_w);
+      in = in && between_h == 0 && between_w == 0;
     }
     at = (int64_t)((q_pix[p] * (int)d.Ho + ho) * (int)d.Wo + wo) * d.Cout + chan;
     return in && ho < d.Ho && wo < d.Wo;
@@ -474,7 +478,7 @@ struct ConvRows {
           const int tap = (MODE == CONV_FWD ? g.by_cin : g.by_cout).divmod((int)k + e, chan);
           const int rr = g.by_s.divmod(tap, s);
           int64_t at;
-          const bool in = ok[p] && k + e < k_end && where(d, p, rr, s, chan, at);
+          const bool in = ok[p] && k + e < k_end && where(g, p, rr, s, chan, at);
           const float v = g.a[in ? at : 0];
           x[e] = in ? v : 0.f;
         }
@@ -499,7 +503,7 @@ struct ConvRows {
         if (!IS_A) {  // dgrad: w[r, s, j, co]
           at = ((int64_t)(t_r[p] * (int)d.S + t_s[p]) * d.Cin + m) * d.Cout + t_c[p];
         } else {
-          in = in && where(d, p, t_r[p], t_s[p], t_c[p], at);
+          in = in && where(g, p, t_r[p], t_s[p], t_c[p], at);
         }
         // (what lies outside reads the first numbers of the tensor: no branch around the request)
         const float* src = (IS_A ? g.a : g.b) + (in ? at : 0);
@@ -572,22 +576,36 @@ __global__ __launch_bounds__(NWM * NWN * 64) void conv_split_kernel(const ConvAr
     lb.template store<SET>(conv_lds + SET * TILE + BM * 12);               \
   } while (0)
 #define CONV_MULTIPLY(SET) acc.template multiply<BM, BN, SET>(conv_lds + SET * TILE, conv_lds + SET * TILE + BM * 12, wm, wn, lane)
+  // (one or two tiles without requests past the end: where every number has a tap of its own, one costs more than
+  // the tile's multiplication.  With conditions in the loop it became slower by up to half.)
   CONV_LOAD(0, 0);
-  CONV_LOAD(1, 1);  // (past the end: zeros)
-  CONV_STORE(0);
-  __syncthreads();
-  int kt = 0;
-  for (; kt + 1 < nk; kt += 2) {
-    CONV_LOAD(0, kt + 2);
-    CONV_MULTIPLY(0);
-    CONV_STORE(1);
-    __syncthreads();
-    CONV_LOAD(1, kt + 3);
-    CONV_MULTIPLY(1);
+  if (nk > 2) {
+    CONV_LOAD(1, 1);
     CONV_STORE(0);
     __syncthreads();
+    int kt = 0;
+    for (; kt + 1 < nk; kt += 2) {
+      CONV_LOAD(0, kt + 2);  // (past the end: zeros)
+      CONV_MULTIPLY(0);
+      CONV_STORE(1);
+      __syncthreads();
+      CONV_LOAD(1, kt + 3);
+      CONV_MULTIPLY(1);
+      CONV_STORE(0);
+      __syncthreads();
+    }
+    if (kt < nk) CONV_MULTIPLY(0);
+  } else {
+    if (nk == 2) CONV_LOAD(1, 1);
+    CONV_STORE(0);
+    __syncthreads();
+    CONV_MULTIPLY(0);
+    if (nk == 2) {
+      CONV_STORE(1);
+      __syncthreads();
+      CONV_MULTIPLY(1);
+    }
   }
-  if (kt < nk) CONV_MULTIPLY(0);
 #undef CONV_MULTIPLY
 #undef CONV_STORE
 #undef CONV_LOAD
@@ -734,7 +752,8 @@ static int conv_launch_tile(ConvArgs& a, hipStream_t st) {
 // x 16, 128 -> 256, 67 / 100, its input gradient (128 columns: 128 tiles) 108 / 80; 90 x 20 x 20, 56 -> 120 72 / 71.
 // Up to 32 channels of results, tiles of 128 x 32 from one per CU on: 50 x 28 x 28, 1 -> 24 9.1 against 11.0,
 // input gradient of 24 -> 40 23 against 29; below that 1 x 32 x 32, 16 -> 32 12.0 against 10.3.
-// (128 x 64 tiles: 5 % less than 64 x 64 at best.)
+// (128 x 64 tiles: 5 % less than 64 x 64 at best.)  Number by number, the gather is most of a forward tile, and two of 64
+// x 64 have no third beside them: 1.5 there (32 x 64 x 64, 12 -> 130 129 / 155).
 template <int MODE, bool FAST>
 static int conv_launch(ConvArgs& a, hipStream_t st) {
   a.set_divisors();
@@ -742,7 +761,7 @@ static int conv_launch(ConvArgs& a, hipStream_t st) {
   const int64_t t64 = ((a.M + 63) / 64) * ((a.Ng + 63) / 64);
   if (a.Ng <= 32 && m128 >= cus) return conv_launch_tile<MODE, FAST, 128, 32, 4, 1>(a, st);
   const int64_t rounds_128 = (m128 * ((a.Ng + 127) / 128) + cus - 1) / cus, rounds_64 = (t64 + 2 * cus - 1) / (2 * cus);
-  if (rounds_128 * 17 <= rounds_64 * 10) return conv_launch_tile<MODE, FAST, 128, 128, 2, 4>(a, st);
+  if (rounds_128 * (MODE == CONV_FWD && !FAST ? 15 : 17) <= rounds_64 * 10) return conv_launch_tile<MODE, FAST, 128, 128, 2, 4>(a, st);
   return conv_launch_tile<MODE, FAST, 64, 64, 2, 2>(a, st);
 }
 

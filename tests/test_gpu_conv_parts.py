@@ -88,6 +88,30 @@ def test_numbers_without_parts(hip, n, hw, cin, cout):
     assert (np.abs(got[ok] - want[ok]) <= 1e-5 * np.abs(want[ok])).all()
 
 
+def descriptor(n, hw, cin, cout, r):
+    from nabla_amd.backend import lib
+    d = lib.ConvDesc()
+    d.N, d.H, d.W, d.Cin, d.R, d.S, d.Cout, d.Ho, d.Wo = n, hw, hw, cin, r, r, cout, hw, hw
+    d.stride_h = d.stride_w = 1
+    d.pad_t = d.pad_b = d.pad_l = d.pad_r = r // 2
+    return d
+
+
+def test_few_output_channels_cost_no_more_than_eight(hip):
+    """Input gradients number by number, of one and two K tiles: with requests past the last tile those of four
+    channels took 1.6 times as long as those of eight."""
+    from nabla_amd.backend import lib
+    from test_gpu_gemm_f32_parts import seconds
+    st = lib.C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    times = []
+    for cout in (8, 3, 4):
+        d = descriptor(64, 32, 128, cout, 3)
+        y, w, x = (torch.ones(s, device="cuda") for s in ((64, 32, 32, cout), (3, 3, 128, cout), (64, 32, 32, 128)))
+        times.append(min(seconds(lambda: lib.check(lib.load().nbk_conv2d_dgrad(
+            lib.C.byref(d), *(lib.C.c_void_p(t.data_ptr()) for t in (y, w, x)), st))) for _ in range(3)))
+    assert max(times[1:]) <= 1.3 * times[0], times
+
+
 @pytest.mark.parametrize("cin,cout", [(64, 128), (20, 40)])
 def test_numbers_without_parts_cost_one_more_pass(hip, cin, cout):
     """Images of NaN throughout: every wave runs its tile again on the float32 instruction and gathers number by
