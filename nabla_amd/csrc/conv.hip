@@ -847,8 +847,12 @@ extern "C" int nbk_conv2d_dgrad(const nbk_conv_desc* d, const void* dy, const vo
 // K steps each.
 static void wgrad_split(const nbk_conv_desc* d, int* splits, int64_t* k_per_split) {
   const int64_t M = d->R * d->S * d->Cin, K = d->N * d->Ho * d->Wo;
-  const int64_t tiles = ((M + 127) / 128) * ((d->Cout + 127) / 128);
-  int64_t want = 2 * (int64_t)nbk_num_cus() / tiles;
+  // (conv_launch_wgrad's tiles: 64 x 64 out of bf16 parts.  Slices for tiles of 128 gave those up to four rounds of
+  // workgroups on short slices: us, 81 x 14 x 14, 140 -> 114 channels at stride 2 51 / 37, 16 x 28 x 28, 50 -> 50 38 / 29, 64 x
+  // 28 x 28, 30 -> 60 63 / 48.  A CU holds three: for two 41 / 30 / 54, for four 41 / 38 / 57)
+  const int64_t edge = M > 32 && (d->Cin % 8 != 0 || d->Cout % 8 != 0) ? 64 : 128;
+  const int64_t tiles = ((M + edge - 1) / edge) * ((d->Cout + edge - 1) / edge);
+  int64_t want = (edge == 64 ? 3 : 2) * (int64_t)nbk_num_cus() / tiles;
   const int64_t most = K / 64 > 0 ? K / 64 : 1;
   if (want > most) want = most;
   if (want < 1) want = 1;

@@ -112,6 +112,16 @@ def test_few_output_channels_cost_no_more_than_eight(hip):
     assert max(times[1:]) <= 1.3 * times[0], times
 
 
+@pytest.mark.parametrize("n,hw,cin,cout,r", [(81, 14, 140, 114, 3), (16, 28, 50, 50, 3), (64, 28, 30, 60, 3), (10, 30, 27, 237, 3)])
+def test_slices_of_odd_filter_gradients_are_one_round(hip, n, hw, cin, cout, r):
+    from nabla_amd.backend import lib
+    d = descriptor(n, hw, cin, cout, r)
+    rows = r * r * cin
+    slices = lib.load().nbk_conv2d_wgrad_workspace(lib.C.byref(d)) // (4 * rows * cout)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert 1 < slices and slices * -(-rows // 64) * -(-cout // 64) <= 3 * cus
+
+
 @pytest.mark.parametrize("cin,cout", [(64, 128), (20, 40)])
 def test_numbers_without_parts_cost_one_more_pass(hip, cin, cout):
     """Images of NaN throughout: every wave runs its tile again on the float32 instruction and gathers number by
