@@ -2441,12 +2441,15 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
   // is what a launch waits for, and four waves that share a fragment of 32 x 32 on the float32
   // instruction have the shorter one.  us, 32 x 32 / 64 x 64 out of parts: 1024 x 512 x 512 (128 tiles of 64)
   // 12.9 / 15.9, 512 x 2048 x 1024 (256) 34 / 27 and as x^T dy 40 / 27, 1024 x 1024 x 200 (256) 15.1 / 10.3.
+  // Tiles of 64 that are half padding are no more work than two of 32: 300 x (20 x 20 x 64) 4.8 / 7.4, 128 x (32 x 128 x
+  // 64) 5.1 / 6.9, 32 x 16384 x 1024 20 / 26, 64 x (16 x 224 x 704) 16.5 / 20; past two of 32 to a CU the two are even (8 x
+  // 32768 x 256 12.6 / 12.5, 64 x (40 x 224 x 704) 27 / 21).
   // 128 x 128 tiles run one to a CU, two of 64 x 64 do; a round of the former does the work of two of the
   // latter in 1.7 of one's time: 4096 x 4096 x 1024 (4 rounds / 8) 197 / 251, 4096 x 1024 x 64 (1 / 2) 12.4 /
   // 14.2, 64 x (333 x 333 x 64) (3 / 5) 33 / 29, 2048 x 1024 x 1024 (1 / 1) 44 / 39.
   auto tiles = [&](int64_t edge) { return ((d->M + edge - 1) / edge) * ((d->N + edge - 1) / edge) * d->batch; };
   const int64_t cus = nbk_num_cus(), t64 = tiles(64);
-  if (t64 * 4 < cus * 3) return launch_f32(a, akc, bkc, d->batch, st);
+  if (t64 * 4 < cus * 3 || tiles(32) <= 2 * cus) return launch_f32(a, akc, bkc, d->batch, st);
   const int64_t rounds_64 = (t64 + 2 * cus - 1) / (2 * cus), rounds_128 = (tiles(128) + cus - 1) / cus;
   if (rounds_128 * 17 <= rounds_64 * 10) return launch_f32_split<128, 128, 2, 4, 2>(a, akc, bkc, d->batch, st);
   return launch_f32_split<64, 64, 2, 2, 2>(a, akc, bkc, d->batch, st);
