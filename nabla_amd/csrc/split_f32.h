@@ -2,14 +2,16 @@
 //
 // A float32 is three bf16 exactly, x = x1 + x2 + x3 (8 bits of the significand each, by two
 // subtractions that are exact), and a product of two is
-//   x1 y1 + (x1 y2 + x2 y1) + (x1 y3 + x2 y2 + x3 y1) + what lies below 2^-25 of it:
-// six bf16 products, each exact in the instruction's float32 sums.  The bf16 instruction has sixteen
+//   x1 y1 + (x1 y2 + x2 y1) + (x1 y3 + x2 y2 + x3 y1) + what is at most 2^-24 of it:
+// (|x2| <= 2^-8 and |x3| <= 2^-17 of x, so x2 y3 + x3 y2 is up to 2^-24 together: 0.99 of that at x = y = 1 + 2^-8 - 2^-17.)
+// Six bf16 products, each exact in the instruction's float32 sums.  The bf16 instruction has sixteen
 // times the rate of the float32 one, so six of them take 0.38 of its time.
 //   The first product is summed apart from the five small ones, whose roundings are then 2^-8 of its
 // own, and one instruction adds 32 of a row's products where the float32 one adds two.  Error against
 // float64, relative 2-norm, of a row of K normal / uniform positive numbers: K = 1024 2.0e-7 / 1.6e-7, K
 // = 16384 8.2e-7 / 5.9e-7; the float32 instruction in one chain 5.9e-7 / 4.4e-7 and 2.2e-6 / 1.7e-6, in
-// four 2.9e-7 / 1.2e-7 and 1.2e-6 / 4.4e-7.  (All six in one accumulator: as the one chain.)
+// four 2.9e-7 / 1.2e-7 and 1.2e-6 / 4.4e-7.  (All six in one accumulator: as the one chain.)  K = 2 2.6e-8 against 3.1e-8;
+// K = 1 is one product and one rounding, 2.53e-8, where the parts have 2.60e-8: the kernels multiply it as it is.
 //   A number that is not finite, or rounds to infinity as a bf16, has no such parts and its sums come out
 // as NaN: a wave with a sum that is not finite runs its tile again on the float32 instruction (SplitAcc::again)
 // and stores those of it that the parts did not give.

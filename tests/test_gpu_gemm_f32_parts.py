@@ -29,7 +29,8 @@ def product(a, b, layout, alpha=1.0, **fields):
 
 
 # A sum is rounded once per K tile of 32 and accumulator (2^-24 of what has been summed, at most the sum of
-# magnitudes) and once in each of the five small products; what the six leave out is 2^-25 of a product.
+# magnitudes), the five small products as often at 2^-8 of their size, and three additions at the end; what the six
+# products leave out is up to 2^-24 of one.
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
 @pytest.mark.parametrize("M,N,K", [(1025, 769, 31), (897, 1024, 64), (1100, 1200, 65), (1024, 1000, 129),   # 64 x 64
                                    (2047, 2050, 95), (2100, 1990, 160), (4097, 1921, 33)])                 # 128 x 128
@@ -45,6 +46,17 @@ def test_against_float64(hip, layout, M, N, K):
     got = product(a, b, layout, alpha=0.5, bias=bd.data_ptr(), act=1)  # relu
     want = np.maximum(0.5 * want + bias, 0.0)
     assert (np.abs(got - want) <= tol + 2.0 ** -23 * (np.abs(want) + np.abs(bias))).all()
+
+
+@pytest.mark.parametrize("M,N", [(1024, 1024), (2048, 2048)])
+@pytest.mark.parametrize("x", [1 + 2.0 ** -8 - 2.0 ** -17, 1 - 2.0 ** -8 + 2.0 ** -17, 1 + 2.0 ** -9 + 2.0 ** -18])
+def test_numbers_whose_left_out_products_add_up(hip, M, N, x):
+    """All of one sign and size: x2 y3 + x3 y2 are 2^-24 of the first product, K times over."""
+    K = 96
+    a, b = np.full((M, K), x, np.float32), np.full((K, N), x, np.float32)
+    want = K * float(np.float32(x)) ** 2
+    tol = (-(-K // 32) + 4) * 2.0 ** -24 * want + 2.0 ** -23 * want
+    assert (np.abs(product(a, b, "nn") - want) <= tol).all()
 
 
 @pytest.mark.parametrize("M,N", [(1024, 1024), (2048, 2048)])
