@@ -1,6 +1,6 @@
-"""Every compiled row kernel at sizes, alignments and immediates it was not generated from, against the
-interpreter on the same inputs: rows shorter and longer than a lane's chunks, odd ones, operands that
-start at an odd element, up to four leading dimensions."""
+"""Every compiled row kernel, in every form that it has, at sizes, alignments and immediates it was not
+generated from, against the interpreter on the same inputs: rows shorter and longer than a lane's chunks, odd
+ones, operands that start at an odd element, up to four leading dimensions."""
 import ctypes as C
 
 import numpy as np
@@ -25,7 +25,7 @@ def test_against_the_interpreter(hip, programs, cols):
     st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
     compared = 0
     for a in programs:
-        if a["n_stage"] and cols > 4096:
+        if a["n_stage"] and cols > 4096:  # (longer than what the generic form stages: in test_every_form)
             a = dict(a, n_stage=0, operands=[type(o)(**{**vars(o), "stage_slot": -1}) for o in a["operands"]])
         rp = _program_record(a)
         dims = [3, 2, 5, 2][:rp.n_lead]
@@ -80,8 +80,114 @@ def test_against_the_interpreter(hip, programs, cols):
             scale = torch.where(w.isfinite(), w.abs(), 0).max()
             assert (same | ((g - w).abs() <= tol * torch.maximum(w.abs(), scale))).all(), name
             compared += 1
-        assert rows >= 1
     assert compared >= 30
+
+
+def form(a, generic, rp):
+    """What nbk_rowprog_launch runs of a kernel for a reduction program (the rule in rowprog.hip)."""
+    chunks = -(-rp.C // 4)
+    need = -(-chunks // rp.block)
+    cpt = next((c for c in (1, 2, 4, 8) if need <= c), 0)
+    if cpt in specialize.resident_variants(a):
+        if rp.C != 4 * cpt * rp.block:
+            return cpt, "masked"
+        rows = int(np.prod([rp.lead_dim[k] for k in range(rp.n_lead)]))
+        moved = sum(rows * rp.C * o.dtype.size_in_bytes for o in generic["operands"] if o.col_stride)
+        return cpt, "stream" if moved > 256 << 20 else "full"
+    if specialize.stage16_operand(generic) is not None and rp.n_stage == 0 and rp.C % 4 == 0:
+        return 0, "stage16"
+    return 0, "generic"
+
+
+def streams(generic):
+    """Whether rows enough for the streaming forms can be had."""
+    return bool(generic["lead"]) and any(o.col_stride for o in generic["operands"])
+
+
+def launches(a, generic):
+    """(row length, workgroup, whether to exceed the last-level cache) for every form of the kernel."""
+    cpts = specialize.resident_variants(a)
+    for cpt in cpts:
+        yield 4 * cpt * 64 - 8, 64, False
+        yield 4 * cpt * 64, 64, False
+        if streams(generic):
+            yield 4 * cpt * 256, 256, True
+    yield 4 * cpts[-1] * 64 + (8 if "approx_hash" in a else 5), 64, False  # (the generic form)
+    if specialize.stage16_operand(generic) is not None:
+        yield 4 * cpts[-1] * 64 + 8, 64, False
+
+
+def test_every_form(hip):
+    L = lib.load()
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    pool = torch.randn(80 << 20, generator=gen, device="cuda")
+    kernels = [k for k in specialize.kernels_of(specialize.collect_programs()) if k[2]["has_reduce"]]
+    assert len(kernels) >= 60
+    for _, name, a, generic in kernels:
+        ran = set()
+        # the kernels of one program alone are found by its alignment, too; the others start at an odd element
+        shift = 0 if "approx_hash" in a else 1
+        for cols, block, large in launches(a, generic):
+            rp = _program_record(generic)
+            rp.C, rp.block = cols, block
+            dims = [1] * rp.n_lead
+            if dims:
+                dims[0], dims[-1] = 2, dims[-1] * 5
+            if large:
+                per_row = sum(cols * o.dtype.size_in_bytes for o in generic["operands"] if o.col_stride)
+                dims[-1] = (256 << 20) // (per_row * int(np.prod(dims[:-1]))) + 3
+            for k, d in enumerate(dims):
+                rp.lead_dim[k] = d
+            written = {i[1] for i in a["ins"] if i[0] in (isa.STG, isa.STR)}
+            operands, outs = [], []
+            for i, o in enumerate(generic["operands"]):
+                od = rp.operand[i]
+                at, strides = (cols if o.col_stride else 1), []
+                for d, s in reversed(list(zip(dims, o.lead_strides))):
+                    strides.insert(0, at if s else 0)
+                    at *= d if s else 1
+                for k, s in enumerate(strides):
+                    od.lead_stride[k] = s
+                dt = o.dtype.to_torch()
+                if o.dtype.is_float():
+                    n = at + shift
+                    x = torch.cat([pool] * -(-n // pool.numel()))[:n].to(dt) if n > pool.numel() else pool[i * 3:n + i * 3].to(dt)
+                    if x.data_ptr() % 16 or x._base is not None or i in written:
+                        x = x.clone()
+                else:
+                    x = torch.randint(0, 2 if dt in (torch.bool, torch.uint8) else cols + 1, (at + shift,), generator=gen, device="cuda").to(dt)
+                operands.append(x)
+                od.ptr = x.data_ptr() + shift * x.element_size()
+                od.vec_ok = 0 if shift else int(o.vec_ok)
+                if i in written:
+                    outs.append(x)
+            results = []
+            for rp.reserved in (0, 1):
+                for x in outs:
+                    x.zero_()
+                assert rp.reserved or L.nbk_rowprog_is_specialized(C.byref(rp)) == (3 if "approx_hash" in a else 1), name
+                lib.check(L.nbk_rowprog_launch(C.byref(rp), st))
+                results.append([x.clone() for x in outs])
+            what = form(a, generic, rp)
+            ran.add(what)
+            for got, want in zip(*results):
+                where = f"{name} {what} C {cols} ({' '.join(a['members'])[:60]})"
+                if not got.dtype.is_floating_point:
+                    assert torch.equal(got, want), where
+                    continue
+                # (tolerances as above)
+                tol = (2.0 ** -7 if got.dtype == torch.bfloat16 else 2e-4 if any(
+                    o.dtype.to_torch() == torch.bfloat16 for o in a["operands"]) else 2e-5)
+                g, w = got.float(), want.float()
+                same = (g == w) | (g.isnan() & w.isnan())
+                scale = torch.where(w.isfinite(), w.abs(), 0).max()
+                assert (same | ((g - w).abs() <= tol * torch.maximum(w.abs(), scale))).all(), where
+        forms = {(c, f) for c in specialize.resident_variants(a) for f in ("masked", "full") + (("stream",) if streams(generic) else ())}
+        forms.add((0, "generic"))
+        if specialize.stage16_operand(generic) is not None:
+            forms.add((0, "stage16"))
+        assert ran == forms, name
 
 
 def test_functions_are_the_interpreters(hip, programs):
