@@ -1974,17 +1974,19 @@ class Planner:
             # apart: 1024 x 4096 x 8192 113 -> 82 us, plus 10 us for the sum of the halves (four
             # slices: 67 us and 25)
             return 2
-        # The partial products and their sum cost 6 to 10 us, and a split product carries no
+        # The partial products and their sum cost 4 to 10 us, and a split product carries no
         # epilogue.  What a launch on few workgroups waits for is its K loop, on 64 x 64 tiles while
         # there are at most two per CU.  Measured, us whole / in two / four / eight, the sum
-        # included, with eight products of one size in a step:
+        # included, eight products of one size behind each other as x^T dy.  (The lines were drawn when whole
+        # products had two tile buffers and took up to 1.8 times as long; with four, results of 144 to 256 tiles
+        # are as fast whole up to 4096, and the lines have not moved yet.)
         small = ((M + 63) // 64) * ((N + 63) // 64)
         if small > 256 and K < 8192:
-            return 1  # (1024 x 1536 x 2048 22 / 24 / 26, 1792 x 1024 x 4096 38 / 42 / 38 / 49)
+            return 1  # (1024 x 1536 x 2048 17.3 / 21.4 / 23.7, 1792 x 1024 x 4096 27 / 29 / 31 / 40)
         if small > 32 and K < 4096:
-            # Up to about 512 workgroups with slices of 512 and more: 512 x 512 x 2048 21.7 / 16.0 /
-            # 14.7 / 15.3, 512 x 512 x 3072 29 / 19 / 15 / 15, 768 x 768 x 2048 21.7 / 17.0 / 16.9 / 19.5,
-            # 1024 x 1024 x 2048 22.0 / 18.5 / 21.1; at 1024 the two are even (512 x 512 x 1024 15.3 / 15.1).
+            # Up to about 512 workgroups with slices of 512 and more: 512 x 512 x 2048 12.1 / 11.6 /
+            # 12.9 / 13.6, 512 x 512 x 3072 16.4 / 13.7 / 12.4 / 13.7, 768 x 768 x 2048 12.1 / 15.1 / 17.0 / 19.3,
+            # 1024 x 1024 x 2048 12.5 / 18.1 / 19.2; at 1024 whole (512 x 512 x 1024 8.3 / 11.0 / 10.8).
             # An epilogue of its own is another launch of 5 us, so one that can be folded keeps the
             # product whole up to 2048.
             if K <= (2048 if epilogue else 1024):
@@ -1993,9 +1995,9 @@ class Planner:
             while small * ks * 2 <= 576 and K // (ks * 2) >= 512 and (rows_contiguous or K % (ks * 2 * 64) == 0):
                 ks *= 2
             return ks
-        # Longer ones down to slices of 1024 (512 x 1024 x 4096 37 / 24 / 19 / 21, 1024 x 1024 x 6144
-        # 52 / 45 / 38 / 38), the longest and the smallest results to slices of 512 (512 x 512 x 4096
-        # 37 / 23 / 17 / 15, 256 x 256 x 4096 36 / 22 / 15 / 14, 1024 x 1024 x 8192 90 / 56 / 46 / 43).
+        # Longer ones down to slices of 1024 (512 x 1024 x 4096 19.7 / 15.8 / 15.9 / 19.3, 1024 x 1024 x 6144
+        # 28 / 26 / 29 / 34), the longest and the smallest results to slices of 512 (512 x 512 x 4096
+        # 20.4 / 15.6 / 13.4 / 15.3, 256 x 256 x 4096 19.2 / 14.5 / 11.0 / 11.2, 1024 x 1024 x 8192 41 / 37 / 35 / 40).
         least = 1024 if small > 64 and K < 8192 else 512
         ks = 1
         while tiles * ks < 512 and tiles < 128 and K // (ks * 2) >= least and \

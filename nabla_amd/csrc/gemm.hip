@@ -14,8 +14,8 @@
 // both operands row-contiguous) copies global memory straight into LDS
 // (global_load_lds_dwordx4); gemm_bf16_kernel takes every other shape through guarded loads and
 // registers.
-// fp32 path: v_mfma_f32_32x32x2f32 with a 128 x 128 x 16 tile, operands kept
-// k-major in LDS.
+// fp32 path: out of bf16 parts (split_f32.h) on tiles of 128 x 128 or 64 x 64, small results on
+// v_mfma_f32_32x32x2f32 with 32 x 32 a workgroup.
 #include "nbk_common.h"
 #include "split_f32.h"
 
