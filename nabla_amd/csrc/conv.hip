@@ -545,8 +545,14 @@ struct ConvRows {
   }
 };
 
-template <int MODE, bool FAST, int BM, int BN, int NWM, int NWN>
-__global__ __launch_bounds__(NWM * NWN * 64) void conv_split_kernel(const ConvArgs g) {
+// SHORT: contractions of up to SPLIT_SHORT tiles, without requests past the end.  us, in the loop / so: forward 83 x 32 x 32, 3 ->
+// 172 channels, 5 x 5 taps 85 / 59, 64 x 32 x 32, 3 -> 64 26 / 21.5, 32 x 64 x 64, 12 -> 130 (four tiles) 155 / 112, input gradients
+// 90 x 53 x 53, 78 -> 3 111 / 68; with channels in pieces of eight 64 x 32 x 32, 128 -> 16, one tap 12.2 / 10.7.
+constexpr int SPLIT_SHORT = 4;
+// (Three workgroups of 64 x 64 share a CU where the gather leaves the registers for it: input gradients 64 x 56 x 56, 36 ->
+// 100 459 us, with two 534.)
+template <int MODE, bool FAST, int BM, int BN, int NWM, int NWN, bool SHORT>
+__global__ __launch_bounds__(NWM * NWN * 64, BM == 64 && (MODE != CONV_FWD || FAST) ? 3 : 1) void conv_split_kernel(const ConvArgs g) {
   constexpr int NT = NWM * NWN * 64, WM = BM / NWM, WN = BN / NWN, TM = WM / 16, TN = WN / 16;
   constexpr int TILE = (BM + BN) * 12;
   extern __shared__ __align__(16) sp_u4 conv_lds[];
@@ -576,16 +582,38 @@ __global__ __launch_bounds__(NWM * NWN * 64) void conv_split_kernel(const ConvAr
     lb.template store<SET>(conv_lds + SET * TILE + BM * 12);               \
   } while (0)
 #define CONV_MULTIPLY(SET) acc.template multiply<BM, BN, SET>(conv_lds + SET * TILE, conv_lds + SET * TILE + BM * 12, wm, wn, lane)
-  // (one or two tiles without requests past the end: where every number has a tap of its own, one costs more than
-  // the tile's multiplication.  With conditions in the loop it became slower by up to half.)
+  // (past the end: zeros.  Where every number has a tap of its own, such a request costs more than a tile's
+  // multiplication; but with conditions in front of them the loop became slower by up to half.)
   CONV_LOAD(0, 0);
-  if (nk > 2) {
+  if constexpr (SHORT) {
+    if (nk > 1) CONV_LOAD(1, 1);
+    CONV_STORE(0);
+    __syncthreads();
+    if (nk > 2) CONV_LOAD(0, 2);
+    CONV_MULTIPLY(0);
+    if (nk > 1) {
+      CONV_STORE(1);
+      __syncthreads();
+      if (nk > 3) CONV_LOAD(1, 3);
+      CONV_MULTIPLY(1);
+    }
+    if (nk > 2) {
+      CONV_STORE(0);
+      __syncthreads();
+      CONV_MULTIPLY(0);
+    }
+    if (nk > 3) {
+      CONV_STORE(1);
+      __syncthreads();
+      CONV_MULTIPLY(1);
+    }
+  } else {
     CONV_LOAD(1, 1);
     CONV_STORE(0);
     __syncthreads();
     int kt = 0;
     for (; kt + 1 < nk; kt += 2) {
-      CONV_LOAD(0, kt + 2);  // (past the end: zeros)
+      CONV_LOAD(0, kt + 2);
       CONV_MULTIPLY(0);
       CONV_STORE(1);
       __syncthreads();
@@ -595,16 +623,6 @@ __global__ __launch_bounds__(NWM * NWN * 64) void conv_split_kernel(const ConvAr
       __syncthreads();
     }
     if (kt < nk) CONV_MULTIPLY(0);
-  } else {
-    if (nk == 2) CONV_LOAD(1, 1);
-    CONV_STORE(0);
-    __syncthreads();
-    CONV_MULTIPLY(0);
-    if (nk == 2) {
-      CONV_STORE(1);
-      __syncthreads();
-      CONV_MULTIPLY(1);
-    }
   }
 #undef CONV_MULTIPLY
 #undef CONV_STORE
@@ -731,14 +749,14 @@ static int conv_check(const nbk_conv_desc* d) {
 
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-template <int MODE, bool FAST, int BM, int BN, int NWM, int NWN>
+template <int MODE, bool FAST, int BM, int BN, int NWM, int NWN, bool SHORT = false>
 static int conv_launch_tile(ConvArgs& a, hipStream_t st) {
   a.tiles_m = (int)((a.M + BM - 1) / BM);
   a.tiles_n = (int)((a.Ng + BN - 1) / BN);
   const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n;
   NBK_REQUIRE(blocks <= 0x7fffffffLL, "conv2d: launch too large");
   const size_t lds = 2 * (size_t)(BM + BN) * 12 * 16;
-  auto kern = conv_split_kernel<MODE, FAST, BM, BN, NWM, NWN>;
+  auto kern = conv_split_kernel<MODE, FAST, BM, BN, NWM, NWN, SHORT>;
   static bool attr_set = false; /* idempotent, so a race only repeats the call */
   if (!attr_set) {
     NBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -753,16 +771,21 @@ static int conv_launch_tile(ConvArgs& a, hipStream_t st) {
 // Up to 32 channels of results, tiles of 128 x 32 from one per CU on: 50 x 28 x 28, 1 -> 24 9.1 against 11.0,
 // input gradient of 24 -> 40 23 against 29; below that 1 x 32 x 32, 16 -> 32 12.0 against 10.3.
 // (128 x 64 tiles: 5 % less than 64 x 64 at best.)  Number by number, the gather is most of a forward tile, and two of 64
-// x 64 have no third beside them: 1.5 there (32 x 64 x 64, 12 -> 130 129 / 155).
+// x 64 have no third beside them: 1.5 there (32 x 64 x 64, 12 -> 130 129 / 155 in the loop).
+template <int MODE, bool FAST, bool SHORT>
+static int conv_launch_length(ConvArgs& a, hipStream_t st) {
+  const int64_t cus = nbk_num_cus(), m128 = (a.M + 127) / 128;
+  const int64_t t64 = ((a.M + 63) / 64) * ((a.Ng + 63) / 64);
+  if (a.Ng <= 32 && m128 >= cus) return conv_launch_tile<MODE, FAST, 128, 32, 4, 1, SHORT>(a, st);
+  const int64_t rounds_128 = (m128 * ((a.Ng + 127) / 128) + cus - 1) / cus, rounds_64 = (t64 + 2 * cus - 1) / (2 * cus);
+  if (rounds_128 * (MODE == CONV_FWD && !FAST ? 15 : 17) <= rounds_64 * 10)
+    return conv_launch_tile<MODE, FAST, 128, 128, 2, 4, SHORT>(a, st);
+  return conv_launch_tile<MODE, FAST, 64, 64, 2, 2, SHORT>(a, st);
+}
 template <int MODE, bool FAST>
 static int conv_launch(ConvArgs& a, hipStream_t st) {
   a.set_divisors();
-  const int64_t cus = nbk_num_cus(), m128 = (a.M + 127) / 128;
-  const int64_t t64 = ((a.M + 63) / 64) * ((a.Ng + 63) / 64);
-  if (a.Ng <= 32 && m128 >= cus) return conv_launch_tile<MODE, FAST, 128, 32, 4, 1>(a, st);
-  const int64_t rounds_128 = (m128 * ((a.Ng + 127) / 128) + cus - 1) / cus, rounds_64 = (t64 + 2 * cus - 1) / (2 * cus);
-  if (rounds_128 * (MODE == CONV_FWD && !FAST ? 15 : 17) <= rounds_64 * 10) return conv_launch_tile<MODE, FAST, 128, 128, 2, 4>(a, st);
-  return conv_launch_tile<MODE, FAST, 64, 64, 2, 2>(a, st);
+  return a.K <= SPLIT_SHORT * SPLIT_BK ? conv_launch_length<MODE, FAST, true>(a, st) : conv_launch_length<MODE, FAST, false>(a, st);
 }
 
 // The filter gradient of channel counts that are multiples of 8 stays on the float32 instruction: its pieces
@@ -779,7 +802,9 @@ static int conv_launch_wgrad(ConvArgs& a, bool fast, hipStream_t st) {
     else hipLaunchKernelGGL((conv_wgrad_few_kernel<2>), grid, dim3(256), 0, st, a);
     return nbk_check_launch("conv_wgrad_few_kernel");
   }
-  if (!fast) return conv_launch_tile<CONV_WGRAD, true, 64, 64, 2, 2>(a, st);
+  if (!fast)
+    return a.k_per_split <= SPLIT_SHORT * SPLIT_BK ? conv_launch_tile<CONV_WGRAD, true, 64, 64, 2, 2, true>(a, st)
+                                                   : conv_launch_tile<CONV_WGRAD, true, 64, 64, 2, 2>(a, st);
   // the narrow workgroup tile when the last 128-wide column tile would be at most half full,
   // or when the wide tiling gives fewer workgroups than the GPU has CUs
   const int64_t wide = ((a.M + 127) / 128) * ((a.Ng + 127) / 128) * a.splits;

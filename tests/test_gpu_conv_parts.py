@@ -48,6 +48,20 @@ def test_against_float64(hip, n, hw, cin, cout, r, pad, stride):
         assert (np.abs(a - c) <= (terms + 6) * 2.0 ** -24 * s + 2.0 ** -23 * np.abs(c)).all()
 
 
+@pytest.mark.parametrize("n,hw", [(3, 7), (130, 16)])
+@pytest.mark.parametrize("cin,cout,r", [(33, 64, 1), (64, 33, 1), (65, 96, 1), (97, 72, 1), (128, 100, 1), (100, 128, 1),
+                                        (129, 136, 1), (136, 129, 1), (3, 37, 5), (11, 12, 3), (14, 15, 3)])
+def test_contractions_of_one_to_five_tiles(hip, n, hw, cin, cout, r):
+    """Those of up to four K tiles request no more than they have; filter gradients in short slices, too."""
+    rng = np.random.default_rng(cin)
+    x, g = (rng.standard_normal((n, hw, hw, c)).astype(np.float32) for c in (cin, cout))
+    w = rng.standard_normal((r, r, cin, cout)).astype(np.float32)
+    a, b = (r // 2, 1), (np.abs(x), np.abs(w), np.abs(g))
+    for got, want, size, terms in zip(ours(x, w, g, *a), reference(x, w, g, *a), reference(*b, *a),
+                                      (r * r * cin / 32, r * r * cout / 32, n * hw * hw / 2)):
+        assert (np.abs(got - want) <= (terms + 6) * 2.0 ** -24 * size + 2.0 ** -23 * np.abs(want)).all()
+
+
 @pytest.mark.parametrize("n,hw,cin", [(33, 32, 8), (32, 32, 128), (2, 9, 65)])
 def test_a_result_of_one_product_is_rounded_once(hip, n, hw, cin):
     """Input gradients of one output channel and one tap; filter gradients of one pixel."""
