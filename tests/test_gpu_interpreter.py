@@ -99,3 +99,38 @@ def test_elementwise_over_broadcast_and_transposed_operands(interpreted, shape):
     assert ((stored(out) - want).abs() <= 2e-6 * (1 + want.abs())).all()
     sure = want.abs() > 1e-4
     assert (torch.tensor(big.numpy())[sure] == (want > 0)[sure]).all()
+
+
+@pytest.mark.parametrize("cols", [255, 256, 257, 262, 511, 512, 513, 519, 2046, 4095, 4096])
+@pytest.mark.parametrize("live", [3, 12])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_one_and_two_chunks_a_lane(interpreted, cols, live, dtype):
+    """Up to 64 chunks a lane holds one, from there on two if the program has at most eight vectors alive at a
+    time.  Whole numbers below 256: exact in both types."""
+    rows = 70
+    rng = np.random.default_rng(cols + live)
+    xs = [rng.integers(-3, 4, (rows, cols)).astype(np.float32) for _ in range(live)]
+
+    def f(*xs):
+        total = xs[0]
+        for i, x in enumerate(xs[1:]):
+            total = total + x if i % 2 else total - x
+        top = nb.reduce_max(total, axis=1, keepdims=True)
+        low = nb.reduce_min(total, axis=1, keepdims=True)
+        out = top - total
+        for x in xs:
+            out = out + (x - nb.relu(x)) * nb.where(x > low, x, low * 0.0)
+        return out, top, low
+
+    got = f(*(tensor(x, dtype) for x in xs))
+    nb.realize_all(*got)
+    total = xs[0].copy()
+    for i, x in enumerate(xs[1:]):
+        total = total + x if i % 2 else total - x
+    top, low = total.max(1, keepdims=True), total.min(1, keepdims=True)
+    out = top - total
+    for x in xs:
+        out = out + np.minimum(x, 0) * np.where(x > low, x, 0)
+    assert np.abs(out).max() < 256
+    for g, w in zip(got, (out, top, low)):
+        np.testing.assert_array_equal(stored(g).numpy(), w)
