@@ -1640,22 +1640,26 @@ using f32_piece = float __attribute__((ext_vector_type(N)));
 template <int N>
 using f32_piece_any = float __attribute__((ext_vector_type(N), aligned(4)));
 __device__ __forceinline__ int f32_at(int row, int chunk, int ld) { return row * ld + (chunk ^ (row >> 4 & 3)) * 4; }
-template <int ROWS, int BK, bool KC>
+template <int ROWS, int BK, bool KC, int NT>
 struct F32Rows {
   static constexpr int LD = BK + 4;
   static constexpr int RB = 2;  // row-contiguous operand: blocks of RB rows x 2 k
   static constexpr int V = KC ? 4 : RB, Q = KC ? 1 : 2;  // a piece: Q accesses of V floats
   static constexpr int PAD = KC ? 0 : V - 1;  // LDS rows in front of the tile (place)
-  static constexpr int PIECES = ROWS * BK / 256 / (V * Q);
+  static constexpr int PIECES = ROWS * BK / NT / (V * Q);
   static_assert(PIECES >= 1, "at least one piece per lane");
   f32_piece<V> r[2][PIECES][Q];  // two K tiles in flight
+  // Where the pieces of the next K tile begin: worked out once (a product of 64 bits per request and
+  // tile was a tenth of the kernel: 128 x 256 x 784 11.3 us, then 10.7).
+  const float* at[PIECES];
+  int64_t stride;
 
   // Where a piece lies in the tile.  The pieces of a row-contiguous operand past its end lie where its
   // last one does, which ends with the last row (and may begin before the tile): the edge of a
   // result is loaded like the rest of it.  Element by element, the workgroups there took half as long
   // again as the others: 79 x 150 x 1188 as x^T dy 29.0 us, 16.5 now, 576 x 248 x 2608 54.0 -> 29.9.
   __device__ static __forceinline__ void place(int p, int64_t left, bool whole, int& row, int& kk) {
-    const int idx = (int)threadIdx.x + 256 * p;
+    const int idx = (int)threadIdx.x + NT * p;
     if constexpr (KC) {
       row = idx / (BK / 4);
       kk = idx % (BK / 4) * 4;
@@ -1667,25 +1671,33 @@ struct F32Rows {
   }
   // Whether the operand has rows for a whole piece.
   __device__ static __forceinline__ bool pieces(int64_t rows) { return KC || rows >= V; }
-  // A K tile that lies inside K, in whole pieces.  `stride`: between rows (KC) or between k
-  // (row-contiguous).  Rows past the end repeat the last one or are left as they are in LDS (their results
-  // are not stored).
-  template <int SET>
-  __device__ __forceinline__ void load(const float* P, int64_t stride, int64_t row0, int64_t rows, int64_t k0) {
+  // `stride`: between rows (KC) or between k (row-contiguous).  Rows past the end repeat the last one or
+  // are left as they are in LDS (their results are not stored).
+  __device__ __forceinline__ void init(const float* P, int64_t stride_, int64_t row0, int64_t rows) {
+    stride = stride_;
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
       int row, kk;
-      place(p, rows - row0, true, row, kk);
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        const float* src = KC ? P + min(row0 + row, rows - 1) * stride + k0 + kk : P + (k0 + kk + q) * stride + row0 + row;
-        r[SET][p][q] = *(const f32_piece_any<V>*)src;
-      }
+      place(p, rows - row0, pieces(rows), row, kk);
+      at[p] = KC ? P + min(row0 + row, rows - 1) * stride + kk : P + kk * stride + row0 + row;
     }
   }
-  // Any other K tile, element by element; k past the end reads as zero.
+  __device__ __forceinline__ void next() {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) at[p] += KC ? (int64_t)BK : BK * stride;
+  }
+  // A K tile that lies inside K, in whole pieces.
   template <int SET>
-  __device__ __forceinline__ void load_each(const float* P, int64_t stride, int64_t row0, int64_t rows, int64_t k0, int64_t K) {
+  __device__ __forceinline__ void load() {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p)
+#pragma unroll
+      for (int q = 0; q < Q; ++q) r[SET][p][q] = *(const f32_piece_any<V>*)(KC || q == 0 ? at[p] : at[p] + stride);
+    next();
+  }
+  // Any other K tile, element by element, `left` k before the end; k past it reads as zero.
+  template <int SET>
+  __device__ __forceinline__ void load_each(int64_t row0, int64_t rows, int64_t left) {
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
       int row, kk;
@@ -1694,10 +1706,12 @@ struct F32Rows {
       for (int q = 0; q < Q; ++q)
 #pragma unroll
         for (int e = 0; e < V; ++e) {
-          const int64_t k = k0 + kk + (KC ? e : q), m = min(row0 + row + (KC ? 0 : e), rows - 1);
-          r[SET][p][q][e] = k < K ? P[KC ? m * stride + k : k * stride + m] : 0.f;
+          const int64_t over = KC ? 0 : min(row0 + row + e, rows - 1) - (row0 + row);  // (past the last row: the last)
+          const float* src = KC ? at[p] + e : at[p] + q * stride + over;
+          r[SET][p][q][e] = kk + (KC ? e : q) < left ? *src : 0.f;
         }
     }
+    next();
   }
   template <int SET>
   __device__ __forceinline__ void store(float* S, int64_t row0, int64_t rows) {
@@ -1720,22 +1734,25 @@ struct F32Rows {
   }
 };
 
-// Small results: a workgroup of four waves owns a tile of 32 x 32 and splits every K tile of 64 (two steps of
-// 8 each); their sums meet in LDS at the end.  Bound by the length of a workgroup's K loop: two K tiles
-// are requested ahead, one workgroup's 8 instructions a wave and tile are shorter than a trip to memory.
-// Lane l of a v_mfma_f32_32x32x2f32 supplies A[row l % 32][k = l / 32] and B[k = l / 32][col l % 32];
-// which two k values share an instruction is free as long as A and B agree, so the lane with half
-// h = l / 32 owns k = 8 s + 4 h .. + 3 of step s and issues four instructions per step.  us: 1024 x 512 x 512
-// 12.9, 32 x (256 x 64 x 256) 9.6, 128 x 256 x 784 11.2.  Two workgroups have to fit a CU (four waves
-// each: the second launch bound); with no row-contiguous operand that costs two to five per cent more on
-// contractions of 64 to 512: no bound there.
-template <bool A_KC, bool B_KC>
-__global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(const GemmArgs g) {
-  constexpr int BM = 32, BN = 32, WK = 4, KS = 2, BK = 8 * KS * WK, LD = BK + 4;
-  constexpr int A0 = F32Rows<BM, BK, A_KC>::PAD * LD, B0 = A0 + (BM + F32Rows<BN, BK, B_KC>::PAD) * LD;
+// Small results: a workgroup of WK waves owns a tile of T x T (32 or 16) and splits every K tile of 16 WK; their sums
+// meet in LDS at the end.  Bound by the length of a workgroup's K loop: two K tiles are requested ahead.
+// Lane l of a v_mfma_f32_32x32x2f32 supplies A[row l % 32][k = l / 32] and B[k = l / 32][col l % 32] (of a
+// 16x16x4f32: l % 16, l / 16); which k values share an instruction is free as long as A and B agree, so the lane
+// with part h = l / T owns four consecutive k of a step and issues four instructions.  Where which form
+// runs, and the times: nbk_gemm.  Two workgroups of up to eight waves have to fit a CU (the second launch
+// bound); four waves with no row-contiguous operand are two to five per cent faster without.
+template <bool A_KC, bool B_KC, int T, int WK>
+__global__ __launch_bounds__(64 * WK, WK > 8 || (WK == 4 && A_KC && B_KC) ? 1 : 2) void gemm_f32_kernel(const GemmArgs g) {
+  constexpr int BM = T, BN = T, KS = T / 16, BK = 16 * WK, LD = BK + 4;  // (a step: 8 or 16 k, in four instructions)
+  constexpr int R = T * T / 64;                                           // results of a lane
+  typedef float acc_t __attribute__((ext_vector_type(R)));
+  typedef F32Rows<BM, BK, A_KC, 64 * WK> RowsA;
+  typedef F32Rows<BN, BK, B_KC, 64 * WK> RowsB;
+  constexpr int A0 = RowsA::PAD * LD, B0 = A0 + (BM + RowsB::PAD) * LD;
   constexpr int SET = B0 + BN * LD;  // (two of them)
-  __shared__ __align__(16) float lds[2 * SET];
-  static_assert(4 * 16 * 64 <= 2 * SET, "the partial sums fit");
+  extern __shared__ __align__(16) u32x4 gemm_lds[];
+  float* lds = (float*)gemm_lds;
+  static_assert(WK * R * 64 <= 2 * SET, "the partial sums fit");
   int tm_i, tn_i;
   gemm_tile_coords(blockIdx.x, g.tiles_m, g.tiles_n, tm_i, tn_i);
   const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
@@ -1745,24 +1762,26 @@ __global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(con
   const int64_t c_off = bo * g.c_bs + bi * g.c_bs2;
   const int64_t K = gemm_slice_k(g, bo, bi);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int li = lane & 31, h = lane >> 5;
+  const int li = lane % T, h = lane / T;
   const int64_t a_stride = A_KC ? g.a_rs : g.a_cs, b_stride = B_KC ? g.b_cs : g.b_rs;
 
-  f32x16 acc = (f32x16)(0.f);
+  acc_t acc = (acc_t)(0.f);
 
-  F32Rows<BM, BK, A_KC> la;
-  F32Rows<BN, BK, B_KC> lb;
+  RowsA la;
+  RowsB lb;
   const int64_t nk = (K + BK - 1) / BK;
   const bool pieces = la.pieces(g.M) && lb.pieces(g.N);
   // (one branch for both operands: with a branch each, the second one's requests wait for the
   // data of the first, 576 x 256 x 2608 40 us instead of 31)
-  auto load = [&](auto set, int64_t kt) {
+  la.init(A, a_stride, m0, g.M);
+  lb.init(B, b_stride, n0, g.N);
+  auto load = [&](auto set, int64_t kt) {  // (tile after tile)
     if (pieces && (kt + 1) * BK <= K) {
-      la.template load<set.value>(A, a_stride, m0, g.M, kt * BK);
-      lb.template load<set.value>(B, b_stride, n0, g.N, kt * BK);
+      la.template load<set.value>();
+      lb.template load<set.value>();
     } else {
-      la.template load_each<set.value>(A, a_stride, m0, g.M, kt * BK, K);
-      lb.template load_each<set.value>(B, b_stride, n0, g.N, kt * BK, K);
+      la.template load_each<set.value>(m0, g.M, K - kt * BK);
+      lb.template load_each<set.value>(n0, g.N, K - kt * BK);
     }
   };
   auto store = [&](auto set) {
@@ -1776,10 +1795,13 @@ __global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(con
     const float* Bs = lds + cur.value * SET + B0;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      const f32x4 fa = *(const f32x4*)(As + f32_at(li, (wave * KS + s) * 2 + h, LD));
-      const f32x4 fb = *(const f32x4*)(Bs + f32_at(li, (wave * KS + s) * 2 + h, LD));
+      const f32x4 fa = *(const f32x4*)(As + f32_at(li, (wave * KS + s) * (64 / T) + h, LD));
+      const f32x4 fb = *(const f32x4*)(Bs + f32_at(li, (wave * KS + s) * (64 / T) + h, LD));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], acc, 0, 0, 0);
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (T == 32) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], acc, 0, 0, 0);
+        else acc = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], fb[e], acc, 0, 0, 0);
+      }
     }
     if (kt + 1 < nk) store(next);
     __syncthreads();
@@ -1795,7 +1817,7 @@ __global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(con
     if (kt + 1 < nk) tile(s1, s0, kt + 1);
   }
 
-  // D register r of lane (col li, half h) is row (r / 4) * 8 + h * 4 + r % 4
+  // D register r of lane (col li, part h) is row (r / 4) * 8 + h * 4 + r % 4
   float* C = (float*)g.C;
   auto put = [&](int r, float sum) {
     const int64_t row = m0 + (r >> 2) * 8 + h * 4 + (r & 3), col = n0 + li;
@@ -1815,14 +1837,27 @@ __global__ __launch_bounds__(256, A_KC && B_KC ? 1 : 2) void gemm_f32_kernel(con
   };
   // (every read of the last K tile lies before its barrier) each wave sums its share of the registers
 #pragma unroll
-  for (int r = 0; r < 16; ++r) lds[(wave * 16 + r) * 64 + lane] = acc[r];
+  for (int r = 0; r < R; ++r) lds[(wave * R + r) * 64 + lane] = acc[r];
   __syncthreads();
   const float* part = lds + lane;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int r = wave * 4 + q;
-    put(r, (part[r * 64] + part[(16 + r) * 64]) + (part[(32 + r) * 64] + part[(48 + r) * 64]));
+  for (int q = 0; q < (R + WK - 1) / WK; ++q) {
+    const int r = q * WK + wave;
+    if (r >= R) break;
+    float sum[WK];
+#pragma unroll
+    for (int w = 0; w < WK; ++w) sum[w] = part[(w * R + r) * 64];
+#pragma unroll
+    for (int n = WK / 2; n > 0; n /= 2)
+#pragma unroll
+      for (int w = 0; w < n; ++w) sum[w] = sum[2 * w] + sum[2 * w + 1];
+    put(r, sum[0]);
   }
+}
+// LDS of a workgroup of gemm_f32_kernel: two K tiles, each with rows in front of a row-contiguous operand.
+template <bool A_KC, bool B_KC, int T, int WK>
+constexpr size_t gemm_f32_lds() {
+  return 2 * (size_t)(2 * T + !A_KC + !B_KC) * (16 * WK + 4) * sizeof(float);
 }
 
 // --------------------------------------------------------------- fp32 out of bf16 parts
@@ -2143,17 +2178,30 @@ static int launch_bf16_dl_colsum(const GemmArgs& a, int64_t batch, hipStream_t s
   return nbk_check_launch("gemm_bf16_dl_kernel (column sums)");
 }
 
+template <int T, int WK>
 static int launch_f32(const GemmArgs& args, bool akc, bool bkc, int64_t batch, hipStream_t st) {
   GemmArgs a = args;
-  const int64_t tiles_m = (a.M + 31) / 32, tiles_n = (a.N + 31) / 32;
+  const int64_t tiles_m = (a.M + T - 1) / T, tiles_n = (a.N + T - 1) / T;
   NBK_REQUIRE(tiles_m * tiles_n <= 0x7fffffffLL, "gemm: launch too large");
   a.tiles_m = (int)tiles_m;
   a.tiles_n = (int)tiles_n;
   const dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch);
-  if (akc && bkc) hipLaunchKernelGGL((gemm_f32_kernel<true, true>), grid, dim3(256), 0, st, a);
-  else if (akc) hipLaunchKernelGGL((gemm_f32_kernel<true, false>), grid, dim3(256), 0, st, a);
-  else if (bkc) hipLaunchKernelGGL((gemm_f32_kernel<false, true>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((gemm_f32_kernel<false, false>), grid, dim3(256), 0, st, a);
+#define NBK_LAUNCH_F32(AK, BK_)                                                                              \
+  do {                                                                                                       \
+    auto kern = gemm_f32_kernel<AK, BK_, T, WK>;                                                             \
+    constexpr size_t lds = gemm_f32_lds<AK, BK_, T, WK>();                                                   \
+    static bool attr_set = false; /* idempotent, so a race only repeats the call */                          \
+    if (!attr_set) {                                                                                         \
+      NBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
+      attr_set = true;                                                                                       \
+    }                                                                                                        \
+    hipLaunchKernelGGL(kern, grid, dim3(64 * WK), lds, st, a);                                               \
+  } while (0)
+  if (akc && bkc) NBK_LAUNCH_F32(true, true);
+  else if (akc) NBK_LAUNCH_F32(true, false);
+  else if (bkc) NBK_LAUNCH_F32(false, true);
+  else NBK_LAUNCH_F32(false, false);
+#undef NBK_LAUNCH_F32
   return nbk_check_launch("gemm_f32_kernel");
 }
 
@@ -2449,7 +2497,23 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
   // 14.2, 64 x (333 x 333 x 64) (3 / 5) 33 / 29, 2048 x 1024 x 1024 (1 / 1) 44 / 39.
   auto tiles = [&](int64_t edge) { return ((d->M + edge - 1) / edge) * ((d->N + edge - 1) / edge) * d->batch; };
   const int64_t cus = nbk_num_cus(), t64 = tiles(64);
-  if (t64 * 4 < cus * 3 || tiles(32) <= 2 * cus) return launch_f32(a, akc, bkc, d->batch, st);
+  const int64_t t32 = tiles(32);
+  if (t64 * 4 < cus * 3 || t32 <= 2 * cus) {
+    // The float32 instruction does 256 operations a cycle and CU, so a tile's K loop on one CU is bound by it:
+    // tiles of 16 x 16 while two to a CU hold the result spread it over four times as many.  us, tiles of 32
+    // by four waves / 16 by eight: 128 x 256 x 784 (128 tiles of 16) 10.8 / 6.1, 300 x 300 x 300 (361) 7.0 / 5.6,
+    // 2048 x 64 x 1024 (512) 12.2 / 8.2, 784 x 256 x 128 (784) 4.8 / 5.8; the longest contractions by sixteen waves:
+    // 128 x 128 x 4096 36.7 / 15.6 / 13.3.  Tiles of 32 by eight waves, where a CU holds all its workgroups and
+    // a K tile of 128 is filled: 512 x 512 x 1024 (256 tiles) 12.0 / 10.8, 1024 x 512 x 2048 (512) 32.1 / 31.1 (K-contiguous
+    // 28.9 / 26.5); 64 x (96 x 64 x 96) (384) 6.2 / 6.9, 16 x (300 x 64 x 300) (320) 9.0 / 9.4.
+    const int64_t t16 = tiles(16);
+    if (t16 <= 2 * cus)
+      return t16 <= cus && d->K >= 2048 ? launch_f32<16, 16>(a, akc, bkc, d->batch, st)
+                                        : launch_f32<16, 8>(a, akc, bkc, d->batch, st);
+    if (d->K >= 128 && (t32 <= cus || (t32 <= 2 * cus && d->K % 128 == 0)))
+      return launch_f32<32, 8>(a, akc, bkc, d->batch, st);
+    return launch_f32<32, 4>(a, akc, bkc, d->batch, st);
+  }
   const int64_t rounds_64 = (t64 + 2 * cus - 1) / (2 * cus), rounds_128 = (tiles(128) + cus - 1) / cus;
   if (rounds_128 * 17 <= rounds_64 * 10) return launch_f32_split<128, 128, 2, 4, 2>(a, akc, bkc, d->batch, st);
   return launch_f32_split<64, 64, 2, 2, 2>(a, akc, bkc, d->batch, st);
