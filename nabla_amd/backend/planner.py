@@ -1963,8 +1963,12 @@ class Planner:
         ``epilogue``: what follows the product could be folded into it if it stays whole."""
         if dtype is not DType.bfloat16:
             return 1
-        if a_k_contiguous and N <= 32 and M >= 1024 and K % 64 == 0:
-            return 1  # tall products with a few columns have a kernel that splits K by itself
+        if a_k_contiguous and N <= 32 and M >= 16 and K % 64 == 0 and K * (1 if N <= 16 else 2) <= 2048:
+            # Products with a few columns have a kernel that splits K by itself.  Each of its workgroups
+            # reads all of B, which decides where it ends; us, whole / in the slices below and their sum:
+            # 1000 x 8 x 1024 6.5 / 8.7, 8192 x 16 x 2048 10.7 / 11.2, 1000 x 32 x 1024 7.7 / 8.8; 2000 x 32 x 2048
+            # 12.1 / 9.0, 1500 x 16 x 4096 20.2 / 8.9.
+            return 1
         tiles = ((M + 127) // 128) * ((N + 127) // 128)
         if rows_contiguous and 128 <= tiles <= 256 and K >= 4096:
             # x^T dy with one workgroup per CU at most: every workgroup walks the same rows of

@@ -2315,7 +2315,9 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
   // (checked before any kernel is chosen: no path may take the product and drop the sums)
   NBK_REQUIRE(d->colsum == nullptr || (d->dtype_ab == NBK_BF16 && !akc && !bkc),
               "gemm: column sums need bf16 operands that are both row-contiguous (a_rs == b_cs == 1)");
-  if (!tail && d->k_last == 0 && d->dtype_ab == NBK_BF16 && d->N <= 32 && d->M >= 1024 && d->K >= 256 && d->K % 64 == 0 &&
+  // (few rows too, where a workgroup's share of B is small: 1000 x 8 x 1024 6.5 us, in two slices and their sum 8.7)
+  const bool tall = d->M >= 1024 || (d->M >= 16 && d->K * (d->N <= 16 ? 1 : 2) <= 2048);
+  if (!tail && d->k_last == 0 && d->dtype_ab == NBK_BF16 && d->N <= 32 && tall && d->K >= 256 && d->K % 64 == 0 &&
       akc && a.a_vec && d->batch == 1 && d->bias == nullptr && d->residual == nullptr &&
       d->act == NBK_ACT_NONE && (bkc ? (bool)a.b_vec : (d->b_cs == 1 && d->N % 8 == 0 && a.b_vec))) {
     // 32 rows per workgroup, K split over its eight waves
