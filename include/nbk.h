@@ -310,6 +310,12 @@ typedef struct nbk_gemm_desc {
   nbk_gemm_term term[NBK_GEMM_MAX_TERMS];
 } nbk_gemm_desc;
 int nbk_gemm(const nbk_gemm_desc* d, void* stream);
+/* 2 to 4 products of one A in one launch (the projections of a layer to queries, keys and values:
+ * nabla/nn/functional/layers.py): product i has B[i], bias[i] (NULL: none) and C[i]; sizes, strides, dtypes, alpha
+ * and act are d's and the same for all (d->B, d->bias and d->C are not read).  batch 1, no residual, second
+ * result, column sums, further operand pairs or k_last, and the C lie a multiple of 16 bytes apart. */
+int nbk_gemm_members(const nbk_gemm_desc* d, int32_t n, const void* const* B, const void* const* bias,
+                     void* const* C, void* stream);
 
 /* C = alpha * A @ W or alpha * A @ W^T for a weight W [w_rows, w_cols] that is stored NF4-coded
  * as quantize_nf4 leaves it (nabla/nn/finetune/qlora.py:41-75): `codes`, one uint8 per weight in

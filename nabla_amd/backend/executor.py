@@ -196,7 +196,22 @@ class BoundPlan:
                     t.K = term["K"]
                     t.a_rs, t.a_cs, t.b_rs, t.b_cs = term["a_rs"], term["a_cs"], term["b_rs"], term["b_cs"]
                     d.n_terms = ti + 1
-                self.calls.append((L.nbk_gemm, [C.byref(d)], patches, d))
+                if a.get("members"):
+                    # (three arrays of pointers in one struct, whose fields can be patched by name)
+                    ptrs = lib.GemmMembers()
+                    for mi, m in enumerate(a["members"]):
+                        for field, ref in (("B", m["b"]), ("bias", m["bias"]), ("C", m["dst"])):
+                            if ref is None:
+                                continue
+                            if ref.dtype is not rc.dtype:
+                                raise TypeError(f"matmul member {mi}: its {field} is {ref.dtype}, the result {rc.dtype}")
+                            ptr_field(ptrs, f"{field}{mi}", ref.buf, ref.offset * ref.dtype.size_in_bytes)
+                    self.calls.append((L.nbk_gemm_members, [
+                        C.byref(d), len(a["members"]), C.byref(ptrs, lib.GemmMembers.B0.offset),
+                        C.byref(ptrs, lib.GemmMembers.bias0.offset), C.byref(ptrs, lib.GemmMembers.C0.offset)],
+                        patches, (d, ptrs)))
+                else:
+                    self.calls.append((L.nbk_gemm, [C.byref(d)], patches, d))
             elif k == "gemm_nf4":
                 d = lib.GemmNf4Desc()
                 rx, rcodes, rsc, rc = a["x"], a["codes"], a["scales"], a["dst"]

@@ -81,6 +81,11 @@ class GemmDesc(C.Structure):
     ]
 
 
+class GemmMembers(C.Structure):
+    """The three arrays of pointers of nbk_gemm_members, one behind the other."""
+    _fields_ = [(f"{name}{i}", C.c_void_p) for name in ("B", "bias", "C") for i in range(4)]
+
+
 class GemmNf4Desc(C.Structure):
     _fields_ = [
         ("A", C.c_void_p), ("codes", C.c_void_p), ("scales", C.c_void_p), ("C", C.c_void_p),
@@ -185,6 +190,7 @@ _SIGNATURES = {
                           C.c_void_p], C.c_int),
     "nbk_fill": ([C.c_void_p, C.c_int32, C.c_int64, C.c_double, C.c_void_p], C.c_int),
     "nbk_gemm": ([C.POINTER(GemmDesc), C.c_void_p], C.c_int),
+    "nbk_gemm_members": ([C.POINTER(GemmDesc), C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p], C.c_int),
     "nbk_gemm_nf4": ([C.POINTER(GemmNf4Desc), C.c_void_p], C.c_int),
     "nbk_conv2d_fwd": ([C.POINTER(ConvDesc), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                         C.c_void_p], C.c_int),

@@ -46,6 +46,7 @@ constexpr int share(int total, int parts, int i) {
   return total * (i + 1) / parts - total * i / parts;
 }
 
+constexpr int GEMM_MAX_MEMBERS = 4;
 struct GemmArgs {
   const void* A; const void* B; void* C; const void* bias; const void* residual;
   int64_t M, N, K;
@@ -72,7 +73,16 @@ struct GemmArgs {
   struct Deep { const void* A; const void* B; int64_t K; } deep[2];
   int32_t n_shallow, n_deep;
   int64_t k_last;        // contraction length of the last slice of a product split along K; 0: K
+  // Products of one A in one launch, the outer batch index: their B, bias and, in elements from C, their results.
+  struct Member { const void* B; const void* bias; int64_t c_off; } member[GEMM_MAX_MEMBERS];
+  int32_t n_members;     // 0: none
 };
+// The right operand, bias and result of this workgroup's batch member.
+struct GemmMember { const void* B; const void* bias; int64_t c_off; };
+__device__ __forceinline__ GemmMember gemm_member(const GemmArgs& g, int64_t bo, int64_t bi, int elem) {
+  if (g.n_members > 0) return {g.member[bo].B, g.member[bo].bias, g.member[bo].c_off};
+  return {(const char*)g.B + (bo * g.b_bs + bi * g.b_bs2) * elem, g.bias, bo * g.c_bs + bi * g.c_bs2};
+}
 
 // Contraction length of this workgroup's batch member (the slice is the inner batch index where there
 // are two levels).
@@ -351,8 +361,8 @@ __device__ __forceinline__ void gemm_residual_prefetch(const GemmArgs& g, int64_
 
 template <int TM, int WN, bool FAST, int EPI, typename Scatter>
 __device__ __forceinline__ void gemm_epilogue_bands(Scatter&& scatter, const GemmArgs& g, int64_t m0,
-                                                    int64_t n0, int wm, int wn, int64_t c_off, int wave,
-                                                    int lane, const uint4* pre = nullptr) {
+                                                    int64_t n0, int wm, int wn, int64_t c_off, const void* bias,
+                                                    int wave, int lane, const uint4* pre = nullptr) {
   constexpr int SLAB_LD = WN + 4;  // floats per slab row (padding spreads the row groups)
   float* slab = (float*)gemm_lds + wave * (32 * SLAB_LD);
   const bool out_f32 = g.dtype_c == NBK_F32;
@@ -365,9 +375,9 @@ __device__ __forceinline__ void gemm_epilogue_bands(Scatter&& scatter, const Gem
   float bias_v[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) bias_v[e] = 0.f;
-  if (EPI != 0 && g.bias) {
-    if (!out_f32 && col + 8 <= g.N && (((uintptr_t)g.bias + 2 * (uintptr_t)col) & 15) == 0) {
-      const uint4 bu = *(const uint4*)((const uint16_t*)g.bias + col);  // eight 16-bit values at once
+  if (EPI != 0 && bias) {
+    if (!out_f32 && col + 8 <= g.N && (((uintptr_t)bias + 2 * (uintptr_t)col) & 15) == 0) {
+      const uint4 bu = *(const uint4*)((const uint16_t*)bias + col);  // eight 16-bit values at once
       bias_v[0] = __uint_as_float(bu.x << 16); bias_v[1] = __uint_as_float(bu.x & 0xffff0000u);
       bias_v[2] = __uint_as_float(bu.y << 16); bias_v[3] = __uint_as_float(bu.y & 0xffff0000u);
       bias_v[4] = __uint_as_float(bu.z << 16); bias_v[5] = __uint_as_float(bu.z & 0xffff0000u);
@@ -375,7 +385,7 @@ __device__ __forceinline__ void gemm_epilogue_bands(Scatter&& scatter, const Gem
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        if (col + e < g.N) bias_v[e] = nbk_load_as_f32(g.bias, col + e, g.dtype_c);
+        if (col + e < g.N) bias_v[e] = nbk_load_as_f32(bias, col + e, g.dtype_c);
     }
   }
   constexpr int NP = 32 / ROWS_PER_PASS;
@@ -524,8 +534,8 @@ __device__ __forceinline__ void gemm_epilogue_bands(Scatter&& scatter, const Gem
 // 32x32 MFMA blocks: D[i][j] lives in lane (j, (i / 4) % 2), register (i / 8) * 4 + i % 4.
 template <int TM, int TN, int WN, bool FAST, int EPI>
 __device__ __forceinline__ void gemm_epilogue(f32x16 (&acc)[TM][TN], const GemmArgs& g, int64_t m0,
-                                              int64_t n0, int wm, int wn, int64_t c_off, int wave,
-                                              int lane, const uint4* pre = nullptr) {
+                                              int64_t n0, int wm, int wn, int64_t c_off, const void* bias,
+                                              int wave, int lane, const uint4* pre = nullptr) {
   const int li = lane & 31, kg = lane >> 5;
   gemm_epilogue_bands<TM, WN, FAST, EPI>(
       [&](auto ti, float* slab) {
@@ -538,7 +548,7 @@ __device__ __forceinline__ void gemm_epilogue(f32x16 (&acc)[TM][TN], const GemmA
             slab[((r >> 2) * 8 + kg * 4 + (r & 3)) * (WN + 4) + j * 32 + li] = a[r];
         });
       },
-      g, m0, n0, wm, wn, c_off, wave, lane, pre);
+      g, m0, n0, wm, wn, c_off, bias, wave, lane, pre);
 }
 
 // 16x16 MFMA blocks: D[i][j] lives in lane (j, i / 4), register i % 4; a band is two block rows.
@@ -547,8 +557,8 @@ __device__ __forceinline__ void gemm_epilogue(f32x16 (&acc)[TM][TN], const GemmA
 // than the slab round trip with its whole 128-byte lines.)
 template <int TM, int TN, int WN, bool FAST, int EPI>
 __device__ __forceinline__ void gemm_epilogue(f32x4 (&acc)[TM][TN], const GemmArgs& g, int64_t m0,
-                                              int64_t n0, int wm, int wn, int64_t c_off, int wave,
-                                              int lane) {
+                                              int64_t n0, int wm, int wn, int64_t c_off, const void* bias,
+                                              int wave, int lane) {
   static_assert(TM % 2 == 0, "block rows per wave tile");
   const int p = lane & 15, q = lane >> 4;
   gemm_epilogue_bands<TM / 2, WN, FAST, EPI>(
@@ -561,7 +571,7 @@ __device__ __forceinline__ void gemm_epilogue(f32x4 (&acc)[TM][TN], const GemmAr
           for (int r = 0; r < 4; ++r) slab[(ib * 16 + 4 * q + r) * (WN + 4) + j * 16 + p] = a[r];
         });
       },
-      g, m0, n0, wm, wn, c_off, wave, lane);
+      g, m0, n0, wm, wn, c_off, bias, wave, lane);
 }
 
 // NW waves: 4 as 2 x 2, or 8 as 2 x 4 (two waves per SIMD, each with half the accumulators:
@@ -586,8 +596,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_kernel(const GemmArgs g) {
   const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
   const int64_t bo = (int64_t)blockIdx.y / g.batch_inner, bi = (int64_t)blockIdx.y % g.batch_inner;
   const uint16_t* A = (const uint16_t*)g.A + bo * g.a_bs + bi * g.a_bs2;
-  const uint16_t* B = (const uint16_t*)g.B + bo * g.b_bs + bi * g.b_bs2;
-  const int64_t c_off = bo * g.c_bs + bi * g.c_bs2;
+  const GemmMember mem = gemm_member(g, bo, bi, 2);
+  const uint16_t* B = (const uint16_t*)mem.B;
+  const int64_t c_off = mem.c_off;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = (wave / WGN) * WM, wn = (wave % WGN) * WN;
   const int li = lane & 31, kg = lane >> 5;
@@ -781,7 +792,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_kernel(const GemmArgs g) {
   }
   __syncthreads();  // the epilogue reuses the tile buffers as per-wave slabs
 
-  gemm_epilogue<TM, TN, WN, false, EPI ? 2 : 0>(acc, g, m0, n0, wm, wn, c_off, wave, lane);
+  gemm_epilogue<TM, TN, WN, false, EPI ? 2 : 0>(acc, g, m0, n0, wm, wn, c_off, mem.bias, wave, lane);
 }
 
 // ------------------------------------------------------------- bf16, direct-to-LDS loads
@@ -939,8 +950,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g)
   const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
   const int64_t bo = (int64_t)blockIdx.y / g.batch_inner, bi = (int64_t)blockIdx.y % g.batch_inner;
   const uint16_t* A = (const uint16_t*)g.A + bo * g.a_bs + bi * g.a_bs2;
-  const uint16_t* B = (const uint16_t*)g.B + bo * g.b_bs + bi * g.b_bs2;
-  const int64_t c_off = bo * g.c_bs + bi * g.c_bs2;
+  const GemmMember mem = gemm_member(g, bo, bi, 2);
+  const uint16_t* B = (const uint16_t*)mem.B;
+  const int64_t c_off = mem.c_off;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = (wave / WGN) * WM, wn = (wave % WGN) * WN;
@@ -1272,7 +1284,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g)
   }
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): no copy may land in a slab
   __syncthreads();  // the epilogue reuses the tile buffers as per-wave slabs
-  gemm_epilogue<TM, TN, WN, true, EPI>(acc, g, m0, n0, wm, wn, c_off, wave, lane);
+  gemm_epilogue<TM, TN, WN, true, EPI>(acc, g, m0, n0, wm, wn, c_off, mem.bias, wave, lane);
 #undef GEMM_COPY_TILE
 #undef GEMM_SRC_A
 #undef GEMM_SRC_B
@@ -1359,7 +1371,7 @@ __global__ __launch_bounds__(256) void gemm_skinny_k_kernel(const GemmArgs g) {
 #pragma unroll
     for (int j = 0; j < TN; ++j)
       acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa, fb[j], (f32x16)(0.f), 0, 0, 0);
-    gemm_epilogue<1, TN, WN, true, EPI>(acc, g, m0, n0, wm + i * 32, wn, 0, wave, lane,
+    gemm_epilogue<1, TN, WN, true, EPI>(acc, g, m0, n0, wm + i * 32, wn, 0, g.bias, wave, lane,
                                         EPI == 4 ? pre : nullptr);
   }
 }
@@ -1758,8 +1770,9 @@ __global__ __launch_bounds__(64 * WK, WK > 8 || (WK == 4 && A_KC && B_KC) ? 1 : 
   const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
   const int64_t bo = (int64_t)blockIdx.y / g.batch_inner, bi = (int64_t)blockIdx.y % g.batch_inner;
   const float* A = (const float*)g.A + bo * g.a_bs + bi * g.a_bs2;
-  const float* B = (const float*)g.B + bo * g.b_bs + bi * g.b_bs2;
-  const int64_t c_off = bo * g.c_bs + bi * g.c_bs2;
+  const GemmMember mem = gemm_member(g, bo, bi, 4);
+  const float* B = (const float*)mem.B;
+  const int64_t c_off = mem.c_off;
   const int64_t K = gemm_slice_k(g, bo, bi);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int li = lane % T, h = lane / T;
@@ -1823,7 +1836,7 @@ __global__ __launch_bounds__(64 * WK, WK > 8 || (WK == 4 && A_KC && B_KC) ? 1 : 
     const int64_t row = m0 + (r >> 2) * 8 + h * 4 + (r & 3), col = n0 + li;
     if (row >= g.M || col >= g.N) return;
     const int64_t idx = c_off + row * g.ldc + col;
-    const float x = sum * g.alpha + (g.bias ? ((const float*)g.bias)[col] : 0.f);
+    const float x = sum * g.alpha + (mem.bias ? ((const float*)mem.bias)[col] : 0.f);
     float v;
     if (g.C2) {
       float dv;
@@ -1961,8 +1974,9 @@ __global__ __launch_bounds__(NWM * NWN * 64) void gemm_f32_split_kernel(const Ge
   const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
   const int64_t bo = (int64_t)blockIdx.y / g.batch_inner, bi = (int64_t)blockIdx.y % g.batch_inner;
   const float* A = (const float*)g.A + bo * g.a_bs + bi * g.a_bs2;
-  const float* B = (const float*)g.B + bo * g.b_bs + bi * g.b_bs2;
-  const int64_t c_off = bo * g.c_bs + bi * g.c_bs2;
+  const GemmMember mem = gemm_member(g, bo, bi, 4);
+  const float* B = (const float*)mem.B;
+  const int64_t c_off = mem.c_off;
   const int64_t K = gemm_slice_k(g, bo, bi);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / NWN * WM, wn = wave % NWN * WN;
@@ -2015,7 +2029,7 @@ __global__ __launch_bounds__(NWM * NWN * 64) void gemm_f32_split_kernel(const Ge
       for (int j = 0; j < TN; ++j) {
         const int64_t col = n0 + wn + j * 16 + (lane & 15);
         if (col >= g.N) continue;
-        const float bias = g.bias ? ((const float*)g.bias)[col] : 0.f;
+        const float bias = mem.bias ? ((const float*)mem.bias)[col] : 0.f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int64_t row = m0 + wm + i * 16 + (lane >> 4) * 4 + r;
@@ -2239,7 +2253,10 @@ static int launch_f32_split(const GemmArgs& args, bool akc, bool bkc, int64_t ba
   return nbk_check_launch("gemm_f32_split_kernel");
 }
 
-extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
+// What the products of one A have of their own (nbk_gemm_members).
+struct GemmMembers { int n; const void* const* B; const void* const* bias; void* const* C; };
+
+static int gemm_launch(const nbk_gemm_desc* d, const GemmMembers& own, void* stream) {
   NBK_REQUIRE(d != nullptr, "gemm: null descriptor");
   NBK_REQUIRE(d->A && d->B && d->C, "gemm: null operand pointer");
   NBK_REQUIRE(d->M > 0 && d->N > 0 && d->K > 0, "gemm: empty problem %lld x %lld x %lld",
@@ -2258,6 +2275,12 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
               (long long)d->b_rs, (long long)d->b_cs);
   NBK_REQUIRE(d->ldc >= d->N, "gemm: ldc %lld < N %lld", (long long)d->ldc, (long long)d->N);
   NBK_REQUIRE(d->batch_reduce == 0, "gemm: batch_reduce is folded into K by the caller");
+  const int members = own.n;
+  NBK_REQUIRE(members == 0 || (d->batch == 1 && d->residual == nullptr && d->C_aux == nullptr && d->colsum == nullptr &&
+                               d->n_terms == 0 && d->k_last == 0),
+              "gemm: several products of one A go without batches, residual, second result, column sums, "
+              "further operand pairs and k_last");
+  const int64_t batch = members > 0 ? members : d->batch;
   hipStream_t st = (hipStream_t)stream;
   GemmArgs a = {};
   a.A = d->A; a.B = d->B; a.C = d->C; a.bias = d->bias; a.residual = d->residual;
@@ -2275,7 +2298,7 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
   // streamed (non-temporal stores), which leaves the cache to the operands.  Smaller results are
   // stored normally: measured inside the decoder step, streaming them takes as much from the
   // kernels that read them next as it gives the product.
-  a.c_stream = d->M * d->N * d->batch * (d->dtype_c == NBK_F32 ? 4 : 2) > (256ll << 20) ? 1 : 0;
+  a.c_stream = d->M * d->N * batch * (d->dtype_c == NBK_F32 ? 4 : 2) > (256ll << 20) ? 1 : 0;
   NBK_REQUIRE(d->aux_op == NBK_AUX_NONE || d->aux_op == NBK_AUX_ACT_GRAD, "gemm: aux_op %d", d->aux_op);
   NBK_REQUIRE((d->aux_op == NBK_AUX_NONE) == (d->C_aux == nullptr),
               "gemm: C_aux and aux_op go together");
@@ -2296,7 +2319,7 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
   NBK_REQUIRE(d->n_terms >= 0 && d->n_terms <= NBK_GEMM_MAX_TERMS, "gemm: n_terms %d", d->n_terms);
   const bool tail = d->n_terms > 0;
   if (tail) {
-    NBK_REQUIRE(d->dtype_ab == NBK_BF16 && d->batch == 1 && d->colsum == nullptr,
+    NBK_REQUIRE(d->dtype_ab == NBK_BF16 && batch == 1 && d->colsum == nullptr,
                 "gemm: more operand pairs go with one bf16 product without column sums");
     for (int i = 0; i < d->n_terms; ++i) {
       const nbk_gemm_term& t = d->term[i];
@@ -2312,13 +2335,21 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
   };
   a.a_vec = vec_ok(d->A, akc ? d->a_rs : d->a_cs, d->a_bs, a.a_bs2);
   a.b_vec = vec_ok(d->B, bkc ? d->b_cs : d->b_rs, d->b_bs, a.b_bs2);
+  const int esz_c = d->dtype_c == NBK_F32 ? 4 : 2;
+  a.n_members = members;
+  for (int i = 0; i < members; ++i) {
+    NBK_REQUIRE(own.B[i] && own.C[i] && ((uintptr_t)own.C[i] - (uintptr_t)d->C) % 16 == 0, "gemm: product %d of one A", i);
+    a.member[i] = {own.B[i], own.bias[i], (int64_t)((intptr_t)own.C[i] - (intptr_t)d->C) / esz_c};
+    if (own.bias[i]) a.bias = own.bias[i];  // (whether there is one at all)
+    a.b_vec = a.b_vec && (uintptr_t)own.B[i] % 16 == 0;
+  }
   // (checked before any kernel is chosen: no path may take the product and drop the sums)
   NBK_REQUIRE(d->colsum == nullptr || (d->dtype_ab == NBK_BF16 && !akc && !bkc),
               "gemm: column sums need bf16 operands that are both row-contiguous (a_rs == b_cs == 1)");
   // (few rows too, where a workgroup's share of B is small: 1000 x 8 x 1024 6.5 us, in two slices and their sum 8.7)
   const bool tall = d->M >= 1024 || (d->M >= 16 && d->K * (d->N <= 16 ? 1 : 2) <= 2048);
   if (!tail && d->k_last == 0 && d->dtype_ab == NBK_BF16 && d->N <= 32 && tall && d->K >= 256 && d->K % 64 == 0 &&
-      akc && a.a_vec && d->batch == 1 && d->bias == nullptr && d->residual == nullptr &&
+      akc && a.a_vec && batch == 1 && d->bias == nullptr && d->residual == nullptr &&
       d->act == NBK_ACT_NONE && (bkc ? (bool)a.b_vec : (d->b_cs == 1 && d->N % 8 == 0 && a.b_vec))) {
     // 32 rows per workgroup, K split over its eight waves
     const int pitch_chunks = d->N <= 16 ? 2 : 4;
@@ -2342,7 +2373,7 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
       return nbk_check_launch("gemm_skinny_n_kernel");
     }
   }
-  if (!tail && d->k_last == 0 && d->dtype_ab == NBK_BF16 && d->K <= 16 && akc && d->batch == 1 && d->N % 8 == 0 &&
+  if (!tail && d->k_last == 0 && d->dtype_ab == NBK_BF16 && d->K <= 16 && akc && batch == 1 && d->N % 8 == 0 &&
       d->ldc % 8 == 0 && ((uintptr_t)d->C & 15) == 0 && ((uintptr_t)d->residual & 15) == 0 &&
       (d->K == 16 ? a.a_vec : d->K == 8 && (d->a_rs % 8 == 0) && ((uintptr_t)d->A & 15) == 0)) {
     // (the vector path reads whole 16-byte pieces of A rows: K = 16 or 8)
@@ -2438,8 +2469,8 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
     // 512) as x^T dy 14.0 / 10.4, x 128 7.1 / 6.3), and on long contractions (128 x (128 x 128 x 512)
     // 13.5 / 12.1, x 128 7.2 / 7.5).
     const bool ragged = (!akc && d->M % 64 != 0) || (!bkc && d->N % 64 != 0);
-    const int64_t tiles_64 = ((d->M + 63) / 64) * ((d->N + 63) / 64) * d->batch;
-    const bool one_each = d->batch > 1 && d->M <= 128 && d->N <= 128 && tiles_64 > 256 &&
+    const int64_t tiles_64 = ((d->M + 63) / 64) * ((d->N + 63) / 64) * batch;
+    const bool one_each = batch > 1 && d->M <= 128 && d->N <= 128 && tiles_64 > 256 &&
                           (d->M > 64 || d->N > 64) &&
                           ((ragged && d->K >= 128) || (d->K >= 512 && d->M % 64 == 0 && d->N % 64 == 0));
     const bool small = tiles_64 <= 512 && !one_each;
@@ -2453,39 +2484,39 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
     const int64_t cus = nbk_num_cus();
     const bool deep = d->K > 512;
     const bool wide = tiles_64 > cus && d->K >= 512 && d->N > 64;
-    const bool one_round = ((d->M + 127) / 128) * ((d->N + 127) / 128) * d->batch <= cus && d->K > 256;
+    const bool one_round = ((d->M + 127) / 128) * ((d->N + 127) / 128) * batch <= cus && d->K > 256;
     if (d->colsum != nullptr) {
       NBK_REQUIRE(fast && !akc && !bkc && d->bias == nullptr &&
                       d->residual == nullptr && d->act == NBK_ACT_NONE && d->alpha == 1.f,
                   "gemm: column sums go with a plain bf16 product of two row-contiguous, 16-byte "
                   "aligned operands (M %% 8 == 0, N %% 8 == 0)");
-      if (small && wide) return launch_bf16_dl_colsum<64, 128, 4, 4>(a, d->batch, st);
-      if (small) return deep ? launch_bf16_dl_colsum<64, 64, 4, 4>(a, d->batch, st)
-                             : launch_bf16_dl_colsum<64, 64, 4>(a, d->batch, st);
-      return one_round ? launch_bf16_dl_colsum<128, 128, 4, 4>(a, d->batch, st)
-                       : launch_bf16_dl_colsum<128, 128, 4>(a, d->batch, st);
+      if (small && wide) return launch_bf16_dl_colsum<64, 128, 4, 4>(a, batch, st);
+      if (small) return deep ? launch_bf16_dl_colsum<64, 64, 4, 4>(a, batch, st)
+                             : launch_bf16_dl_colsum<64, 64, 4>(a, batch, st);
+      return one_round ? launch_bf16_dl_colsum<128, 128, 4, 4>(a, batch, st)
+                       : launch_bf16_dl_colsum<128, 128, 4>(a, batch, st);
     }
-    if (!fast) return launch_bf16<128, 128>(a, akc, bkc, d->batch, st);
+    if (!fast) return launch_bf16<128, 128>(a, akc, bkc, batch, st);
     // 256 x 256 tiles run at about twice the rate of 128 x 128 ones per CU, one workgroup
     // per CU at a time: take them when the rounds of workgroups they need are at least
     // 60 % full (256 tiles on 256 CUs is the ideal case, 128 or 300 tiles are not).
-    const int64_t big_tiles = ((d->M + 255) / 256) * ((d->N + 255) / 256) * d->batch;
+    const int64_t big_tiles = ((d->M + 255) / 256) * ((d->N + 255) / 256) * batch;
     const int64_t rounds = (big_tiles + cus - 1) / cus;
     // (a K loop of one or two iterations is all prologue and epilogue: there two co-resident
     // 128 x 128 workgroups per CU overlap better than one 256 x 256)
     // (eight waves on the big tile: 8-16 % faster than four on every shape measured)
     if (big_tiles * 10 >= rounds * cus * 6 && d->M >= 256 && d->N >= 256 && d->K > 128)
-      return launch_bf16_dl<256, 256, 8, 1, true>(a, akc, bkc, d->batch, st);
-    if (small && wide) return launch_bf16_dl<64, 128, 4, 1, true, 4>(a, akc, bkc, d->batch, st);
-    if (small) return deep ? launch_bf16_dl<64, 64, 4, 1, true, 4>(a, akc, bkc, d->batch, st)
-                           : launch_bf16_dl<64, 64, 4, 1, true>(a, akc, bkc, d->batch, st);
+      return launch_bf16_dl<256, 256, 8, 1, true>(a, akc, bkc, batch, st);
+    if (small && wide) return launch_bf16_dl<64, 128, 4, 1, true, 4>(a, akc, bkc, batch, st);
+    if (small) return deep ? launch_bf16_dl<64, 64, 4, 1, true, 4>(a, akc, bkc, batch, st)
+                           : launch_bf16_dl<64, 64, 4, 1, true>(a, akc, bkc, batch, st);
     // (a 256 x 128 tile was measured and is no faster than 128 x 128 on mid-sized problems:
     // with one workgroup per CU a short K loop is bound by load latency, and two co-resident
     // 128 x 128 workgroups hide it better)
     // (the 16 x 16 x 32 instruction is 3-8 % faster on every shape and layout of the big tile; on
     // this one it gains 4-9 % with a row-contiguous operand and loses 5-10 % with two K-contiguous)
-    return one_round ? launch_bf16_dl<128, 128, 4, 1, false, 4>(a, akc, bkc, d->batch, st)
-                     : launch_bf16_dl<128, 128, 4, 1, false>(a, akc, bkc, d->batch, st);
+    return one_round ? launch_bf16_dl<128, 128, 4, 1, false, 4>(a, akc, bkc, batch, st)
+                     : launch_bf16_dl<128, 128, 4, 1, false>(a, akc, bkc, batch, st);
   }
   // Out of bf16 parts where a launch gives most CUs a tile of 64 x 64; below that the K loop of one workgroup
   // is what a launch waits for, and four waves that share a fragment of 32 x 32 on the float32
@@ -2497,7 +2528,7 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
   // 128 x 128 tiles run one to a CU, two of 64 x 64 do; a round of the former does the work of two of the
   // latter in 1.7 of one's time: 4096 x 4096 x 1024 (4 rounds / 8) 197 / 251, 4096 x 1024 x 64 (1 / 2) 12.4 /
   // 14.2, 64 x (333 x 333 x 64) (3 / 5) 33 / 29, 2048 x 1024 x 1024 (1 / 1) 44 / 39.
-  auto tiles = [&](int64_t edge) { return ((d->M + edge - 1) / edge) * ((d->N + edge - 1) / edge) * d->batch; };
+  auto tiles = [&](int64_t edge) { return ((d->M + edge - 1) / edge) * ((d->N + edge - 1) / edge) * batch; };
   const int64_t cus = nbk_num_cus(), t64 = tiles(64);
   const int64_t t32 = tiles(32);
   if (t64 * 4 < cus * 3 || t32 <= 2 * cus) {
@@ -2510,15 +2541,28 @@ extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) {
     // 28.9 / 26.5); 64 x (96 x 64 x 96) (384) 6.2 / 6.9, 16 x (300 x 64 x 300) (320) 9.0 / 9.4.
     const int64_t t16 = tiles(16);
     if (t16 <= 2 * cus)
-      return t16 <= cus && d->K >= 2048 ? launch_f32<16, 16>(a, akc, bkc, d->batch, st)
-                                        : launch_f32<16, 8>(a, akc, bkc, d->batch, st);
+      return t16 <= cus && d->K >= 2048 ? launch_f32<16, 16>(a, akc, bkc, batch, st)
+                                        : launch_f32<16, 8>(a, akc, bkc, batch, st);
     if (d->K >= 128 && (t32 <= cus || (t32 <= 2 * cus && d->K % 128 == 0)))
-      return launch_f32<32, 8>(a, akc, bkc, d->batch, st);
-    return launch_f32<32, 4>(a, akc, bkc, d->batch, st);
+      return launch_f32<32, 8>(a, akc, bkc, batch, st);
+    return launch_f32<32, 4>(a, akc, bkc, batch, st);
   }
   const int64_t rounds_64 = (t64 + 2 * cus - 1) / (2 * cus), rounds_128 = (tiles(128) + cus - 1) / cus;
-  if (rounds_128 * 17 <= rounds_64 * 10) return launch_f32_split<128, 128, 2, 4, 2>(a, akc, bkc, d->batch, st);
-  return launch_f32_split<64, 64, 2, 2, 2>(a, akc, bkc, d->batch, st);
+  if (rounds_128 * 17 <= rounds_64 * 10) return launch_f32_split<128, 128, 2, 4, 2>(a, akc, bkc, batch, st);
+  return launch_f32_split<64, 64, 2, 2, 2>(a, akc, bkc, batch, st);
+}
+
+extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) { return gemm_launch(d, {}, stream); }
+
+extern "C" int nbk_gemm_members(const nbk_gemm_desc* d, int32_t n, const void* const* B, const void* const* bias,
+                                void* const* C, void* stream) {
+  NBK_REQUIRE(d != nullptr && B != nullptr && bias != nullptr && C != nullptr, "gemm_members: null argument");
+  NBK_REQUIRE(n >= 2 && n <= GEMM_MAX_MEMBERS, "gemm_members: %d products", n);
+  nbk_gemm_desc first = *d;
+  first.B = B[0];
+  first.bias = bias[0];
+  first.C = C[0];
+  return gemm_launch(&first, {n, B, bias, C}, stream);
 }
 
 // ------------------------------------------------------------------ NF4-coded weights

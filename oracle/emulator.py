@@ -296,6 +296,10 @@ def _view(mem, ref: ViewRef) -> torch.Tensor:
 
 
 def _gemm(a, mem):
+    if a.get("members"):  # products of one left operand, each with a right operand, a bias and a result
+        for m in a["members"]:
+            _gemm(dict(a, members=None, b=m["b"], bias=m["bias"], dst=m["dst"]), mem)
+        return
     bi = max(1, a.get("batch_inner", 1))
     bo = a["batch"] // bi
 

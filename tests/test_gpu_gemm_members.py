@@ -1,0 +1,50 @@
+"""Several products of one left operand in one launch (nbk_gemm_members), on every kernel that carries them: tiles of 64, 128
+and 256 in bf16, the guarded one, small and large float32 tiles; with and without biases.  Whole numbers: exact
+in float32, and in bf16 as far as they are below 256."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(200, 72, 64), (129, 64, 129), (384, 256, 640), (513, 1000, 96), (2048, 1536, 128)]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("layout", ["nn", "nt"])
+@pytest.mark.parametrize("M,N,K", SIZES)
+@pytest.mark.parametrize("n", [2, 3, 4])
+def test_against_the_products_alone(hip, M, N, K, n, layout, dtype):
+    from nabla_amd.backend import lib
+    rng = np.random.default_rng(M + N + K + n)
+    t = getattr(torch, dtype)
+    a = torch.tensor(rng.integers(-1, 2, (M, K)) * (rng.random((M, K)) < 0.3), dtype=t).cuda()
+    bs = [torch.tensor(rng.integers(-1, 2, (K, N)), dtype=t) for _ in range(n)]
+    bias = [torch.tensor(rng.integers(-9, 10, N), dtype=t).cuda() if i % 2 else None for i in range(n)]
+    dev = [(b.t().contiguous() if layout == "nt" else b).cuda() for b in bs]
+    room = torch.full((n, M * N + 64), 7.0, dtype=t, device="cuda")  # (results in no order of their addresses)
+    order = rng.permutation(n)
+    d = lib.GemmDesc()
+    d.A, d.M, d.N, d.K, d.a_rs, d.a_cs, d.ldc = a.data_ptr(), M, N, K, K, 1, N
+    d.b_rs, d.b_cs = (1, K) if layout == "nt" else (N, 1)
+    d.batch, d.dtype_ab, d.dtype_c, d.alpha = 1, int(dtype == "bfloat16"), int(dtype == "bfloat16"), 1.0
+    p = lib.GemmMembers()
+    for i in range(n):
+        setattr(p, f"B{i}", dev[i].data_ptr())
+        setattr(p, f"bias{i}", None if bias[i] is None else bias[i].data_ptr())
+        setattr(p, f"C{i}", room[order[i]].data_ptr())
+    L = lib.load()
+    at = [C.byref(p, getattr(lib.GemmMembers, f).offset) for f in ("B0", "bias0", "C0")]
+    lib.check(L.nbk_gemm_members(C.byref(d), n, *at, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    for i in range(n):
+        want = a.double() @ bs[i].double().cuda()
+        want = want + bias[i].double() if bias[i] is not None else want
+        assert want.abs().max() < 256
+        got = room[order[i]]
+        assert torch.equal(got[:M * N].view(M, N).double(), want) and (got[M * N:] == 7).all(), i
+    d.batch = 2
+    assert L.nbk_gemm_members(C.byref(d), n, *at, None) != 0
+    d.batch = 1
+    assert L.nbk_gemm_members(C.byref(d), 5, *at, None) != 0 and L.nbk_gemm_members(C.byref(d), 1, *at, None) != 0
