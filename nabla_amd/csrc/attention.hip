@@ -236,12 +236,16 @@ constexpr float AT_LN2 = 0.6931471805599453f;
 // tile buffers, maxima, sums and accumulators of their own, which meet in LDS at the end.  A wave's tile is
 // a chain of latencies, and a launch with few workgroups waits for the one with the most tiles: B1 H8
 // S1800 hd128, causal (120 workgroups of 128 queries, up to 29 tiles) 45 us in one part.
-template <int HD, bool RAG, int PARTS, int QW>
-__global__ __launch_bounds__(64 * QW * PARTS, PARTS > 1 ? 1 : HD == 64 ? (RAG ? 3 : 4) : 2) void attn_fwd_kernel(const AttnArgs g) {
+// HALVES 2: of every part one group of waves takes the first 32 keys of a tile, one the others: twice the
+// waves on the tile buffers of one, each with half the chain.
+template <int HD, bool RAG, int PARTS, int QW, int HALVES = 1>
+__global__ __launch_bounds__(64 * QW * PARTS * HALVES, PARTS > 1 ? 1 : HD == 64 ? (RAG ? 3 : 4) : 2) void attn_fwd_kernel(const AttnArgs g) {
   constexpr int KSTEPS = HD / 16, DT = HD / 32, NCH = HD / 8;
   constexpr int TILE = 64 * HD * 2, STAGE = 2 * TILE;
   extern __shared__ __align__(16) unsigned char at_lds[];
-  const int part = PARTS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * QW)) : 0;
+  constexpr int GROUPS = PARTS * HALVES;
+  const int group = GROUPS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * QW)) : 0;
+  const int part = group / HALVES, half = group % HALVES;
   auto k_tile = [&](int buf) { return (at_u32x4*)(at_lds + (part * 2 + buf) * STAGE); };
   auto v_tile = [&](int buf) { return (at_u32x4*)(at_lds + (part * 2 + buf) * STAGE + TILE); };
 
@@ -286,11 +290,13 @@ __global__ __launch_bounds__(64 * QW * PARTS, PARTS > 1 ? 1 : HD == 64 ? (RAG ? 
   // K and V tiles go from memory into LDS without passing through registers: a wave instruction
   // deposits 64 x 16 bytes in a row (four rows of a 128-wide tile, eight of a 64-wide one), so
   // the swizzle is applied to the address each lane fetches from.
-  constexpr int PER_WAVE = 64 * NCH / 64 / QW;  // instructions per wave and tile
+  constexpr int KT2 = 2 / HALVES;                         // 32-key blocks of a tile that a wave takes, from `half` on
+  const int copier = wave + QW * half;
+  constexpr int PER_WAVE = 64 * NCH / 64 / QW / HALVES;  // instructions per wave and tile
   int src_off_k[PER_WAVE], src_off_v[PER_WAVE];  // element offsets of this lane's chunks in a tile
 #pragma unroll
   for (int j = 0; j < PER_WAVE; ++j) {
-    const int slot = (wave * PER_WAVE + j) * 64 + lane, row = slot / NCH, c = (slot % NCH) ^ at_sw<NCH>(row);
+    const int slot = (copier * PER_WAVE + j) * 64 + lane, row = slot / NCH, c = (slot % NCH) ^ at_sw<NCH>(row);
     src_off_k[j] = row * (int)g.k.ss + c * 8;
     src_off_v[j] = row * (int)g.v.ss + c * 8;
   }
@@ -300,21 +306,21 @@ __global__ __launch_bounds__(64 * QW * PARTS, PARTS > 1 ? 1 : HD == 64 ? (RAG ? 
     if (RAG && kt * 64 + 63 > last) {  // (the last tile: rows past the end repeat the last one)
 #pragma unroll
       for (int j = 0; j < PER_WAVE; ++j) {
-        const int slot = (wave * PER_WAVE + j) * 64 + lane, row = slot / NCH;
+        const int slot = (copier * PER_WAVE + j) * 64 + lane, row = slot / NCH;
         const int back = max(kt * 64 + row - last, 0);
         __builtin_amdgcn_global_load_lds((at_glb_void*)(ks + src_off_k[j] - back * (int)g.k.ss),
-                                         (at_lds_void*)(k_tile(buf) + (wave * PER_WAVE + j) * 64), 16, 0, 0);
+                                         (at_lds_void*)(k_tile(buf) + (copier * PER_WAVE + j) * 64), 16, 0, 0);
         __builtin_amdgcn_global_load_lds((at_glb_void*)(vs + src_off_v[j] - back * (int)g.v.ss),
-                                         (at_lds_void*)(v_tile(buf) + (wave * PER_WAVE + j) * 64), 16, 0, 0);
+                                         (at_lds_void*)(v_tile(buf) + (copier * PER_WAVE + j) * 64), 16, 0, 0);
       }
       return;
     }
 #pragma unroll
     for (int j = 0; j < PER_WAVE; ++j) {
       __builtin_amdgcn_global_load_lds((at_glb_void*)(ks + src_off_k[j]),
-                                       (at_lds_void*)(k_tile(buf) + (wave * PER_WAVE + j) * 64), 16, 0, 0);
+                                       (at_lds_void*)(k_tile(buf) + (copier * PER_WAVE + j) * 64), 16, 0, 0);
       __builtin_amdgcn_global_load_lds((at_glb_void*)(vs + src_off_v[j]),
-                                       (at_lds_void*)(v_tile(buf) + (wave * PER_WAVE + j) * 64), 16, 0, 0);
+                                       (at_lds_void*)(v_tile(buf) + (copier * PER_WAVE + j) * 64), 16, 0, 0);
     }
   };
   // a workgroup barrier behind which every wave's copies have landed
@@ -355,13 +361,13 @@ __global__ __launch_bounds__(64 * QW * PARTS, PARTS > 1 ? 1 : HD == 64 ? (RAG ? 
     auto tile = [&](auto masked) {
       constexpr bool MASK = decltype(masked)::value;
       // transposed scores: rows = keys (two 32-row tiles), columns = the wave's queries
-      at_f32x16 st[2];
+      at_f32x16 st[KT2];
 #pragma unroll
-      for (int kt2 = 0; kt2 < 2; ++kt2) {
+      for (int kt2 = 0; kt2 < KT2; ++kt2) {
         // all fragments of the 32 keys are requested before the first MFMA waits for one
         at_bf16x8 kfr[KSTEPS];
 #pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) kfr[s] = frag(Ks, kt2 * 32 + li, 2 * s + h);
+        for (int s = 0; s < KSTEPS; ++s) kfr[s] = frag(Ks, (half + kt2) * 32 + li, 2 * s + h);
         __builtin_amdgcn_sched_barrier(0);  // keeps the scheduler from sinking each read to its MFMA
         at_f32x16 acc = (at_f32x16)(0.f);
 #pragma unroll
@@ -371,11 +377,11 @@ __global__ __launch_bounds__(64 * QW * PARTS, PARTS > 1 ? 1 : HD == 64 ? (RAG ? 
       }
       float mx = at_neg_big();
 #pragma unroll
-      for (int kt2 = 0; kt2 < 2; ++kt2)
+      for (int kt2 = 0; kt2 < KT2; ++kt2)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           if (MASK) {
-            const int key = k0 + kt2 * 32 + (r >> 2) * 8 + 4 * h + (r & 3);
+            const int key = k0 + (half + kt2) * 32 + (r >> 2) * 8 + 4 * h + (r & 3);
             if (key > seen) st[kt2][r] = at_neg_big();
           }
           mx = fmaxf(mx, st[kt2][r]);
@@ -392,7 +398,7 @@ __global__ __launch_bounds__(64 * QW * PARTS, PARTS > 1 ? 1 : HD == 64 ? (RAG ? 
       }
       float sum = 0.f;
 #pragma unroll
-      for (int kt2 = 0; kt2 < 2; ++kt2)
+      for (int kt2 = 0; kt2 < KT2; ++kt2)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt2][r], c, -m_i));
@@ -402,29 +408,31 @@ __global__ __launch_bounds__(64 * QW * PARTS, PARTS > 1 ? 1 : HD == 64 ? (RAG ? 
       l_i += sum;  // each half of the lane pair keeps the sum of its own keys
       // O^T[d, q] += V^T[d, key] P^T[key, q]
 #pragma unroll
-      for (int kt2 = 0; kt2 < 2; ++kt2)
+      for (int kt2 = 0; kt2 < KT2; ++kt2)
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const at_bf16x8 pf = at_regs_frag(st[kt2], t);
 #pragma unroll
           for (int d = 0; d < DT; ++d)
-            o_acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(Vs, d, 2 * kt2 + t), pf, o_acc[d], 0, 0, 0);
+            o_acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(Vs, d, 2 * (half + kt2) + t), pf, o_acc[d], 0, 0, 0);
           l_r = at_sum_bf16x8(pf, l_r);
         }
     };
-    // keys of this tile against the wave's queries: all visible, some, or none
+    // keys of this tile (of its half) against the wave's queries: all visible, some, or none.  (None is left out:
+    // every query that takes part in a tile sees a key of it, so its maximum is a score.)
     const bool whole = !RAG || k0 + 63 <= last;
-    if ((RAG && wq0 > last) || (PARTS > 1 && kt >= n_tiles)) {}
+    const int first = HALVES > 1 ? k0 + 32 * half : k0;
+    if ((RAG && wq0 > last) || (PARTS > 1 && kt >= n_tiles) || (HALVES > 1 && RAG && first > last)) {}
     else if (whole && (!g.causal || k0 + 63 <= wq0)) tile(std::false_type{});
-    else if (!g.causal || k0 <= wq0 + 31) tile(std::true_type{});
+    else if (!g.causal || first <= wq0 + 31) tile(std::true_type{});
     tile_barrier();
   }
-  if constexpr (PARTS > 1) {
-    // the other parts' rows through the tile buffers, which are free behind the last barrier
+  if constexpr (GROUPS > 1) {
+    // the other groups' rows through the tile buffers, which are free behind the last barrier
     constexpr int NR = DT * 16 + 3;
     float* rows = (float*)at_lds + wave * 64 + lane;
-    if (part > 0) {
-      float* mine = rows + (part - 1) * NR * (64 * QW);
+    if (group > 0) {
+      float* mine = rows + (group - 1) * NR * (64 * QW);
 #pragma unroll
       for (int d = 0; d < DT; ++d)
 #pragma unroll
@@ -434,12 +442,12 @@ __global__ __launch_bounds__(64 * QW * PARTS, PARTS > 1 ? 1 : HD == 64 ? (RAG ? 
       mine[(DT * 16 + 2) * (64 * QW)] = l_r;
     }
     __syncthreads();
-    if (part > 0) return;
+    if (group > 0) return;
 #pragma unroll
-    for (int q = 0; q < PARTS - 1; ++q) {
+    for (int q = 0; q < GROUPS - 1; ++q) {
       const float* other = rows + q * NR * (64 * QW);
       const float m_o = other[DT * 16 * (64 * QW)], m_new = fmaxf(m_i, m_o);
-      // (a part without a key that this query sees still has its first maximum: its factor is zero)
+      // (a group without a key that this query sees still has its first maximum: its factor is zero)
       const float mine = __builtin_amdgcn_exp2f(m_i - m_new), theirs = __builtin_amdgcn_exp2f(m_o - m_new);
       m_i = m_new;
       l_i = l_i * mine + other[(DT * 16 + 1) * (64 * QW)] * theirs;
@@ -1087,26 +1095,35 @@ extern "C" int nbk_attention_fwd(const nbk_attn_desc* d, const nbk_attn_tensor* 
   a.lse = (float*)lse;
   hipStream_t st = (hipStream_t)stream;
   const bool rag = d->S % 128 != 0;
-  auto launch = [&](auto kern, int parts, int waves) -> int {
+  auto launch = [&](auto kern, int parts, int waves, int halves) -> int {
     const dim3 grid((unsigned)(d->B * d->H), (unsigned)((d->S + 32 * waves - 1) / (32 * waves)));
     // two stages of a row-major K and V tile each
-    const size_t lds = (size_t)parts * 2 * 2 * 64 * (size_t)d->hd * 2;
+    // (and, behind the last tile, the rows of all groups of waves but one: attn_fwd_kernel's NR numbers a lane)
+    const size_t tiles = (size_t)parts * 2 * 2 * 64 * (size_t)d->hd * 2;
+    const size_t rows = (size_t)(parts * halves - 1) * (size_t)(d->hd / 2 + 3) * (size_t)(64 * waves) * sizeof(float);
+    const size_t lds = tiles > rows ? tiles : rows;
     const int lrc = attn_set_lds(kern, lds);
-    if (lrc == NBK_OK) hipLaunchKernelGGL(kern, grid, dim3(64 * waves * parts), lds, st, a);
+    if (lrc == NBK_OK) hipLaunchKernelGGL(kern, grid, dim3(64 * waves * parts * halves), lds, st, a);
     return lrc;
   };
-#define ATTN_FWD(PARTS, QW)                                                                                          \
-  (d->hd == 64 ? (rag ? launch(attn_fwd_kernel<64, true, PARTS, QW>, PARTS, QW) : launch(attn_fwd_kernel<64, false, PARTS, QW>, PARTS, QW)) \
-               : (rag ? launch(attn_fwd_kernel<128, true, PARTS, QW>, PARTS, QW) : launch(attn_fwd_kernel<128, false, PARTS, QW>, PARTS, QW)))
+#define ATTN_FWD_OF(HD, RAG, PARTS, QW, HALVES) launch(attn_fwd_kernel<HD, RAG, PARTS, QW, HALVES>, PARTS, QW, HALVES)
+#define ATTN_FWD(PARTS, QW, HALVES)                                                                                   \
+  (d->hd == 64 ? (rag ? ATTN_FWD_OF(64, true, PARTS, QW, HALVES) : ATTN_FWD_OF(64, false, PARTS, QW, HALVES))          \
+               : (rag ? ATTN_FWD_OF(128, true, PARTS, QW, HALVES) : ATTN_FWD_OF(128, false, PARTS, QW, HALVES)))
   // 64 queries in two parts while that gives no CU a second workgroup (with causal 64-wide heads, whose workgroups
   // end at different times, a third), then 128 in two parts while a CU holds no more than two of those and a part
   // has three tiles, else 128 in one.  us, one part of 128 / two of 128 / two of 64: B1 H8 S1800 hd128 causal 45 /
   // 38 / 33, B1 H16 S1024 hd64 causal 20 / 17 / 14.5, B2 21 / 18 / 17, B1 H4 S256 8.5 / 8.7 / 7.2, B3 H8 S700 hd64 16.1
   // / 14.7 / 16.8, B2 H16 S2048 hd128 causal 58 / 56 / 82, B8 H16 S1024 hd64 causal 38 / 47 / 48.
+  // The first of these in halves of tiles too where there are enough of them for the sum of four groups' rows, us
+  // two of 64 / in halves: B1 H8 S1800 hd128 causal 32.1 / 27.1, S1000 20.8 / 19.2, S500 12.5 / 13.2; hd64 causal B1
+  // H16 S1800 (464 workgroups) 23.8 / 21.0, S1024 (256) 13.3 / 12.9, B2 H16 S1024 (512) 14.9 / 15.4.
   const int64_t heads = d->B * d->H, cus = nbk_num_cus(), g64 = heads * ((d->S + 63) / 64), g128 = heads * ((d->S + 127) / 128);
-  if (g64 <= cus * (d->hd == 64 && d->causal ? 2 : 1)) rc = ATTN_FWD(2, 2);
-  else if (g128 <= 2 * cus && d->S > 320) rc = ATTN_FWD(2, 4);
-  else rc = ATTN_FWD(1, 4);
+  if (g64 <= cus * (d->hd == 64 && d->causal ? 2 : 1))
+    rc = d->S >= (g64 <= cus ? 768 : 1280) ? ATTN_FWD(2, 2, 2) : ATTN_FWD(2, 2, 1);
+  else if (g128 <= 2 * cus && d->S > 320) rc = ATTN_FWD(2, 4, 1);
+  else rc = ATTN_FWD(1, 4, 1);
+#undef ATTN_FWD_OF
 #undef ATTN_FWD
   if (rc) return rc;
   return nbk_check_launch("attn_fwd_kernel");
