@@ -1721,7 +1721,10 @@ class Planner:
         vec = 16 // x.dtype.size_in_bytes if inner % (16 // x.dtype.size_in_bytes) == 0 else 1
         blocks = outer * ((inner + 64 * vec - 1) // (64 * vec))
         split = 1
-        if blocks < 256 and red >= 768 and x.dtype.is_float():  # (partials are fp32)
+        # (a column of numbers behind each other is read by 16 bytes a lane: one workgroup takes 65536 of them in
+        # less time than a second launch, by element 8192)
+        line = inner == 1 and red <= (65536 if red % (16 // x.dtype.size_in_bytes) == 0 else 8192)
+        if blocks < 256 and red >= 768 and x.dtype.is_float() and not line:  # (partials are fp32)
             want = min(256, red // 64, max(1, 1024 // max(blocks, 1)))
             for s in range(want, 1, -1):
                 if red % s == 0 and outer * s <= 65535:

@@ -208,13 +208,15 @@ struct RedAny {
 };
 constexpr int RED_FLIGHT = 8;  // rows in flight per lane
 
-template <typename P, int kind>
+// LINE: rows of one element, read 16 bytes at a time as if N of them were a row; the N sums meet at the end.
+template <typename P, int kind, bool LINE>
 __device__ __forceinline__ void reduce_strip_kind(const void* __restrict__ in, void* __restrict__ out,
                                                   int dti, int dto, int64_t red, int64_t inner,
                                                   int64_t bx, int64_t o, int lxs, float* part) {
   constexpr int N = P::N;
-  const int LX = 1 << lxs, RY = 256 >> lxs;
-  const int64_t pieces = inner / N;
+  if constexpr (LINE) red /= N;
+  const int LX = LINE ? 1 : 1 << lxs, RY = LINE ? 256 : 256 >> lxs;
+  const int64_t pieces = LINE ? 1 : inner / N;
   const int64_t at = bx * LX + (threadIdx.x & (LX - 1));
   const int64_t base = o * red * pieces + (at < pieces ? at : pieces - 1);
   const float ident = kind == NBK_RED_SUM ? 0.f : (kind == NBK_RED_MAX ? -INFINITY : INFINITY);
@@ -280,6 +282,18 @@ __device__ __forceinline__ void reduce_strip_kind(const void* __restrict__ in, v
 #pragma unroll
       for (int e = 0; e < N; ++e) acc[c][e] = red_comb(acc[c][e], acc[c + w][e], kind);
   float(&sum)[N] = acc[0];
+  if constexpr (LINE) {
+#pragma unroll
+    for (int w = N / 2; w > 0; w /= 2)
+#pragma unroll
+      for (int e = 0; e < w; ++e) sum[e] = red_comb(sum[e], sum[e + w], kind);
+    for (int s = 1; s < 64; s <<= 1) sum[0] = red_comb(sum[0], __shfl_xor(sum[0], s), kind);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sum[0];
+    __syncthreads();
+    if (threadIdx.x == 0)
+      nbk_store_from_f32(out, o, dto, red_comb(red_comb(part[0], part[1], kind), red_comb(part[2], part[3], kind), kind));
+    return;
+  }
   if (RY == 1) {  // a column is one lane's: no partial sums to meet
     if (at >= pieces) return;
     const int64_t to = o * pieces + at;
@@ -316,11 +330,11 @@ __device__ __forceinline__ void reduce_strip_kind(const void* __restrict__ in, v
 }
 // (a function chosen anew for every number was two thirds of the instructions: us, 2 x (3287x2624) bf16 27.4 / 12.7,
 // 33 x (7479x56) 53 / 13.3, 42 x (105x4664) 16.6 / 11.0)
-template <typename P>
+template <typename P, bool LINE = false>
 __device__ __forceinline__ void reduce_strip_body(const void* __restrict__ in, void* __restrict__ out,
                                                   int dti, int dto, int64_t red, int64_t inner, int kind,
                                                   int64_t bx, int64_t o, int lxs, float* part) {
-#define REDUCE_KIND(K) reduce_strip_kind<P, K>(in, out, dti, dto, red, inner, bx, o, lxs, part)
+#define REDUCE_KIND(K) reduce_strip_kind<P, K, LINE>(in, out, dti, dto, red, inner, bx, o, lxs, part)
   if (kind == NBK_RED_SUM) REDUCE_KIND(NBK_RED_SUM);
   else if (kind == NBK_RED_MAX) REDUCE_KIND(NBK_RED_MAX);
   else REDUCE_KIND(NBK_RED_MIN);
@@ -329,7 +343,8 @@ __device__ __forceinline__ void reduce_strip_body(const void* __restrict__ in, v
 // How a reduction is laid out, a function of its own shape alone: the order of summation, and so
 // the result, does not depend on how reductions are grouped into launches.
 struct RedLayout {
-  int mode;  // 1: bf16 by 16 bytes, 2: fp32 by 16 bytes; by element 3: bf16, 4: fp32, 0: other types
+  int mode;  // 1: bf16 by 16 bytes, 2: fp32 by 16 bytes; by element 3: bf16, 4: fp32, 0: other types; rows of one
+             // element by 16 bytes 5: bf16, 6: fp32
   int lxs;   // log2 of the strip's width in pieces
   int64_t blocks_x;
 };
@@ -342,6 +357,14 @@ static RedLayout reduce_layout(const void* in, int dti, int64_t outer, int64_t r
   RedLayout L;
   const bool aligned = ((uintptr_t)in & 15) == 0;
   L.mode = dti == NBK_BF16 ? (aligned && inner % 8 == 0 ? 1 : 3) : dti == NBK_F32 ? (aligned && inner % 4 == 0 ? 2 : 4) : 0;
+  // (a column of numbers behind each other, the sum of a loss: one workgroup by 16 bytes takes up to 16384 of them
+  // in one trip to memory, where slices of 64 took a launch more; us, 8192 bf16 9.2 / 4.7)
+  if (inner == 1 && aligned && red >= 512 && (dti == NBK_BF16 ? red % 8 == 0 : dti == NBK_F32 && red % 4 == 0)) {
+    L.mode = dti == NBK_BF16 ? 5 : 6;
+    L.lxs = 0;
+    L.blocks_x = 1;
+    return L;
+  }
   const int64_t pieces = inner / (L.mode == 1 ? 8 : L.mode == 2 ? 4 : 1);
   // (by element, two rows abreast at least: sixteen chains with the eight of a lane)
   const int widest = (L.mode == 1 || L.mode == 2 || red <= RED_FLIGHT) ? 8 : 7;
@@ -361,12 +384,12 @@ static RedLayout reduce_layout(const void* in, int dti, int64_t outer, int64_t r
   L.blocks_x = (pieces + (1ll << s) - 1) >> s;
   return L;
 }
-template <typename P>
+template <typename P, bool LINE = false>
 __global__ __launch_bounds__(256) void reduce_strip_kernel(const void* __restrict__ in, void* __restrict__ out,
                                                            int dti, int dto, int64_t red, int64_t inner, int kind,
                                                            int lxs) {
   __shared__ float part[4 * 64 * P::N];
-  reduce_strip_body<P>(in, out, dti, dto, red, inner, kind, blockIdx.x, blockIdx.y, lxs, part);
+  reduce_strip_body<P, LINE>(in, out, dti, dto, red, inner, kind, blockIdx.x, blockIdx.y, lxs, part);
 }
 
 // Integer tensors: exact, with a 64-bit accumulator.  The same [outer, red, inner] layout and
@@ -419,13 +442,15 @@ __global__ __launch_bounds__(256) void reduce_batch_kernel(const ReduceBatchArgs
   const nbk_reduce_task& t = B.t[i];
   const int lb = (int)blockIdx.x - B.first_block[i];
   const int64_t bx = lb % B.blocks_x[i], o = lb / B.blocks_x[i];
-#define REDUCE_STRIP(P)                                                                                           \
-  reduce_strip_body<P>(t.in, t.out, t.dtype_in, t.dtype_out, t.red, t.inner, t.kind, bx, o, B.lxs[i], part)
+#define REDUCE_STRIP(...)                                                                                         \
+  reduce_strip_body<__VA_ARGS__>(t.in, t.out, t.dtype_in, t.dtype_out, t.red, t.inner, t.kind, bx, o, B.lxs[i], part)
   switch (B.mode[i]) {
     case 1: REDUCE_STRIP(RedBf16x8); break;
     case 2: REDUCE_STRIP(RedF32x4); break;
     case 3: REDUCE_STRIP(RedBf16); break;
     case 4: REDUCE_STRIP(RedF32); break;
+    case 5: REDUCE_STRIP(RedBf16x8, true); break;
+    case 6: REDUCE_STRIP(RedF32x4, true); break;
     default: REDUCE_STRIP(RedAny);
   }
 #undef REDUCE_STRIP
@@ -463,14 +488,16 @@ static int reduce_mid_slab(const RedLayout& L, const void* in, void* out, int32_
     return nbk_check_launch("reduce_mid_int_kernel");
   }
   dim3 grid((unsigned)L.blocks_x, (unsigned)outer);
-#define REDUCE_STRIP(P)                                                                                          \
-  hipLaunchKernelGGL(reduce_strip_kernel<P>, grid, dim3(256), 0, (hipStream_t)stream, in, out, dti, dto, red, inner, \
-                     kind, L.lxs)
+#define REDUCE_STRIP(...)                                                                                         \
+  hipLaunchKernelGGL((reduce_strip_kernel<__VA_ARGS__>), grid, dim3(256), 0, (hipStream_t)stream, in, out, dti, dto, red, \
+                     inner, kind, L.lxs)
   switch (L.mode) {
     case 1: REDUCE_STRIP(RedBf16x8); break;
     case 2: REDUCE_STRIP(RedF32x4); break;
     case 3: REDUCE_STRIP(RedBf16); break;
     case 4: REDUCE_STRIP(RedF32); break;
+    case 5: REDUCE_STRIP(RedBf16x8, true); break;
+    case 6: REDUCE_STRIP(RedF32x4, true); break;
     default: REDUCE_STRIP(RedAny);
   }
 #undef REDUCE_STRIP
