@@ -60,6 +60,7 @@ class BoundPlan:
         L = self.ex.lib
         plan = self.plan
         dyn = set(self.dynamic)
+        group_open = None  # the last launch, if products of its group may join it
         for st in plan.steps:
             a = st.attrs
             k = st.kind
@@ -210,6 +211,17 @@ class BoundPlan:
                         C.byref(d), len(a["members"]), C.byref(ptrs, lib.GemmMembers.B0.offset),
                         C.byref(ptrs, lib.GemmMembers.bias0.offset), C.byref(ptrs, lib.GemmMembers.C0.offset)],
                         patches, (d, ptrs)))
+                elif "group" in a and group_open is not None and group_open[0] == a["group"]:
+                    # (one more product of the launch before)
+                    _, descs, grouped, kept = group_open
+                    kept.append(d)
+                    grouped.extend(patches)
+                    descs[len(kept) - 1] = C.pointer(d)
+                    self.calls[-1][1][1] = len(kept)
+                elif "group" in a:
+                    descs, kept = (C.POINTER(lib.GemmDesc) * 8)(C.pointer(d)), [d]
+                    self.calls.append((L.nbk_gemm_group, [descs, 1], patches, (descs, kept)))
+                    group_open = (a["group"], descs, patches, kept)
                 else:
                     self.calls.append((L.nbk_gemm, [C.byref(d)], patches, d))
             elif k == "gemm_nf4":

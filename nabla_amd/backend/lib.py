@@ -190,6 +190,7 @@ _SIGNATURES = {
                           C.c_void_p], C.c_int),
     "nbk_fill": ([C.c_void_p, C.c_int32, C.c_int64, C.c_double, C.c_void_p], C.c_int),
     "nbk_gemm": ([C.POINTER(GemmDesc), C.c_void_p], C.c_int),
+    "nbk_gemm_group": ([C.POINTER(C.POINTER(GemmDesc)), C.c_int32, C.c_void_p], C.c_int),
     "nbk_gemm_members": ([C.POINTER(GemmDesc), C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p], C.c_int),
     "nbk_gemm_nf4": ([C.POINTER(GemmNf4Desc), C.c_void_p], C.c_int),
     "nbk_conv2d_fwd": ([C.POINTER(ConvDesc), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,

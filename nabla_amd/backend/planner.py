@@ -1363,6 +1363,7 @@ class Planner:
             # the step drew random numbers: its last launch moves the generator on, so that
             # the next run (a replay of the recording included) draws new ones
             self._emit(Step("rng_advance", [], [], {}))
+        self._group_products()
         arena = self._assign_arena()
         stats = {"steps": len(self.steps), "units": len(units),
                  "fused_groups": sum(1 for u in units if u.fused)}
@@ -1371,6 +1372,68 @@ class Planner:
         if self.n_split:
             stats["split_groups"] = self.n_split
         return Plan(self.bufs, self.steps, len(self.b.inputs), outs, arena, stats)
+
+    # Products in one launch (as many as its arguments hold), and the steps between the first and the last of them:
+    # what a product reads stays in memory until its launch.
+    GROUP_PRODUCTS, GROUP_WINDOW = 7, 24
+
+    def _group_products(self) -> None:
+        """Products x^T dy that leave most of the GPU idle, and that nothing reads for a while, go out together
+        (``nbk_gemm_group``): the weight gradients of small layers and of adapters.  A product moves behind
+        later steps, to the last one of its group; their buffers live as if they ran at once."""
+        steps = self.steps
+
+        def tiles(a) -> int:
+            return -(-a["M"] // 64) * -(-a["N"] // 64) * a["batch"]
+
+        def small(st: Step) -> bool:
+            a = st.attrs
+            return (st.kind == "gemm" and a["a_cs"] != 1 and a["b_rs"] != 1 and a["K"] > 1 and tiles(a) <= 512 and
+                    not any(a.get(f) for f in ("bias", "residual", "terms", "act", "aux_dst", "members")))
+
+        def apart(x: Step, y: Step) -> bool:
+            return set(x.writes).isdisjoint(y.reads + y.writes) and set(x.reads).isdisjoint(y.writes)
+
+        groups: list[list[int]] = []
+        open_: list[int] = []
+        for j, st in enumerate(steps):
+            if not small(st):
+                continue
+            first = steps[open_[0]].attrs if open_ else None
+            fits = (open_ and len(open_) < self.GROUP_PRODUCTS and j - open_[0] <= self.GROUP_WINDOW and
+                    first["a"].dtype is st.attrs["a"].dtype and
+                    sum(tiles(steps[i].attrs) for i in open_) + tiles(st.attrs) <= 2048 and
+                    all(apart(steps[i], steps[k]) for i in open_ for k in range(i + 1, j + 1) if k not in open_) and
+                    all(apart(steps[i], st) for i in open_))
+            if not fits:
+                open_ = []
+                groups.append(open_)
+            open_.append(j)
+        groups = [g for g in groups if len(g) > 1]
+        if not groups:
+            return
+        moved = {i for g in groups for i in g}
+        order, spans = [], []
+        tail = {g[-1]: g for g in groups}
+        for j in range(len(steps)):
+            if j in tail:
+                spans.append((len(order), len(order) + len(tail[j]) - 1))
+                for i in tail[j]:
+                    steps[i].attrs["group"] = len(spans)
+                    order.append(steps[i])
+            elif j not in moved:
+                order.append(steps[j])
+        self.steps = order
+        now = {id(st): idx for idx, st in enumerate(order)}
+        span_of = {i: s for s in spans for i in range(s[0], s[1] + 1)}
+        touched: dict[int, list[int]] = {}
+        for st in steps:
+            for b in st.reads + st.writes:
+                touched.setdefault(b, []).append(now[id(st)])
+        for b, at in touched.items():
+            buf = self.bufs[b]
+            lo, hi = min(at), max(max(at), now[id(steps[buf.last])])
+            buf.first, buf.last = span_of.get(lo, (lo,))[0], span_of.get(hi, (hi, hi))[1]
 
     def _assign_arena(self) -> int:
         """First-fit offsets for temps whose live ranges overlap."""

@@ -86,8 +86,8 @@ __device__ __forceinline__ GemmMember gemm_member(const GemmArgs& g, int64_t bo,
 
 // Contraction length of this workgroup's batch member (the slice is the inner batch index where there
 // are two levels).
-__device__ __forceinline__ int64_t gemm_slice_k(const GemmArgs& g, int64_t bo, int64_t bi) {
-  const bool last = g.batch_inner > 1 ? bi == g.batch_inner - 1 : bo == (int64_t)gridDim.y - 1;
+__device__ __forceinline__ int64_t gemm_slice_k(const GemmArgs& g, int64_t bo, int64_t bi, int batch) {
+  const bool last = g.batch_inner > 1 ? bi == g.batch_inner - 1 : bo == (int64_t)batch - 1;
   return g.k_last > 0 && last ? g.k_last : g.K;
 }
 
@@ -611,7 +611,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_kernel(const GemmArgs g) {
 
   TileLoader<BM, A_KC, NT> la;
   TileLoader<BN, B_KC, NT> lb;
-  const int64_t K = gemm_slice_k(g, bo, bi);
+  const int64_t K = gemm_slice_k(g, bo, bi, gridDim.y);
   const int64_t nk = (K + 63) / 64;
   // A is rows = m; for the loader a K-contiguous operand has (rs = row stride, k unit),
   // a row-contiguous one has (cs = k stride, row unit).
@@ -936,8 +936,9 @@ struct DirectLoader {
 // multiply a fragment of ones into one more accumulator per block column, from the B fragments
 // that are in registers for the product -- no byte is read twice.
 // STAGES: tile buffers (a power of two).  With more than two a copy has STAGES - 1 tiles' time to land.
-template <int BM, int BN, bool A_KC, bool B_KC, int EPI, int NW, int KSS, bool MI16, bool COLSUM = false, int STAGES = 2>
-__global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g) {
+// (bx, by: tile and batch member, of ny)
+template <int BM, int BN, bool A_KC, bool B_KC, int EPI, int NW, int KSS, bool MI16, bool COLSUM, int STAGES>
+__device__ __forceinline__ void gemm_bf16_dl_body(const GemmArgs& g, int bx, int by, int ny) {
   static_assert((STAGES & (STAGES - 1)) == 0, "tile t is in buffer t % STAGES");
   constexpr int WGN = NW / 2;
   constexpr int WM = BM / 2, WN = BN / WGN;  // wave tile
@@ -946,9 +947,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g)
   constexpr int TM = WM / FM, TN = WN / FM;
   constexpr int CA = BM * 8, TILE_CHUNKS = (BM + BN) * 8;
   int tm_i, tn_i;
-  gemm_tile_coords(blockIdx.x, g.tiles_m, g.tiles_n, tm_i, tn_i);
+  gemm_tile_coords(bx, g.tiles_m, g.tiles_n, tm_i, tn_i);
   const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
-  const int64_t bo = (int64_t)blockIdx.y / g.batch_inner, bi = (int64_t)blockIdx.y % g.batch_inner;
+  const int64_t bo = (int64_t)by / g.batch_inner, bi = (int64_t)by % g.batch_inner;
   const uint16_t* A = (const uint16_t*)g.A + bo * g.a_bs + bi * g.a_bs2;
   const GemmMember mem = gemm_member(g, bo, bi, 2);
   const uint16_t* B = (const uint16_t*)mem.B;
@@ -971,7 +972,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g)
   if constexpr (COLSUM) {
 #pragma unroll
     for (int j = 0; j < TN; ++j) cs[j] = (f32x4)(0.f);
-    do_cs = tm_i == 0 && wm == 0;  // (uniform over the wave)
+    do_cs = tm_i == 0 && wm == 0 && g.colsum != nullptr;  // (uniform over the wave)
   }
 
   using LA = DirectLoader<BM, A_KC, NW, MI16>;
@@ -984,7 +985,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g)
   // (tile numbers are 32-bit: the scalar unit compares those, 64-bit ones go through vector registers)
   // Two row-contiguous operands take any K: what is left over a multiple of 64 (of this slice, where
   // the product is split along K) is the first tile, like a shallow pair.
-  const int64_t K = gemm_slice_k(g, bo, bi);
+  const int64_t K = gemm_slice_k(g, bo, bi, ny);
   const int k_over = !A_KC && !B_KC ? (int)(K & 63) : 0;
   const int ns = k_over ? 1 : g.n_shallow;
   const int e0 = ns + (int)(K / 64);                                     // first tile past A and B
@@ -1275,7 +1276,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g)
       for (int j = 0; j < TN; ++j) {
         const int64_t col = n0 + wn + j * 16 + lane;
         if (col < g.N) {
-          const int64_t at = (int64_t)blockIdx.y * g.N + col;
+          const int64_t at = (int64_t)by * g.N + col;
           if (g.dtype_c == NBK_F32) ((float*)g.colsum)[at] = cs[j][0];
           else ((uint16_t*)g.colsum)[at] = nbk_f32_to_bf16(cs[j][0]);
         }
@@ -1288,6 +1289,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g)
 #undef GEMM_COPY_TILE
 #undef GEMM_SRC_A
 #undef GEMM_SRC_B
+}
+template <int BM, int BN, bool A_KC, bool B_KC, int EPI, int NW, int KSS, bool MI16, bool COLSUM = false, int STAGES = 2>
+__global__ __launch_bounds__(NW * 64) void gemm_bf16_dl_kernel(const GemmArgs g) {
+  gemm_bf16_dl_body<BM, BN, A_KC, B_KC, EPI, NW, KSS, MI16, COLSUM, STAGES>(g, blockIdx.x, blockIdx.y, gridDim.y);
 }
 
 // ------------------------------------------------------------------- bf16, K <= 16
@@ -1754,7 +1759,7 @@ struct F32Rows {
 // runs, and the times: nbk_gemm.  Two workgroups of up to eight waves have to fit a CU (the second launch
 // bound); four waves with no row-contiguous operand are two to five per cent faster without.
 template <bool A_KC, bool B_KC, int T, int WK>
-__global__ __launch_bounds__(64 * WK, WK > 8 || (WK == 4 && A_KC && B_KC) ? 1 : 2) void gemm_f32_kernel(const GemmArgs g) {
+__device__ __forceinline__ void gemm_f32_body(const GemmArgs& g, int bx, int by, int ny) {
   constexpr int BM = T, BN = T, KS = T / 16, BK = 16 * WK, LD = BK + 4;  // (a step: 8 or 16 k, in four instructions)
   constexpr int R = T * T / 64;                                           // results of a lane
   typedef float acc_t __attribute__((ext_vector_type(R)));
@@ -1766,14 +1771,14 @@ __global__ __launch_bounds__(64 * WK, WK > 8 || (WK == 4 && A_KC && B_KC) ? 1 : 
   float* lds = (float*)gemm_lds;
   static_assert(WK * R * 64 <= 2 * SET, "the partial sums fit");
   int tm_i, tn_i;
-  gemm_tile_coords(blockIdx.x, g.tiles_m, g.tiles_n, tm_i, tn_i);
+  gemm_tile_coords(bx, g.tiles_m, g.tiles_n, tm_i, tn_i);
   const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
-  const int64_t bo = (int64_t)blockIdx.y / g.batch_inner, bi = (int64_t)blockIdx.y % g.batch_inner;
+  const int64_t bo = (int64_t)by / g.batch_inner, bi = (int64_t)by % g.batch_inner;
   const float* A = (const float*)g.A + bo * g.a_bs + bi * g.a_bs2;
   const GemmMember mem = gemm_member(g, bo, bi, 4);
   const float* B = (const float*)mem.B;
   const int64_t c_off = mem.c_off;
-  const int64_t K = gemm_slice_k(g, bo, bi);
+  const int64_t K = gemm_slice_k(g, bo, bi, ny);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int li = lane % T, h = lane / T;
   const int64_t a_stride = A_KC ? g.a_rs : g.a_cs, b_stride = B_KC ? g.b_cs : g.b_rs;
@@ -1866,6 +1871,10 @@ __global__ __launch_bounds__(64 * WK, WK > 8 || (WK == 4 && A_KC && B_KC) ? 1 : 
       for (int w = 0; w < n; ++w) sum[w] = sum[2 * w] + sum[2 * w + 1];
     put(r, sum[0]);
   }
+}
+template <bool A_KC, bool B_KC, int T, int WK>
+__global__ __launch_bounds__(64 * WK, WK > 8 || (WK == 4 && A_KC && B_KC) ? 1 : 2) void gemm_f32_kernel(const GemmArgs g) {
+  gemm_f32_body<A_KC, B_KC, T, WK>(g, blockIdx.x, blockIdx.y, gridDim.y);
 }
 // LDS of a workgroup of gemm_f32_kernel: two K tiles, each with rows in front of a row-contiguous operand.
 template <bool A_KC, bool B_KC, int T, int WK>
@@ -1964,20 +1973,20 @@ struct SplitRows {
 
 // C = A B of float32 numbers: tiles of BM x BN, NWM x NWN waves, two K tiles of 32 in LDS.
 template <int BM, int BN, int NWM, int NWN, int NM, bool A_KC, bool B_KC, bool FULL>
-__global__ __launch_bounds__(NWM * NWN * 64) void gemm_f32_split_kernel(const GemmArgs g) {
+__device__ __forceinline__ void gemm_f32_split_body(const GemmArgs& g, int bx, int by, int ny) {
   constexpr int NT = NWM * NWN * 64, WM = BM / NWM, WN = BN / NWN, TM = WM / 16, TN = WN / 16;
   constexpr int TILE = (BM + BN) * 12;  // 16-byte chunks: three parts of four chunks a row
   extern __shared__ __align__(16) u32x4 gemm_lds[];
   sp_u4* lds = (sp_u4*)gemm_lds;
   int tm_i, tn_i;
-  gemm_tile_coords(blockIdx.x, g.tiles_m, g.tiles_n, tm_i, tn_i);
+  gemm_tile_coords(bx, g.tiles_m, g.tiles_n, tm_i, tn_i);
   const int64_t m0 = (int64_t)tm_i * BM, n0 = (int64_t)tn_i * BN;
-  const int64_t bo = (int64_t)blockIdx.y / g.batch_inner, bi = (int64_t)blockIdx.y % g.batch_inner;
+  const int64_t bo = (int64_t)by / g.batch_inner, bi = (int64_t)by % g.batch_inner;
   const float* A = (const float*)g.A + bo * g.a_bs + bi * g.a_bs2;
   const GemmMember mem = gemm_member(g, bo, bi, 4);
   const float* B = (const float*)mem.B;
   const int64_t c_off = mem.c_off;
-  const int64_t K = gemm_slice_k(g, bo, bi);
+  const int64_t K = gemm_slice_k(g, bo, bi, ny);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / NWN * WM, wn = wave % NWN * WN;
   SplitRows<BM, NT, A_KC> la;
@@ -2091,6 +2100,10 @@ __global__ __launch_bounds__(NWM * NWN * 64) void gemm_f32_split_kernel(const Ge
               [&](int j, int64_t k, auto inside) { return at(pb[j], k, B_KC ? 1 : g.b_rs, inside); });
     store([&](int i, int j, int r) { return acc.sum_again(i, j, r); }, [&](float, uint32_t bit) { return (left & bit) != 0; });
   }
+}
+template <int BM, int BN, int NWM, int NWN, int NM, bool A_KC, bool B_KC, bool FULL>
+__global__ __launch_bounds__(NWM * NWN * 64) void gemm_f32_split_kernel(const GemmArgs g) {
+  gemm_f32_split_body<BM, BN, NWM, NWN, NM, A_KC, B_KC, FULL>(g, blockIdx.x, blockIdx.y, gridDim.y);
 }
 
 template <int BM, int BN, int NW = 4>
@@ -2256,7 +2269,8 @@ static int launch_f32_split(const GemmArgs& args, bool akc, bool bkc, int64_t ba
 // What the products of one A have of their own (nbk_gemm_members).
 struct GemmMembers { int n; const void* const* B; const void* const* bias; void* const* C; };
 
-static int gemm_launch(const nbk_gemm_desc* d, const GemmMembers& own, void* stream) {
+// Checks a description and fills the kernels' arguments.
+static int gemm_prepare(const nbk_gemm_desc* d, const GemmMembers& own, GemmArgs& a) {
   NBK_REQUIRE(d != nullptr, "gemm: null descriptor");
   NBK_REQUIRE(d->A && d->B && d->C, "gemm: null operand pointer");
   NBK_REQUIRE(d->M > 0 && d->N > 0 && d->K > 0, "gemm: empty problem %lld x %lld x %lld",
@@ -2281,8 +2295,7 @@ static int gemm_launch(const nbk_gemm_desc* d, const GemmMembers& own, void* str
               "gemm: several products of one A go without batches, residual, second result, column sums, "
               "further operand pairs and k_last");
   const int64_t batch = members > 0 ? members : d->batch;
-  hipStream_t st = (hipStream_t)stream;
-  GemmArgs a = {};
+  a = {};
   a.A = d->A; a.B = d->B; a.C = d->C; a.bias = d->bias; a.residual = d->residual;
   a.M = d->M; a.N = d->N; a.K = d->K;
   a.a_rs = d->a_rs; a.a_cs = d->a_cs; a.b_rs = d->b_rs; a.b_cs = d->b_cs; a.ldc = d->ldc;
@@ -2346,6 +2359,26 @@ static int gemm_launch(const nbk_gemm_desc* d, const GemmMembers& own, void* str
   // (checked before any kernel is chosen: no path may take the product and drop the sums)
   NBK_REQUIRE(d->colsum == nullptr || (d->dtype_ab == NBK_BF16 && !akc && !bkc),
               "gemm: column sums need bf16 operands that are both row-contiguous (a_rs == b_cs == 1)");
+  return NBK_OK;
+}
+
+// Whether the direct-to-LDS kernels take a product.
+static bool gemm_direct(const nbk_gemm_desc* d, const GemmArgs& a) {
+  // (they keep per-lane byte offsets within a tile in 32 bits: 256 rows or 64 k-rows times the stride)
+  const bool akc = d->a_cs == 1, bkc = d->b_rs == 1;
+  const int64_t a_stride = akc ? d->a_rs : d->a_cs, b_stride = bkc ? d->b_cs : d->b_rs;
+  const bool k_whole = d->K % 64 == 0 && d->k_last % 64 == 0;
+  return a.a_vec && a.b_vec && (k_whole || (!akc && !bkc && d->n_terms == 0)) && (akc || d->M % 8 == 0) &&
+         (bkc || d->N % 8 == 0) && d->M >= 8 && d->N >= 8 &&
+         a_stride >= 0 && b_stride >= 0 && a_stride < (1 << 22) && b_stride < (1 << 22);
+}
+
+static int gemm_launch(const nbk_gemm_desc* d, const GemmMembers& own, void* stream) {
+  GemmArgs a;
+  { const int rc = gemm_prepare(d, own, a); if (rc != NBK_OK) return rc; }
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t batch = own.n > 0 ? own.n : d->batch;
+  const bool akc = d->a_cs == 1, bkc = d->b_rs == 1, tail = d->n_terms > 0;
   // (few rows too, where a workgroup's share of B is small: 1000 x 8 x 1024 6.5 us, in two slices and their sum 8.7)
   const bool tall = d->M >= 1024 || (d->M >= 16 && d->K * (d->N <= 16 ? 1 : 2) <= 2048);
   if (!tail && d->k_last == 0 && d->dtype_ab == NBK_BF16 && d->N <= 32 && tall && d->K >= 256 && d->K % 64 == 0 &&
@@ -2404,13 +2437,7 @@ static int gemm_launch(const nbk_gemm_desc* d, const GemmMembers& own, void* str
     return nbk_check_launch("gemm_skinny_k_kernel");
   }
   if (d->dtype_ab == NBK_BF16) {
-    // (the direct kernel keeps per-lane byte offsets within a tile in 32 bits: 256 rows or
-    // 64 k-rows times the stride)
-    const int64_t a_stride = akc ? d->a_rs : d->a_cs, b_stride = bkc ? d->b_cs : d->b_rs;
-    const bool k_whole = d->K % 64 == 0 && d->k_last % 64 == 0;
-    const bool fast = a.a_vec && a.b_vec && (k_whole || (!akc && !bkc && !tail)) && (akc || d->M % 8 == 0) &&
-                      (bkc || d->N % 8 == 0) && d->M >= 8 && d->N >= 8 &&
-                      a_stride >= 0 && b_stride >= 0 && a_stride < (1 << 22) && b_stride < (1 << 22);
+    const bool fast = gemm_direct(d, a);
     if (tail) {
       // In the accumulator of the direct-to-LDS kernels when every pair is laid out like A and B
       // and 16-byte aligned: shallow pairs (one K tile each, at most two) and deep pairs with
@@ -2553,6 +2580,117 @@ static int gemm_launch(const nbk_gemm_desc* d, const GemmMembers& own, void* str
 }
 
 extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) { return gemm_launch(d, {}, stream); }
+
+// ------------------------------------------------------------------ products that share a launch
+// Weight gradients of small layers: each has a fraction of the workgroups the GPU holds, and nothing reads
+// them before the end of a step.  A workgroup finds its product from the running counts and runs the
+// body of the kernel that the product would have had to itself.  us, one after the other / together: 4096 x 8,
+// 8 x 1024, 1024 x 8 and 8 x 4096 over 1000 rows in bf16 32 / 10.5; six of 512 x 512 to 512 x 2048 over 1998 rows 52 / 27, over
+// 1024 rows in float32 117 / 64; the adapters of a decoder layer over 8192 rows 44 / 34.
+constexpr int GEMM_GROUP_MAX = 7;
+struct GemmGroup {
+  int32_t n;
+  int32_t first[GEMM_GROUP_MAX + 1];  // workgroups before each product
+  int32_t batch[GEMM_GROUP_MAX];
+  GemmArgs a[GEMM_GROUP_MAX];
+};
+static_assert(sizeof(GemmGroup) <= 4096, "kernel arguments");
+template <typename Body>
+__device__ __forceinline__ void gemm_group_run(const GemmGroup& G, Body&& body) {
+  int i = 0;
+  while (i + 1 < G.n && (int)blockIdx.x >= G.first[i + 1]) ++i;
+  const GemmArgs& g = G.a[i];
+  const int local = (int)blockIdx.x - G.first[i], tiles = g.tiles_m * g.tiles_n;
+  const int by = local / tiles;
+  body(g, local - by * tiles, by, G.batch[i]);
+}
+template <int BM, int BN, int STAGES>
+__global__ __launch_bounds__(256) void gemm_bf16_group_kernel(const GemmGroup G) {
+  gemm_group_run(G, [](const GemmArgs& g, int bx, int by, int ny) {
+    gemm_bf16_dl_body<BM, BN, false, false, 0, 4, 1, true, true, STAGES>(g, bx, by, ny);
+  });
+}
+template <int T, int WK>
+__global__ __launch_bounds__(64 * WK, 2) void gemm_f32_group_kernel(const GemmGroup G) {
+  gemm_group_run(G, [](const GemmArgs& g, int bx, int by, int ny) { gemm_f32_body<false, false, T, WK>(g, bx, by, ny); });
+}
+__global__ __launch_bounds__(256) void gemm_f32_split_group_kernel(const GemmGroup G) {
+  gemm_group_run(G, [](const GemmArgs& g, int bx, int by, int ny) {
+    gemm_f32_split_body<64, 64, 2, 2, 2, false, false, false>(g, bx, by, ny);
+  });
+}
+template <typename Kern>
+static int launch_group(Kern kern, GemmGroup& G, int bm, int bn, int threads, size_t lds, hipStream_t st) {
+  int64_t blocks = 0;
+  for (int i = 0; i < G.n; ++i) {
+    GemmArgs& a = G.a[i];
+    a.tiles_m = (int)((a.M + bm - 1) / bm);
+    a.tiles_n = (int)((a.N + bn - 1) / bn);
+    G.first[i] = (int32_t)blocks;
+    blocks += (int64_t)a.tiles_m * a.tiles_n * G.batch[i];
+    NBK_REQUIRE(blocks <= 0x7fffffffLL, "gemm_group: launch too large");
+  }
+  G.first[G.n] = (int32_t)blocks;
+  NBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3((unsigned)threads), lds, st, G);
+  return nbk_check_launch("gemm group kernel");
+}
+template <int BM, int BN, int STAGES>
+static int launch_bf16_group(GemmGroup& G, hipStream_t st) {
+  const size_t pipe = STAGES * (size_t)(BM + BN) * 8 * 16, slabs = 4 * 32 * (size_t)(BN / 2 + 4) * sizeof(float);
+  return launch_group(gemm_bf16_group_kernel<BM, BN, STAGES>, G, BM, BN, 256, pipe > slabs ? pipe : slabs, st);
+}
+template <int T, int WK>
+static int launch_f32_group(GemmGroup& G, hipStream_t st) {
+  return launch_group(gemm_f32_group_kernel<T, WK>, G, T, T, 64 * WK, gemm_f32_lds<false, false, T, WK>(), st);
+}
+
+extern "C" int nbk_gemm_group(const nbk_gemm_desc* const* d, int32_t n, void* stream) {
+  NBK_REQUIRE(d != nullptr && n > 0, "gemm_group: no products");
+  for (int32_t base = 0; base < n; base += GEMM_GROUP_MAX) {
+    GemmGroup G;
+    G.n = n - base < GEMM_GROUP_MAX ? n - base : GEMM_GROUP_MAX;
+    bool together = G.n > 1, narrow = false, deep = false, long_k = true, whole_k = true;
+    int64_t t16 = 0, t32 = 0, t64 = 0, t128 = 0;
+    const int ab = d[base] != nullptr ? d[base]->dtype_ab : -1;
+    for (int i = 0; i < G.n; ++i) {
+      const nbk_gemm_desc* p = d[base + i];
+      const int rc = gemm_prepare(p, {}, G.a[i]);
+      if (rc != NBK_OK) return rc;
+      // (x^T dy: both operands row-contiguous, nothing behind the product)
+      together = together && p->dtype_ab == ab && p->a_cs != 1 && p->b_rs != 1 && p->n_terms == 0 && p->bias == nullptr &&
+                 p->residual == nullptr && p->act == NBK_ACT_NONE && p->K > 1 &&
+                 (ab == NBK_F32 || (gemm_direct(p, G.a[i]) && (p->colsum == nullptr || p->alpha == 1.f)));
+      G.batch[i] = (int32_t)p->batch;
+      auto tiles = [&](int64_t edge) { return ((p->M + edge - 1) / edge) * ((p->N + edge - 1) / edge) * p->batch; };
+      t16 += tiles(16); t32 += tiles(32); t64 += tiles(64); t128 += tiles(128);
+      narrow = narrow || p->M <= 64 || p->N <= 64;
+      deep = deep || p->K > 512;
+      long_k = long_k && p->K >= 512;
+      whole_k = whole_k && p->K % 128 == 0;
+    }
+    int rc = NBK_OK;
+    hipStream_t st = (hipStream_t)stream;
+    const int64_t cus = nbk_num_cus();
+    if (!together) {
+      for (int i = 0; rc == NBK_OK && i < G.n; ++i) rc = nbk_gemm(d[base + i], stream);
+    } else if (ab == NBK_BF16) {  // (the lines of nbk_gemm, for all products together)
+      if (narrow || (t64 <= 2 * cus && !(t64 > cus && long_k)))
+        rc = deep ? launch_bf16_group<64, 64, 4>(G, st) : launch_bf16_group<64, 64, 2>(G, st);
+      else if (t64 <= 2 * cus) rc = launch_bf16_group<64, 128, 4>(G, st);
+      else if (t128 <= cus) rc = launch_bf16_group<128, 128, 4>(G, st);
+      else rc = launch_bf16_group<128, 128, 2>(G, st);
+    } else if (t16 <= 2 * cus) {
+      rc = launch_f32_group<16, 8>(G, st);
+    } else if (t64 * 4 < cus * 3 || t32 <= 2 * cus) {
+      rc = t32 <= cus || whole_k ? launch_f32_group<32, 8>(G, st) : launch_f32_group<32, 4>(G, st);
+    } else {
+      rc = launch_group(gemm_f32_split_group_kernel, G, 64, 64, 256, 2 * (64 + 64) * 12 * 16, st);
+    }
+    if (rc != NBK_OK) return rc;
+  }
+  return NBK_OK;
+}
 
 extern "C" int nbk_gemm_members(const nbk_gemm_desc* d, int32_t n, const void* const* B, const void* const* bias,
                                 void* const* C, void* stream) {
