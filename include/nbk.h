@@ -345,6 +345,10 @@ typedef struct nbk_gemm_nf4_desc {
   int64_t workspace_bytes;
 } nbk_gemm_nf4_desc;
 int nbk_gemm_nf4(const nbk_gemm_nf4_desc* d, void* stream);
+/* The same plus further operand pairs, as nbk_gemm_desc.term (qlora_linear's update on its base product,
+ * nabla/nn/finetune/qlora.py:77-113): inside the product where the weight is decoded into a workspace, else
+ * as products that add themselves. */
+int nbk_gemm_nf4_terms(const nbk_gemm_nf4_desc* d, const nbk_gemm_term* term, int32_t n_terms, void* stream);
 
 /* ===================================================================== */
 /*  Convolution / pooling (NHWC x HWIO)                                   */

@@ -45,6 +45,7 @@ class BoundPlan:
                     self.base[b.id] = a0 + b.offset
         self.dynamic = [b.id for b in plan.bufs if b.role in ("input", "output")]
         self.calls: list[tuple] = []  # (fn, args tuple, patch list)
+        self._call_step: list[int] = []  # the (first) step of every call: products of a group share one
         self.has_gather = any(st.kind in ("gather", "scatter") for st in plan.steps)
         self._graphs: dict = {}  # pointer tuple -> recorded launch sequence (at most eight)
         self._seen: set = set()  # pointer tuples that have run once already
@@ -61,7 +62,8 @@ class BoundPlan:
         plan = self.plan
         dyn = set(self.dynamic)
         group_open = None  # the last launch, if products of its group may join it
-        for st in plan.steps:
+        for step_index, st in enumerate(plan.steps):
+            self._call_step.extend([step_index - 1] * (len(self.calls) - len(self._call_step)))
             a = st.attrs
             k = st.kind
             patches: list = []  # (setter(addr_of_buf)) closures
@@ -246,7 +248,17 @@ class BoundPlan:
                 if ws is not None:
                     ptr_field(d, "workspace", ws.buf, 0)
                     d.workspace_bytes = a["workspace_bytes"]
-                self.calls.append((L.nbk_gemm_nf4, [C.byref(d)], patches, d))
+                if a.get("terms"):
+                    terms = (lib.GemmTerm * len(a["terms"]))()
+                    for t, term in zip(terms, a["terms"]):
+                        for field, ref in (("A", term["a"]), ("B", term["b"])):
+                            if ref.dtype is not rx.dtype:
+                                raise TypeError(f"matmul_nf4: a further operand is {ref.dtype}, the first {rx.dtype}")
+                            ptr_field(t, field, ref.buf, ref.offset * ref.dtype.size_in_bytes)
+                        t.K, t.a_rs, t.a_cs, t.b_rs, t.b_cs = (term[f] for f in ("K", "a_rs", "a_cs", "b_rs", "b_cs"))
+                    self.calls.append((L.nbk_gemm_nf4_terms, [C.byref(d), terms, len(terms)], patches, (d, terms)))
+                else:
+                    self.calls.append((L.nbk_gemm_nf4, [C.byref(d)], patches, d))
             elif k in ("conv2d", "conv2d_dgrad", "conv2d_wgrad"):
                 d = lib.ConvDesc()
                 xs, ws, ys = a["x_shape"], a["w_shape"], a["y_shape"]
@@ -627,8 +639,11 @@ class BoundPlan:
         plan = self.plan
         base = self.base
         check = lib.check
-        for si, (fn, args, patches, _keep) in enumerate(self.calls):
-            after = timer(si, plan.steps[si].kind, stream) if timer is not None else None
+        for ci, (fn, args, patches, _keep) in enumerate(self.calls):
+            after = None
+            if timer is not None:
+                si = self._call_step[ci] if ci < len(self._call_step) else len(plan.steps) - 1
+                after = timer(si, plan.steps[si].kind, stream)
             for obj, fieldname, buf, off in patches:
                 setattr(obj, fieldname, base[buf] + off)
             if args[0] is _LATE:

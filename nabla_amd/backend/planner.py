@@ -1015,6 +1015,40 @@ class Planner:
             users[t_out.id] = []
             users[inner.outputs[0].id] = []
 
+    def _fold_thin_pair_into_nf4(self) -> None:
+        """The same on a base product whose weight is NF4-coded: the weight is decoded into scratch memory for it
+        (contractions of 128 and more), and the product out of that takes the adapter's update as one
+        more K tile.  The sum, a row kernel's or its part of one, and the thin product's launch go."""
+        nodes = self._live_nodes()
+        n_users: dict[int, int] = {}
+        for n in nodes:
+            for i in n.inputs:
+                n_users[i.id] = n_users.get(i.id, 0) + 1
+        out_ids = {v.id for v in self.outputs}
+        for n in nodes:
+            if not (n.kind == "ew" and n.fn == "add" and len(n.inputs) == 2 and
+                    all(isinstance(x, ir.Value) for x in n.attrs["operands"])):
+                continue
+            for p, t in ((n.inputs[0], n.inputs[1]), (n.inputs[1], n.inputs[0])):
+                base, thin = p.node, t.node
+                if not (base.kind == "matmul_nf4" and len(base.inputs) == 3 and thin.kind == "matmul" and
+                        len(thin.inputs) == 2 and len(thin.outputs) == 1 and
+                        not (set(thin.attrs or {}) & {"res_in", "bias_in", "act", "terms_in"}) and
+                        (thin.attrs or {}).get("alpha", 1.0) == 1.0):
+                    continue
+                u, v = thin.inputs
+                x, k2 = base.inputs[0], u.shape[-1]
+                if not (n_users.get(p.id) == n_users.get(t.id) == 1 and p.id not in out_ids and t.id not in out_ids and
+                        k2 <= 64 and k2 % 8 == 0 and v.rank == 2 and x.shape[-1] % 64 == 0 and x.shape[-1] >= 128 and
+                        u.shape[:-1] == x.shape[:-1] and p.shape == t.shape == n.outputs[0].shape and
+                        _numel(x.shape[:-1]) >= 128 and p.shape[-1] >= 128 and
+                        all(z.dtype is DType.bfloat16 for z in (x, u, v, p, t, n.outputs[0]))):
+                    continue
+                n.kind, n.fn = "matmul_nf4", None
+                n.inputs = list(base.inputs) + [u, v]
+                n.attrs = dict(base.attrs)
+                break
+
     def _fold_product_sums(self) -> None:
         """``x1 @ W1 + x2 @ W2 (+ x3 @ W3)``: a value that several products contribute to (the
         gradient of an activation that feeds the query, key and value projections:
@@ -1526,13 +1560,23 @@ class Planner:
                     writes.append(wbuf.id)
             self._emit(Step(k, [i.buf for i in ins], writes, attrs))
         elif k == "matmul_nf4":
-            x, codes, scales = (self._contig(i) for i in n.inputs)
+            x, codes, scales = (self._contig(i) for i in n.inputs[:3])
+            terms = []
+            for u, v in zip(n.inputs[3::2], n.inputs[4::2]):
+                ru, rv = self._contig(u), self._resolve(v)
+                pv = None if isinstance(rv, Const) else self._mat_operand(rv)
+                if pv is None:
+                    rv = self._materialize(rv)
+                    pv = self._mat_operand(rv)
+                terms.append(dict(a=ru, b=rv, K=u.shape[-1], a_rs=u.shape[-1], a_cs=1, b_rs=pv[1], b_cs=pv[2]))
             dst = self._alloc_value(out)
             kdim = n.inputs[0].shape[-1]
             writes = [dst.buf]
             attrs = dict(x=x, codes=codes, scales=scales, dst=dst, M=_numel(n.inputs[0].shape[:-1]), K=kdim,
                          N=out.shape[-1], w_shape=n.attrs["w_shape"], block=n.attrs["block"],
                          transpose=n.attrs["transpose"])
+            if terms:
+                attrs["terms"] = terms
             if kdim >= 128:
                 # room for the weight of this one product, decoded (the launch's rule: nbk_gemm_nf4)
                 shape = tuple(n.attrs["w_shape"])
@@ -1540,7 +1584,7 @@ class Planner:
                 attrs["workspace"] = ViewRef(wbuf.id, 0, shape, contiguous_strides(shape), out.dtype)
                 attrs["workspace_bytes"] = _numel(shape) * out.dtype.size_in_bytes
                 writes.append(wbuf.id)
-            self._emit(Step("gemm_nf4", [x.buf, codes.buf, scales.buf], writes, attrs))
+            self._emit(Step("gemm_nf4", [x.buf, codes.buf, scales.buf] + self._epi_bufs(attrs), writes, attrs))
         elif k in ("attention", "attention_bwd"):
             self._lower_attention(n)
         elif k in ("maxpool2d", "maxpool2d_bwd", "avgpool2d", "avgpool2d_bwd"):
@@ -3037,6 +3081,7 @@ def plan_graph(builder: ir.Builder, outputs: Sequence[ir.Value]) -> Plan:
         pre._fold_sum_into_matmul(thin_only=not config.FOLD_RESIDUAL)
         if config.FOLD_THIN_PAIR:
             pre._fold_thin_pair_into_matmul()
+            pre._fold_thin_pair_into_nf4()
             if config.FOLD_PRODUCT_SUMS:
                 pre._fold_product_sums()
         pre._fold_bias_into_matmul()  # (a bias on top of a sum that has just become a product)

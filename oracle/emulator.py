@@ -365,7 +365,12 @@ def _gemm_nf4(a, mem):
         w = w.to(torch.bfloat16).float()
     x = _view(mem, a["x"]).reshape(a["M"], a["K"]).double()
     w = w.double().t() if a["transpose"] else w.double()
-    dst.copy_((x @ w).reshape(dst.shape).to(dst.dtype))
+    prod = x @ w
+    for t in a.get("terms") or ():  # more operand pairs in the same accumulator
+        At = torch.as_strided(mem[t["a"].buf], (a["M"], t["K"]), (t["a_rs"], t["a_cs"]), t["a"].offset)
+        Bt = torch.as_strided(mem[t["b"].buf], (t["K"], a["N"]), (t["b_rs"], t["b_cs"]), t["b"].offset)
+        prod = prod + At.double() @ Bt.double()
+    dst.copy_(prod.reshape(dst.shape).to(dst.dtype))
 
 
 def _update_list(kind, a, mem):
