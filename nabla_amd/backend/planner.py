@@ -2067,17 +2067,20 @@ class Planner:
 
     @staticmethod
     def _split_k(M: int, N: int, K: int, dtype: DType, a_k_contiguous: bool = False,
-                 rows_contiguous: bool = False, epilogue: bool = False) -> int:
+                 rows_contiguous: bool = False, epilogue: bool = False, b_k_contiguous: bool = False) -> int:
         """Slices of the contraction axis for a product whose output has too few 128 x 128
         tiles to occupy the GPU while K is long (weight gradients: K = batch x sequence).
         ``epilogue``: what follows the product could be folded into it if it stays whole."""
         if dtype is not DType.bfloat16:
             return 1
-        if a_k_contiguous and N <= 32 and M >= 16 and K % 64 == 0 and K * (1 if N <= 16 else 2) <= 2048:
+        if a_k_contiguous and N <= 32 and M >= 16 and K % 64 == 0 and K * (1 if N <= 16 else 2) <= 4096 and (
+                b_k_contiguous or K * (1 if N == 8 else 2 if N <= 16 else 4) <= (4096 if M < 8192 or N != 8 else 2048)):
             # Products with a few columns have a kernel that splits K by itself.  Each of its workgroups
-            # reads all of B, which decides where it ends; us, whole / in the slices below and their sum:
-            # 1000 x 8 x 1024 6.5 / 8.7, 8192 x 16 x 2048 10.7 / 11.2, 1000 x 32 x 1024 7.7 / 8.8; 2000 x 32 x 2048
-            # 12.1 / 9.0, 1500 x 16 x 4096 20.2 / 8.9.
+            # reads all of B, and keeps a copy of one whose rows are columns of the result, which decides where
+            # it ends; us, whole / in the slices below and their sum.  B K-contiguous: 1000 x 8 x 4096 7.8 / 8.5,
+            # 8192 x 16 x 4096 16.5 / 18.2, 1000 x 32 x 2048 6.9 / 8.5, 2000 x 32 x 4096 11.3 / 10.1.  The other:
+            # 1000 x 8 x 1024 4.4 / 8.7, 1000 x 8 x 4096 8.3 / 8.7, 8192 x 8 x 4096 18.9 / 18.0, 8192 x 16 x 2048
+            # 8.6 / 11.1, 2000 x 16 x 4096 20.3 / 9.1, 1000 x 32 x 1024 5.7 / 8.8, 2000 x 32 x 2048 12.3 / 8.9.
             return 1
         tiles = ((M + 127) // 128) * ((N + 127) // 128)
         if rows_contiguous and 128 <= tiles <= 256 and K >= 4096:
@@ -2152,9 +2155,13 @@ class Planner:
                          out: ir.Value, epi: dict | None = None) -> None:
         """One unbatched product into contiguous storage for ``out``; split along K into fp32
         partial products plus their sum when the output alone gives too few workgroups."""
+        # (long rows that 16-byte loads cannot take stay in slices)
+        whole_chunks = pa[1] % 8 == 0 and ra.offset % 8 == 0 and rb.offset % 8 == 0 and (
+            pb[2] % 8 == 0 if pb[1] == 1 else pb[1] % 8 == 0)
         ks = self._split_k(M, N, K, ra.dtype if ra.dtype is rb.dtype else DType.float32,
-                           a_k_contiguous=pa[2] == 1,
-                           rows_contiguous=pa[1] == 1 and pa[2] != 1 and pb[2] == 1 and pb[1] != 1)
+                           a_k_contiguous=pa[2] == 1 and (K * (1 if N <= 16 else 2) <= 2048 or whole_chunks),
+                           rows_contiguous=pa[1] == 1 and pa[2] != 1 and pb[2] == 1 and pb[1] != 1,
+                           b_k_contiguous=pb[1] == 1)
         dst = self._alloc_value(out)
         common = dict(a=ra, b=rb, M=M, N=N, a_rs=pa[1], a_cs=pa[2], b_rs=pb[1], b_cs=pb[2],
                       batch_inner=1, a_bs2=0, b_bs2=0, c_bs2=0, ldc=N, c_bs=M * N, alpha=1.0)

@@ -1529,11 +1529,14 @@ __global__ __launch_bounds__(SKN_WAVES * 64) void gemm_skinny_n_kernel(const Gem
 #pragma unroll
   for (int r = 0; r < 16; ++r) red[(wave * 16 + r) * 64 + lane] = acc[r];
   __syncthreads();
-  if (wave != 0) return;
   const int64_t col = li;
   if (col >= g.N) return;
+  // Every wave adds up its share of the tile: left to one wave, the 128 reads in a row are a quarter of the launch
+  // (1000 x 8 x 1024 8.1 -> 4.4 us with the form for few rows, 8192 x 16 x 1024 7.7 -> 5.5, 8192 x 16 x 2048 10.7 ->
+  // 8.6, 20000 x 16 x 1024 15.5 -> 11.2).  Sixteen waves that halve the K of each gain nothing (4.4, 5.0, 7.4, 13.8).
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
+  for (int r0 = 0; r0 < 16 / SKN_WAVES; ++r0) {
+    const int r = wave * (16 / SKN_WAVES) + r0;
     float v = 0.f;
 #pragma unroll
     for (int w = 0; w < SKN_WAVES; ++w) v += red[(w * 16 + r) * 64 + lane];
@@ -2379,13 +2382,16 @@ static int gemm_launch(const nbk_gemm_desc* d, const GemmMembers& own, void* str
   hipStream_t st = (hipStream_t)stream;
   const int64_t batch = own.n > 0 ? own.n : d->batch;
   const bool akc = d->a_cs == 1, bkc = d->b_rs == 1, tail = d->n_terms > 0;
-  // (few rows too, where a workgroup's share of B is small: 1000 x 8 x 1024 6.5 us, in two slices and their sum 8.7)
-  const bool tall = d->M >= 1024 || (d->M >= 16 && d->K * (d->N <= 16 ? 1 : 2) <= 2048);
+  // (few rows too, where a workgroup's share of B is small, us on this kernel / on 64 x 64 tiles: 1000 x 8 x 1024
+  // 4.4 / 8.1, 1000 x 8 x 4096 8.3 / 20.3, 1000 x 32 x 2048 6.9 / 11.8; and many rows until a workgroup's copy of a
+  // B of eight columns fills the LDS: 8192 x 8 x 4096 18.9 / 20.3, 20000 x 8 x 4096 41.0 / 31.7)
+  const bool tall = d->M >= 1024 ? d->M <= 8192 || bkc || d->N > 8 || d->K < 4096
+                                 : d->M >= 16 && d->K * (d->N <= 16 ? 1 : 2) <= 4096;
   if (!tail && d->k_last == 0 && d->dtype_ab == NBK_BF16 && d->N <= 32 && tall && d->K >= 256 && d->K % 64 == 0 &&
       akc && a.a_vec && batch == 1 && d->bias == nullptr && d->residual == nullptr &&
       d->act == NBK_ACT_NONE && (bkc ? (bool)a.b_vec : (d->b_cs == 1 && d->N % 8 == 0 && a.b_vec))) {
     // 32 rows per workgroup, K split over its eight waves
-    const int pitch_chunks = d->N <= 16 ? 2 : 4;
+    const int pitch_chunks = d->N <= 8 ? 1 : d->N <= 16 ? 2 : 4;
     const size_t red = SKN_WAVES * 16 * 64 * sizeof(float);
     const size_t stage = bkc ? 0 : (size_t)d->K * pitch_chunks * 16 + 64;
     if (red + stage <= 160 * 1024 - 512 && (d->M + 31) / 32 <= 0x7fffffff) {
