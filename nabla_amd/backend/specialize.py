@@ -699,7 +699,7 @@ def write_sources(programs: dict[int, dict]) -> list[Path]:
     items = kernels_of(programs)
     files = []
     for fi in range(N_FILES):
-        chunk = items[fi::N_FILES]
+        chunk = [item for item in items if item[0] % N_FILES == fi]  # (by key: a new program changes one file)
         src = [_PRELUDE]
         for _, name, a, generic in chunk:
             src.append(f"// members: {' '.join(a.get('members', []))}")
