@@ -349,6 +349,8 @@ int nbk_gemm_nf4(const nbk_gemm_nf4_desc* d, void* stream);
  * nabla/nn/finetune/qlora.py:77-113): inside the product where the weight is decoded into a workspace, else
  * as products that add themselves. */
 int nbk_gemm_nf4_terms(const nbk_gemm_nf4_desc* d, const nbk_gemm_term* term, int32_t n_terms, void* stream);
+/* The same with a float32 C whatever the dtype, for a row program that computes on with the sum. */
+int nbk_gemm_nf4_terms_f32(const nbk_gemm_nf4_desc* d, const nbk_gemm_term* term, int32_t n_terms, void* stream);
 
 /* ===================================================================== */
 /*  Convolution / pooling (NHWC x HWIO)                                   */

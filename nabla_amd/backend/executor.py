@@ -231,7 +231,8 @@ class BoundPlan:
                 rx, rcodes, rsc, rc = a["x"], a["codes"], a["scales"], a["dst"]
                 if rcodes.dtype is not DType.uint8 or rsc.dtype is not DType.float32:
                     raise TypeError(f"matmul_nf4 wants uint8 codes and float32 scales, got {rcodes.dtype}, {rsc.dtype}")
-                if rx.dtype is not rc.dtype or rx.dtype not in (DType.bfloat16, DType.float32):
+                wide = rc.dtype is DType.float32 and rx.dtype is DType.bfloat16 and bool(a.get("terms"))
+                if not wide and (rx.dtype is not rc.dtype or rx.dtype not in (DType.bfloat16, DType.float32)):
                     raise TypeError(f"matmul_nf4 computes in bfloat16 or float32, got {rx.dtype} -> {rc.dtype}")
                 ptr_field(d, "A", rx.buf, rx.offset * rx.dtype.size_in_bytes)
                 ptr_field(d, "codes", rcodes.buf, rcodes.offset)
@@ -256,7 +257,8 @@ class BoundPlan:
                                 raise TypeError(f"matmul_nf4: a further operand is {ref.dtype}, the first {rx.dtype}")
                             ptr_field(t, field, ref.buf, ref.offset * ref.dtype.size_in_bytes)
                         t.K, t.a_rs, t.a_cs, t.b_rs, t.b_cs = (term[f] for f in ("K", "a_rs", "a_cs", "b_rs", "b_cs"))
-                    self.calls.append((L.nbk_gemm_nf4_terms, [C.byref(d), terms, len(terms)], patches, (d, terms)))
+                    self.calls.append((L.nbk_gemm_nf4_terms_f32 if wide else L.nbk_gemm_nf4_terms,
+                                       [C.byref(d), terms, len(terms)], patches, (d, terms)))
                 else:
                     self.calls.append((L.nbk_gemm_nf4, [C.byref(d)], patches, d))
             elif k in ("conv2d", "conv2d_dgrad", "conv2d_wgrad"):

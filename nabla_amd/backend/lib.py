@@ -193,6 +193,7 @@ _SIGNATURES = {
     "nbk_gemm_group": ([C.POINTER(C.POINTER(GemmDesc)), C.c_int32, C.c_void_p], C.c_int),
     "nbk_gemm_members": ([C.POINTER(GemmDesc), C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p], C.c_int),
     "nbk_gemm_nf4_terms": ([C.POINTER(GemmNf4Desc), C.POINTER(GemmTerm), C.c_int32, C.c_void_p], C.c_int),
+    "nbk_gemm_nf4_terms_f32": ([C.POINTER(GemmNf4Desc), C.POINTER(GemmTerm), C.c_int32, C.c_void_p], C.c_int),
     "nbk_gemm_nf4": ([C.POINTER(GemmNf4Desc), C.c_void_p], C.c_int),
     "nbk_conv2d_fwd": ([C.POINTER(ConvDesc), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                         C.c_void_p], C.c_int),

@@ -1018,12 +1018,23 @@ class Planner:
     def _fold_thin_pair_into_nf4(self) -> None:
         """The same on a base product whose weight is NF4-coded: the weight is decoded into scratch memory for it
         (contractions of 128 and more), and the product out of that takes the adapter's update as one
-        more K tile.  The sum, a row kernel's or its part of one, and the thin product's launch go."""
+        more K tile.  The thin product's launch goes, and the sum: a row kernel, or its part of one.
+
+        A row program that made the sum computed on with it in float32.  What is left of that program reads
+        the product in float32 and rounds where the sum was stored.  (Rounded to bf16 in between: a GELU of 5000 x
+        1024 2.6e-3 from float64 instead of 2.5e-3, and gradients behind it 3.4e-4 too large throughout.)"""
         nodes = self._live_nodes()
         n_users: dict[int, int] = {}
+        readers: dict[int, list[ir.Node]] = {}
         for n in nodes:
             for i in n.inputs:
                 n_users[i.id] = n_users.get(i.id, 0) + 1
+                readers.setdefault(i.id, []).append(n)
+
+        def computed_on(v: ir.Value) -> bool:
+            return any(r.kind in FUSABLE or (r.kind in VIEW_KINDS and computed_on(r.outputs[0]))
+                       for r in readers.get(v.id, ()))
+
         out_ids = {v.id for v in self.outputs}
         for n in nodes:
             if not (n.kind == "ew" and n.fn == "add" and len(n.inputs) == 2 and
@@ -1044,9 +1055,14 @@ class Planner:
                         _numel(x.shape[:-1]) >= 128 and p.shape[-1] >= 128 and
                         all(z.dtype is DType.bfloat16 for z in (x, u, v, p, t, n.outputs[0]))):
                     continue
-                n.kind, n.fn = "matmul_nf4", None
-                n.inputs = list(base.inputs) + [u, v]
-                n.attrs = dict(base.attrs)
+                whole = n
+                if computed_on(n.outputs[0]):
+                    whole = base if base.pos > thin.pos else thin  # (what both read is there before the later one)
+                    total = whole.outputs[0]
+                    total.dtype = DType.float32
+                    n.fn, n.inputs, n.attrs = "mov", [total], dict(operands=(total,))
+                whole.kind, whole.fn = "matmul_nf4", None
+                whole.inputs, whole.attrs = list(base.inputs) + [u, v], dict(base.attrs)
                 break
 
     def _fold_product_sums(self) -> None:
@@ -1580,9 +1596,9 @@ class Planner:
             if kdim >= 128:
                 # room for the weight of this one product, decoded (the launch's rule: nbk_gemm_nf4)
                 shape = tuple(n.attrs["w_shape"])
-                wbuf = self._new_buf(shape, out.dtype)
-                attrs["workspace"] = ViewRef(wbuf.id, 0, shape, contiguous_strides(shape), out.dtype)
-                attrs["workspace_bytes"] = _numel(shape) * out.dtype.size_in_bytes
+                wbuf = self._new_buf(shape, x.dtype)
+                attrs["workspace"] = ViewRef(wbuf.id, 0, shape, contiguous_strides(shape), x.dtype)
+                attrs["workspace_bytes"] = _numel(shape) * x.dtype.size_in_bytes
                 writes.append(wbuf.id)
             self._emit(Step("gemm_nf4", [x.buf, codes.buf, scales.buf] + self._epi_bufs(attrs), writes, attrs))
         elif k in ("attention", "attention_bwd"):

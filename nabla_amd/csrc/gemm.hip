@@ -2739,14 +2739,15 @@ __global__ __launch_bounds__(256) void nf4_decode_kernel(const uint8_t* codes, c
 }
 
 // Further operand pairs of a product that has been launched: each adds itself to the result.
-static int nf4_add_terms(const nbk_gemm_nf4_desc* d, int64_t N, const nbk_gemm_term* term, int n_terms, void* stream) {
+static int nf4_add_terms(const nbk_gemm_nf4_desc* d, int dtype_c, int64_t N, const nbk_gemm_term* term, int n_terms,
+                         void* stream) {
   for (int i = 0; i < n_terms; ++i) {
     nbk_gemm_desc p = {};
     p.A = term[i].A; p.B = term[i].B; p.C = d->C; p.residual = d->C;
     p.M = d->M; p.N = N; p.K = term[i].K;
     p.a_rs = term[i].a_rs; p.a_cs = term[i].a_cs; p.b_rs = term[i].b_rs; p.b_cs = term[i].b_cs;
     p.ldc = d->ldc; p.batch = 1; p.batch_inner = 1;
-    p.dtype_ab = d->dtype; p.dtype_c = d->dtype; p.alpha = 1.f;
+    p.dtype_ab = d->dtype; p.dtype_c = dtype_c; p.alpha = 1.f;
     const int rc = nbk_gemm(&p, stream);
     if (rc != NBK_OK) return rc;
   }
@@ -2755,7 +2756,7 @@ static int nf4_add_terms(const nbk_gemm_nf4_desc* d, int64_t N, const nbk_gemm_t
 
 // (The update of an adapter as one more K tile of the product out of the workspace: 1000 x 1024 x 4096 with rank 8
 // 17.4 + 9.2 us in two launches and 7 of the sum in a row kernel, then 18.)
-static int gemm_nf4(const nbk_gemm_nf4_desc* d, const nbk_gemm_term* term, int n_terms, void* stream) {
+static int gemm_nf4(const nbk_gemm_nf4_desc* d, bool c_f32, const nbk_gemm_term* term, int n_terms, void* stream) {
   NBK_REQUIRE(d != nullptr, "gemm_nf4: null descriptor");
   NBK_REQUIRE(n_terms >= 0 && n_terms <= NBK_GEMM_MAX_TERMS && (n_terms == 0 || (term != nullptr && d->alpha == 1.f)),
               "gemm_nf4: %d further pairs, with alpha 1 only", n_terms);
@@ -2766,6 +2767,7 @@ static int gemm_nf4(const nbk_gemm_nf4_desc* d, const nbk_gemm_term* term, int n
               "gemm_nf4: the block length (%d) and the weight's width (%lld) must be multiples of 8",
               d->block, (long long)d->w_cols);
   NBK_REQUIRE(((uintptr_t)d->codes & 7) == 0, "gemm_nf4: codes must be 8-byte aligned");
+  const int dtype_c = c_f32 ? NBK_F32 : d->dtype;
   // C = A @ W (K = rows of W, N = its columns) or A @ W^T (K = columns of W, N = its rows)
   const int64_t K = d->transpose_w ? d->w_cols : d->w_rows;
   const int64_t N = d->transpose_w ? d->w_rows : d->w_cols;
@@ -2796,14 +2798,14 @@ static int gemm_nf4(const nbk_gemm_nf4_desc* d, const nbk_gemm_term* term, int n
     p.b_rs = d->transpose_w ? 1 : d->w_cols;
     p.b_cs = d->transpose_w ? d->w_cols : 1;
     p.ldc = d->ldc; p.batch = 1; p.batch_inner = 1;
-    p.dtype_ab = d->dtype; p.dtype_c = d->dtype; p.alpha = d->alpha;
+    p.dtype_ab = d->dtype; p.dtype_c = dtype_c; p.alpha = d->alpha;
     if (d->dtype == NBK_BF16) {
       p.n_terms = n_terms;
       for (int i = 0; i < n_terms; ++i) p.term[i] = term[i];
       return nbk_gemm(&p, stream);
     }
     const int prc = nbk_gemm(&p, stream);
-    return prc != NBK_OK ? prc : nf4_add_terms(d, N, term, n_terms, stream);
+    return prc != NBK_OK ? prc : nf4_add_terms(d, dtype_c, N, term, n_terms, stream);
   }
   GemmArgs a = {};
   a.A = d->A; a.B = d->codes; a.C = d->C;
@@ -2813,7 +2815,7 @@ static int gemm_nf4(const nbk_gemm_nf4_desc* d, const nbk_gemm_term* term, int n
   a.b_rs = d->transpose_w ? 1 : d->w_cols;
   a.b_cs = d->transpose_w ? d->w_cols : 1;
   a.ldc = d->ldc; a.batch_inner = 1;
-  a.dtype_c = d->dtype; a.act = NBK_ACT_NONE; a.alpha = d->alpha;
+  a.dtype_c = dtype_c; a.act = NBK_ACT_NONE; a.alpha = d->alpha;
   a.b_scales = (const float*)d->scales; a.b_block = d->block;
   a.a_vec = ((uintptr_t)d->A % 16 == 0) && (d->lda % (d->dtype == NBK_F32 ? 4 : 8) == 0);
   a.b_vec = 0;
@@ -2827,7 +2829,7 @@ static int gemm_nf4(const nbk_gemm_nf4_desc* d, const nbk_gemm_term* term, int n
     if (bkc) hipLaunchKernelGGL((gemm_f32_nf4_kernel<true>), grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL((gemm_f32_nf4_kernel<false>), grid, dim3(256), 0, st, a);
     const int krc = nbk_check_launch("gemm_f32_nf4_kernel");
-    return krc != NBK_OK ? krc : nf4_add_terms(d, N, term, n_terms, stream);
+    return krc != NBK_OK ? krc : nf4_add_terms(d, dtype_c, N, term, n_terms, stream);
   }
   const size_t pipe = 2 * (size_t)(TileGeom<128, true>::CHUNKS +
                                    (bkc ? TileGeom<128, true>::CHUNKS : TileGeom<128, false>::CHUNKS)) * 16;
@@ -2848,10 +2850,13 @@ static int gemm_nf4(const nbk_gemm_nf4_desc* d, const nbk_gemm_term* term, int n
   else NBK_LAUNCH_NF4(false);
 #undef NBK_LAUNCH_NF4
   const int krc = nbk_check_launch("gemm_bf16_kernel (nf4)");
-  return krc != NBK_OK ? krc : nf4_add_terms(d, N, term, n_terms, stream);
+  return krc != NBK_OK ? krc : nf4_add_terms(d, dtype_c, N, term, n_terms, stream);
 }
 
-extern "C" int nbk_gemm_nf4(const nbk_gemm_nf4_desc* d, void* stream) { return gemm_nf4(d, nullptr, 0, stream); }
+extern "C" int nbk_gemm_nf4(const nbk_gemm_nf4_desc* d, void* stream) { return gemm_nf4(d, false, nullptr, 0, stream); }
 extern "C" int nbk_gemm_nf4_terms(const nbk_gemm_nf4_desc* d, const nbk_gemm_term* term, int32_t n_terms, void* stream) {
-  return gemm_nf4(d, term, n_terms, stream);
+  return gemm_nf4(d, false, term, n_terms, stream);
+}
+extern "C" int nbk_gemm_nf4_terms_f32(const nbk_gemm_nf4_desc* d, const nbk_gemm_term* term, int32_t n_terms, void* stream) {
+  return gemm_nf4(d, true, term, n_terms, stream);
 }

@@ -361,7 +361,7 @@ def _gemm_nf4(a, mem):
     scales = _view(mem, a["scales"]).reshape(-1).float()
     w = (_NF4_LEVELS[codes].reshape(-1, a["block"]) * scales[:, None]).reshape(a["w_shape"])
     dst = _view(mem, a["dst"])
-    if dst.dtype == torch.bfloat16:  # level * scale is rounded to bf16 once, as in the kernel
+    if _view(mem, a["x"]).dtype == torch.bfloat16:  # level * scale is rounded to bf16 once, as in the kernel
         w = w.to(torch.bfloat16).float()
     x = _view(mem, a["x"]).reshape(a["M"], a["K"]).double()
     w = w.double().t() if a["transpose"] else w.double()

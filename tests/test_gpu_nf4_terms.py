@@ -51,3 +51,34 @@ def test_update_inside(hip, M, rows, cols, ranks, workspace, dtype, transpose):
     # once more for each pair that does not go inside it
     rounds = (2.0 ** -9 * (1 + len(ranks)) if dtype == "bfloat16" else 0.0)
     assert ((out.double() - want).abs() <= 2.0 ** -20 * size + rounds * size.clamp(min=1e-6).minimum(want.abs() + 2.0 ** -1 * size)).all()
+
+
+@pytest.mark.parametrize("transpose", [0, 1])
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("M,rows,cols,rank", [(1000, 256, 640, 8), (129, 128, 136, 64), (77, 64, 136, 8), (300, 320, 192, 5)])
+def test_float32_result_of_bf16_operands(hip, M, rows, cols, rank, workspace, transpose):
+    """Nothing is rounded to bf16 but the operands."""
+    import nabla_amd as nb
+    from nabla_amd.backend import lib
+    gen = torch.Generator(device="cuda").manual_seed(M + cols)
+    K, N = (cols, rows) if transpose else (rows, cols)
+    codes = torch.randint(0, 16, (rows * cols,), generator=gen, device="cuda").to(torch.uint8)
+    scales = torch.rand(rows * cols // 64, generator=gen, device="cuda") + 0.5
+    level = torch.from_numpy(np.asarray(nb.nn.finetune.qlora.NF4_CODEBOOK, np.float32)).cuda()
+    w = (level[codes.long()].view(-1, 64) * scales[:, None]).view(rows, cols).to(torch.bfloat16).double()
+    w = w.t().contiguous() if transpose else w
+    x, u, v = (torch.randn(s, generator=gen, device="cuda").to(torch.bfloat16) for s in ((M, K), (M, rank), (rank, N)))
+    stored = v.t().contiguous() if transpose else v
+    out, ws = torch.full((M, N), float("nan"), device="cuda"), torch.empty(rows * cols, dtype=torch.bfloat16, device="cuda")
+    d = lib.GemmNf4Desc()
+    d.A, d.codes, d.scales, d.C = x.data_ptr(), codes.data_ptr(), scales.data_ptr(), out.data_ptr()
+    d.M, d.w_rows, d.w_cols, d.lda, d.ldc, d.block, d.transpose_w, d.dtype, d.alpha = M, rows, cols, K, N, 64, transpose, 1, 1.0
+    if workspace:
+        d.workspace, d.workspace_bytes = ws.data_ptr(), 2 * ws.numel()
+    terms = (lib.GemmTerm * 1)()
+    terms[0].A, terms[0].B, terms[0].K, terms[0].a_rs, terms[0].a_cs = u.data_ptr(), stored.data_ptr(), rank, rank, 1
+    terms[0].b_rs, terms[0].b_cs = (1, rank) if transpose else (N, 1)
+    lib.check(lib.load().nbk_gemm_nf4_terms_f32(C.byref(d), terms, 1, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    size = x.double().abs() @ w.abs() + u.double().abs() @ v.double().abs()
+    # (704 exact products at most, added in float32: 2^-24 of all that is added for each of up to 16 steps of a chain)
+    assert ((out.double() - (x.double() @ w + u.double() @ v.double())).abs() <= 2.0 ** -20 * size).all()
