@@ -317,7 +317,7 @@ int nbk_gemm(const nbk_gemm_desc* d, void* stream);
 int nbk_gemm_group(const nbk_gemm_desc* const* d, int32_t n, void* stream);
 /* 2 to 4 products of one A in one launch (the projections of a layer to queries, keys and values:
  * nabla/nn/functional/layers.py): product i has B[i], bias[i] (NULL: none) and C[i]; sizes, strides, dtypes, alpha
- * and act are d's and the same for all (d->B, d->bias and d->C are not read).  batch 1, no residual, second
+ * and act are d's and the same for all (d->B, d->bias, d->C and batch strides are not read).  batch 1, no residual, second
  * result, column sums, further operand pairs or k_last, and the C lie a multiple of 16 bytes apart. */
 int nbk_gemm_members(const nbk_gemm_desc* d, int32_t n, const void* const* B, const void* const* bias,
                      void* const* C, void* stream);

@@ -2308,7 +2308,9 @@ static int gemm_prepare(const nbk_gemm_desc* d, const GemmMembers& own, GemmArgs
   a.A = d->A; a.B = d->B; a.C = d->C; a.bias = d->bias; a.residual = d->residual;
   a.M = d->M; a.N = d->N; a.K = d->K;
   a.a_rs = d->a_rs; a.a_cs = d->a_cs; a.b_rs = d->b_rs; a.b_cs = d->b_cs; a.ldc = d->ldc;
-  a.a_bs = d->a_bs; a.b_bs = d->b_bs; a.c_bs = d->c_bs;
+  if (members == 0) {  // (the products of one A have one A and their own pointers to the rest)
+    a.a_bs = d->a_bs; a.b_bs = d->b_bs; a.c_bs = d->c_bs;
+  }
   a.batch_inner = d->batch_inner > 1 ? d->batch_inner : 1;
   NBK_REQUIRE(d->batch % a.batch_inner == 0, "gemm: batch %lld is not a multiple of batch_inner %lld",
               (long long)d->batch, (long long)a.batch_inner);
@@ -2355,8 +2357,8 @@ static int gemm_prepare(const nbk_gemm_desc* d, const GemmMembers& own, GemmArgs
     const int64_t q = 16 / esz;
     return ((uintptr_t)p % 16 == 0) && (other_stride % q == 0) && (bs % q == 0) && (bs2 % q == 0);
   };
-  a.a_vec = vec_ok(d->A, akc ? d->a_rs : d->a_cs, d->a_bs, a.a_bs2);
-  a.b_vec = vec_ok(d->B, bkc ? d->b_cs : d->b_rs, d->b_bs, a.b_bs2);
+  a.a_vec = vec_ok(d->A, akc ? d->a_rs : d->a_cs, a.a_bs, a.a_bs2);
+  a.b_vec = vec_ok(d->B, bkc ? d->b_cs : d->b_rs, a.b_bs, a.b_bs2);
   const int esz_c = d->dtype_c == NBK_F32 ? 4 : 2;
   a.n_members = members;
   for (int i = 0; i < members; ++i) {

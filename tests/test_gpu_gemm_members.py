@@ -48,3 +48,41 @@ def test_against_the_products_alone(hip, M, N, K, n, layout, dtype):
     assert L.nbk_gemm_members(C.byref(d), n, *at, None) != 0
     d.batch = 1
     assert L.nbk_gemm_members(C.byref(d), 5, *at, None) != 0 and L.nbk_gemm_members(C.byref(d), 1, *at, None) != 0
+
+
+def launched(lib, a, bs, layout="nn", **fields):
+    """Products of ``a`` with each of ``bs`` in one launch (one: nbk_gemm)."""
+    M, K = a.shape
+    N = bs[0].shape[0] if layout == "nt" else bs[0].shape[1]
+    out = torch.full((len(bs), M, N), float("nan"), dtype=a.dtype, device="cuda")
+    d = lib.GemmDesc()
+    d.A, d.M, d.N, d.K, d.a_rs, d.a_cs, d.ldc = a.data_ptr(), M, N, K, K, 1, N
+    d.b_rs, d.b_cs = (1, K) if layout == "nt" else (N, 1)
+    code = int(a.dtype == torch.bfloat16)
+    d.batch, d.dtype_ab, d.dtype_c, d.alpha = 1, code, code, 1.0
+    for field, value in fields.items():
+        setattr(d, field, value)
+    L, stream = lib.load(), C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    if len(bs) == 1:
+        d.B, d.C = bs[0].data_ptr(), out.data_ptr()
+        lib.check(L.nbk_gemm(C.byref(d), stream))
+        return out
+    p = lib.GemmMembers()
+    for i, b in enumerate(bs):
+        setattr(p, f"B{i}", b.data_ptr())
+        setattr(p, f"C{i}", out[i].data_ptr())
+    at = [C.byref(p, getattr(lib.GemmMembers, f).offset) for f in ("B0", "bias0", "C0")]
+    lib.check(L.nbk_gemm_members(C.byref(d), len(bs), *at, stream))
+    return out
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_batch_strides_are_not_looked_at(hip, dtype):
+    """There is no batch: strides left in the description reach neither A nor the choice of a kernel."""
+    from nabla_amd.backend import lib
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    t = getattr(torch, dtype)
+    room = torch.randn(4 * 200 * 64, generator=gen, device="cuda").to(t)  # (as far as three strides of A reach)
+    a, bs = room[:200 * 64].view(200, 64), [torch.randn(64, 72, generator=gen, device="cuda").to(t) for _ in range(3)]
+    got = launched(lib, a, bs, a_bs=200 * 64, b_bs=3, c_bs=5)
+    assert torch.equal(got, launched(lib, a, bs)) and not got.isnan().any()
