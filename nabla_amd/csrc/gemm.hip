@@ -2384,6 +2384,32 @@ static bool gemm_direct(const nbk_gemm_desc* d, const GemmArgs& a) {
          a_stride >= 0 && b_stride >= 0 && a_stride < (1 << 22) && b_stride < (1 << 22);
 }
 
+// How a float32 product is added up: tiles of 16 or 32 by so many waves, each with a share of K, on the float32
+// instruction, or out of bf16 parts.  A function of the product alone: products that share a launch (nbk_gemm_members,
+// nbk_gemm_group) have the sums they have by themselves.
+enum F32Form { F32_16_BY_16, F32_16_BY_8, F32_32_BY_8, F32_32_BY_4, F32_PARTS };
+static F32Form gemm_f32_form(int64_t M, int64_t N, int64_t K, int64_t batch) {
+  // Out of bf16 parts where a launch gives most CUs a tile of 64 x 64; below that the K loop of one workgroup
+  // is what a launch waits for, and four waves that share a fragment of 32 x 32 on the float32
+  // instruction have the shorter one.  us, 32 x 32 / 64 x 64 out of parts: 1024 x 512 x 512 (128 tiles of 64)
+  // 12.9 / 15.9, 512 x 2048 x 1024 (256) 34 / 27 and as x^T dy 40 / 27, 1024 x 1024 x 200 (256) 15.1 / 10.3.
+  // Tiles of 64 that are half padding are no more work than two of 32: 300 x (20 x 20 x 64) 4.8 / 7.4, 128 x (32 x 128 x
+  // 64) 5.1 / 6.9, 32 x 16384 x 1024 20 / 26, 64 x (16 x 224 x 704) 16.5 / 20; past two of 32 to a CU the two are even (8 x
+  // 32768 x 256 12.6 / 12.5, 64 x (40 x 224 x 704) 27 / 21).
+  auto tiles = [&](int64_t edge) { return ((M + edge - 1) / edge) * ((N + edge - 1) / edge) * batch; };
+  const int64_t cus = nbk_num_cus(), t16 = tiles(16), t32 = tiles(32);
+  if (tiles(64) * 4 >= cus * 3 && t32 > 2 * cus) return F32_PARTS;
+  // The float32 instruction does 256 operations a cycle and CU, so a tile's K loop on one CU is bound by it:
+  // tiles of 16 x 16 while two to a CU hold the result spread it over four times as many.  us, tiles of 32
+  // by four waves / 16 by eight: 128 x 256 x 784 (128 tiles of 16) 10.8 / 6.1, 300 x 300 x 300 (361) 7.0 / 5.6,
+  // 2048 x 64 x 1024 (512) 12.2 / 8.2, 784 x 256 x 128 (784) 4.8 / 5.8; the longest contractions by sixteen waves:
+  // 128 x 128 x 4096 36.7 / 15.6 / 13.3.  Tiles of 32 by eight waves, where a CU holds all its workgroups and
+  // a K tile of 128 is filled: 512 x 512 x 1024 (256 tiles) 12.0 / 10.8, 1024 x 512 x 2048 (512) 32.1 / 31.1 (K-contiguous
+  // 28.9 / 26.5); 64 x (96 x 64 x 96) (384) 6.2 / 6.9, 16 x (300 x 64 x 300) (320) 9.0 / 9.4.
+  if (t16 <= 2 * cus) return t16 <= cus && K >= 2048 ? F32_16_BY_16 : F32_16_BY_8;
+  return K >= 128 && (t32 <= cus || (t32 <= 2 * cus && K % 128 == 0)) ? F32_32_BY_8 : F32_32_BY_4;
+}
+
 static int gemm_launch(const nbk_gemm_desc* d, const GemmMembers& own, void* stream) {
   GemmArgs a;
   { const int rc = gemm_prepare(d, own, a); if (rc != NBK_OK) return rc; }
@@ -2559,36 +2585,19 @@ static int gemm_launch(const nbk_gemm_desc* d, const GemmMembers& own, void* str
     return one_round ? launch_bf16_dl<128, 128, 4, 1, false, 4>(a, akc, bkc, batch, st)
                      : launch_bf16_dl<128, 128, 4, 1, false>(a, akc, bkc, batch, st);
   }
-  // Out of bf16 parts where a launch gives most CUs a tile of 64 x 64; below that the K loop of one workgroup
-  // is what a launch waits for, and four waves that share a fragment of 32 x 32 on the float32
-  // instruction have the shorter one.  us, 32 x 32 / 64 x 64 out of parts: 1024 x 512 x 512 (128 tiles of 64)
-  // 12.9 / 15.9, 512 x 2048 x 1024 (256) 34 / 27 and as x^T dy 40 / 27, 1024 x 1024 x 200 (256) 15.1 / 10.3.
-  // Tiles of 64 that are half padding are no more work than two of 32: 300 x (20 x 20 x 64) 4.8 / 7.4, 128 x (32 x 128 x
-  // 64) 5.1 / 6.9, 32 x 16384 x 1024 20 / 26, 64 x (16 x 224 x 704) 16.5 / 20; past two of 32 to a CU the two are even (8 x
-  // 32768 x 256 12.6 / 12.5, 64 x (40 x 224 x 704) 27 / 21).
+  const int64_t cus = nbk_num_cus();
+  switch (gemm_f32_form(d->M, d->N, d->K, d->batch)) {
+    case F32_16_BY_16: return launch_f32<16, 16>(a, akc, bkc, batch, st);
+    case F32_16_BY_8: return launch_f32<16, 8>(a, akc, bkc, batch, st);
+    case F32_32_BY_8: return launch_f32<32, 8>(a, akc, bkc, batch, st);
+    case F32_32_BY_4: return launch_f32<32, 4>(a, akc, bkc, batch, st);
+    default: break;
+  }
   // 128 x 128 tiles run one to a CU, two of 64 x 64 do; a round of the former does the work of two of the
   // latter in 1.7 of one's time: 4096 x 4096 x 1024 (4 rounds / 8) 197 / 251, 4096 x 1024 x 64 (1 / 2) 12.4 /
-  // 14.2, 64 x (333 x 333 x 64) (3 / 5) 33 / 29, 2048 x 1024 x 1024 (1 / 1) 44 / 39.
+  // 14.2, 64 x (333 x 333 x 64) (3 / 5) 33 / 29, 2048 x 1024 x 1024 (1 / 1) 44 / 39.  (A sum is the same in either.)
   auto tiles = [&](int64_t edge) { return ((d->M + edge - 1) / edge) * ((d->N + edge - 1) / edge) * batch; };
-  const int64_t cus = nbk_num_cus(), t64 = tiles(64);
-  const int64_t t32 = tiles(32);
-  if (t64 * 4 < cus * 3 || t32 <= 2 * cus) {
-    // The float32 instruction does 256 operations a cycle and CU, so a tile's K loop on one CU is bound by it:
-    // tiles of 16 x 16 while two to a CU hold the result spread it over four times as many.  us, tiles of 32
-    // by four waves / 16 by eight: 128 x 256 x 784 (128 tiles of 16) 10.8 / 6.1, 300 x 300 x 300 (361) 7.0 / 5.6,
-    // 2048 x 64 x 1024 (512) 12.2 / 8.2, 784 x 256 x 128 (784) 4.8 / 5.8; the longest contractions by sixteen waves:
-    // 128 x 128 x 4096 36.7 / 15.6 / 13.3.  Tiles of 32 by eight waves, where a CU holds all its workgroups and
-    // a K tile of 128 is filled: 512 x 512 x 1024 (256 tiles) 12.0 / 10.8, 1024 x 512 x 2048 (512) 32.1 / 31.1 (K-contiguous
-    // 28.9 / 26.5); 64 x (96 x 64 x 96) (384) 6.2 / 6.9, 16 x (300 x 64 x 300) (320) 9.0 / 9.4.
-    const int64_t t16 = tiles(16);
-    if (t16 <= 2 * cus)
-      return t16 <= cus && d->K >= 2048 ? launch_f32<16, 16>(a, akc, bkc, batch, st)
-                                        : launch_f32<16, 8>(a, akc, bkc, batch, st);
-    if (d->K >= 128 && (t32 <= cus || (t32 <= 2 * cus && d->K % 128 == 0)))
-      return launch_f32<32, 8>(a, akc, bkc, batch, st);
-    return launch_f32<32, 4>(a, akc, bkc, batch, st);
-  }
-  const int64_t rounds_64 = (t64 + 2 * cus - 1) / (2 * cus), rounds_128 = (tiles(128) + cus - 1) / cus;
+  const int64_t rounds_64 = (tiles(64) + 2 * cus - 1) / (2 * cus), rounds_128 = (tiles(128) + cus - 1) / cus;
   if (rounds_128 * 17 <= rounds_64 * 10) return launch_f32_split<128, 128, 2, 4, 2>(a, akc, bkc, batch, st);
   return launch_f32_split<64, 64, 2, 2, 2>(a, akc, bkc, batch, st);
 }
@@ -2625,7 +2634,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_group_kernel(const GemmGroup G)
   });
 }
 template <int T, int WK>
-__global__ __launch_bounds__(64 * WK, 2) void gemm_f32_group_kernel(const GemmGroup G) {
+__global__ __launch_bounds__(64 * WK, WK > 8 ? 1 : 2) void gemm_f32_group_kernel(const GemmGroup G) {
   gemm_group_run(G, [](const GemmArgs& g, int bx, int by, int ny) { gemm_f32_body<false, false, T, WK>(g, bx, by, ny); });
 }
 __global__ __launch_bounds__(256) void gemm_f32_split_group_kernel(const GemmGroup G) {
@@ -2664,8 +2673,9 @@ extern "C" int nbk_gemm_group(const nbk_gemm_desc* const* d, int32_t n, void* st
   for (int32_t base = 0; base < n; base += GEMM_GROUP_MAX) {
     GemmGroup G;
     G.n = n - base < GEMM_GROUP_MAX ? n - base : GEMM_GROUP_MAX;
-    bool together = G.n > 1, narrow = false, deep = false, long_k = true, whole_k = true;
-    int64_t t16 = 0, t32 = 0, t64 = 0, t128 = 0;
+    bool together = G.n > 1, narrow = false, deep = false, long_k = true;
+    int64_t t64 = 0, t128 = 0;
+    F32Form form[GEMM_GROUP_MAX];
     const int ab = d[base] != nullptr ? d[base]->dtype_ab : -1;
     for (int i = 0; i < G.n; ++i) {
       const nbk_gemm_desc* p = d[base + i];
@@ -2677,11 +2687,11 @@ extern "C" int nbk_gemm_group(const nbk_gemm_desc* const* d, int32_t n, void* st
                  (ab == NBK_F32 || (gemm_direct(p, G.a[i]) && (p->colsum == nullptr || p->alpha == 1.f)));
       G.batch[i] = (int32_t)p->batch;
       auto tiles = [&](int64_t edge) { return ((p->M + edge - 1) / edge) * ((p->N + edge - 1) / edge) * p->batch; };
-      t16 += tiles(16); t32 += tiles(32); t64 += tiles(64); t128 += tiles(128);
+      t64 += tiles(64); t128 += tiles(128);
+      form[i] = gemm_f32_form(p->M, p->N, p->K, p->batch);
       narrow = narrow || p->M <= 64 || p->N <= 64;
       deep = deep || p->K > 512;
       long_k = long_k && p->K >= 512;
-      whole_k = whole_k && p->K % 128 == 0;
     }
     int rc = NBK_OK;
     hipStream_t st = (hipStream_t)stream;
@@ -2694,12 +2704,26 @@ extern "C" int nbk_gemm_group(const nbk_gemm_desc* const* d, int32_t n, void* st
       else if (t64 <= 2 * cus) rc = launch_bf16_group<64, 128, 4>(G, st);
       else if (t128 <= cus) rc = launch_bf16_group<128, 128, 4>(G, st);
       else rc = launch_bf16_group<128, 128, 2>(G, st);
-    } else if (t16 <= 2 * cus) {
-      rc = launch_f32_group<16, 8>(G, st);
-    } else if (t64 * 4 < cus * 3 || t32 <= 2 * cus) {
-      rc = t32 <= cus || whole_k ? launch_f32_group<32, 8>(G, st) : launch_f32_group<32, 4>(G, st);
-    } else {
-      rc = launch_group(gemm_f32_split_group_kernel, G, 64, 64, 256, 2 * (64 + 64) * 12 * 16, st);
+    } else {  // (those that are added up alike share a launch)
+      for (F32Form of : {F32_16_BY_16, F32_16_BY_8, F32_32_BY_8, F32_32_BY_4, F32_PARTS}) {
+        GemmGroup F;
+        F.n = 0;
+        int last = 0;
+        for (int i = 0; i < G.n; ++i) {
+          if (form[i] != of) continue;
+          F.a[F.n] = G.a[i];
+          F.batch[F.n++] = G.batch[i];
+          last = i;
+        }
+        if (F.n == 0) continue;
+        if (F.n == 1) rc = nbk_gemm(d[base + last], stream);
+        else if (of == F32_16_BY_16) rc = launch_f32_group<16, 16>(F, st);
+        else if (of == F32_16_BY_8) rc = launch_f32_group<16, 8>(F, st);
+        else if (of == F32_32_BY_8) rc = launch_f32_group<32, 8>(F, st);
+        else if (of == F32_32_BY_4) rc = launch_f32_group<32, 4>(F, st);
+        else rc = launch_group(gemm_f32_split_group_kernel, F, 64, 64, 256, 2 * (64 + 64) * 12 * 16, st);
+        if (rc != NBK_OK) return rc;
+      }
     }
     if (rc != NBK_OK) return rc;
   }

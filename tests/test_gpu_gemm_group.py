@@ -102,3 +102,35 @@ def test_a_step_reads_its_groups(hip):
             assert np.abs(g.numpy() - w.grad.numpy()).max() <= 1e-5 * w.grad.abs().max()
     groups = [s.attrs["group"] for bp in engine._PLAN_CACHE.values() for s in bp.plan.steps if s.attrs.get("group")]
     assert len(groups) >= 4
+
+
+def products(lib, dtype, pairs, alpha=1.0, together=True):
+    """x^T dy of every pair, in one call or one by one."""
+    L, stream = lib.load(), C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    outs, ptrs = [], (C.POINTER(lib.GemmDesc) * len(pairs))()
+    for i, (a, b) in enumerate(pairs):
+        (K, M), N = a.shape, b.shape[1]
+        outs.append(torch.full((M, N), float("nan"), device="cuda"))
+        d = lib.GemmDesc()
+        d.A, d.B, d.C = a.data_ptr(), b.data_ptr(), outs[i].data_ptr()
+        d.M, d.N, d.K, d.a_rs, d.a_cs, d.b_rs, d.b_cs, d.ldc = M, N, K, 1, M, N, 1, N
+        d.batch, d.batch_inner, d.dtype_ab, d.dtype_c, d.alpha = 1, 1, dtype, 0, alpha
+        ptrs[i] = C.pointer(d)
+        if not together:
+            lib.check(L.nbk_gemm(ptrs[i], stream))
+    if together:
+        lib.check(L.nbk_gemm_group(ptrs, len(pairs), stream))
+    return outs
+
+
+FORMS = [(512, 512, 1024), (512, 2048, 1024), (200, 100, 300), (64, 64, 3000), (500, 400, 131), (512, 512, 640), (33, 1, 57),
+         (128, 32, 2200), (2048, 512, 1024), (400, 600, 100)]
+
+
+def test_float32_sums_are_those_of_the_products_alone(hip):
+    """Bit for bit, whatever else is in the launch."""
+    from nabla_amd.backend import lib
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    pairs = [tuple(torch.rand(K, n, generator=gen, device="cuda") for n in (M, N)) for M, N, K in FORMS]
+    for got, alone in zip(products(lib, 0, pairs), products(lib, 0, pairs, together=False)):
+        assert torch.equal(got, alone), tuple(got.shape)

@@ -86,3 +86,12 @@ def test_batch_strides_are_not_looked_at(hip, dtype):
     a, bs = room[:200 * 64].view(200, 64), [torch.randn(64, 72, generator=gen, device="cuda").to(t) for _ in range(3)]
     got = launched(lib, a, bs, a_bs=200 * 64, b_bs=3, c_bs=5)
     assert torch.equal(got, launched(lib, a, bs)) and not got.isnan().any()
+
+
+@pytest.mark.parametrize("M,N,K", [(1024, 512, 512), (200, 72, 300), (300, 320, 2100), (500, 400, 131), (513, 1000, 96)])
+def test_float32_sums_are_those_of_the_products_alone(hip, M, N, K):
+    """Bit for bit, on both sides of the lines between the kernels."""
+    from nabla_amd.backend import lib
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    a, bs = torch.rand(M, K, generator=gen, device="cuda"), [torch.rand(K, N, generator=gen, device="cuda") for _ in range(3)]
+    assert torch.equal(launched(lib, a, bs), torch.cat([launched(lib, a, [b]) for b in bs]))
