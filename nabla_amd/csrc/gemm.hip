@@ -2642,8 +2642,8 @@ __global__ __launch_bounds__(256) void gemm_f32_split_group_kernel(const GemmGro
     gemm_f32_split_body<64, 64, 2, 2, 2, false, false, false>(g, bx, by, ny);
   });
 }
-template <typename Kern>
-static int launch_group(Kern kern, GemmGroup& G, int bm, int bn, int threads, size_t lds, hipStream_t st) {
+template <auto KERN>
+static int launch_group(GemmGroup& G, int bm, int bn, int threads, size_t lds, hipStream_t st) {
   int64_t blocks = 0;
   for (int i = 0; i < G.n; ++i) {
     GemmArgs& a = G.a[i];
@@ -2654,18 +2654,22 @@ static int launch_group(Kern kern, GemmGroup& G, int bm, int bn, int threads, si
     NBK_REQUIRE(blocks <= 0x7fffffffLL, "gemm_group: launch too large");
   }
   G.first[G.n] = (int32_t)blocks;
-  NBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3((unsigned)threads), lds, st, G);
+  static bool attr_set = false; /* idempotent, so a race only repeats the call */
+  if (!attr_set) {
+    NBK_HIP(hipFuncSetAttribute((const void*)KERN, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(KERN, dim3((unsigned)blocks), dim3((unsigned)threads), lds, st, G);
   return nbk_check_launch("gemm group kernel");
 }
 template <int BM, int BN, int STAGES>
 static int launch_bf16_group(GemmGroup& G, hipStream_t st) {
   const size_t pipe = STAGES * (size_t)(BM + BN) * 8 * 16, slabs = 4 * 32 * (size_t)(BN / 2 + 4) * sizeof(float);
-  return launch_group(gemm_bf16_group_kernel<BM, BN, STAGES>, G, BM, BN, 256, pipe > slabs ? pipe : slabs, st);
+  return launch_group<gemm_bf16_group_kernel<BM, BN, STAGES>>(G, BM, BN, 256, pipe > slabs ? pipe : slabs, st);
 }
 template <int T, int WK>
 static int launch_f32_group(GemmGroup& G, hipStream_t st) {
-  return launch_group(gemm_f32_group_kernel<T, WK>, G, T, T, 64 * WK, gemm_f32_lds<false, false, T, WK>(), st);
+  return launch_group<gemm_f32_group_kernel<T, WK>>(G, T, T, 64 * WK, gemm_f32_lds<false, false, T, WK>(), st);
 }
 
 extern "C" int nbk_gemm_group(const nbk_gemm_desc* const* d, int32_t n, void* stream) {
@@ -2721,7 +2725,7 @@ extern "C" int nbk_gemm_group(const nbk_gemm_desc* const* d, int32_t n, void* st
         else if (of == F32_16_BY_8) rc = launch_f32_group<16, 8>(F, st);
         else if (of == F32_32_BY_8) rc = launch_f32_group<32, 8>(F, st);
         else if (of == F32_32_BY_4) rc = launch_f32_group<32, 4>(F, st);
-        else rc = launch_group(gemm_f32_split_group_kernel, F, 64, 64, 256, 2 * (64 + 64) * 12 * 16, st);
+        else rc = launch_group<gemm_f32_split_group_kernel>(F, 64, 64, 256, 2 * (64 + 64) * 12 * 16, st);
         if (rc != NBK_OK) return rc;
       }
     }
