@@ -966,8 +966,10 @@ class Decoder {
     in.dst = (uint8_t)code(id);
     if (v.a >= 0) in.a = (uint8_t)code(v.a);
     if (v.op >= NBK_OP_MOV) {
-      if (v.b >= 0) in.b = (uint8_t)code(v.b);
-      if (v.c >= 0) in.c = (uint8_t)code(v.c);
+      // (an instruction of scalars reads all three: an operand that it does not have is the first)
+      const uint8_t none = v.scalar ? in.a : 0;
+      in.b = v.b >= 0 ? (uint8_t)code(v.b) : none;
+      in.c = v.c >= 0 ? (uint8_t)code(v.c) : none;
       in.two = v.b >= 0;
     } else {
       in.b = (uint8_t)v.y;

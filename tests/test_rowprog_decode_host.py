@@ -385,3 +385,19 @@ def test_a_reduction_of_its_neighbours_result(kinds):
     last = S + (len(kinds) - 1) % 2
     ins += body((isa.STG, 1, last, 0, 0, 0))
     assert check(program(ins, 2, 1003, True, [0, 1]))[ROW] is not None
+
+
+def test_instructions_of_scalars_name_scalars_only():
+    """All three operands are read, whatever the instruction has: a register number below the scalars would be
+    an index outside their file."""
+    rng, seen = random.Random(5), 0
+    for _ in range(200):
+        rp = random_program(rng)
+        for mode in [ROW, LOOP] if rp.has_reduce else [FLAT]:
+            vm = decode(rp, mode)
+            for q in range(vm.n_ins if vm is not None else 0):
+                n = vm.ins[q]
+                if n.op >= isa.UNARY["mov"] and SCALAR <= n.dst < NONE:
+                    assert all(SCALAR <= r < SCALAR + isa.NSCL for r in (n.a, n.b, n.c)), (n.op, n.a, n.b, n.c)
+                    seen += 1
+    assert seen > 200
