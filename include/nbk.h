@@ -310,6 +310,8 @@ typedef struct nbk_gemm_desc {
   nbk_gemm_term term[NBK_GEMM_MAX_TERMS];
 } nbk_gemm_desc;
 int nbk_gemm(const nbk_gemm_desc* d, void* stream);
+/* 1 if nbk_gemm launches the kernel for few columns, which splits K over the waves of a workgroup; 0 otherwise. */
+int nbk_gemm_few_columns(const nbk_gemm_desc* d);
 /* n products, none of which reads or overwrites what another one writes, in any order: what nbk_gemm makes of each.
  * Products x^T dy (both operands row-contiguous) of one dtype with nothing behind them but alpha and column sums
  * share a launch, seven at a time (the weight gradients of small layers: MatmulOp.vjp_rule, nabla/ops/binary.py:

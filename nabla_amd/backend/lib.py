@@ -190,6 +190,7 @@ _SIGNATURES = {
                           C.c_void_p], C.c_int),
     "nbk_fill": ([C.c_void_p, C.c_int32, C.c_int64, C.c_double, C.c_void_p], C.c_int),
     "nbk_gemm": ([C.POINTER(GemmDesc), C.c_void_p], C.c_int),
+    "nbk_gemm_few_columns": ([C.POINTER(GemmDesc)], C.c_int),
     "nbk_gemm_group": ([C.POINTER(C.POINTER(GemmDesc)), C.c_int32, C.c_void_p], C.c_int),
     "nbk_gemm_members": ([C.POINTER(GemmDesc), C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p], C.c_int),
     "nbk_gemm_nf4_terms": ([C.POINTER(GemmNf4Desc), C.POINTER(GemmTerm), C.c_int32, C.c_void_p], C.c_int),

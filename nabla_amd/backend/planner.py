@@ -2086,17 +2086,20 @@ class Planner:
                  rows_contiguous: bool = False, epilogue: bool = False, b_k_contiguous: bool = False) -> int:
         """Slices of the contraction axis for a product whose output has too few 128 x 128
         tiles to occupy the GPU while K is long (weight gradients: K = batch x sequence).
-        ``epilogue``: what follows the product could be folded into it if it stays whole."""
+        ``epilogue``: what follows the product could be folded into it if it stays whole.
+        ``a_k_contiguous``: up to 32 columns, also that the kernel for few columns takes it (_few_columns)."""
         if dtype is not DType.bfloat16:
             return 1
-        if a_k_contiguous and N <= 32 and M >= 16 and K % 64 == 0 and K * (1 if N <= 16 else 2) <= 4096 and (
+        if a_k_contiguous and N <= 32 and K * (1 if N <= 16 else 2) <= 4096 and (
                 b_k_contiguous or K * (1 if N == 8 else 2 if N <= 16 else 4) <= (4096 if M < 8192 or N != 8 else 2048)):
             # Products with a few columns have a kernel that splits K by itself.  Each of its workgroups
             # reads all of B, and keeps a copy of one whose rows are columns of the result, which decides where
             # it ends; us, whole / in the slices below and their sum.  B K-contiguous: 1000 x 8 x 4096 7.8 / 8.5,
             # 8192 x 16 x 4096 16.5 / 18.2, 1000 x 32 x 2048 6.9 / 8.5, 2000 x 32 x 4096 11.3 / 10.1.  The other:
             # 1000 x 8 x 1024 4.4 / 8.7, 1000 x 8 x 4096 8.3 / 8.7, 8192 x 8 x 4096 18.9 / 18.0, 8192 x 16 x 2048
-            # 8.6 / 11.1, 2000 x 16 x 4096 20.3 / 9.1, 1000 x 32 x 1024 5.7 / 8.8, 2000 x 32 x 2048 12.3 / 8.9.
+            # 8.6 / 11.1, 2000 x 16 x 4096 20.3 / 9.1, 1000 x 32 x 1024 5.7 / 8.8, 2000 x 32 x 2048 12.3 / 8.9.  Few rows
+            # take as long as many, in either: 16 x 8 x 1024 3.9 / 6.4, 16 x 16 x 2048 6.2 / 6.5, 16 x 32 x 1024 5.3 / 6.5,
+            # 64 x 12 x 2048 5.3 / 7.3, 200 x 4 x 4096 7.1 / 14.3.
             return 1
         tiles = ((M + 127) // 128) * ((N + 127) // 128)
         if rows_contiguous and 128 <= tiles <= 256 and K >= 4096:
@@ -2139,6 +2142,24 @@ class Planner:
         return ks
 
     @staticmethod
+    def _few_columns(M: int, N: int, K: int, pa, pb, a_offset: int, b_offset: int) -> bool:
+        """Whether a plain bf16 product is launched on the kernel for few columns: the condition of ``nbk_gemm``
+        (``nbk_gemm_few_columns``), which loads 16 bytes at a time.  What that refuses runs on tiles with guarded loads,
+        where slices are all that helps: 1000 x 4 x 2048 54 us whole and 15 in eight slices with their sum, 16 x 12 x 1024 27
+        and 13, 200 x 20 x 4096 104 and 23."""
+        _, a_rs, a_cs = pa
+        _, b_rs, b_cs = pb
+        if not (N <= 32 and K >= 256 and K % 64 == 0 and a_cs == 1 and a_rs % 8 == 0 and a_offset % 8 == b_offset % 8 == 0):
+            return False
+        if not (b_cs % 8 == 0 if b_rs == 1 else b_cs == 1 and b_rs % 8 == 0 and N % 8 == 0):
+            return False
+        if b_rs != 1 and K * (1 if N <= 8 else 2 if N <= 16 else 4) > 8156:
+            return False  # (a workgroup's copy of B in LDS)
+        if M >= 1024:
+            return M <= 8192 or b_rs == 1 or N > 8 or K < 4096
+        return M >= 16 and K * (1 if N <= 16 else 2) <= 4096
+
+    @staticmethod
     def _slices(K: int, ks: int) -> tuple[int, int, int]:
         """(slices, length of a slice, length of the last one) for ``K`` cut into about ``ks`` whole
         numbers of 64; rounding a slice up can leave fewer of them (8200 in sixteen: fifteen of
@@ -2171,11 +2192,8 @@ class Planner:
                          out: ir.Value, epi: dict | None = None) -> None:
         """One unbatched product into contiguous storage for ``out``; split along K into fp32
         partial products plus their sum when the output alone gives too few workgroups."""
-        # (long rows that 16-byte loads cannot take stay in slices)
-        whole_chunks = pa[1] % 8 == 0 and ra.offset % 8 == 0 and rb.offset % 8 == 0 and (
-            pb[2] % 8 == 0 if pb[1] == 1 else pb[1] % 8 == 0)
         ks = self._split_k(M, N, K, ra.dtype if ra.dtype is rb.dtype else DType.float32,
-                           a_k_contiguous=pa[2] == 1 and (K * (1 if N <= 16 else 2) <= 2048 or whole_chunks),
+                           a_k_contiguous=pa[2] == 1 and (N > 32 or self._few_columns(M, N, K, pa, pb, ra.offset, rb.offset)),
                            rows_contiguous=pa[1] == 1 and pa[2] != 1 and pb[2] == 1 and pb[1] != 1,
                            b_k_contiguous=pb[1] == 1)
         dst = self._alloc_value(out)

@@ -2410,41 +2410,48 @@ static F32Form gemm_f32_form(int64_t M, int64_t N, int64_t K, int64_t batch) {
   return K >= 128 && (t32 <= cus || (t32 <= 2 * cus && K % 128 == 0)) ? F32_32_BY_8 : F32_32_BY_4;
 }
 
+// LDS of gemm_skinny_n_kernel: the partial sums of its waves, and a copy of a B that is not K-contiguous, in rows of so
+// many 16-byte chunks.
+constexpr size_t SKN_SUMS = SKN_WAVES * 16 * 64 * sizeof(float);
+static int skn_pitch(int64_t N) { return N <= 8 ? 1 : N <= 16 ? 2 : 4; }
+static size_t skn_stage(int64_t N, int64_t K) { return (size_t)K * skn_pitch(N) * 16 + 64; }
+// Whether gemm_skinny_n_kernel takes a product.  Planner._few_columns (backend/planner.py) asks the same.
+static bool gemm_few_columns(const nbk_gemm_desc* d, const GemmArgs& a, int64_t batch) {
+  const bool akc = d->a_cs == 1, bkc = d->b_rs == 1;
+  // (few rows too, where a workgroup's share of B is small, us on this kernel / on 64 x 64 tiles: 1000 x 8 x 1024
+  // 4.4 / 8.1, 1000 x 8 x 4096 8.3 / 20.3, 1000 x 32 x 2048 6.9 / 11.8; and many rows until a workgroup's copy of a
+  // B of eight columns fills the LDS: 8192 x 8 x 4096 18.9 / 20.3, 20000 x 8 x 4096 41.0 / 31.7)
+  const bool tall = d->M >= 1024 ? d->M <= 8192 || bkc || d->N > 8 || d->K < 4096
+                                 : d->M >= 16 && d->K * (d->N <= 16 ? 1 : 2) <= 4096;
+  return d->n_terms == 0 && d->k_last == 0 && d->dtype_ab == NBK_BF16 && d->N <= 32 && tall && d->K >= 256 && d->K % 64 == 0 &&
+         akc && a.a_vec && batch == 1 && d->bias == nullptr && d->residual == nullptr && d->act == NBK_ACT_NONE &&
+         a.b_vec && (bkc || (d->N % 8 == 0 && SKN_SUMS + skn_stage(d->N, d->K) <= 160 * 1024 - 512)) &&
+         (d->M + 31) / 32 <= 0x7fffffff;
+}
+
 static int gemm_launch(const nbk_gemm_desc* d, const GemmMembers& own, void* stream) {
   GemmArgs a;
   { const int rc = gemm_prepare(d, own, a); if (rc != NBK_OK) return rc; }
   hipStream_t st = (hipStream_t)stream;
   const int64_t batch = own.n > 0 ? own.n : d->batch;
   const bool akc = d->a_cs == 1, bkc = d->b_rs == 1, tail = d->n_terms > 0;
-  // (few rows too, where a workgroup's share of B is small, us on this kernel / on 64 x 64 tiles: 1000 x 8 x 1024
-  // 4.4 / 8.1, 1000 x 8 x 4096 8.3 / 20.3, 1000 x 32 x 2048 6.9 / 11.8; and many rows until a workgroup's copy of a
-  // B of eight columns fills the LDS: 8192 x 8 x 4096 18.9 / 20.3, 20000 x 8 x 4096 41.0 / 31.7)
-  const bool tall = d->M >= 1024 ? d->M <= 8192 || bkc || d->N > 8 || d->K < 4096
-                                 : d->M >= 16 && d->K * (d->N <= 16 ? 1 : 2) <= 4096;
-  if (!tail && d->k_last == 0 && d->dtype_ab == NBK_BF16 && d->N <= 32 && tall && d->K >= 256 && d->K % 64 == 0 &&
-      akc && a.a_vec && batch == 1 && d->bias == nullptr && d->residual == nullptr &&
-      d->act == NBK_ACT_NONE && (bkc ? (bool)a.b_vec : (d->b_cs == 1 && d->N % 8 == 0 && a.b_vec))) {
+  if (gemm_few_columns(d, a, batch)) {
     // 32 rows per workgroup, K split over its eight waves
-    const int pitch_chunks = d->N <= 8 ? 1 : d->N <= 16 ? 2 : 4;
-    const size_t red = SKN_WAVES * 16 * 64 * sizeof(float);
-    const size_t stage = bkc ? 0 : (size_t)d->K * pitch_chunks * 16 + 64;
-    if (red + stage <= 160 * 1024 - 512 && (d->M + 31) / 32 <= 0x7fffffff) {
-      dim3 grid((unsigned)((d->M + 31) / 32));
-      if (bkc) {
-        hipLaunchKernelGGL((gemm_skinny_n_kernel<true>), grid, dim3(SKN_WAVES * 64), red, st, a,
-                           pitch_chunks);
-      } else {
-        static bool attr_set = false; /* idempotent, so a race only repeats the call */
-        if (!attr_set) {
-          NBK_HIP(hipFuncSetAttribute((const void*)gemm_skinny_n_kernel<false>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-          attr_set = true;
-        }
-        hipLaunchKernelGGL((gemm_skinny_n_kernel<false>), grid, dim3(SKN_WAVES * 64), red + stage, st, a,
-                           pitch_chunks);
+    const int pitch_chunks = skn_pitch(d->N);
+    dim3 grid((unsigned)((d->M + 31) / 32));
+    if (bkc) {
+      hipLaunchKernelGGL((gemm_skinny_n_kernel<true>), grid, dim3(SKN_WAVES * 64), SKN_SUMS, st, a, pitch_chunks);
+    } else {
+      static bool attr_set = false; /* idempotent, so a race only repeats the call */
+      if (!attr_set) {
+        NBK_HIP(hipFuncSetAttribute((const void*)gemm_skinny_n_kernel<false>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        attr_set = true;
       }
-      return nbk_check_launch("gemm_skinny_n_kernel");
+      hipLaunchKernelGGL((gemm_skinny_n_kernel<false>), grid, dim3(SKN_WAVES * 64), SKN_SUMS + skn_stage(d->N, d->K), st,
+                         a, pitch_chunks);
     }
+    return nbk_check_launch("gemm_skinny_n_kernel");
   }
   if (!tail && d->k_last == 0 && d->dtype_ab == NBK_BF16 && d->K <= 16 && akc && batch == 1 && d->N % 8 == 0 &&
       d->ldc % 8 == 0 && ((uintptr_t)d->C & 15) == 0 && ((uintptr_t)d->residual & 15) == 0 &&
@@ -2603,6 +2610,10 @@ static int gemm_launch(const nbk_gemm_desc* d, const GemmMembers& own, void* str
 }
 
 extern "C" int nbk_gemm(const nbk_gemm_desc* d, void* stream) { return gemm_launch(d, {}, stream); }
+extern "C" int nbk_gemm_few_columns(const nbk_gemm_desc* d) {
+  GemmArgs a;
+  return gemm_prepare(d, {}, a) == NBK_OK && gemm_few_columns(d, a, d->batch) ? 1 : 0;
+}
 
 // ------------------------------------------------------------------ products that share a launch
 // Weight gradients of small layers: each has a fraction of the workgroups the GPU holds, and nothing reads
