@@ -1844,9 +1844,13 @@ class Planner:
         vec = 16 // x.dtype.size_in_bytes if inner % (16 // x.dtype.size_in_bytes) == 0 else 1
         blocks = outer * ((inner + 64 * vec - 1) // (64 * vec))
         split = 1
-        # (a column of numbers behind each other is read by 16 bytes a lane: one workgroup takes 65536 of them in
-        # less time than a second launch, by element 8192)
-        line = inner == 1 and red <= (65536 if red % (16 // x.dtype.size_in_bytes) == 0 else 8192)
+        # A column of numbers behind each other: one workgroup takes so many of them in less time than slices and a second
+        # launch.  us, whole / in slices: by 16 bytes a lane (bf16 and float32 where they lie on such) 65536 floats 4.3 / 5.0,
+        # by element 8192 2.8 / 5.0 and 65536 6.9 / 5.4, float16, converted one by one, 2048 3.6 / 5.5 and 8192 8.0 / 6.0.
+        chunk = 16 // x.dtype.size_in_bytes
+        limit = 4096 if x.dtype not in (DType.bfloat16, DType.float32) else \
+            65536 if red % chunk == 0 and src.offset % chunk == 0 else 8192
+        line = inner == 1 and red <= limit
         if blocks < 256 and red >= 768 and x.dtype.is_float() and not line:  # (partials are fp32)
             want = min(256, red // 64, max(1, 1024 // max(blocks, 1)))
             for s in range(want, 1, -1):
