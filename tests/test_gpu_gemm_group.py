@@ -134,3 +134,30 @@ def test_float32_sums_are_those_of_the_products_alone(hip):
     pairs = [tuple(torch.rand(K, n, generator=gen, device="cuda") for n in (M, N)) for M, N, K in FORMS]
     for got, alone in zip(products(lib, 0, pairs), products(lib, 0, pairs, together=False)):
         assert torch.equal(got, alone), tuple(got.shape)
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_scaled(hip, dtype):
+    from nabla_amd.backend import lib
+    rng = np.random.default_rng(dtype)
+    pairs = [tuple(torch.tensor(rng.integers(-3, 4, (K, n)), dtype=torch.bfloat16 if dtype else torch.float32).cuda() for n in (M, N))
+             for M, N, K in [(64, 72, 96), (512, 2048, 256), (72, 80, 100), (512, 1024, 33), (400, 600, 100)]]
+    for (a, b), got in zip(pairs, products(lib, dtype, pairs, alpha=0.25)):
+        assert torch.equal(got.double(), 0.25 * (a.double().t().contiguous() @ b.double()))
+
+
+def test_bf16_contractions_below_a_tile(hip):
+    run(hip, 1, [(64, 72, 40, 1), (128, 64, 8, 1), (72, 80, 56, 1), (512, 520, 24, 1)], colsum=(1, 3))
+
+
+def test_numbers_without_parts(hip):
+    """Infinities and NaN as in the products alone, in every form."""
+    from nabla_amd.backend import lib
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    pairs = [tuple(torch.randn(K, n, generator=gen, device="cuda") for n in (M, N)) for M, N, K in FORMS]
+    for i, (a, b) in enumerate(pairs):
+        a[i % a.shape[0], i % a.shape[1]] = float("inf")
+        b[-1, i % b.shape[1]] = float("nan") if i % 2 else -3e38
+    for got, alone in zip(products(lib, 0, pairs), products(lib, 0, pairs, together=False)):
+        assert got.isnan().any() or got.isinf().any()
+        assert torch.equal(got.nan_to_num(7e37, 8e37, 9e37), alone.nan_to_num(7e37, 8e37, 9e37))

@@ -95,3 +95,30 @@ def test_float32_sums_are_those_of_the_products_alone(hip, M, N, K):
     gen = torch.Generator(device="cuda").manual_seed(K)
     a, bs = torch.rand(M, K, generator=gen, device="cuda"), [torch.rand(K, N, generator=gen, device="cuda") for _ in range(3)]
     assert torch.equal(launched(lib, a, bs), torch.cat([launched(lib, a, [b]) for b in bs]))
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt"])
+@pytest.mark.parametrize("M,N,K", [(1024, 512, 300), (2048, 1536, 128), (200, 72, 64)])
+def test_numbers_without_parts(hip, M, N, K, layout):
+    """Infinities and NaN as in the products alone: the second pass of a tile reads the operand of its own product."""
+    from nabla_amd.backend import lib
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    a, bs = torch.randn(M, K, generator=gen, device="cuda"), [torch.randn(K, N, generator=gen, device="cuda") for _ in range(3)]
+    a[5, 7] = float("inf")
+    bs[1][3, 9], bs[2][K - 1, N - 1] = float("nan"), -3e38
+    if layout == "nt":
+        bs = [b.t().contiguous() for b in bs]
+    got, alone = launched(lib, a, bs, layout), torch.cat([launched(lib, a, [b], layout) for b in bs])
+    assert got[1].isnan().any() and got[0].isinf().any()
+    assert torch.equal(got.nan_to_num(7e37, 8e37, 9e37), alone.nan_to_num(7e37, 8e37, 9e37))
+
+
+@pytest.mark.parametrize("K", [8, 40, 56])
+def test_bf16_contractions_below_a_tile(hip, K):
+    from nabla_amd.backend import lib
+    rng = np.random.default_rng(K)
+    a, *bs = (torch.tensor(rng.integers(-2, 3, s), dtype=torch.bfloat16).cuda() for s in [(384, K)] + [(K, 256)] * 3)
+    for layout in ("nn", "nt"):
+        got = launched(lib, a, bs if layout == "nn" else [b.t().contiguous() for b in bs], layout)
+        for g, b in zip(got, bs):
+            assert torch.equal(g.double(), a.double() @ b.double())

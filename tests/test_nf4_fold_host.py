@@ -63,3 +63,27 @@ def test_a_sum_that_nothing_computes_on_is_rounded_by_its_product(emulator):
     steps = planned(pre)
     assert [s.attrs["dst"].dtype for s in folded(steps)] == [BF16] and not any(s.kind == "rowprog" for s in steps)
     assert ((pre.to_torch().double() - p.exact()).abs() <= 2.0 ** -8 * p.exact().abs() + 2e-5).all()
+
+
+@pytest.mark.parametrize("tokens,rows,cols,rank,inside", [
+    (128, 128, 128, 8, 1), (127, 128, 128, 8, 0), (128, 64, 128, 8, 0), (128, 192, 128, 64, 1), (128, 160, 128, 8, 0),
+    (128, 128, 64, 8, 0), (128, 128, 192, 72, 0), (128, 128, 192, 4, 0)])
+def test_where_the_update_goes_inside(emulator, tokens, rows, cols, rank, inside):
+    """From 128 rows, columns and numbers of a sum on, for contractions of whole K tiles and ranks of whole chunks up to one."""
+    p = Pair(tokens, rows, cols, rank)
+    y = p.linear(nb.Tensor.from_dlpack(p.x))
+    steps = planned(y)
+    assert len(folded(steps)) == inside
+    # (a sum that is no part of the product: base and update rounded by themselves, and what they come to)
+    size = p.exact().abs() + 2.0 * (p.x.double().abs() @ p.a.double().abs()) @ p.b.double().abs()
+    assert ((y.to_torch().double() - p.exact()).abs() <= 2.0 ** (-8 if inside else -7) * size + 2e-5).all()
+
+
+def test_an_update_that_is_used_twice_stays_a_product(emulator):
+    p = Pair(160, 128, 192, 8)
+    x = nb.Tensor.from_dlpack(p.x)
+    base = p.linear(x, {k: nb.zeros_like(v) for k, v in p.adapter.items()})
+    thin = (x @ p.adapter["A"]) @ p.adapter["B"]
+    steps = planned(base + thin, thin)
+    assert not any(t["K"] == 8 and s.attrs["N"] != 192 for s in folded(steps) for t in s.attrs["terms"])
+    assert any(s.kind == "gemm" and s.attrs["N"] == 192 for s in steps)
