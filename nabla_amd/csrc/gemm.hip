@@ -2627,6 +2627,7 @@ struct GemmGroup {
   int32_t n;
   int32_t first[GEMM_GROUP_MAX + 1];  // workgroups before each product
   int32_t batch[GEMM_GROUP_MAX];
+  int32_t bm[GEMM_GROUP_MAX], bn[GEMM_GROUP_MAX];  // tile of each product
   GemmArgs a[GEMM_GROUP_MAX];
 };
 static_assert(sizeof(GemmGroup) <= 4096, "kernel arguments");
@@ -2637,30 +2638,36 @@ __device__ __forceinline__ void gemm_group_run(const GemmGroup& G, Body&& body) 
   const GemmArgs& g = G.a[i];
   const int local = (int)blockIdx.x - G.first[i], tiles = g.tiles_m * g.tiles_n;
   const int by = local / tiles;
-  body(g, local - by * tiles, by, G.batch[i]);
+  body(g, local - by * tiles, by, G.batch[i], G.bm[i]);
 }
 template <int BM, int BN, int STAGES>
 __global__ __launch_bounds__(256) void gemm_bf16_group_kernel(const GemmGroup G) {
-  gemm_group_run(G, [](const GemmArgs& g, int bx, int by, int ny) {
+  gemm_group_run(G, [](const GemmArgs& g, int bx, int by, int ny, int) {
     gemm_bf16_dl_body<BM, BN, false, false, 0, 4, 1, true, true, STAGES>(g, bx, by, ny);
   });
 }
-template <int T, int WK>
+// (tiles of 16 and of 32 by eight waves: one kernel for both)
+template <int WK>
 __global__ __launch_bounds__(64 * WK, WK > 8 ? 1 : 2) void gemm_f32_group_kernel(const GemmGroup G) {
-  gemm_group_run(G, [](const GemmArgs& g, int bx, int by, int ny) { gemm_f32_body<false, false, T, WK>(g, bx, by, ny); });
+  gemm_group_run(G, [](const GemmArgs& g, int bx, int by, int ny, int tile) {
+    if constexpr (WK == 16) gemm_f32_body<false, false, 16, WK>(g, bx, by, ny);
+    else if constexpr (WK == 4) gemm_f32_body<false, false, 32, WK>(g, bx, by, ny);
+    else if (tile == 16) gemm_f32_body<false, false, 16, WK>(g, bx, by, ny);
+    else gemm_f32_body<false, false, 32, WK>(g, bx, by, ny);
+  });
 }
 __global__ __launch_bounds__(256) void gemm_f32_split_group_kernel(const GemmGroup G) {
-  gemm_group_run(G, [](const GemmArgs& g, int bx, int by, int ny) {
+  gemm_group_run(G, [](const GemmArgs& g, int bx, int by, int ny, int) {
     gemm_f32_split_body<64, 64, 2, 2, 2, false, false, false>(g, bx, by, ny);
   });
 }
 template <auto KERN>
-static int launch_group(GemmGroup& G, int bm, int bn, int threads, size_t lds, hipStream_t st) {
+static int launch_group(GemmGroup& G, int threads, size_t lds, hipStream_t st) {
   int64_t blocks = 0;
   for (int i = 0; i < G.n; ++i) {
     GemmArgs& a = G.a[i];
-    a.tiles_m = (int)((a.M + bm - 1) / bm);
-    a.tiles_n = (int)((a.N + bn - 1) / bn);
+    a.tiles_m = (int)((a.M + G.bm[i] - 1) / G.bm[i]);
+    a.tiles_n = (int)((a.N + G.bn[i] - 1) / G.bn[i]);
     G.first[i] = (int32_t)blocks;
     blocks += (int64_t)a.tiles_m * a.tiles_n * G.batch[i];
     NBK_REQUIRE(blocks <= 0x7fffffffLL, "gemm_group: launch too large");
@@ -2677,11 +2684,13 @@ static int launch_group(GemmGroup& G, int bm, int bn, int threads, size_t lds, h
 template <int BM, int BN, int STAGES>
 static int launch_bf16_group(GemmGroup& G, hipStream_t st) {
   const size_t pipe = STAGES * (size_t)(BM + BN) * 8 * 16, slabs = 4 * 32 * (size_t)(BN / 2 + 4) * sizeof(float);
-  return launch_group<gemm_bf16_group_kernel<BM, BN, STAGES>>(G, BM, BN, 256, pipe > slabs ? pipe : slabs, st);
+  for (int i = 0; i < G.n; ++i) { G.bm[i] = BM; G.bn[i] = BN; }
+  return launch_group<gemm_bf16_group_kernel<BM, BN, STAGES>>(G, 256, pipe > slabs ? pipe : slabs, st);
 }
-template <int T, int WK>
+template <int WK>
 static int launch_f32_group(GemmGroup& G, hipStream_t st) {
-  return launch_group<gemm_f32_group_kernel<T, WK>>(G, T, T, 64 * WK, gemm_f32_lds<false, false, T, WK>(), st);
+  constexpr int T = WK > 8 ? 16 : 32;  // (the larger where there are two)
+  return launch_group<gemm_f32_group_kernel<WK>>(G, 64 * WK, gemm_f32_lds<false, false, T, WK>(), st);
 }
 
 extern "C" int nbk_gemm_group(const nbk_gemm_desc* const* d, int32_t n, void* stream) {
@@ -2720,24 +2729,24 @@ extern "C" int nbk_gemm_group(const nbk_gemm_desc* const* d, int32_t n, void* st
       else if (t64 <= 2 * cus) rc = launch_bf16_group<64, 128, 4>(G, st);
       else if (t128 <= cus) rc = launch_bf16_group<128, 128, 4>(G, st);
       else rc = launch_bf16_group<128, 128, 2>(G, st);
-    } else {  // (those that are added up alike share a launch)
-      for (F32Form of : {F32_16_BY_16, F32_16_BY_8, F32_32_BY_8, F32_32_BY_4, F32_PARTS}) {
+    } else {  // (those of as many waves share a launch)
+      for (F32Form of : {F32_16_BY_16, F32_16_BY_8, F32_32_BY_4, F32_PARTS}) {
         GemmGroup F;
         F.n = 0;
         int last = 0;
         for (int i = 0; i < G.n; ++i) {
-          if (form[i] != of) continue;
+          if (form[i] != of && !(of == F32_16_BY_8 && form[i] == F32_32_BY_8)) continue;
           F.a[F.n] = G.a[i];
+          F.bm[F.n] = F.bn[F.n] = form[i] <= F32_16_BY_8 ? 16 : form[i] == F32_PARTS ? 64 : 32;
           F.batch[F.n++] = G.batch[i];
           last = i;
         }
         if (F.n == 0) continue;
         if (F.n == 1) rc = nbk_gemm(d[base + last], stream);
-        else if (of == F32_16_BY_16) rc = launch_f32_group<16, 16>(F, st);
-        else if (of == F32_16_BY_8) rc = launch_f32_group<16, 8>(F, st);
-        else if (of == F32_32_BY_8) rc = launch_f32_group<32, 8>(F, st);
-        else if (of == F32_32_BY_4) rc = launch_f32_group<32, 4>(F, st);
-        else rc = launch_group<gemm_f32_split_group_kernel>(F, 64, 64, 256, 2 * (64 + 64) * 12 * 16, st);
+        else if (of == F32_16_BY_16) rc = launch_f32_group<16>(F, st);
+        else if (of == F32_16_BY_8) rc = launch_f32_group<8>(F, st);
+        else if (of == F32_32_BY_4) rc = launch_f32_group<4>(F, st);
+        else rc = launch_group<gemm_f32_split_group_kernel>(F, 256, 2 * (64 + 64) * 12 * 16, st);
         if (rc != NBK_OK) return rc;
       }
     }

@@ -357,8 +357,9 @@ static RedLayout reduce_layout(const void* in, int dti, int64_t outer, int64_t r
   RedLayout L;
   const bool aligned = ((uintptr_t)in & 15) == 0;
   L.mode = dti == NBK_BF16 ? (aligned && inner % 8 == 0 ? 1 : 3) : dti == NBK_F32 ? (aligned && inner % 4 == 0 ? 2 : 4) : 0;
-  // (a column of numbers behind each other, the sum of a loss: one workgroup by 16 bytes takes up to 16384 of them
-  // in one trip to memory, where slices of 64 took a launch more; us, 8192 bf16 9.2 / 4.7)
+  // (a column of numbers behind each other, the sum of a loss, by 16 bytes a lane: 16384 bf16 are one trip to memory, and
+  // up to 65536 one workgroup is faster than slices and the launch that adds them, which is where the planner's line is;
+  // us, 8192 bf16 9.2 in slices / 4.7)
   if (inner == 1 && aligned && red >= 512 && (dti == NBK_BF16 ? red % 8 == 0 : dti == NBK_F32 && red % 4 == 0)) {
     L.mode = dti == NBK_BF16 ? 5 : 6;
     L.lxs = 0;

@@ -1177,7 +1177,9 @@ int rp_vm_launch(const nbk_rowprog* p, int64_t rows, hipStream_t stream) {
     if (dt != NBK_F32 && dt != NBK_I32) flags &= ~(uint32_t)RPVM_WORDS;
   }
   // Two chunks a lane where a row has more than one wavefront's and the program up to eight vector registers: half
-  // the decoding per element (20000 rows of 270 floats 383 -> 212 us, 3000 of 4001 510 -> 413).
+  // the decoding per element (20000 rows of 270 floats 383 -> 212 us, 3000 of 4001 510 -> 413).  On few rows too, where
+  // half the wavefronts of a row are a longer chain each and share the scalar unit with fewer others (two programs, us:
+  // 32 x 300 floats 17.2 + 12.8 -> 15.9 + 10.7, 250 x 2051 24.6 + 17.2 -> 21.7 + 14.5, 250 x 300 bf16 16.6 + 12.5 -> 16.8 + 11.4).
   // (Looped programs keep one: their accumulators and offsets leave no room, 4096 rows of 12000 bfloat16 3477 -> 3684 us.)
   const bool wide = mode == RPVM_ROW && chunks > 64 && top_reg < RPVM_WIDE_REGS;
 #define RPVM_PICK(K, N) (d->rare ? (const void*)rp_vm_kernel<K, true, N> : (const void*)rp_vm_kernel<K, false, N>)
