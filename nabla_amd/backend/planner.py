@@ -2243,7 +2243,7 @@ class Planner:
         that launch (``nbk_gemm_members``) if nothing since has written what it reads: the projections to
         queries, keys and values of a short sequence have fewer tiles than the GPU has places each.  Three of 1800
         x 1024 x 1024: 38 -> 23 us, of 1998 x 512 x 512 27 -> 13, of 8192 x 1024 x 1024 (512 tiles of 128 x 128, two a CU)
-        81 -> 71, in float32 of 1024 x 512 x 512 39 -> 23; larger ones fill
+        81 -> 71, in float32 of 1024 x 512 x 512 31 -> 27; larger ones fill
         the GPU alone.  (Up to one tile of rows, 128, each keeps its launch.)"""
         M, N = common["M"], common["N"]
         bias = epi.get("bias")

@@ -2621,7 +2621,7 @@ extern "C" int nbk_gemm_few_columns(const nbk_gemm_desc* d) {
 // them before the end of a step.  A workgroup finds its product from the running counts and runs the
 // body of the kernel that the product would have had to itself.  us, one after the other / together: 4096 x 8,
 // 8 x 1024, 1024 x 8 and 8 x 4096 over 1000 rows in bf16 32 / 10.5; six of 512 x 512 to 512 x 2048 over 1998 rows 52 / 27, over
-// 1024 rows in float32 117 / 64; the adapters of a decoder layer over 8192 rows 44 / 34.
+// 1024 rows in float32 102 / 75; the adapters of a decoder layer over 8192 rows 44 / 34.
 constexpr int GEMM_GROUP_MAX = 7;
 struct GemmGroup {
   int32_t n;
