@@ -314,8 +314,8 @@ int nbk_gemm(const nbk_gemm_desc* d, void* stream);
 int nbk_gemm_few_columns(const nbk_gemm_desc* d);
 /* n products, none of which reads or overwrites what another one writes, in any order: what nbk_gemm makes of each.
  * Products x^T dy (both operands row-contiguous) of one dtype with nothing behind them but alpha and column sums
- * share a launch, seven at a time, float32 ones with those that are added up alike, as each is by itself (the weight gradients of small layers: MatmulOp.vjp_rule, nabla/ops/binary.py:
- * 303-314); others get one each. */
+ * share a launch, seven at a time, float32 ones with those that are added up alike, as each is by itself (the
+ * weight gradients of small layers: MatmulOp.vjp_rule, nabla/ops/binary.py:303-314); others get one each. */
 int nbk_gemm_group(const nbk_gemm_desc* const* d, int32_t n, void* stream);
 /* 2 to 4 products of one A in one launch (the projections of a layer to queries, keys and values:
  * nabla/nn/functional/layers.py): product i has B[i], bias[i] (NULL: none) and C[i]; sizes, strides, dtypes, alpha
